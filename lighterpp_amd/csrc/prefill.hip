@@ -570,42 +570,45 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
     // reads and the next tile's writes.
     static_assert(kStages >= 3 && kStageBytes / 4 >= 32 * 144, "room for a transposed tile per wavefront");
     char* room = pipe_lds + ((trips + 1) % kStages) * kStageBytes + wave * (kStageBytes / 4);
-    const int row8 = lane >> 3, part8 = lane & 7;
     if constexpr (kMode == 2) {
-        static_assert(kFi == 4, "a wavefront's gate and up tiles: two of each");
+        static_assert(kFi % 2 == 0, "a wavefront's gate and up tiles: as many of each");
         typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-        constexpr int kPitch = 72;  // binary16 per token row of the transposed tile: 64 features + padding
+        constexpr int kPairs = kFi / 2, kWide = 32 * kPairs;  // features of the wavefront's output
+        constexpr int kPitch = kWide + 8;                     // binary16 per token row of the transposed tile, padding included
+        constexpr int kLanes = kWide / 8, kRowsAtOnce = 64 / kLanes;
+        const int part = lane % kLanes, row_of = lane / kLanes;
         half_t* tile = reinterpret_cast<half_t*>(room);
 #pragma unroll
         for (int j = 0; j < kTj; ++j) {
-            half4_t h[2][4], l[2][4];
+            half4_t h[kPairs][4], l[kPairs][4];
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < kPairs; ++i)
 #pragma unroll
                 for (int e4 = 0; e4 < 4; ++e4) {
                     const float gate[4] = {acc[i][j][4 * e4], acc[i][j][4 * e4 + 1], acc[i][j][4 * e4 + 2], acc[i][j][4 * e4 + 3]};
-                    const float up[4] = {acc[i + 2][j][4 * e4], acc[i + 2][j][4 * e4 + 1], acc[i + 2][j][4 * e4 + 2],
-                                         acc[i + 2][j][4 * e4 + 3]};
+                    const float up[4] = {acc[i + kPairs][j][4 * e4], acc[i + kPairs][j][4 * e4 + 1], acc[i + kPairs][j][4 * e4 + 2],
+                                         acc[i + kPairs][j][4 * e4 + 3]};
                     swiglu_split4(h[i][e4], l[i][e4], gate, up);
                 }
-            const size_t at = static_cast<size_t>(t_base + wt * 32 * kTj + 32 * j) * job.out_ld + f_base + wf * 64 + 8 * part8;
+            const size_t at = static_cast<size_t>(t_base + wt * 32 * kTj + 32 * j) * job.out_ld + f_base + wf * kWide + 8 * part;
 #pragma unroll
-            for (int part = 0; part < (kLo ? 2 : 1); ++part) {  // (without kLo the next GEMM reads no remainders either)
+            for (int which_half = 0; which_half < (kLo ? 2 : 1); ++which_half) {  // (without kLo the next GEMM reads no remainders either)
 #pragma unroll
-                for (int i = 0; i < 2; ++i)
+                for (int i = 0; i < kPairs; ++i)
 #pragma unroll
                     for (int e4 = 0; e4 < 4; ++e4)
-                        *reinterpret_cast<half4_t*>(tile + r * kPitch + 32 * i + 8 * e4 + 4 * g) = part == 0 ? h[i][e4] : l[i][e4];
-                half_t* out = part == 0 ? job.out_hi : job.out_lo;
+                        *reinterpret_cast<half4_t*>(tile + r * kPitch + 32 * i + 8 * e4 + 4 * g) = which_half == 0 ? h[i][e4] : l[i][e4];
+                half_t* out = which_half == 0 ? job.out_hi : job.out_lo;
 #pragma unroll
-                for (int pass = 0; pass < 4; ++pass) {
-                    const int n = 8 * pass + row8;
+                for (int pass = 0; pass < 32 / kRowsAtOnce; ++pass) {
+                    const int n = kRowsAtOnce * pass + row_of;
                     *reinterpret_cast<half8_t*>(out + at + static_cast<size_t>(n) * job.out_ld) =
-                        *reinterpret_cast<const half8_t*>(tile + n * kPitch + 8 * part8);
+                        *reinterpret_cast<const half8_t*>(tile + n * kPitch + 8 * part);
                 }
             }
         }
     } else {
+        const int row8 = lane >> 3, part8 = lane & 7;
         constexpr int kPitch = 36;  // floats per token row of the transposed tile: 32 features + padding
         float* tile = reinterpret_cast<float*>(room);
         float* __restrict__ y = (which == 2 ? job.y[2] : (which == 1 ? job.y[1] : job.y[0])) + static_cast<size_t>(split) * job.split_stride;
@@ -631,6 +634,210 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
                     *out = v;
                 }
             }
+    }
+}
+
+// The same product for a batch of few tokens, where the weights are the traffic and the tiles above would leave most
+// of the device without a workgroup.
+//
+// A tile is 32 kFi features x 32 kTj tokens (kTj: the whole batch up to 128 tokens), so that a matrix of a few thousand
+// rows still makes a workgroup per compute unit.  Such a tile is too small to be cut among four wavefronts: each would
+// read its operands from LDS for a quarter of the products.  The four multiplying wavefronts take the whole tile each
+// and share out K instead -- a trip is 64 columns, four k-steps, one per wavefront -- and their sums meet in LDS at the
+// end, added in wavefront order.  Per k-step a wavefront reads kFi + 2 kTj fragments for 2 kFi kTj MFMAs.
+//
+// The stages, the requesting wavefronts, the order of the pieces and the barrier are those of k_gemm_pipe; there are
+// more and smaller stages, because what has to be in flight is weight bytes (4 KiB kFi a stage).
+// kMode 2: the first half of the tile's rows are features of W1, the second half the same features of W3.
+//
+// What bounds it: the weights from HBM up to 64 tokens (W1+W3 of the 1B shape, 67 MB, 32 tokens: 49.6 us with the tile of
+// 256 x 128 on 64 compute units, 15.4 here, of which launch, first data and epilogue are 4 to 5), the activations from L2
+// into LDS beyond (128 tokens: 26 us, 268 MB in requests).  The workgroups of a die start their walk over K at different
+// trips: in step, all of them would read the same columns of rows 4 KiB apart at once (W1+W3, 32 tokens: 19.4 -> 16.3 us).
+// 32 prompt ids of the 1B shape: 1.90 -> 0.90 ms.
+template <int kFi, int kTj, bool kLo>
+struct FewShape {
+    static constexpr int kRowBytes = 128;
+    static constexpr int kRowsA = 32 * kFi, kRowsB = 32 * kTj, kRows = kRowsA + (kLo ? 2 : 1) * kRowsB;
+    static constexpr int kStageBytes = kRows * kRowBytes;
+    static constexpr int kLoads = kStageBytes / 4096;  // requests of 1 KiB per requesting wavefront and stage
+    static constexpr int kStages = (160 * 1024) / kStageBytes > 10 ? 10 : (160 * 1024) / kStageBytes;
+    static constexpr int kPitch = 36;  // floats per token row of a 32 x 32 tile of sums
+    static constexpr int kSumBytes = 4 * kFi * kTj * 32 * kPitch * 4;
+    static constexpr int kLdsBytes = kStages * kStageBytes > kSumBytes ? kStages * kStageBytes : kSumBytes;
+    static_assert(kLdsBytes <= 160 * 1024 && kStages >= 3, "LDS of a workgroup");
+};
+
+template <int kFi, int kTj, int kMode, bool kLo>
+__global__ __launch_bounds__(512) void k_gemm_few(PipeJob job) {
+    typedef FewShape<kFi, kTj, kLo> Shape;
+    constexpr int kRowsA = Shape::kRowsA, kRowsB = Shape::kRowsB, kStages = Shape::kStages, kLoads = Shape::kLoads;
+    constexpr int kStageBytes = Shape::kStageBytes, kRowBytes = Shape::kRowBytes, kPitch = Shape::kPitch;
+    static_assert(kMode != 2 || kFi % 2 == 0, "as many tiles of W1 as of W3");
+    extern __shared__ __align__(1024) char few_lds[];
+    const int lane = lane_id();
+    const int wave_of_8 = __builtin_amdgcn_readfirstlane(wave_index());
+    const int wave = wave_of_8 & 3;
+    const int id = static_cast<int>(blockIdx.x), die = id & 7, within = id >> 3;
+    const int group = (within / job.token_tiles) * 8 + die;
+    if (group >= job.groups) return;
+    const int token_tile = within % job.token_tiles;
+    const int tile_all = group % job.feature_tiles, split = group / job.feature_tiles;
+    const int which = tile_all >= job.first_tile[2] ? 2 : (tile_all >= job.first_tile[1] ? 1 : 0);
+    const int tile_x = tile_all - (which == 2 ? job.first_tile[2] : (which == 1 ? job.first_tile[1] : 0));
+    const half_t* __restrict__ w = which == 2 ? job.w[2] : (which == 1 ? job.w[1] : job.w[0]);
+    const int K = job.K, k_first = split * job.k_len, trips = job.k_len / 64;
+    constexpr int kFeaturesPerTile = kMode == 2 ? 16 * kFi : 32 * kFi;
+    const int f_base = tile_x * kFeaturesPerTile, t_base = token_tile * kRowsB;
+
+    floatx16 acc[kFi][kTj];
+    if (wave_of_8 >= 4) {
+        const char* src[kLoads];
+#pragma unroll
+        for (int q = 0; q < kLoads; ++q) {
+            const int row = 8 * (wave + 4 * q) + (lane >> 3);
+            const int piece = (lane & 7) ^ ((row >> 1) & 7);
+            const half_t* from;
+            if (row < kRowsA) {
+                if constexpr (kMode == 2) from = (row >= 16 * kFi ? job.w[1] : job.w[0]) + static_cast<size_t>(f_base + row % (16 * kFi)) * K;
+                else from = w + static_cast<size_t>(f_base + row) * K;
+            } else if (!kLo || row < kRowsA + kRowsB) {
+                from = job.xh + static_cast<size_t>(t_base + row - kRowsA) * K;
+            } else {
+                from = job.xl + static_cast<size_t>(t_base + row - kRowsA - kRowsB) * K;
+            }
+            src[q] = reinterpret_cast<const char*>(from + k_first) + 16 * piece;
+        }
+        const unsigned lds_base = static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)few_lds));
+        const int turn0 = (group >> 3) % trips;
+        auto request = [&](int trip) {
+            const unsigned at = __builtin_amdgcn_readfirstlane(lds_base + (trip % kStages) * kStageBytes + wave * 1024);
+            const int rot = trip + turn0 < trips ? trip + turn0 : trip + turn0 - trips;
+            const int column = __builtin_amdgcn_readfirstlane(rot * kRowBytes);
+#pragma unroll
+            for (int q = 0; q < kLoads; ++q)
+                asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off\n" ::"v"(src[q] + column), "s"(at + q * 4096)
+                             : "memory");
+        };
+        auto landed = [&](int trip) {
+            if (trips - 1 - trip >= kStages - 2) wait_requests<(kStages - 2) * kLoads>();
+            else wait_requests<0>();
+        };
+#pragma unroll
+        for (int t = 0; t < kStages - 1; ++t)
+            if (t < trips) request(t);
+        landed(0);
+        __syncthreads();
+        if (kStages - 1 < trips) request(kStages - 1);
+        for (int t = 0; t < trips; ++t) {
+            landed(t + 1);
+            __syncthreads();
+            if (t + kStages < trips) request(t + kStages);
+        }
+    } else {
+        const int r = lane & 31, g = lane >> 5;
+        const int piece = (2 * wave + g) ^ ((r >> 1) & 7);  // this wavefront's k-step of every trip
+        const int a_off = r * kRowBytes + 16 * piece, b_off = a_off + kRowsA * kRowBytes;
+#pragma unroll
+        for (int i = 0; i < kFi; ++i)
+#pragma unroll
+            for (int j = 0; j < kTj; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+        struct Frags {
+            half8_t a[kFi], bh[kTj], bl[kTj];
+        };
+        auto read = [&](Frags& f, int trip) {
+            const char* stage = few_lds + (trip % kStages) * kStageBytes;
+#pragma unroll
+            for (int i = 0; i < kFi; ++i) f.a[i] = *reinterpret_cast<const half8_t*>(stage + a_off + i * 32 * kRowBytes);
+#pragma unroll
+            for (int j = 0; j < kTj; ++j) {
+                f.bh[j] = *reinterpret_cast<const half8_t*>(stage + b_off + j * 32 * kRowBytes);
+                if constexpr (kLo) f.bl[j] = *reinterpret_cast<const half8_t*>(stage + b_off + (kRowsB + j * 32) * kRowBytes);
+            }
+        };
+        auto multiply = [&](const Frags& f) {
+#pragma unroll
+            for (int i = 0; i < kFi; ++i)
+#pragma unroll
+                for (int j = 0; j < kTj; ++j) {
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.a[i], f.bh[j], acc[i][j], 0, 0, 0);
+                    if constexpr (kLo) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.a[i], f.bl[j], acc[i][j], 0, 0, 0);
+                }
+        };
+        // (the trip's fragments are read behind the barrier that says they are there and multiplied behind the next
+        // one: the reads travel while the trip before is multiplied.  The read past the last trip is of a stage nobody uses.)
+        Frags even, odd;
+        __syncthreads();
+        read(even, 0);
+        for (int t = 0; t < trips; t += 2) {
+            __syncthreads();
+            read(odd, t + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(even);
+            __builtin_amdgcn_sched_barrier(0);
+            if (t + 1 < trips) {
+                __syncthreads();
+                read(even, t + 2);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(odd);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    }
+    // the four wavefronts' sums through LDS, tile by tile as [token][feature] (the stages are free: every wavefront has
+    // read its last fragments, no request is outstanding), then whole lines to memory by all eight
+    __syncthreads();
+    float* sums = reinterpret_cast<float*>(few_lds);
+    constexpr int kTile = 32 * kPitch;
+    if (wave_of_8 < 4) {
+        const int r = lane & 31, g = lane >> 5;
+#pragma unroll
+        for (int i = 0; i < kFi; ++i)
+#pragma unroll
+            for (int j = 0; j < kTj; ++j)
+#pragma unroll
+                for (int e4 = 0; e4 < 4; ++e4)
+                    *reinterpret_cast<floatx4*>(sums + (wave * kFi * kTj + i * kTj + j) * kTile + r * kPitch + 8 * e4 + 4 * g) =
+                        floatx4{acc[i][j][4 * e4], acc[i][j][4 * e4 + 1], acc[i][j][4 * e4 + 2], acc[i][j][4 * e4 + 3]};
+    }
+    __syncthreads();
+    const int row8 = lane >> 3, part8 = lane & 7;
+    auto summed = [&](int tile, int n) {
+        floatx4 v[4];
+#pragma unroll
+        for (int z = 0; z < 4; ++z) v[z] = *reinterpret_cast<const floatx4*>(sums + (z * kFi * kTj + tile) * kTile + n * kPitch + 4 * part8);
+        floatx4 sum;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum[e] = (v[0][e] + v[1][e]) + (v[2][e] + v[3][e]);
+        return sum;
+    };
+    // (a wavefront and turn: eight tokens of one tile)
+    if constexpr (kMode == 2) {
+        for (int turn = wave_of_8; turn < 2 * kFi * kTj; turn += 8) {
+            const int tile = turn >> 2, i = tile / kTj, j = tile % kTj, n = 8 * (turn & 3) + row8;
+            const floatx4 g4 = summed(tile, n), u4 = summed(kFi / 2 * kTj + tile, n);
+            const float gate[4] = {g4[0], g4[1], g4[2], g4[3]}, up[4] = {u4[0], u4[1], u4[2], u4[3]};
+            half4_pf_t h, l;
+            swiglu_split4(h, l, gate, up);
+            const size_t at = static_cast<size_t>(t_base + 32 * j + n) * job.out_ld + f_base + 32 * i + 4 * part8;
+            *reinterpret_cast<half4_pf_t*>(job.out_hi + at) = h;
+            if constexpr (kLo) *reinterpret_cast<half4_pf_t*>(job.out_lo + at) = l;
+        }
+    } else {
+        float* __restrict__ y = (which == 2 ? job.y[2] : (which == 1 ? job.y[1] : job.y[0])) + static_cast<size_t>(split) * job.split_stride;
+        const int ldy = which == 2 ? job.ldy[2] : (which == 1 ? job.ldy[1] : job.ldy[0]);
+        for (int turn = wave_of_8; turn < 4 * kFi * kTj; turn += 8) {
+            const int tile = turn >> 2, i = tile / kTj, j = tile % kTj, n = 8 * (turn & 3) + row8;
+            floatx4 v = summed(tile, n);
+            floatx4* out = reinterpret_cast<floatx4*>(y + static_cast<size_t>(t_base + 32 * j + n) * ldy + f_base + 32 * i + 4 * part8);
+            if constexpr (kMode == 1) {
+                const floatx4 old = *out;
+                v = floatx4{old[0] + v[0], old[1] + v[1], old[2] + v[2], old[3] + v[3]};
+            }
+            *out = v;
+        }
     }
 }
 
@@ -1018,9 +1225,17 @@ __global__ __launch_bounds__(256) void k_split(const float* __restrict__ x, half
 
 namespace {
 
-// Buffers of a chunk of t_pad tokens, in lpp_model::pf_buf order.
-enum { kBufTokens, kBufX, kBufQ, kBufK, kBufV, kBufGate, kBufUp, kBufHi, kBufLo, kBufHi2, kBufLo2, kBufCount };
+// Buffers of a chunk of t_pad tokens, in lpp_model::pf_buf order: parts of one allocation, which kBufAll names.
+enum { kBufTokens, kBufX, kBufQ, kBufK, kBufV, kBufPartials, kBufHi, kBufLo, kBufHi2, kBufLo2, kBufAll, kBufCount };
 static_assert(kBufCount <= static_cast<int>(sizeof(lpp_model::pf_buf) / sizeof(void*)), "lpp_model::pf_buf is too small");
+
+// Floats of kBufPartials: the partial products of the GEMM before (read by the kernel that follows it, so one area does
+// for all of a layer's), or the gate and up projections where those are not fused.
+size_t partial_floats(const lpp_model* m, int t_pad) {
+    const size_t t = static_cast<size_t>(t_pad), few = t < 256 ? t : 256;  // (small batches are cut along K the most)
+    const size_t pair = 2 * t * m->cfg.hidden_dim, ranges = 8 * few * (m->cfg.dim + 2 * m->kv_dim);
+    return pair > ranges ? pair : ranges;
+}
 
 const char* unsupported_reason(const lpp_model* m) {
     const lpp_config& c = m->cfg;
@@ -1038,25 +1253,24 @@ lpp_status ensure_scratch(lpp_model* m, int t_pad) {
     const lpp_config& c = m->cfg;
     const size_t t = static_cast<size_t>(t_pad);
     const size_t widest = static_cast<size_t>(c.hidden_dim > c.dim ? c.hidden_dim : c.dim);
-    const size_t bytes[kBufCount] = {t * sizeof(int),
-                                     t * c.dim * sizeof(float),
-                                     t * c.dim * sizeof(float),
-                                     t * m->kv_dim * sizeof(float),
-                                     t * m->kv_dim * sizeof(float),
-                                     t * c.hidden_dim * sizeof(float),
-                                     t * c.hidden_dim * sizeof(float),
-                                     t * widest * sizeof(pf::half_t),
-                                     t * widest * sizeof(pf::half_t),
-                                     // the feed-forward activations, written while hi/lo are still being read
-                                     t * c.hidden_dim * sizeof(pf::half_t),
-                                     t * c.hidden_dim * sizeof(pf::half_t)};
-    for (int i = 0; i < kBufCount; ++i) {
-        lpp_status st = lpp_malloc(&m->pf_buf[i], bytes[i]);
-        if (st != LPP_OK) {
-            prefill_release(m);
-            return st;
-        }
+    const size_t bytes[kBufAll] = {t * sizeof(int),
+                                   t * c.dim * sizeof(float),
+                                   t * c.dim * sizeof(float),
+                                   t * m->kv_dim * sizeof(float),
+                                   t * m->kv_dim * sizeof(float),
+                                   partial_floats(m, t_pad) * sizeof(float),
+                                   t * widest * sizeof(pf::half_t),
+                                   t * widest * sizeof(pf::half_t),
+                                   // the feed-forward activations, written while hi/lo are still being read
+                                   t * c.hidden_dim * sizeof(pf::half_t),
+                                   t * c.hidden_dim * sizeof(pf::half_t)};
+    size_t offset[kBufAll], total = 0;
+    for (int i = 0; i < kBufAll; ++i) {
+        offset[i] = total;
+        total += (bytes[i] + 255) / 256 * 256;
     }
+    LPP_TRY(lpp_malloc(&m->pf_buf[kBufAll], total));
+    for (int i = 0; i < kBufAll; ++i) m->pf_buf[i] = static_cast<char*>(m->pf_buf[kBufAll]) + offset[i];
     m->pf_cap = t_pad;
     return LPP_OK;
 }
@@ -1068,18 +1282,26 @@ struct Product {
     int n;
 };
 
-// The kernel's LDS need, told to the runtime once per device (the attribute belongs to the device's copy of the kernel).
-template <int kFi, int kTj, int kMode, int kTripK, bool kLo = true>
-lpp_status size_pipe() {
-    static bool sized[64] = {};
+// A kernel's LDS need, told to the runtime once per device (the attribute belongs to the device's copy of the kernel).
+lpp_status size_lds(const void* kernel, int bytes, bool (&sized)[64]) {
     int device = 0;
     LPP_HIP(hipGetDevice(&device));
     if (device < 0 || device >= 64 || !sized[device]) {
-        LPP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&pf::k_gemm_pipe<kFi, kTj, kMode, kTripK, kLo>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, pf::PipeShape<kFi, kTj, kTripK, kLo>::kLdsBytes));
+        LPP_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
         if (device >= 0 && device < 64) sized[device] = true;
     }
     return LPP_OK;
+}
+template <int kFi, int kTj, int kMode, int kTripK, bool kLo = true>
+lpp_status size_pipe() {
+    static bool sized[64] = {};
+    return size_lds(reinterpret_cast<const void*>(&pf::k_gemm_pipe<kFi, kTj, kMode, kTripK, kLo>),
+                    pf::PipeShape<kFi, kTj, kTripK, kLo>::kLdsBytes, sized);
+}
+template <int kFi, int kTj, int kMode, bool kLo>
+lpp_status size_few() {
+    static bool sized[64] = {};
+    return size_lds(reinterpret_cast<const void*>(&pf::k_gemm_few<kFi, kTj, kMode, kLo>), pf::FewShape<kFi, kTj, kLo>::kLdsBytes, sized);
 }
 
 template <int kFi, int kTj, int kMode, int kTripK, bool kLo>
@@ -1097,6 +1319,114 @@ lpp_status launch_pipe(const pf::PipeJob& job, hipStream_t s) {
     return job.xl != nullptr ? launch_pipe_as<kFi, kTj, kMode, kTripK, true>(job, s) : launch_pipe_as<kFi, kTj, kMode, kTripK, false>(job, s);
 }
 
+template <int kFi, int kTj, int kMode, bool kLo>
+lpp_status launch_few_as(const pf::PipeJob& job, hipStream_t s) {
+    constexpr int kLds = pf::FewShape<kFi, kTj, kLo>::kLdsBytes;
+    LPP_TRY((size_few<kFi, kTj, kMode, kLo>()));
+    const int per_die = (job.groups + 7) / 8;
+    hipLaunchKernelGGL((pf::k_gemm_few<kFi, kTj, kMode, kLo>), dim3(per_die * 8 * job.token_tiles), dim3(512), kLds, s, job);
+    LPP_CHECK_LAUNCH("k_gemm_few");
+    return LPP_OK;
+}
+template <int kFi, int kTj, int kMode>
+lpp_status launch_few(const pf::PipeJob& job, hipStream_t s) {
+    return job.xl != nullptr ? launch_few_as<kFi, kTj, kMode, true>(job, s) : launch_few_as<kFi, kTj, kMode, false>(job, s);
+}
+
+// How a product is laid out on the device: what a workgroup's tile is and in how many ranges K is cut.
+struct Plan {
+    bool few;          // k_gemm_few (rows = 32 fi, tokens = 32 tj), otherwise k_gemm_pipe (rows = 64 fi, tokens = 64 tj)
+    int fi, tj;
+    int splits;
+    int tile_rows() const { return (few ? 32 : 64) * fi; }
+    int tile_tokens() const { return (few ? 32 : 64) * tj; }
+};
+
+// Rows the activations of n tokens are padded to: whole tiles of 128 tokens, or of 32 up to that many.
+int padded_tokens(int n) {
+    const int unit = n <= 128 && test_option(LPP_OPT_PREFILL_STAGED_GEMM) != 0 ? 32 : pf::kTileTokens;
+    return (n + unit - 1) / unit * unit;
+}
+
+// More than 256 tokens: k_gemm_pipe, 256 rows a tile where that leaves no compute unit without a workgroup (always for
+// a pair), otherwise 128 and K in as many ranges as the device takes at once.
+//
+// Up to 256 tokens the choice is made by what a launch of each would take.  A workgroup of k_gemm_few is paced by its
+// bytes from L2 into LDS (57 bytes a nanosecond), one of k_gemm_pipe by its bytes (88) and its MFMA clocks; a last round
+// of workgroups that does not fill the device counts almost whole; no launch is faster than its weights at 3.9 TB/s;
+// every partial product of a cut K is written (2.5 TB/s, in many short runs) and read (5 TB/s) once more.  The constants
+// are a fit to 1100 timed launches (ten weight matrices of the TinyLlama, 1B and 8B shapes, 32 to 2048 tokens, both
+// modes, every tile below): 14 % rms, and the launch picked is 2.2 % slower than the fastest one on average.
+//
+// `max_splits`: ranges K may be cut into.  `row_step`: every matrix is a whole number of row_step rows.  `pair`: W1 and W3
+// side by side in a tile (total_n counts both).
+Plan plan_gemm(int total_n, int K, int t_pad, int max_splits, bool lo, int row_step, bool pair) {
+    static constexpr struct {
+        bool few;
+        int fi, tj;
+    } kTiles[] = {{true, 1, 1}, {true, 1, 2}, {true, 1, 3}, {true, 1, 4}, {true, 2, 1}, {true, 2, 2}, {true, 2, 3}, {true, 2, 4},
+                  {true, 4, 1}, {true, 4, 2}, {false, 2, 2}, {false, 4, 2}};
+    Plan best = {false, 2, 2, 1};
+    const bool wide_allowed = row_step % 256 == 0 && test_option(LPP_OPT_PREFILL_WIDE_TILES) != 0;
+    if (t_pad > 256) {
+        const int token_tiles = t_pad / 128;
+        if (pair || (wide_allowed && total_n / 256 * token_tiles >= compute_units())) best.fi = 4;
+        while (2 * best.splits <= max_splits && total_n / best.tile_rows() * token_tiles * best.splits * 2 <= compute_units() &&
+               K % (64 * 2 * best.splits) == 0 && K / (2 * best.splits) >= 512)
+            best.splits *= 2;
+        return best;
+    }
+    float best_us = 1e30f;
+    for (const auto& t : kTiles) {
+        const Plan p = {t.few, t.fi, t.tj, 1};
+        const int rows = p.tile_rows(), tokens = p.tile_tokens();
+        if (row_step % rows != 0 || t_pad % tokens != 0 || (pair && t.fi == 1)) continue;
+        if (!t.few && t.fi == 4 && !wide_allowed) continue;
+        for (int splits = 1; splits <= max_splits; splits *= 2) {
+            if (splits > 1 && (K % (64 * splits) != 0 || K / splits < 512)) continue;
+            const int wgs = total_n / rows * (t_pad / tokens) * splits;
+            const int rounds = (wgs + compute_units() - 1) / compute_units();
+            const float k = static_cast<float>(K) / splits, copies = lo ? 2.0f : 1.0f;
+            const float bytes = k * 2.0f * (rows + copies * tokens), clocks = k * copies * rows * tokens / 1024.0f;
+            const float busy = t.few ? bytes / 57e3f : bytes / 88e3f + clocks / 5.7e6f;
+            float us = (t.few || t_pad > 128 ? 1.9f : 2.9f) + fmaxf(fmaxf(1.0f, 0.87f * rounds + 0.13f * wgs / compute_units()) * busy, 2.0f * total_n * K / 3.9e6f);
+            if (splits > 1) us += 4.0f * t_pad * total_n * (splits / 2.5e6f + (splits - 1) / 5e6f);
+            if (us < best_us) {
+                best_us = us;
+                best = p;
+                best.splits = splits;
+            }
+        }
+    }
+    return best;
+}
+
+template <int kMode>
+lpp_status launch_plan(const Plan& p, const pf::PipeJob& job, hipStream_t s) {
+    if (!p.few) {
+        if (p.fi == 4) return launch_pipe<4, 2, kMode, 32>(job, s);
+        return launch_pipe<2, 2, kMode>(job, s);
+    }
+    if (p.fi == 4) return p.tj == 1 ? launch_few<4, 1, kMode>(job, s) : launch_few<4, 2, kMode>(job, s);
+    if (p.fi == 2) {
+        switch (p.tj) {
+            case 1: return launch_few<2, 1, kMode>(job, s);
+            case 2: return launch_few<2, 2, kMode>(job, s);
+            case 3: return launch_few<2, 3, kMode>(job, s);
+            default: return launch_few<2, 4, kMode>(job, s);
+        }
+    }
+    if constexpr (kMode != 2) {
+        switch (p.tj) {
+            case 1: return launch_few<1, 1, kMode>(job, s);
+            case 2: return launch_few<1, 2, kMode>(job, s);
+            case 3: return launch_few<1, 3, kMode>(job, s);
+            default: return launch_few<1, 4, kMode>(job, s);
+        }
+    }
+    return fail(LPP_ERR_STATE, "prefill GEMM: no kernel for a pair of matrices in one row tile");
+}
+
 // `partials` (optional, partial_floats long): room for the partial products of a split K.  A product
 // with too few output tiles for the compute units is cut along K into ranges, each multiplied by
 // its own workgroups into `partials`: range z of matrix i lies at partials + z * t_pad * (n_0 + n_1 +
@@ -1106,29 +1436,24 @@ lpp_status launch_pipe(const pf::PipeJob& job, hipStream_t s) {
 lpp_status gemm(const Product* prods, int count, const pf::half_t* xh, const pf::half_t* xl, int K, int t_pad, bool accumulate,
                 hipStream_t s, float* partials = nullptr, size_t partial_floats = 0, int* left_split = nullptr,
                 bool remainder = true) {
-    LPP_REQUIRE(count >= 1 && count <= 3 && t_pad % pf::kTileTokens == 0 && K % 32 == 0, "prefill GEMM: %d products, K %d, T %d",
+    LPP_REQUIRE(count >= 1 && count <= 3 && t_pad > 0 && t_pad % 32 == 0 && K % 32 == 0, "prefill GEMM: %d products, K %d, T %d",
                 count, K, t_pad);
     if (left_split != nullptr) *left_split = 1;
     int total_n = 0;
-    bool wide = true;  // every matrix a whole number of 256-row tiles
+    int step = 256;  // largest tile height every matrix is a whole number of
     for (int i = 0; i < count; ++i) {
         LPP_REQUIRE(prods[i].n > 0 && prods[i].n % pf::kTileFeatures == 0, "prefill GEMM: n %d", prods[i].n);
         total_n += prods[i].n;
-        wide = wide && prods[i].n % 256 == 0;
+        if (prods[i].n % 256 != 0) step = 128;
     }
     const bool staged = K % pf::kPipeTripK == 0 && test_option(LPP_OPT_PREFILL_STAGED_GEMM) != 0;
+    LPP_REQUIRE(staged || t_pad % pf::kTileTokens == 0, "prefill GEMM: T %d, K %d", t_pad, K);
     if (staged) {
-        const int token_tiles = t_pad / pf::kTileTokens;
-        wide = wide && (total_n / 256) * token_tiles >= compute_units() && test_option(LPP_OPT_PREFILL_WIDE_TILES) != 0;
-        const int tile = wide ? 256 : 128;
-        const int feature_tiles = total_n / tile;
         const size_t stride = static_cast<size_t>(t_pad) * total_n;
-        int splits = 1;
-        if (partials != nullptr && (count == 1 || left_split != nullptr)) {
-            while (splits < 8 && feature_tiles * token_tiles * splits * 2 <= compute_units() &&
-                   K % (2 * pf::kPipeTripK * splits) == 0 && K / (2 * splits) >= 512 && stride * 2 * splits <= partial_floats)
-                splits *= 2;
-        }
+        int most = 1;
+        while (partials != nullptr && (count == 1 || left_split != nullptr) && most < 8 && stride * 2 * most <= partial_floats) most *= 2;
+        const Plan plan = plan_gemm(total_n, K, t_pad, most, remainder, step, false);
+        const int tile = plan.tile_rows(), feature_tiles = total_n / tile, token_tiles = t_pad / plan.tile_tokens(), splits = plan.splits;
         pf::PipeJob job = {};
         int at = 0;
         size_t before = 0;
@@ -1152,13 +1477,8 @@ lpp_status gemm(const Product* prods, int count, const pf::half_t* xh, const pf:
         job.token_tiles = token_tiles;
         job.groups = feature_tiles * splits;
         const bool add_in_kernel = accumulate && splits == 1;
-        if (wide) {
-            if (add_in_kernel) LPP_TRY((launch_pipe<4, 2, 1, 32>(job, s)));
-            else LPP_TRY((launch_pipe<4, 2, 0, 32>(job, s)));
-        } else {
-            if (add_in_kernel) LPP_TRY((launch_pipe<2, 2, 1>(job, s)));
-            else LPP_TRY((launch_pipe<2, 2, 0>(job, s)));
-        }
+        if (add_in_kernel) LPP_TRY(launch_plan<1>(plan, job, s));
+        else LPP_TRY(launch_plan<0>(plan, job, s));
         if (splits > 1 && left_split != nullptr) {
             *left_split = splits;
         } else if (splits > 1) {
@@ -1236,20 +1556,21 @@ lpp_status gate_up_swiglu(const void* w1, const void* w3, int hidden, const pf::
     job.xl = remainder ? xl : nullptr;
     job.K = K;
     job.k_len = K;
-    job.feature_tiles = hidden / 128;  // 128 features a tile: 128 rows of W1 and the same 128 of W3
-    job.token_tiles = t_pad / pf::kTileTokens;
+    const Plan plan = plan_gemm(2 * hidden, K, t_pad, 1, remainder, hidden % 128 == 0 ? 256 : 128, true);
+    job.feature_tiles = 2 * hidden / plan.tile_rows();  // half of a tile's rows from either matrix
+    job.token_tiles = t_pad / plan.tile_tokens();
     job.groups = job.feature_tiles;
     job.out_hi = out_hi;
     job.out_lo = out_lo;
     job.out_ld = hidden;
-    return launch_pipe<4, 2, 2, 32>(job, s);
+    return launch_plan<2>(plan, job, s);
 }
 
 // One chunk: tokens[0..n) at positions pos0 .. pos0 + n - 1; n <= kChunk.
 lpp_status prefill_chunk(lpp_model* m, const int* tokens, int n, int pos0) {
     const lpp_config& c = m->cfg;
     const int dim = c.dim, kv = m->kv_dim, hidden = c.hidden_dim, hs = m->head_size;
-    const int t_pad = (n + pf::kTileTokens - 1) / pf::kTileTokens * pf::kTileTokens;
+    const int t_pad = padded_tokens(n);
     LPP_TRY(ensure_scratch(m, t_pad));
     hipStream_t s = stream();
     int* d_tokens = static_cast<int*>(m->pf_buf[kBufTokens]);
@@ -1257,8 +1578,7 @@ lpp_status prefill_chunk(lpp_model* m, const int* tokens, int n, int pos0) {
     float* q = static_cast<float*>(m->pf_buf[kBufQ]);
     float* k = static_cast<float*>(m->pf_buf[kBufK]);
     float* v = static_cast<float*>(m->pf_buf[kBufV]);
-    float* gate = static_cast<float*>(m->pf_buf[kBufGate]);
-    float* up = static_cast<float*>(m->pf_buf[kBufUp]);
+    float* partials = static_cast<float*>(m->pf_buf[kBufPartials]);
     pf::half_t* hi = static_cast<pf::half_t*>(m->pf_buf[kBufHi]);
     pf::half_t* lo = static_cast<pf::half_t*>(m->pf_buf[kBufLo]);
     LPP_HIP(hipMemcpyAsync(d_tokens, tokens, static_cast<size_t>(n) * sizeof(int), hipMemcpyHostToDevice, s));
@@ -1271,9 +1591,7 @@ lpp_status prefill_chunk(lpp_model* m, const int* tokens, int n, int pos0) {
     };
     pf::half_t* hi2 = static_cast<pf::half_t*>(m->pf_buf[kBufHi2]);
     pf::half_t* lo2 = static_cast<pf::half_t*>(m->pf_buf[kBufLo2]);
-    // The fp32 gate and up buffers double as room for the partial products of the GEMMs whose K is
-    // split (each is t_pad * hidden floats): up for Wq/Wk/Wv, gate for Wo and then for W2.
-    const size_t room = static_cast<size_t>(t_pad) * hidden;
+    const size_t room = partial_floats(m, t_pad);
     // LPP_PREFILL_EXACT: every product takes the activations as binary16 head + remainder.  LPP_PREFILL_FAST: the head
     // alone, in the staged kernels (what a GEMM sees of its input is then what the reference's own GPU GEMV sees,
     // matmul.cu:85-98; accumulation stays fp32).
@@ -1286,7 +1604,7 @@ lpp_status prefill_chunk(lpp_model* m, const int* tokens, int n, int pos0) {
     int pending = 0;  // ranges of the product before (W2's, then Wo's) still to be added to x
     for (int l = 0; l < c.n_layers; ++l) {
         // attention block, model.cpp:216-218
-        LPP_TRY(norm_split(x, static_cast<const float*>(m->w[LPP_T_RMS_ATT]) + static_cast<size_t>(l) * dim, hi, lo, dim, n, t_pad, gate,
+        LPP_TRY(norm_split(x, static_cast<const float*>(m->w[LPP_T_RMS_ATT]) + static_cast<size_t>(l) * dim, hi, lo, dim, n, t_pad, partials,
                            pending > 1 ? pending : 0, static_cast<size_t>(t_pad) * dim, s, !lean));
         // What a prefill leaves behind is the cache: the last layer needs its K and V rows only, and
         // nothing reads what the rest of that layer would compute.
@@ -1295,11 +1613,11 @@ lpp_status prefill_chunk(lpp_model* m, const int* tokens, int n, int pos0) {
                                 {layer_of(LPP_T_WV, l, kv, dim), v, kv}};
         const int q_dim = last_layer ? 0 : dim;
         int qkv_split = 1;
-        LPP_TRY(gemm(qkv + (last_layer ? 1 : 0), last_layer ? 2 : 3, hi, lo, dim, t_pad, false, s, up, room, &qkv_split, exact));
+        LPP_TRY(gemm(qkv + (last_layer ? 1 : 0), last_layer ? 2 : 3, hi, lo, dim, t_pad, false, s, partials, room, &qkv_split, exact));
         const size_t qkv_stride = static_cast<size_t>(t_pad) * (q_dim + 2 * kv);
-        const float* qs = qkv_split > 1 ? up : q;
-        const float* ks = qkv_split > 1 ? up + static_cast<size_t>(t_pad) * q_dim : k;
-        const float* vs = qkv_split > 1 ? up + static_cast<size_t>(t_pad) * (q_dim + kv) : v;
+        const float* qs = qkv_split > 1 ? partials : q;
+        const float* ks = qkv_split > 1 ? partials + static_cast<size_t>(t_pad) * q_dim : k;
+        const float* vs = qkv_split > 1 ? partials + static_cast<size_t>(t_pad) * (q_dim + kv) : v;
         hipLaunchKernelGGL(pf::k_rope_scatter, dim3(n), dim3(256), 0, s, q, qs, ks, vs, m->rope, m->key_cache, m->value_cache, l,
                            pos0, q_dim, kv, hs, c.seq_len, qkv_split, qkv_stride);
         LPP_CHECK_LAUNCH("k_rope_scatter");
@@ -1330,21 +1648,22 @@ lpp_status prefill_chunk(lpp_model* m, const int* tokens, int n, int pos0) {
                                m->value_cache, hi, lo, l, pos0, dim, kv, hs, m->gqa, c.seq_len, n);
         LPP_CHECK_LAUNCH("k_attention");
         const Product wo = {layer_of(LPP_T_WO, l, dim, dim), x, dim};
-        LPP_TRY(gemm(&wo, 1, hi, lo, dim, t_pad, true, s, gate, room, &pending, exact));
+        LPP_TRY(gemm(&wo, 1, hi, lo, dim, t_pad, true, s, partials, room, &pending, exact));
         // feed-forward block, model.cpp:221-226
-        LPP_TRY(norm_split(x, static_cast<const float*>(m->w[LPP_T_RMS_FFN]) + static_cast<size_t>(l) * dim, hi, lo, dim, n, t_pad, gate,
+        LPP_TRY(norm_split(x, static_cast<const float*>(m->w[LPP_T_RMS_FFN]) + static_cast<size_t>(l) * dim, hi, lo, dim, n, t_pad, partials,
                            pending > 1 ? pending : 0, static_cast<size_t>(t_pad) * dim, s, !lean));
         if (fused_ffn) {
             LPP_TRY(gate_up_swiglu(layer_of(LPP_T_W1, l, hidden, dim), layer_of(LPP_T_W3, l, hidden, dim), hidden, hi, lo, dim, t_pad,
                                    hi2, lo2, s, exact));
         } else {
+            float *gate = partials, *up = partials + static_cast<size_t>(t_pad) * hidden;
             const Product gate_up[2] = {{layer_of(LPP_T_W1, l, hidden, dim), gate, hidden}, {layer_of(LPP_T_W3, l, hidden, dim), up, hidden}};
             LPP_TRY(gemm(gate_up, 2, hi, lo, dim, t_pad, false, s, nullptr, 0, nullptr, exact));
             hipLaunchKernelGGL(pf::k_swiglu_split, dim3((hidden + 255) / 256, t_pad), dim3(256), 0, s, gate, up, hi2, lo2, hidden, n);
             LPP_CHECK_LAUNCH("k_swiglu_split");
         }
         const Product w2 = {layer_of(LPP_T_W2, l, dim, hidden), x, dim};
-        LPP_TRY(gemm(&w2, 1, hi2, lo2, hidden, t_pad, true, s, gate, room, &pending, exact));
+        LPP_TRY(gemm(&w2, 1, hi2, lo2, hidden, t_pad, true, s, partials, room, &pending, exact));
     }
     LPP_HIP(hipStreamSynchronize(s));
     return LPP_OK;
@@ -1353,10 +1672,8 @@ lpp_status prefill_chunk(lpp_model* m, const int* tokens, int n, int pos0) {
 }  // namespace
 
 void prefill_release(lpp_model* m) {
-    for (void*& p : m->pf_buf) {
-        lpp_free(p);
-        p = nullptr;
-    }
+    lpp_free(m->pf_buf[kBufAll]);
+    for (void*& p : m->pf_buf) p = nullptr;
     m->pf_cap = 0;
 }
 
@@ -1458,11 +1775,28 @@ namespace {
 int g_setup_state[kMaxDevices] = {};
 char g_setup_message[kMaxDevices][256] = {};
 
+// (every tile plan_gemm may give whole tiles of 128 tokens)
+template <int kMode>
+lpp_status size_few_for() {
+    LPP_TRY((size_few<1, 1, kMode, true>()));
+    LPP_TRY((size_few<1, 2, kMode, true>()));
+    LPP_TRY((size_few<1, 3, kMode, true>()));
+    LPP_TRY((size_few<1, 4, kMode, true>()));
+    LPP_TRY((size_few<2, 1, kMode, true>()));
+    LPP_TRY((size_few<2, 2, kMode, true>()));
+    LPP_TRY((size_few<2, 3, kMode, true>()));
+    LPP_TRY((size_few<2, 4, kMode, true>()));
+    LPP_TRY((size_few<4, 1, kMode, true>()));
+    return size_few<4, 2, kMode, true>();
+}
+
 lpp_status run_scratch_setup() {
     LPP_TRY((size_pipe<4, 2, 0, 32>()));
     LPP_TRY((size_pipe<4, 2, 1, 32>()));
     LPP_TRY((size_pipe<2, 2, 0, pf::kPipeTripK>()));
     LPP_TRY((size_pipe<2, 2, 1, pf::kPipeTripK>()));
+    LPP_TRY((size_few_for<0>()));
+    LPP_TRY((size_few_for<1>()));
     void* p = nullptr;
     return scratch_address(&p);
 }

@@ -388,6 +388,26 @@ def test_prefill_ragged_lengths_and_a_cache_that_ends_inside_a_block(n):
     b.close()
 
 
+@pytest.mark.parametrize("n", [1, 32, 33, 64, 65, 96, 97, 128, 129, 256, 257])
+def test_small_batches_around_the_edges_of_the_token_tiles(n, test_options):
+    """Batches on either side of every token tile and of the rules that pick a GEMM's tile: two layers of the TinyLlama
+    shape (the second layer's cache entries have been through all five products), against the GEMM that reads its
+    fragments straight from memory.  Both sum in fp32: every entry within one binary16 step, or 2^-11 of the largest."""
+    shape = Shape(2048, 5632, 2, 32, 4, 1024, 320, 10000.0, fp16=True, tied=True)
+    m = Model(shape)
+    m.load_synthetic(3)
+    prompt = capi.synth_token_ids(n, 5, shape.vocab_size)
+    m.prefill(prompt, 0)
+    k, v, kf, vf = caches(m, shape, n)
+    assert not kf[:, :, n:, :].any() and not vf[:, :, n:, :].any(), "slots beyond the prompt were written"
+    test_options(capi.OPT_PREFILL_STAGED_GEMM, 0)
+    m.prefill(prompt, 0)
+    k0, v0, _, _ = caches(m, shape, n)
+    for x, y in ((k, k0), (v, v0)):
+        assert np.all(np.abs(x - y) <= np.maximum(np.abs(y) * 2.0 ** -9, np.abs(y).max() * 2.0 ** -11))
+    m.close()
+
+
 def test_prefill_of_a_long_prompt_at_full_size():
     """Llama-3.2-1B shape with the long-context cache: 1500 prompt ids = three batches (512, 512, 476), the later
     ones attending to the earlier ones' cache entries; caches and the next step against prefill by decode."""
