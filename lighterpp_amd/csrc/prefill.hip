@@ -32,7 +32,7 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int kTileTokens = 128;    // token rows of a workgroup's output tile
 constexpr int kTileFeatures = 128;  // weight rows of it
-constexpr int kChunk = 512;         // prompt tokens per pass over the weights
+constexpr int kChunk = 512;         // prompt tokens per pass over the weights, at most
 constexpr int kMaxGqa = 8;          // query heads per KV head the attention kernel keeps in registers
 
 // ---------------------------------------------------------------------------
@@ -958,92 +958,141 @@ __global__ __launch_bounds__(256) void k_attention(const float* __restrict__ q, 
 // The same attention on the matrix cores
 // ---------------------------------------------------------------------------
 //
-// A workgroup owns 32 query rows = (32 / gqa) consecutive tokens x the gqa query heads of one KV
-// head; its four wavefronts share the cache's blocks of 32 positions among them (wavefront w takes
-// blocks w, w + 4, ..: a row's work is a chain of dependent steps per block, so the longest rows
-// set the kernel's time), each with its own running maximum, sum and output, merged through
-// LDS at the end.  Per block:
-//   S^T[pos][row] = sum_d K[pos][d] Q[row][d]     A = K block (a lane's 8 d-values: one 16-byte
-//                                                 load from the cache row), B = Q (head + remainder)
-//   online softmax: in the result a LANE holds one query row (its column) and 16 of the block's 32
-//                   positions, the lane 32 further on the other 16 -- maximum, sum and rescaling are
-//                   per lane, with one exchange between the two halves of the wavefront
-//   O^T[d][row] += sum_pos V^T[d][pos] P^T[pos][row]   A = V transposed: the wavefront loads its block of
-//                                                      V as the cache holds it (a position's row at a
-//                                                      time, 16 bytes a lane), writes it into a tile of
-//                                                      LDS of its own with positions contiguous, and
-//                                                      reads its fragments from there,
-//                                                      B = P straight from the lane's own registers
-// A lane's 16 positions of a block are {8j + 4g .. 8j + 4g + 3 : j = 0..3} (g = lane / 32), so as
-// B operand of the second product it supplies, per 16-position step, positions 4g..4g+3 and
-// 8+4g..8+4g+3; the V^T fragment is read in the same order (two 8-byte reads).  Any such
-// permutation of k is fine as long as both operands use it.
-// Probabilities and queries are split into binary16 head + remainder like every other activation.
+// A wavefront owns 32 query rows = (32 / gqa) consecutive tokens x the gqa query heads of one KV head, and walks the
+// context in steps of 32 positions.  A workgroup is kR x kP such wavefronts: kR take neighbouring rows and share every
+// step's K and V rows, kP take the steps in turn and merge their running (maximum, sum, output) at the end.  2 x 2 where
+// that makes workgroups enough; a batch of few rows takes 1 x 8 (heads of 128: 1 x 4, for want of LDS).  Per step:
+//   S^T[pos][row] = sum_d K[pos][d] Q[row][d]     A = K rows, B = Q (head + remainder, in registers for the whole walk)
+//   online softmax: in the result a LANE holds one query row (its column) and 16 of the 32 positions, the lane 32 further
+//                   on the other 16 -- maximum and rescaling are per lane, with one exchange between the two halves of
+//                   the wavefront per step; the sums of the two halves meet once, at the end
+//   O^T[d][row] += sum_pos V^T[d][pos] P^T[pos][row]   A = V transposed, B = P straight from the lane's own registers
+// A lane's 16 positions of 32 are {8j + 4g .. 8j + 4g + 3 : j = 0..3} (g = lane / 32), so as B operand of the second
+// product it supplies, per 16 positions, positions 4g..4g+3 and 8+4g..8+4g+3; V is read in the same order (any
+// permutation of k is fine as long as both operands use it).  Queries and probabilities are split into binary16 head +
+// remainder like every other activation; the softmax works in powers of two, log2(e) / sqrt(head size) being multiplied
+// into the queries.
+//
+// K and V rows travel from the cache into LDS by requests of 1 KiB (no registers, and nothing waits but the step that
+// reads them), a step ahead.  The 16-byte pieces of a row are stored in an order that keeps the reads free of bank
+// conflicts (the address each lane requests makes it): K fragments are 16 bytes a lane from 32 rows; V fragments are
+// transposed on the way out (ds_read_b64_tr_b16: 16 lanes read a tile of 4 positions x 16 dimensions and every lane gets
+// the 4 positions of one dimension).  Rows past the tile's last position are the last row again (finite, weight zero).
+
+//
+// What bounds it: a step of 32 positions is 512 MFMA clocks and about as many of the vector units (sixteen v_exp_f32 are
+// 256 of them), and one wavefront does them one after the other, so what counts is wavefronts per SIMD: the stages are
+// kept small enough for two or three workgroups to a compute unit.  (Measured and not better: the next step's scores
+// formed between this step's weights in the same wavefront, at twice the stages; more steps in flight; 128 rows to a
+// workgroup; a short batch's context split over several workgroups with a kernel that merges them.)  1B shape, exact
+// mode: 150 ids behind 3000, 34 -> 22 us a layer; 2048 ids behind 2048, 107 us on average.
 
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+typedef short short4_t __attribute__((ext_vector_type(4)));
 
-template <int kHs, bool kLo>
-__global__ __launch_bounds__(256) void k_attention_mfma(const float* __restrict__ q, const uint16_t* __restrict__ key_cache,
-                                                        const uint16_t* __restrict__ value_cache, half_t* __restrict__ out_hi,
-                                                        half_t* __restrict__ out_lo, int layer, int pos0, int dim, int kv_dim,
-                                                        int gqa, int seq_len, int n_tokens) {
-    constexpr int kDTiles = kHs / 32, kKSteps = kHs / 16;
-    const int lane = lane_id(), wave = wave_index();
+template <int kHs, int kR, int kP>
+struct AttentionShape {
+    static constexpr int kStep = 32;
+    static constexpr int kRowBytes = 2 * kHs, kPieces = kHs / 8;
+    static constexpr int kHalfBytes = kStep * kRowBytes, kStageBytes = 2 * kHalfBytes;  // K rows, then V rows
+    static constexpr int kLoads = kStageBytes / 1024 / kR;                              // requests per wavefront and step
+    static constexpr int kStages = kHs == 64 && kP == 2 ? 3 : 2;  // 2 x 2: 48 / 64 KiB, at least two workgroups to a compute unit
+    static constexpr int kMergeBytes = (kP - 1) * kR * (kHs / 2 + 2) * 64 * 4;
+    static constexpr int kLdsBytes = kP * kStages * kStageBytes > kMergeBytes ? kP * kStages * kStageBytes : kMergeBytes;
+    static_assert(kLdsBytes <= 160 * 1024, "LDS of a workgroup");
+};
+
+// max(v, the other half-wavefront's v) / v + the other half-wavefront's v
+__device__ __forceinline__ float halves_max(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float halves_sum(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// (p0, p1) rounded to binary16, and what is left of each (exact).  The packed pair and the factor -1 are hidden from the
+// compiler, which would otherwise round every value a second time to subtract it: one v_cvt_pk_f16_f32 and two v_fma_mix_f32.
+// (No instruction is written here by hand: one that reads a result of v_exp_f32 needs a wait state, which the compiler
+// counts for its own instructions only.)
+__device__ __forceinline__ half2_t split_pair(float& p0, float& p1, float minus_one) {
+    uint32_t packed = __builtin_bit_cast(uint32_t, half2_t{static_cast<half_t>(p0), static_cast<half_t>(p1)});
+    asm("" : "+v"(packed));
+    const half2_t h = __builtin_bit_cast(half2_t, packed);
+    p0 = fmaf(static_cast<float>(h[0]), minus_one, p0);
+    p1 = fmaf(static_cast<float>(h[1]), minus_one, p1);
+    return h;
+}
+
+template <int kHs, bool kLo, int kR, int kP>
+__global__ __launch_bounds__(64 * kR * kP, 2) void k_attention_mfma(const float* __restrict__ q, const uint16_t* __restrict__ key_cache,
+                                                                 const uint16_t* __restrict__ value_cache,
+                                                                 half_t* __restrict__ out_hi, half_t* __restrict__ out_lo, int layer,
+                                                                 int pos0, int dim, int kv_dim, int gqa, int seq_len, int n_tokens,
+                                                                 int round_tiles) {
+    typedef AttentionShape<kHs, kR, kP> Shape;
+    constexpr int kDTiles = kHs / 32, kKSteps = kHs / 16, kStep = Shape::kStep, kRowBytes = Shape::kRowBytes;
+    constexpr int kPieces = Shape::kPieces, kLoads = Shape::kLoads, kHalfBytes = Shape::kHalfBytes, kStageBytes = Shape::kStageBytes;
+    constexpr int kStages = Shape::kStages;
+    extern __shared__ __align__(1024) char att_lds[];
+    const int lane = lane_id();
+    const int wave = __builtin_amdgcn_readfirstlane(wave_index());
+    const int wr = wave % kR, wp = wave / kR;
     const int r = lane & 31, g = lane >> 5;
-    const int tokens_per_tile = 32 / gqa;
-    // (the tiles with the longest contexts are dispatched first: where not all workgroups are resident at once, the
-    // short ones fill the gaps at the end instead of the long ones starting last)
-    const int t0 = static_cast<int>(gridDim.x - 1 - blockIdx.x) * tokens_per_tile;
-    if (t0 >= n_tokens) return;  // (the whole workgroup)
-    const int kvh = blockIdx.y;
+    const int tokens_per_wave = 32 / gqa;
+    // (one KV head after the other in the workgroup's number: where there are as many KV heads as dies, a head's rows
+    // stay in one die's L2.  The tiles with the longest contexts are dispatched first; where the device takes two rounds of
+    // workgroups at once, the second round's go out shortest first, so that a compute unit has a long and a short one.)
+    const int kvh = blockIdx.x, round = round_tiles > 0 ? static_cast<int>(blockIdx.y) / round_tiles : 0;
+    const int first_of_round = round * round_tiles, after_round = min(first_of_round + round_tiles, static_cast<int>(gridDim.y));
+    const int order = (round & 1) ? after_round - 1 - (static_cast<int>(blockIdx.y) - first_of_round) : static_cast<int>(blockIdx.y);
+    const int tile = static_cast<int>(gridDim.y) - 1 - order;
+    const int first_token = tile * kR * tokens_per_wave;                                         // of the workgroup
+    const int t0 = first_token + wr * tokens_per_wave;                                           // of the wavefront
+    auto end_of = [&](int token) { return pos0 + (token < n_tokens ? token : n_tokens); };       // positions below which `token`s before attend
+    const int limit = end_of(first_token + kR * tokens_per_wave);                // the workgroup reads [0, limit)
+    const int wave_limit = t0 < n_tokens ? end_of(t0 + tokens_per_wave) : 0;     // the wavefront attends to [0, wave_limit)
     const int my_tok = t0 + r / gqa, my_head = r % gqa;
     const bool valid = my_tok < n_tokens;
     const int tok_c = valid ? my_tok : n_tokens - 1;
-    const int last_tok = (t0 + tokens_per_tile < n_tokens ? t0 + tokens_per_tile : n_tokens) - 1;
-    const int limit = pos0 + last_tok + 1;    // positions the tile reads: [0, limit)
-    const int my_limit = pos0 + tok_c + 1;    // positions this lane's row attends to: [0, my_limit)
-    const uint16_t* kbase = key_cache + static_cast<size_t>(layer) * kv_dim * seq_len + static_cast<size_t>(kvh) * seq_len * kHs;
-    const uint16_t* vbase = value_cache + static_cast<size_t>(layer) * kv_dim * seq_len + static_cast<size_t>(kvh) * seq_len * kHs;
-    // this wavefront's tile of the block's V rows, as the cache holds them: [32 positions][kHs], rows 16 bytes
-    // longer than a cache row, so that the rows four positions apart, which the two halves of the wavefront read
-    // side by side, start 16 banks apart
-    constexpr int kTileRow = kHs + 8;  // binary16 per row
-    __shared__ __align__(16) uint16_t vt_tiles[4][32 * kTileRow];
-    uint16_t* vt_tile = vt_tiles[wave];
-    constexpr int kVChunks = kHs / 16;  // 16-byte pieces of the block's V rows per lane
-    const float scale = 1.0f / sqrtf(static_cast<float>(kHs));  // model.cpp:188
+    const int my_limit = pos0 + tok_c + 1;                                       // this lane's row attends to [0, my_limit)
+    const size_t head_base = static_cast<size_t>(layer) * kv_dim * seq_len + static_cast<size_t>(kvh) * seq_len * kHs;
+    const char* kbase = reinterpret_cast<const char*>(key_cache + head_base);
+    const char* vbase = reinterpret_cast<const char*>(value_cache + head_base);
 
-    // The K rows and the V rows of a wavefront's next block are requested a block ahead (the first block's
-    // before q is read), so that they travel while this block is worked on.  (Four blocks ahead measures
-    // slower: a block's time is its ~400 vector instructions, and the registers cost more than the wait.)
-    auto fetch_k = [&](half8_t (&kf)[kKSteps], int p0) {
-        const int prow = (p0 + r < seq_len) ? p0 + r : seq_len - 1;  // (rows past the tile's limit are masked below)
-        const uint16_t* krow = kbase + static_cast<size_t>(prow) * kHs + 8 * g;
+    char* stages = att_lds + wp * kStages * kStageBytes;
+    const unsigned lds_base = static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)stages));
+    const int steps = (limit + kStep - 1) / kStep, turns = (steps + kP - 1) / kP;
+    constexpr int kRowsPerLoad = 1024 / kRowBytes, kLoadsPerHalf = kHalfBytes / 1024;
+    auto request = [&](int turn) {
+        const int p0 = (turn * kP + wp) * kStep;
 #pragma unroll
-        for (int s = 0; s < kKSteps; ++s) kf[s] = as_half8(load16(krow + 16 * s));
-    };
-    // a block's V rows: piece c of the block = 8 dimensions of one position (zero past the context)
-    auto fetch_v = [&](uintx4 (&vr)[kVChunks], int p0) {
-#pragma unroll
-        for (int i = 0; i < kVChunks; ++i) {
-            const int c = lane + 64 * i, p = c / (kHs / 8), d0 = (c % (kHs / 8)) * 8;
-            const int pos = p0 + p;
-            vr[i] = pos < limit ? load16(vbase + static_cast<size_t>(pos) * kHs + d0) : uintx4{0u, 0u, 0u, 0u};
+        for (int i = 0; i < kLoads; ++i) {
+            const int load = wr + kR * i, in_half = load % kLoadsPerHalf;
+            const bool is_v = load >= kLoadsPerHalf;  // (uniform)
+            const int row = in_half * kRowsPerLoad + lane / kPieces;
+            const int swizzle = is_v ? (kHs == 64 ? 4 * ((row >> 1) & 1) : 4 * (row & 3)) : (kHs == 64 ? (row >> 1) & 7 : row & 15);
+            const int pos = p0 + row < limit ? p0 + row : limit - 1;
+            const char* src = (is_v ? vbase : kbase) + static_cast<size_t>(pos) * kRowBytes + 16 * ((lane % kPieces) ^ swizzle);
+            const unsigned at = __builtin_amdgcn_readfirstlane(lds_base + (turn % kStages) * kStageBytes + load * 1024);
+            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off\n" ::"v"(src), "s"(at) : "memory");
         }
     };
-    half8_t k_next[kKSteps];
-    uintx4 v_next[kVChunks];
-    fetch_k(k_next, 32 * wave);
-    fetch_v(v_next, 32 * wave);
+#pragma unroll
+    for (int t = 0; t < kStages - 1; ++t)
+        if (t < turns) request(t);
 
     half8_t qh[kKSteps], ql[kKSteps];
     {
+        const float scale = 1.44269504088896341f / sqrtf(static_cast<float>(kHs));  // model.cpp:188
         const float* qrow = q + static_cast<size_t>(tok_c) * dim + (kvh * gqa + my_head) * kHs + 8 * g;
 #pragma unroll
         for (int s = 0; s < kKSteps; ++s)
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                const float v = qrow[16 * s + e];
+                const float v = qrow[16 * s + e] * scale;
                 const half_t h = static_cast<half_t>(v);
                 qh[s][e] = h;
                 ql[s][e] = static_cast<half_t>(v - static_cast<float>(h));
@@ -1054,127 +1103,144 @@ __global__ __launch_bounds__(256) void k_attention_mfma(const float* __restrict_
     for (int dt = 0; dt < kDTiles; ++dt)
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[dt][e] = 0.0f;
-    float top = -INFINITY, lsum = 0.0f;
+    // Weights are 2^(score - top).  The reference `top` follows the row's maximum lazily: it moves only when a step's
+    // maximum exceeds it by more than kSlack (weights then stay below 2^kSlack, far inside binary16, and any reference
+    // gives the same quotient in the end).  After a row's first steps it hardly ever moves, and a step in which no row's
+    // reference moved rescales nothing.  The products start from -top, so the scores come out relative to it.
+    constexpr float kSlack = 6.0f;
+    float top = 0.0f, lsum = 0.0f;  // (the sum over this lane's own positions)
+    bool seen = false;              // the row has attended to something: top is a score
+    float minus_one = -1.0f;
+    asm("" : "+v"(minus_one));
 
-    for (int p0 = 32 * wave; p0 < limit; p0 += 128) {
+    // where this lane reads its fragments of a step: K row r, pieces 2 s + g; V rows 4 g + (lane % 16) / 4 of the first
+    // sixteen, dimensions 32 dt + 16 (lane / 16 % 2) + 4 (lane % 4) ..
+    int k_at[kKSteps], v_at[kDTiles];
+#pragma unroll
+    for (int s = 0; s < kKSteps; ++s) k_at[s] = r * kRowBytes + 16 * ((2 * s + g) ^ (kHs == 64 ? (r >> 1) & 7 : r & 15));
+    {
+        const int row = 4 * g + ((lane & 15) >> 2);
+#pragma unroll
+        for (int dt = 0; dt < kDTiles; ++dt) {
+            const int piece = 4 * dt + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
+            v_at[dt] = kHalfBytes + row * kRowBytes + 16 * (piece ^ (kHs == 64 ? 4 * ((row >> 1) & 1) : 4 * (row & 3))) + 8 * (lane & 1);
+        }
+    }
+
+    for (int turn = 0; turn < turns; ++turn) {
+        const int p0 = (turn * kP + wp) * kStep;
+        // (the step's rows have landed, and nobody reads the stage the next requests go to any more)
+        if (turns - 1 - turn >= kStages - 2) wait_requests<(kStages - 2) * kLoads>();
+        else wait_requests<0>();
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if constexpr (kR > 1) __syncthreads();
+        if (turn + kStages - 1 < turns) request(turn + kStages - 1);
+        if (p0 >= wave_limit) continue;
+        const char* stage = stages + (turn % kStages) * kStageBytes;
         floatx16 st;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) st[e] = 0.0f;
-        half8_t kf[kKSteps];
-#pragma unroll
-        for (int s = 0; s < kKSteps; ++s) kf[s] = k_next[s];
-        uintx4 vrows[kVChunks];
-#pragma unroll
-        for (int i = 0; i < kVChunks; ++i) vrows[i] = v_next[i];
-        if (p0 + 128 < limit) {
-            fetch_k(k_next, p0 + 128);
-            fetch_v(v_next, p0 + 128);
-        }
+        for (int e = 0; e < 16; ++e) st[e] = -top;
 #pragma unroll
         for (int s = 0; s < kKSteps; ++s) {
-            st = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[s], qh[s], st, 0, 0, 0);
-            if constexpr (kLo) st = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[s], ql[s], st, 0, 0, 0);
+            const half8_t kf = *reinterpret_cast<const half8_t*>(stage + k_at[s]);
+            st = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qh[s], st, 0, 0, 0);
+            if constexpr (kLo) st = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, ql[s], st, 0, 0, 0);
         }
-        float sv[16];
-        float block_top = -INFINITY;
-        if (p0 + 32 <= pos0 + t0 + 1) {  // (uniform) every row of the tile attends to the whole block: nothing to mask
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                sv[e] = st[e] * scale;
-                block_top = fmaxf(block_top, sv[e]);
-            }
-        } else {
+        if (p0 + kStep > pos0 + t0 + 1) {  // (uniform) some row of the wavefront does not attend to the whole step
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const int pos = p0 + 8 * (e >> 2) + 4 * g + (e & 3);
-                sv[e] = (pos < my_limit) ? st[e] * scale : -INFINITY;
-                block_top = fmaxf(block_top, sv[e]);
+                st[e] = pos < my_limit ? st[e] : -INFINITY;
             }
         }
-        block_top = fmaxf(block_top, __shfl_xor(block_top, 32));
-        // The reference the exponentials are taken against follows the row's maximum lazily: it moves only when a
-        // block's maximum exceeds it by more than kSlack (weights then stay below e^kSlack, far inside binary16, and
-        // any reference gives the same quotient in the end).  After a row's first blocks it hardly ever moves, and a
-        // block in which no row's reference moved skips the rescaling of the running sums and outputs altogether.
-        constexpr float kSlack = 4.0f;
-        const bool moves = block_top > top + kSlack;  // (true for the first block: top is -inf; finite from then on: position 0 is in every row's range)
-        const float grown = moves ? block_top : top;
-        const float corr = (top == -INFINITY) ? 0.0f : (moves ? exp_fast(top - grown) : 1.0f);
-        const bool rescale = __builtin_amdgcn_ballot_w64(moves && top != -INFINITY) != 0ull;  // (uniform; outputs are still zero before the first block)
-        half8_t ph[2], pl[2];
-        float block_sum = 0.0f;
-        // (a row that has seen nothing but masked positions so far keeps -inf as its reference: its weights are
-        // exp(-inf - 0) = 0 instead of exp(-inf + inf))
-        const float against = (grown == -INFINITY) ? 0.0f : grown;
+        float step_top = -INFINITY;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const float pw = exp_fast(sv[e] - against);
-            block_sum += pw;
-            const half_t h = static_cast<half_t>(pw);
-            ph[e >> 3][e & 7] = h;
-            pl[e >> 3][e & 7] = static_cast<half_t>(pw - static_cast<float>(h));
-        }
-        block_sum += __shfl_xor(block_sum, 32);
-        lsum = lsum * corr + block_sum;
-        top = grown;
-        // V rows into the tile, 16 bytes a lane (no two lanes of a quarter wavefront on one bank); the LDS serves a
-        // wavefront's accesses in order, so the fragment reads below see them (and the next block's writes come
-        // after these reads)
+        for (int e = 0; e < 16; ++e) step_top = fmaxf(step_top, st[e]);
+        step_top = halves_max(step_top);
+        const bool moves = step_top > (seen ? kSlack : -INFINITY);
+        if (__builtin_amdgcn_ballot_w64(moves) != 0ull) {  // (uniform)
+            const float by = moves ? step_top : 0.0f;
+            const float corr = __builtin_amdgcn_exp2f(seen ? -by : 0.0f);  // (nothing to rescale before a row's first step)
+            top += by;
+            lsum *= corr;
 #pragma unroll
-        for (int i = 0; i < kVChunks; ++i) {
-            const int c = lane + 64 * i, p = c / (kHs / 8), d0 = (c % (kHs / 8)) * 8;
-            *reinterpret_cast<uintx4*>(vt_tile + p * kTileRow + d0) = vrows[i];
-        }
-#pragma unroll
-        for (int dt = 0; dt < kDTiles; ++dt) {
-            if (rescale) {
+            for (int dt = 0; dt < kDTiles; ++dt)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) o[dt][e] *= corr;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) st[e] -= by;
+            seen = seen || moves;
+        }
+#pragma unroll
+        for (int s2 = 0; s2 < 2; ++s2) {
+            half8_t ph, pl;
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) {
+                float p_0 = __builtin_amdgcn_exp2f(st[8 * s2 + e]), p_1 = __builtin_amdgcn_exp2f(st[8 * s2 + e + 1]);
+                lsum += p_0 + p_1;
+                half2_t h;
+                if constexpr (kLo) h = split_pair(p_0, p_1, minus_one);
+                else h = half2_t{static_cast<half_t>(p_0), static_cast<half_t>(p_1)};
+                ph[e] = h[0];
+                ph[e + 1] = h[1];
+                if constexpr (kLo) {
+                    pl[e] = static_cast<half_t>(p_0);
+                    pl[e + 1] = static_cast<half_t>(p_1);
+                }
             }
 #pragma unroll
-            for (int s2 = 0; s2 < 2; ++s2) {
-                // the fragment: dimension 32 dt + r at the eight positions this lane supplies, one 2-byte read each
-                // (32 lanes read 64 consecutive bytes: every bank once per half wavefront)
-                const half_t* vcol = reinterpret_cast<const half_t*>(vt_tile) + (16 * s2 + 4 * g) * kTileRow + 32 * dt + r;
-                half8_t vf;
+            for (int dt = 0; dt < kDTiles; ++dt) {
+                union {
+                    short4_t part[2];
+                    half8_t whole;
+                } vf;
 #pragma unroll
-                for (int j = 0; j < 8; ++j) vf[j] = vcol[((j & 3) + 8 * (j >> 2)) * kTileRow];
-                o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, ph[s2], o[dt], 0, 0, 0);
-                if constexpr (kLo) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pl[s2], o[dt], 0, 0, 0);
+                for (int j = 0; j < 2; ++j)
+                    vf.part[j] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                        (__attribute__((address_space(3))) short4_t*)(stage + v_at[dt] + (16 * s2 + 8 * j) * kRowBytes));
+                o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf.whole, ph, o[dt], 0, 0, 0);
+                if constexpr (kLo) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf.whole, pl, o[dt], 0, 0, 0);
             }
         }
     }
-    // merge: wavefronts 1..3 hand their (maximum, sum, output) to wavefront 0, lane for lane
-    __shared__ float merge_o[3][kDTiles * 16][64];
-    __shared__ float merge_ms[3][2][64];
-    if (wave > 0) {
-        merge_ms[wave - 1][0][lane] = top;
-        merge_ms[wave - 1][1][lane] = lsum;
+    lsum = halves_sum(lsum);
+    if (!seen) top = -INFINITY;
+    if constexpr (kP > 1) {
+        // wavefronts of the later steps hand their (maximum, sum, output) to the first one of their rows, lane for lane
+        __syncthreads();  // (the stages are free)
+        float* merge = reinterpret_cast<float*>(att_lds);
+        constexpr int kPart = (kHs / 2 + 2) * 64;
+        if (wp > 0) {
+            float* mine = merge + ((wp - 1) * kR + wr) * kPart + lane;
+            mine[0] = top;
+            mine[64] = lsum;
+#pragma unroll
+            for (int dt = 0; dt < kDTiles; ++dt)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) mine[64 * (2 + dt * 16 + e)] = o[dt][e];
+        }
+        __syncthreads();
+        if (wp > 0) return;
+        float all_top = top;
+#pragma unroll
+        for (int w = 0; w < kP - 1; ++w) all_top = fmaxf(all_top, merge[(w * kR + wr) * kPart + lane]);
+        if (all_top == -INFINITY) all_top = 0.0f;  // (a row past the last token)
+        const float own = __builtin_amdgcn_exp2f(top - all_top);
+        lsum *= own;
 #pragma unroll
         for (int dt = 0; dt < kDTiles; ++dt)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) merge_o[wave - 1][dt * 16 + e][lane] = o[dt][e];
-    }
-    __syncthreads();
-    if (wave > 0) return;
-    float all_top = top;  // finite: block 0 is wavefront 0's and position 0 is in every row's range
+            for (int e = 0; e < 16; ++e) o[dt][e] *= own;
 #pragma unroll
-    for (int w = 0; w < 3; ++w) all_top = fmaxf(all_top, merge_ms[w][0][lane]);
-    const float own = exp_fast(top - all_top);
-    lsum *= own;
+        for (int w = 0; w < kP - 1; ++w) {
+            const float* theirs = merge + (w * kR + wr) * kPart + lane;
+            const float weight = __builtin_amdgcn_exp2f(theirs[0] - all_top);
+            lsum += theirs[64] * weight;
 #pragma unroll
-    for (int dt = 0; dt < kDTiles; ++dt)
+            for (int dt = 0; dt < kDTiles; ++dt)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) o[dt][e] *= own;
-#pragma unroll
-    for (int w = 0; w < 3; ++w) {
-        const float their_top = merge_ms[w][0][lane];
-        const float weight = (their_top == -INFINITY) ? 0.0f : exp_fast(their_top - all_top);
-        lsum += merge_ms[w][1][lane] * weight;
-#pragma unroll
-        for (int dt = 0; dt < kDTiles; ++dt)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) o[dt][e] += merge_o[w][dt * 16 + e][lane] * weight;
+                for (int e = 0; e < 16; ++e) o[dt][e] += theirs[64 * (2 + dt * 16 + e)] * weight;
+        }
     }
     if (valid) {
         const size_t base = static_cast<size_t>(my_tok) * dim + (kvh * gqa + my_head) * kHs;
@@ -1229,14 +1295,6 @@ namespace {
 enum { kBufTokens, kBufX, kBufQ, kBufK, kBufV, kBufPartials, kBufHi, kBufLo, kBufHi2, kBufLo2, kBufAll, kBufCount };
 static_assert(kBufCount <= static_cast<int>(sizeof(lpp_model::pf_buf) / sizeof(void*)), "lpp_model::pf_buf is too small");
 
-// Floats of kBufPartials: the partial products of the GEMM before (read by the kernel that follows it, so one area does
-// for all of a layer's), or the gate and up projections where those are not fused.
-size_t partial_floats(const lpp_model* m, int t_pad) {
-    const size_t t = static_cast<size_t>(t_pad), few = t < 256 ? t : 256;  // (small batches are cut along K the most)
-    const size_t pair = 2 * t * m->cfg.hidden_dim, ranges = 8 * few * (m->cfg.dim + 2 * m->kv_dim);
-    return pair > ranges ? pair : ranges;
-}
-
 const char* unsupported_reason(const lpp_model* m) {
     const lpp_config& c = m->cfg;
     if (c.weight_precision != LPP_WEIGHT_FP16) return "weights are not binary16";
@@ -1245,34 +1303,6 @@ const char* unsupported_reason(const lpp_model* m) {
     if (m->head_size != 64 && m->head_size != 128) return "head_size must be 64 or 128";
     if (m->gqa > pf::kMaxGqa) return "more than 8 query heads per KV head";
     return nullptr;
-}
-
-lpp_status ensure_scratch(lpp_model* m, int t_pad) {
-    if (m->pf_cap >= t_pad) return LPP_OK;
-    prefill_release(m);
-    const lpp_config& c = m->cfg;
-    const size_t t = static_cast<size_t>(t_pad);
-    const size_t widest = static_cast<size_t>(c.hidden_dim > c.dim ? c.hidden_dim : c.dim);
-    const size_t bytes[kBufAll] = {t * sizeof(int),
-                                   t * c.dim * sizeof(float),
-                                   t * c.dim * sizeof(float),
-                                   t * m->kv_dim * sizeof(float),
-                                   t * m->kv_dim * sizeof(float),
-                                   partial_floats(m, t_pad) * sizeof(float),
-                                   t * widest * sizeof(pf::half_t),
-                                   t * widest * sizeof(pf::half_t),
-                                   // the feed-forward activations, written while hi/lo are still being read
-                                   t * c.hidden_dim * sizeof(pf::half_t),
-                                   t * c.hidden_dim * sizeof(pf::half_t)};
-    size_t offset[kBufAll], total = 0;
-    for (int i = 0; i < kBufAll; ++i) {
-        offset[i] = total;
-        total += (bytes[i] + 255) / 256 * 256;
-    }
-    LPP_TRY(lpp_malloc(&m->pf_buf[kBufAll], total));
-    for (int i = 0; i < kBufAll; ++i) m->pf_buf[i] = static_cast<char*>(m->pf_buf[kBufAll]) + offset[i];
-    m->pf_cap = t_pad;
-    return LPP_OK;
 }
 
 // Y_i[t][f] (+)= sum_k W_i[f][k] * x[t][k] for up to three matrices W_i of n_i rows that share x.
@@ -1399,6 +1429,47 @@ Plan plan_gemm(int total_n, int K, int t_pad, int max_splits, bool lo, int row_s
         }
     }
     return best;
+}
+
+// Floats of kBufPartials that chunks of up to t_pad tokens need: the partial products of the GEMM before (read by the
+// kernel that follows it, so one area does for all of a layer's) -- at most eight of 256 tokens, or one tile of 128 x 128 per
+// compute unit (plan_gemm) -- or the gate and up projections where those are not fused.
+size_t partial_floats(const lpp_model* m, int t_pad) {
+    const size_t t = static_cast<size_t>(t_pad), few = t < 256 ? t : 256;
+    size_t most = 8 * few * (m->cfg.dim + 2 * m->kv_dim);
+    const size_t tiles = static_cast<size_t>(compute_units()) * 128 * 128, pair = 2 * t * m->cfg.hidden_dim;
+    if (t > 256 && tiles > most) most = tiles;
+    const bool fused = test_option(LPP_OPT_PREFILL_STAGED_GEMM) != 0 && test_option(LPP_OPT_PREFILL_FUSED_FFN) != 0;
+    return !fused && pair > most ? pair : most;
+}
+
+lpp_status ensure_scratch(lpp_model* m, int t_pad) {
+    const size_t room = partial_floats(m, t_pad);
+    if (m->pf_cap >= t_pad && m->pf_room >= room) return LPP_OK;
+    prefill_release(m);
+    const lpp_config& c = m->cfg;
+    const size_t t = static_cast<size_t>(t_pad);
+    const size_t bytes[kBufAll] = {t * sizeof(int),
+                                   t * c.dim * sizeof(float),
+                                   t * c.dim * sizeof(float),
+                                   t * m->kv_dim * sizeof(float),
+                                   t * m->kv_dim * sizeof(float),
+                                   room * sizeof(float),
+                                   t * c.dim * sizeof(pf::half_t),
+                                   t * c.dim * sizeof(pf::half_t),
+                                   // the feed-forward activations, written while hi/lo are still being read
+                                   t * c.hidden_dim * sizeof(pf::half_t),
+                                   t * c.hidden_dim * sizeof(pf::half_t)};
+    size_t offset[kBufAll], total = 0;
+    for (int i = 0; i < kBufAll; ++i) {
+        offset[i] = total;
+        total += (bytes[i] + 255) / 256 * 256;
+    }
+    LPP_TRY(lpp_malloc(&m->pf_buf[kBufAll], total));
+    for (int i = 0; i < kBufAll; ++i) m->pf_buf[i] = static_cast<char*>(m->pf_buf[kBufAll]) + offset[i];
+    m->pf_cap = t_pad;
+    m->pf_room = room;
+    return LPP_OK;
 }
 
 template <int kMode>
@@ -1566,6 +1637,32 @@ lpp_status gate_up_swiglu(const void* w1, const void* w3, int hidden, const pf::
     return launch_plan<2>(plan, job, s);
 }
 
+template <int kHs, bool kLo, int kR, int kP>
+lpp_status launch_attention_as(const lpp_model* m, const float* q, pf::half_t* hi, pf::half_t* lo, int layer, int pos0, int n, hipStream_t s) {
+    constexpr int kLds = pf::AttentionShape<kHs, kR, kP>::kLdsBytes;
+    static bool sized[64] = {};
+    LPP_TRY(size_lds(reinterpret_cast<const void*>(&pf::k_attention_mfma<kHs, kLo, kR, kP>), kLds, sized));
+    const int tokens = 32 * kR / m->gqa;
+    hipLaunchKernelGGL((pf::k_attention_mfma<kHs, kLo, kR, kP>), dim3(m->cfg.n_kv_heads, (n + tokens - 1) / tokens), dim3(64 * kR * kP), kLds, s, q,
+                       m->key_cache, m->value_cache, hi, lo, layer, pos0, m->cfg.dim, m->kv_dim, m->gqa, m->cfg.seq_len, n,
+                       compute_units() / m->cfg.n_kv_heads);
+    LPP_CHECK_LAUNCH("k_attention_mfma");
+    return LPP_OK;
+}
+// Up to a tile of 32 rows per compute unit the longest walk is what counts, and eight wavefronts share it.
+template <int kHs, bool kLo>
+lpp_status launch_attention(const lpp_model* m, const float* q, pf::half_t* hi, pf::half_t* lo, int layer, int pos0, int n, hipStream_t s) {
+    const int tokens = 32 / m->gqa, tiles = (n + tokens - 1) / tokens * m->cfg.n_kv_heads;
+    if (tiles <= compute_units()) return launch_attention_as<kHs, kLo, 1, kHs == 64 ? 8 : 4>(m, q, hi, lo, layer, pos0, n, s);
+    return launch_attention_as<kHs, kLo, 2, 2>(m, q, hi, lo, layer, pos0, n, s);
+}
+lpp_status attention(const lpp_model* m, const float* q, pf::half_t* hi, pf::half_t* lo, int layer, int pos0, int n, bool remainders,
+                     hipStream_t s) {
+    if (m->head_size == 64)
+        return remainders ? launch_attention<64, true>(m, q, hi, lo, layer, pos0, n, s) : launch_attention<64, false>(m, q, hi, lo, layer, pos0, n, s);
+    return remainders ? launch_attention<128, true>(m, q, hi, lo, layer, pos0, n, s) : launch_attention<128, false>(m, q, hi, lo, layer, pos0, n, s);
+}
+
 // One chunk: tokens[0..n) at positions pos0 .. pos0 + n - 1; n <= kChunk.
 lpp_status prefill_chunk(lpp_model* m, const int* tokens, int n, int pos0) {
     const lpp_config& c = m->cfg;
@@ -1591,7 +1688,7 @@ lpp_status prefill_chunk(lpp_model* m, const int* tokens, int n, int pos0) {
     };
     pf::half_t* hi2 = static_cast<pf::half_t*>(m->pf_buf[kBufHi2]);
     pf::half_t* lo2 = static_cast<pf::half_t*>(m->pf_buf[kBufLo2]);
-    const size_t room = partial_floats(m, t_pad);
+    const size_t room = m->pf_room;
     // LPP_PREFILL_EXACT: every product takes the activations as binary16 head + remainder.  LPP_PREFILL_FAST: the head
     // alone, in the staged kernels (what a GEMM sees of its input is then what the reference's own GPU GEMV sees,
     // matmul.cu:85-98; accumulation stays fp32).
@@ -1625,21 +1722,8 @@ lpp_status prefill_chunk(lpp_model* m, const int* tokens, int n, int pos0) {
         // (rows n .. t_pad of hi/lo are still the zeros k_norm_split wrote: the attention writes rows < n only)
         const bool matrix_cores = 32 % m->gqa == 0 && test_option(LPP_OPT_PREFILL_MFMA_ATTENTION) != 0;
         if (matrix_cores) {
-            const int tiles = (n + 32 / m->gqa - 1) / (32 / m->gqa);
-            const dim3 grid(tiles, c.n_kv_heads);
-#define LPP_PF_ATTENTION(HS, LO)                                                                                          \
-    hipLaunchKernelGGL((pf::k_attention_mfma<HS, LO>), grid, dim3(256), 0, s, q, m->key_cache, m->value_cache, hi, lo, l, pos0, \
-                       dim, kv, m->gqa, c.seq_len, n)
             // (the fast mode rounds q and the softmax weights to binary16 as it rounds every GEMM input)
-            if (hs == 64) {
-                if (!lean) LPP_PF_ATTENTION(64, true);
-                else LPP_PF_ATTENTION(64, false);
-            } else {
-                if (!lean) LPP_PF_ATTENTION(128, true);
-                else LPP_PF_ATTENTION(128, false);
-            }
-#undef LPP_PF_ATTENTION
-            LPP_CHECK_LAUNCH("k_attention_mfma");
+            LPP_TRY(attention(m, q, hi, lo, l, pos0, n, !lean, s));
         } else if (hs == 64)
             hipLaunchKernelGGL(pf::k_attention<8>, dim3((n + 3) / 4, c.n_kv_heads), dim3(256), 0, s, q, m->key_cache,
                                m->value_cache, hi, lo, l, pos0, dim, kv, hs, m->gqa, c.seq_len, n);
@@ -1675,6 +1759,7 @@ void prefill_release(lpp_model* m) {
     lpp_free(m->pf_buf[kBufAll]);
     for (void*& p : m->pf_buf) p = nullptr;
     m->pf_cap = 0;
+    m->pf_room = 0;
 }
 
 }  // namespace lpp
@@ -1705,10 +1790,11 @@ lpp_status lpp_prefill(lpp_model* m, const int* tokens, int n_tokens, int start_
     for (int t = 0; t < LPP_T_COUNT; ++t)
         if (!m->w_loaded[t]) return fail(LPP_ERR_STATE, "weight tensor %d has not been uploaded", t);
     LPP_TRY(lpp_prefill_supported(m));
-    for (int done = 0; done < n_tokens; done += pf::kChunk) {
-        const int n = n_tokens - done < pf::kChunk ? n_tokens - done : pf::kChunk;
-        LPP_TRY(prefill_chunk(m, tokens + done, n, start_pos + done));
-    }
+    // chunks of equal length, whole token tiles but for the last
+    const int chunks = (n_tokens + pf::kChunk - 1) / pf::kChunk;
+    const int each = chunks > 0 ? padded_tokens((n_tokens + chunks - 1) / chunks) : 0;
+    for (int done = 0; done < n_tokens; done += each)
+        LPP_TRY(prefill_chunk(m, tokens + done, n_tokens - done < each ? n_tokens - done : each, start_pos + done));
     return LPP_OK;
 }
 

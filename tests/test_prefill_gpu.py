@@ -408,6 +408,56 @@ def test_small_batches_around_the_edges_of_the_token_tiles(n, test_options):
     m.close()
 
 
+MANY_HEADS = {  # more than 256 tiles of 32 query rows from 257 (513) ids on: the attention's other workgroup shape
+    "hs64": Shape(2048, 256, 2, 32, 32, 512, 640, 10000.0, fp16=True, tied=True),
+    "hs128": Shape(2048, 256, 2, 16, 16, 512, 640, 10000.0, fp16=True, tied=True),
+    "hs64_gqa4": Shape(1024, 256, 2, 16, 4, 512, 640, 10000.0, fp16=True, tied=True),
+}
+
+
+@pytest.mark.parametrize("name,start,n", [("hs64", 0, 256), ("hs64", 0, 257), ("hs64", 95, 289), ("hs128", 0, 512), ("hs128", 33, 513),
+                                          ("hs64_gqa4", 31, 33), ("hs64_gqa4", 300, 1), ("hs64_gqa4", 64, 520)])
+def test_attention_on_the_matrix_cores_against_the_vector_kernel(name, start, n, test_options):
+    """Both workgroup shapes of the attention, whole and ragged tiles of rows and steps, behind a context and without: the
+    second layer's cache entries against those with the one-wavefront-per-token attention.  Queries and weights are
+    split exactly and summed in fp32 by both: within one binary16 step, or 2^-11 of the largest entry."""
+    shape = MANY_HEADS[name]
+    m = Model(shape)
+    m.load_synthetic(4)
+    ids = capi.synth_token_ids(start + n, 8, shape.vocab_size)
+    if start:
+        m.prefill(ids[:start], 0)
+    m.prefill(ids[start:], start)
+    k, v, kf, vf = caches(m, shape, start + n)
+    assert not kf[:, :, start + n:, :].any() and not vf[:, :, start + n:, :].any(), "slots beyond the prompt were written"
+    test_options(capi.OPT_PREFILL_MFMA_ATTENTION, 0)
+    m.prefill(ids[start:], start)
+    k0, v0, _, _ = caches(m, shape, start + n)
+    for x, y in ((k, k0), (v, v0)):
+        assert np.all(np.abs(x - y) <= np.maximum(np.abs(y) * 2.0 ** -9, np.abs(y).max() * 2.0 ** -11))
+    m.close()
+
+
+@pytest.mark.parametrize("n", [2048, 2049, 2500])
+def test_prompts_around_the_longest_batch(n):
+    """One batch, and two of equal length: the same cache as in calls of 500 ids, to one binary16 step."""
+    shape = Shape(256, 512, 2, 4, 2, 1024, 2600, 10000.0, fp16=True, tied=True)
+    a, b = Model(shape), Model(shape)
+    for m in (a, b):
+        m.load_synthetic(17)
+    ids = capi.synth_token_ids(n, 18, shape.vocab_size)
+    a.prefill(ids, 0)
+    for at in range(0, n, 500):
+        b.prefill(ids[at:at + 500], at)
+    ka, va, kf, vf = caches(a, shape, n)
+    kb, vb, _, _ = caches(b, shape, n)
+    for x, y in ((ka, kb), (va, vb)):
+        assert np.all(np.abs(x - y) <= np.maximum(np.abs(y) * 2.0 ** -9, np.abs(y).max() * 2.0 ** -11))
+    assert not kf[:, :, n:, :].any() and not vf[:, :, n:, :].any(), "slots beyond the prompt were written"
+    a.close()
+    b.close()
+
+
 def test_prefill_of_a_long_prompt_at_full_size():
     """Llama-3.2-1B shape with the long-context cache: 1500 prompt ids = three batches (512, 512, 476), the later
     ones attending to the earlier ones' cache entries; caches and the next step against prefill by decode."""
