@@ -3,9 +3,8 @@
 // Replaces cuda_gemv / gemv_f16_kernel / gemv_kernel / convert_f32_to_f16_kernel
 // (reference src/matmul.cu:9-161).  The reference launches one 256-thread block
 // per output row and, for binary16 weights, first casts x to binary16 and
-// accumulates in half2.  Here a wavefront owns a tile of rows, every lane keeps
-// kRows*kUnroll 16-byte weight loads in flight, x stays fp32 (staged once per
-// workgroup in LDS) and accumulation is fp32.
+// accumulates in half2.  Here every lane keeps kRows*kUnroll 16-byte weight loads
+// in flight, x stays fp32 and accumulation is fp32.
 #include "lpp_device.hpp"
 #include "lpp_internal.hpp"
 
@@ -50,6 +49,62 @@ __global__ __launch_bounds__(kGemvThreads) void gemv_rows_kernel(float* __restri
                 if (lane_id() == r) v = sums[r];
             out[row0 + lane_id()] = v;
         }
+    }
+}
+
+// A workgroup per kRows rows, whose columns are dealt out to its kWaves wavefronts in slices of 1 KiB (a row has at most
+// kWaves * kUnroll of them).  A matrix of some tens of megabytes is a few microseconds of traffic, so what counts is how
+// soon everything is requested: all of a wavefront's weights and its own part of x (straight into registers, no stage in
+// LDS and no barrier ahead of them) go out with the first instructions, and the wavefronts' sums meet in LDS at the end,
+// added in wavefront order.  Rows past the end are the last row again, columns past the end column 0 (not multiplied).
+// Launches back to back, other weights each time, against the kernel above: 8192 x 2048 binary16 9.2 -> 6.9 us,
+// 2048 x 8192 11.0 -> 7.2, 128256 x 2048 81 -> 71 (7.4 TB/s); fp32 2048 x 8192 16.0 -> 12.3.
+template <bool kF16, int kWaves, int kUnroll, int kRows>
+__global__ __launch_bounds__(kWaves* kWave) void gemv_slices_kernel(float* __restrict__ out, const float* __restrict__ x,
+                                                                    const char* __restrict__ w, int n, int d) {
+    constexpr int kPer = WTraits<kF16>::kPerLoad, kSlice = kWave * kPer;
+    __shared__ float part[kWaves][kRows];
+    const int lane = lane_id(), wave = wave_index();
+    const int row0 = static_cast<int>(blockIdx.x) * kRows;
+    const size_t row_bytes = static_cast<size_t>(d) * WTraits<kF16>::kBytes;
+    uintx4 wv[kUnroll][kRows];
+    floatx4 xv[kUnroll][kPer / 4];
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+        const int col = (wave + kWaves * u) * kSlice + lane * kPer, safe = col < d ? col : 0;
+#pragma unroll
+        for (int h = 0; h < kPer / 4; ++h) xv[u][h] = *reinterpret_cast<const floatx4*>(x + safe + 4 * h);
+#pragma unroll
+        for (int r = 0; r < kRows; ++r) {
+            const int row = row0 + r < n ? row0 + r : n - 1;
+            wv[u][r] = load16_stream(w + row * row_bytes + static_cast<size_t>(safe) * WTraits<kF16>::kBytes);
+        }
+    }
+    float acc[kRows];
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) acc[r] = 0.0f;
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+        if ((wave + kWaves * u) * kSlice + lane * kPer < d) {
+#pragma unroll
+            for (int r = 0; r < kRows; ++r) {
+                if constexpr (kF16) acc[r] = dot8(wv[u][r], xv[u][0], xv[u][1], acc[r]);
+                else acc[r] = dot4(wv[u][r], xv[u][0], acc[r]);
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+        const float sum = wave_sum(acc[r]);
+        if (lane == r) part[wave][r] = sum;
+    }
+    __syncthreads();
+    const int r = static_cast<int>(threadIdx.x);
+    if (r < kRows && row0 + r < n) {
+        float v = part[0][r];
+#pragma unroll
+        for (int z = 1; z < kWaves; ++z) v += part[z][r];
+        out[row0 + r] = v;
     }
 }
 
@@ -98,6 +153,14 @@ lpp_status launch_rows(float* out, const float* x, const void* w, int n, int d) 
     return LPP_OK;
 }
 
+template <bool kF16, int kWaves, int kUnroll, int kRows>
+lpp_status launch_slices(float* out, const float* x, const void* w, int n, int d) {
+    hipLaunchKernelGGL((gemv_slices_kernel<kF16, kWaves, kUnroll, kRows>), dim3((n + kRows - 1) / kRows), dim3(kWaves * kWave), 0,
+                       stream(), out, x, static_cast<const char*>(w), n, d);
+    LPP_CHECK_LAUNCH("gemv_slices_kernel");
+    return LPP_OK;
+}
+
 template <bool kF16>
 lpp_status gemv_dispatch(float* out, const float* x, const void* w, int n, int d) {
     constexpr int kPer = WTraits<kF16>::kPerLoad;
@@ -112,9 +175,20 @@ lpp_status gemv_dispatch(float* out, const float* x, const void* w, int n, int d
         LPP_CHECK_LAUNCH("gemv_generic_kernel");
         return LPP_OK;
     }
-    // Tile choice: enough wave tiles to cover every SIMD several times over for
-    // small matrices, more rows per wave (more loads in flight) for large ones.
+    // Rows of 3 to 32 slices: columns dealt out to a workgroup's wavefronts, two rows of up to four slices or four of
+    // more (one to sixteen timed: fewer leave the wavefronts too little to request, more too few workgroups; 2048 x 8192
+    // by 1, 2, 4, 8 rows: 9.0, 7.6, 7.2, 9.7 us).  Shorter rows leave wavefronts without a slice, longer ones need more
+    // registers than a wavefront has, and x is read 16 bytes at a time: those go to the wavefront-per-tile kernel
+    // (768 x 288 fp32: 4.5 us either way, all of it the launch).
     const int chunks = (d + kWave * kPer - 1) / (kWave * kPer);
+    if (chunks > 2 && chunks <= 32 && reinterpret_cast<uintptr_t>(x) % 16 == 0) {
+        if (chunks <= 4) return launch_slices<kF16, 4, 1, 2>(out, x, w, n, d);
+        if (chunks <= 8) return launch_slices<kF16, 8, 1, 4>(out, x, w, n, d);
+        if (chunks <= 16) return launch_slices<kF16, 8, 2, 4>(out, x, w, n, d);
+        return launch_slices<kF16, 16, 2, 4>(out, x, w, n, d);
+    }
+    // Enough wave tiles to cover every SIMD several times over for small matrices, more rows per wave (more loads in
+    // flight) for large ones.
     const long waves_wanted = static_cast<long>(compute_units()) * 8;
     if (chunks >= 8) {
         // Long rows: one or two rows, four chunks in flight each.

@@ -106,6 +106,27 @@ def test_gemv_random(lib, n, d, fp16):
     assert np.max(np.abs(got - want)) <= 2e-3 * np.max(np.abs(want)) + 1e-30
 
 
+@pytest.mark.parametrize("n,d", [(1, 1024), (1, 1032), (3, 2048), (2, 2056), (5, 4096), (7, 4104), (6, 8192), (3, 8200), (5, 16384), (257, 1544)])
+@pytest.mark.parametrize("fp16", [True, False])
+def test_gemv_around_the_slices_of_a_row(lib, n, d, fp16):
+    """Rows of one slice more and less than each workgroup shape takes, ragged last slices and rows; x aligned to 16 bytes and
+    not (two kernels), an infinite weight in column 0 of one row, and a word behind the output that stays as it was."""
+    rng = np.random.default_rng(n + d)
+    x = rng.standard_normal(d).astype(F)
+    w = (rng.standard_normal((n, d)) * 0.02).astype(np.float16 if fp16 else F)
+    w[n - 1, 0] = np.inf
+    x[0] = 1.5
+    exact = w.astype(np.float64) @ x.astype(np.float64)
+    bound = 16 * np.finfo(F).eps * (np.abs(w[: n - 1].astype(np.float64)) @ np.abs(x.astype(np.float64)))
+    dw = DB.from_numpy(w.view(np.uint16) if fp16 else w)
+    for shift in (0, 1):
+        dx, dout = DB.from_numpy(np.concatenate([np.zeros(shift, F), x])), DB.from_numpy(np.full(n + 1, 7.0, F))
+        capi.check(lib.lpp_gemv(dout.ptr, dx.at(4 * shift), dw.ptr, None, n, d, capi.WEIGHT_FP16 if fp16 else capi.WEIGHT_FP32))
+        got = dout.to_numpy(F, n + 1)
+        assert np.all(np.abs(got[: n - 1] - exact[: n - 1]) <= bound + 1e-30)
+        assert got[n - 1] == np.inf and got[n] == 7.0
+
+
 def test_gemv_lm_head_full_size(lib):
     """128256 x 2048 binary16: the largest single launch of the decode step."""
     n, d = 128256, 2048
