@@ -192,7 +192,7 @@ def bench_prefill(args, model, shape, name, cus) -> int:
                vs_baseline=None,
                dtype="f32 accumulate over f16 weights, activations rounded to f16 at each GEMM input" if fast
                else "f32 accumulate over f16 weights, activations split hi+lo", data="synthetic",
-               config=dict(workload=args.config, prompt_ids=n, chunk=512, prefill_mode=args.prefill_mode),
+               config=dict(workload=args.config, prompt_ids=n, chunk=2048, prefill_mode=args.prefill_mode),
                roofline=dict(bound="mfma", achieved=round(tflops, 1), peak=MFMA_F16_PEAK_TFLOPS, unit="TFLOP/s",
                              frac=round(tflops / MFMA_F16_PEAK_TFLOPS, 4), traffic=None,
                              note="algorithmic flops of what the cache depends on (the last layer stops at its K/V "

@@ -358,9 +358,9 @@ lpp_status lpp_run(lpp_model *m, const int *prompt, int n_prompt, int steps, flo
  * start_pos + n_tokens - 1, all layers: what those decode steps leave behind for later
  * steps to read (K and V rounded to binary16, model.cpp:171-176), within one binary16
  * step of it (the GEMMs sum in another order than the decode GEMVs); no logits,
- * no sampling.  The prompt goes through each layer as one batch of up to 512 tokens:
- * GEMMs on the matrix cores, every weight read once per batch.  Needs binary16
- * weights, dim / kv_dim / hidden_dim multiples of 128, head_size 64 or 128, at most 8
+ * no sampling.  The prompt goes through each layer as batches of up to 2048 tokens (512 where
+ * device memory has no room for the buffers of more): GEMMs on the matrix cores, every
+ * weight read once per batch.  Needs binary16 weights, dim / kv_dim / hidden_dim multiples of 128, head_size 64 or 128, at most 8
  * query heads per KV head: lpp_prefill_supported says whether the model qualifies
  * (LPP_ERR_UNSUPPORTED and the reason in lpp_last_error otherwise).  `tokens` is host
  * memory.  Synchronous. */

@@ -5,7 +5,7 @@
 // a time and dropping what the sampler returns (src/main.cpp:163-180), which reads
 // every weight once per prompt token.  Here the prompt's tokens go through each
 // layer together, so the matrix products are GEMMs on the matrix cores
-// (v_mfma_f32_32x32x16_f16) and every weight is read once per chunk of up to 512
+// (v_mfma_f32_32x32x16_f16) and every weight is read once per chunk of up to 2048
 // tokens.  What a prefill leaves behind is exactly what the decode loop reads
 // later: K and V of the prompt positions, rounded to binary16 as the cache store
 // rounds them (model.cpp:171-176, kernels.cuh:34).  The classifier and the sampler
@@ -32,7 +32,13 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int kTileTokens = 128;    // token rows of a workgroup's output tile
 constexpr int kTileFeatures = 128;  // weight rows of it
-constexpr int kChunk = 512;         // prompt tokens per pass over the weights, at most
+// Prompt tokens per pass over the weights, at most.  What a longer chunk saves is the ends of launches: 512 tokens give the
+// 1B shape's W1+W3 one tile per compute unit, whose first data and epilogue (12 of 69 us) overlap nothing, and its other
+// products less than that; norm, RoPE and attention are then launches of 5 to 15 us.  1B shape, exact mode, chunks of at
+// most 512 / 1024 / 2048 / 3072: 2011 ids 10.9 / 9.1 / 8.5 / 8.5 ms, 6000 ids 37.7 / 30.4 / 28.5 / 29.9; fast mode, 2011
+// ids: 8.4 / 6.6 / 5.9 / 5.9.  8B shape, 2011 ids: 60.6 / 57.3 / 53.6 ms.
+constexpr int kChunk = 2048;
+constexpr int kSmallChunk = 512;  // where device memory has no room for the buffers of more
 constexpr int kMaxGqa = 8;          // query heads per KV head the attention kernel keeps in registers
 
 // ---------------------------------------------------------------------------
@@ -1790,9 +1796,14 @@ lpp_status lpp_prefill(lpp_model* m, const int* tokens, int n_tokens, int start_
     for (int t = 0; t < LPP_T_COUNT; ++t)
         if (!m->w_loaded[t]) return fail(LPP_ERR_STATE, "weight tensor %d has not been uploaded", t);
     LPP_TRY(lpp_prefill_supported(m));
-    // chunks of equal length, whole token tiles but for the last
-    const int chunks = (n_tokens + pf::kChunk - 1) / pf::kChunk;
-    const int each = chunks > 0 ? padded_tokens((n_tokens + chunks - 1) / chunks) : 0;
+    // Full chunks and a rest: 2048 tokens are the length that fills the device's rounds best.  (1B shape, exact: one chunk of
+    // 2048 takes 8.6 ms, of 640 3.7, of 1280 or 1408 6.0 or 6.5, so 2600 ids are better cut 2048 + 552 than into halves.)
+    int each = n_tokens < pf::kChunk ? n_tokens : pf::kChunk;
+    if (each > pf::kSmallChunk) {
+        const lpp_status st = ensure_scratch(m, padded_tokens(each));
+        if (st == LPP_ERR_OOM) each = pf::kSmallChunk;
+        else if (st != LPP_OK) return st;
+    }
     for (int done = 0; done < n_tokens; done += each)
         LPP_TRY(prefill_chunk(m, tokens + done, n_tokens - done < each ? n_tokens - done : each, start_pos + done));
     return LPP_OK;

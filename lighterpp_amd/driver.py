@@ -36,7 +36,7 @@ def main(argv=None) -> int:
     ap.add_argument("--seed", type=int, default=1, help="seed of the per-step uniform draws")
     ap.add_argument("--path", default="persistent", choices=list(PATHS))
     ap.add_argument("--batched-prefill", action="store_true",
-                    help="fill the cache for the prompt in one pass per 512 ids (lpp_run_batched_prefill) instead of by decode")
+                    help="fill the cache for the prompt in one pass per 2048 ids (lpp_run_batched_prefill) instead of by decode")
     args = ap.parse_args(argv)
 
     capi.check(capi.load().lpp_init(0))

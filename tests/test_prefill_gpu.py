@@ -132,7 +132,7 @@ def test_prefill_leaves_what_decode_leaves(name, variant, test_options):
 
 
 def test_prefill_in_chunks_and_from_a_later_position():
-    """600 prompt ids = one full chunk of 512 and a ragged one; then a second call that starts
+    """600 prompt ids, a ragged batch; then a second call that starts
     where the first ended (its attention reads the first call's cache entries)."""
     shape = Shape(256, 512, 2, 4, 2, 1024, 1024, 500000.0, fp16=True, tied=True)
     a, b = Model(shape), Model(shape)
@@ -440,7 +440,7 @@ def test_attention_on_the_matrix_cores_against_the_vector_kernel(name, start, n,
 
 @pytest.mark.parametrize("n", [2048, 2049, 2500])
 def test_prompts_around_the_longest_batch(n):
-    """One batch, and two of equal length: the same cache as in calls of 500 ids, to one binary16 step."""
+    """One batch of 2048, and one with a rest behind it: the same cache as in calls of 500 ids, to one binary16 step."""
     shape = Shape(256, 512, 2, 4, 2, 1024, 2600, 10000.0, fp16=True, tied=True)
     a, b = Model(shape), Model(shape)
     for m in (a, b):
@@ -459,8 +459,8 @@ def test_prompts_around_the_longest_batch(n):
 
 
 def test_prefill_of_a_long_prompt_at_full_size():
-    """Llama-3.2-1B shape with the long-context cache: 1500 prompt ids = three batches (512, 512, 476), the later
-    ones attending to the earlier ones' cache entries; caches and the next step against prefill by decode."""
+    """Llama-3.2-1B shape with the long-context cache: 1500 prompt ids in one batch (twelve
+    token tiles); caches and the next step against prefill by decode."""
     shape = CONFIGS["c4_llama32_1b_longctx_fp16"]
     n = 1500
     prompt = capi.synth_token_ids(n, 14, shape.vocab_size)
