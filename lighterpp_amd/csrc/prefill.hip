@@ -1385,7 +1385,10 @@ int padded_tokens(int n) {
 }
 
 // More than 256 tokens: k_gemm_pipe, 256 rows a tile where that leaves no compute unit without a workgroup (always for
-// a pair), otherwise 128 and K in as many ranges as the device takes at once.
+// a pair), otherwise 128 and K in as many ranges as the device takes at once.  In the exact mode also 256 where tiles of
+// 128 rows are more than the device takes at once: a second round of them costs more than compute units left idle, the
+// wider tile being a third more bytes from L2 and not twice as many (8B shape, 1280 ids: 38.2 -> 36.9 ms, 1792: 51.0 ->
+// 49.4).  In the fast mode it is half as many again, and the narrow tiles' rounds stay the faster ones.
 //
 // Up to 256 tokens the choice is made by what a launch of each would take.  A workgroup of k_gemm_few is paced by its
 // bytes from L2 into LDS (57 bytes a nanosecond), one of k_gemm_pipe by its bytes (88) and its MFMA clocks; a last round
@@ -1406,7 +1409,8 @@ Plan plan_gemm(int total_n, int K, int t_pad, int max_splits, bool lo, int row_s
     const bool wide_allowed = row_step % 256 == 0 && test_option(LPP_OPT_PREFILL_WIDE_TILES) != 0;
     if (t_pad > 256) {
         const int token_tiles = t_pad / 128;
-        if (pair || (wide_allowed && total_n / 256 * token_tiles >= compute_units())) best.fi = 4;
+        const bool wide = total_n / 256 * token_tiles >= compute_units() || (lo && total_n / 128 * token_tiles > compute_units());
+        if (pair || (wide_allowed && wide)) best.fi = 4;
         while (2 * best.splits <= max_splits && total_n / best.tile_rows() * token_tiles * best.splits * 2 <= compute_units() &&
                K % (64 * 2 * best.splits) == 0 && K / (2 * best.splits) >= 512)
             best.splits *= 2;

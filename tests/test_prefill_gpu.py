@@ -44,7 +44,8 @@ def rel_err(got, want):
 
 
 @pytest.mark.parametrize("n,k,t", [(128, 32, 128), (256, 2048, 128), (384, 1024, 256), (128, 8192, 512), (16384, 256, 512),
-                                   (256, 64, 128), (16384, 64, 512)])  # the last two: one and two trips through the staged kernels
+                                   (256, 64, 128), (16384, 64, 512),  # one and two trips through the staged kernels
+                                   (12288, 128, 384)])  # 288 tiles of 128 rows: 144 of 256 instead
 @pytest.mark.parametrize("accumulate", [0, 1])
 def test_gemm_against_float64(lib, n, k, t, accumulate):
     rng = np.random.default_rng(1000 * n + k + t)
