@@ -381,6 +381,7 @@ struct PipeJob {
     int k_len;  // columns a workgroup multiplies: split z covers [z * k_len, (z + 1) * k_len) and writes y + z * split_stride
     size_t split_stride;
     int feature_tiles, token_tiles, groups;  // groups = feature_tiles * splits
+    int band;                                // k_gemm_pipe: token tiles a die's workgroups take at a time; divides token_tiles
     half_t* out_hi;                          // kMode 2: [tokens][out_ld]
     half_t* out_lo;
     int out_ld;
@@ -434,9 +435,13 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
     // Workgroups are handed to the eight dies in turn: those that share a weight tile (same features
     // and columns, other tokens) get numbers that are equal modulo 8, so the tile crosses one die's L2.
     const int id = static_cast<int>(blockIdx.x), die = id & 7, within = id >> 3;
-    const int group = (within / job.token_tiles) * 8 + die;
+    // Of many token tiles, job.band at a time: a die's 32 compute units then hold band x 32 / band tiles, whose operands come
+    // from beyond its L2 once for all of them -- at 16 token tiles, all at a time, two weight tiles and 16 activation
+    // tiles; four at a time, eight and four, a third fewer bytes.  (band divides token_tiles.)
+    const int per_band = ((job.groups + 7) >> 3) * job.band, band = within / per_band, in_band = within - band * per_band;
+    const int group = (in_band / job.band) * 8 + die;
     if (group >= job.groups) return;
-    const int token_tile = within % job.token_tiles;
+    const int token_tile = band * job.band + in_band % job.band;
     const int tile_all = group % job.feature_tiles, split = group / job.feature_tiles;
     const int which = tile_all >= job.first_tile[2] ? 2 : (tile_all >= job.first_tile[1] ? 1 : 0);
     const int tile_x = tile_all - (which == 2 ? job.first_tile[2] : (which == 1 ? job.first_tile[1] : 0));
@@ -1482,8 +1487,21 @@ lpp_status ensure_scratch(lpp_model* m, int t_pad) {
     return LPP_OK;
 }
 
+// Token tiles of k_gemm_pipe that a die's workgroups take at a time (PipeJob::band): four or the next larger divisor, bands of
+// different lengths being slower than none (1280 ids in 4 + 4 + 2 tiles, 8B shape, fast mode: 24.5 -> 25.0 ms).  2048 ids,
+// fast mode: 1B shape 5.81 -> 5.47 ms, 8B 37.6 -> 36.0, TinyLlama 6.70 -> 6.27; exact mode, paced by its MFMAs and LDS:
+// 8B 53.8 -> 53.2, TinyLlama 9.53 -> 9.39, and up to 1408 ids between 2.5 % faster and 0.9 % slower, so not there.
+int band_of(int token_tiles, bool lo) {
+    if (token_tiles <= 4 || (lo && token_tiles < 12)) return token_tiles;
+    int band = 4;
+    while (token_tiles % band != 0) ++band;
+    return band;
+}
+
 template <int kMode>
-lpp_status launch_plan(const Plan& p, const pf::PipeJob& job, hipStream_t s) {
+lpp_status launch_plan(const Plan& p, const pf::PipeJob& job_in, hipStream_t s) {
+    pf::PipeJob job = job_in;
+    job.band = band_of(job.token_tiles, job.xl != nullptr);
     if (!p.few) {
         if (p.fi == 4) return launch_pipe<4, 2, kMode, 32>(job, s);
         return launch_pipe<2, 2, kMode>(job, s);
