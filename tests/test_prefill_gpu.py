@@ -20,6 +20,7 @@ import pytest
 import oracle_binding as ob
 from lighterpp_amd import CONFIGS, Model, Shape, capi, synth_tensor
 from lighterpp_amd.capi import DeviceBuffer as DB
+from lighterpp_amd.model import MATRIX_TENSORS
 
 pytestmark = pytest.mark.gpu
 F = np.float32
@@ -489,3 +490,87 @@ def test_prefill_of_a_long_prompt_at_full_size():
     assert rel_err(b.buffer(capi.B_LOGITS), logits_a) <= LOGIT_TOL
     assert tok_a == tok_b
     b.close()
+
+
+@pytest.mark.parametrize("head_size", [64, 128])
+@pytest.mark.parametrize("n", [46, 2200])  # a walk shared by eight (four) wavefronts, and 64 rows to a workgroup
+def test_attention_keeps_the_queries_remainders(head_size, n):
+    """Two positions whose scores are equal in exact arithmetic, with values +1 and -1: the attention's output is
+    tanh((score_0 - score_1) / 2) of the scores as computed, zero but for their error.  Queries are small and keys large, so
+    that a bit lost from a query's remainder shows; every query is a sum of a binary16 head and a binary16 remainder.
+
+    Layer 0: a token owns four coordinates of x, normalized to a power of two (the query tokens' gains 2^-13 instead of 1),
+    so q, k and v are exact sums of weights.  Head dimensions in the first half, which RoPE turns, are zero.  Query = (q, q / 4),
+    key of position 0 = (k, 0), of position 1 = (0, 4 k), all others 0 (weights below e^-100).  Wo brings one output
+    dimension of each head to a free coordinate, and layer 1's Wk copies that into the cache.
+
+    Bound: a score is an fp32 sum of head_size / 4 products of which no partial sum exceeds S; with an addition each for head
+    and remainder that is head_size / 2 roundings of 2^-24 S, and a few more for the scale and the reference, for either of the
+    pair.  (Measured: 0; with log2(e) / sqrt(head_size) multiplied into the query before the split, 5 and 3 times the bound.)"""
+    quarter = head_size // 4
+    dim, heads, kv_heads, vocab = 4 * head_size, 4, 2, 64
+    kv = kv_heads * head_size
+    shape = Shape(dim, 128, 2, heads, kv_heads, vocab, n + 8, 1e30, fp16=True, tied=True)
+    rng = np.random.default_rng(head_size)
+    queries = 40
+    emb = np.zeros((vocab, dim), F)
+    for t in range(queries + 2):
+        emb[t, 4 * t:4 * t + 4] = 1024.0
+    if dim == 512:  # (four more that nothing reads: the root of the mean square is 128 in either dim)
+        emb[:queries + 2, 448:452] = 1024.0
+    xn = 8.0
+    gain = np.ones((2, dim), F)
+    gain[0, 8:4 * (queries + 2)] = 2.0 ** -13
+    wq, wk, wv, wo = (np.zeros((2, r, dim), np.float16) for r in (dim, kv, kv, dim))
+    # tokens 0 and 1: the pair of positions; 2 ..: queries
+    sign = rng.choice([-1.0, 1.0], (kv_heads, quarter))
+    k = (sign * rng.uniform(9000.0, 14000.0, (kv_heads, quarter)) / xn).astype(np.float16)  # key / xn
+    half = head_size // 2
+    for g in range(kv_heads):
+        wk[0, g * head_size + half:g * head_size + half + quarter, 0] = k[g]
+        wk[0, g * head_size + half + quarter:(g + 1) * head_size, 4] = 4.0 * k[g]
+        wv[0, g * head_size:(g + 1) * head_size, 0] = 1.0 / xn
+        wv[0, g * head_size:(g + 1) * head_size, 4] = -1.0 / xn
+    largest = 0.0
+    for h in range(heads):
+        g = h // 2
+        # multiples of 2^-22 of 16 bits: a quarter of one is a multiple of 2^-24, as is its remainder from binary16
+        q = rng.integers(33600, 58700, (queries, quarter)) * 2.0 ** -22 * sign[g]
+        largest = max(largest, float(np.max(np.abs(q) @ np.abs(xn * k[g].astype(np.float64)))))
+        for part, rows in ((q, slice(h * head_size + half, h * head_size + half + quarter)),
+                           (q / 4, slice(h * head_size + half + quarter, (h + 1) * head_size))):
+            w = part * 2.0 ** 13 / xn
+            top = w.astype(np.float16)
+            rest = (w - top.astype(np.float64)).astype(np.float16)
+            assert np.array_equal(top.astype(np.float64) + rest.astype(np.float64), w)
+            for t in range(queries):
+                wq[0, rows, 4 * (t + 2)] = top[t]
+                wq[0, rows, 4 * (t + 2) + 1] = rest[t]
+        wo[0, dim - 4 + h, h * head_size] = 64.0
+        wk[1, half + h, dim - 4 + h] = 128.0
+    m = Model(shape)
+    w = {t: np.zeros(shape.tensor_shape(t), np.uint16) for t in MATRIX_TENSORS if t != capi.T_WCLS}
+    w[capi.T_WQ], w[capi.T_WK], w[capi.T_WV], w[capi.T_WO] = (a.view(np.uint16) for a in (wq, wk, wv, wo))
+    w[capi.T_TOKEN_EMBEDDING] = emb
+    w[capi.T_RMS_ATT] = gain
+    w[capi.T_RMS_FFN] = np.ones((2, dim), F)
+    w[capi.T_RMS_FINAL] = np.ones(dim, F)
+    for t, a in w.items():
+        m.upload(t, a.reshape(shape.tensor_shape(t)))
+    m.tie_classifier()
+    ids = np.concatenate([[0, 1], 2 + np.arange(n - 2) % queries]).astype(np.int32)
+    m.prefill(ids, 0)
+    kc, vc, _, _ = caches(m, shape, n)
+    # the construction: keys and values of layer 0 as meant
+    for g in range(kv_heads):
+        assert np.array_equal(kc[0, g, 0, half:half + quarter], (xn * k[g].astype(np.float64)).astype(F))
+        assert np.array_equal(kc[0, g, 1, half + quarter:], (4 * xn * k[g].astype(np.float64)).astype(F))
+    assert (vc[0, :, 0] == 1.0).all() and (vc[0, :, 1] == -1.0).all()
+    assert not kc[0, :, 2:].any()
+    # o of every head and position >= 2: x takes 64 o, the norm xn / 1024, layer 1's Wk 128
+    o = kc[1, 0, 2:, half:half + heads] / (64.0 * 128.0 * xn / 1024.0)
+    off = np.max(np.abs(2.0 * np.arctanh(o.astype(np.float64))))
+    bound = 2 * (head_size / 2 + 4) * 2.0 ** -24 * largest / np.sqrt(head_size)
+    print(f"head size {head_size}, {n} ids: scores of {largest / np.sqrt(head_size):.0f} differ by {off:.1e}, bound {bound:.1e}", flush=True)
+    assert off <= bound
+    m.close()
