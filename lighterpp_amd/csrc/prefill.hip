@@ -989,8 +989,13 @@ __global__ __launch_bounds__(256) void k_attention(const float* __restrict__ q, 
 // reads them), a step ahead.  The 16-byte pieces of a row are stored in an order that keeps the reads free of bank
 // conflicts (the address each lane requests makes it): K fragments are 16 bytes a lane from 32 rows; V fragments are
 // transposed on the way out (ds_read_b64_tr_b16: 16 lanes read a tile of 4 positions x 16 dimensions and every lane gets
-// the 4 positions of one dimension).  Rows past the tile's last position are the last row again (finite, weight zero).
-
+// the 4 positions of one dimension).  Rows past the workgroup's last position are the last row again.
+//
+// A weight of zero does not keep an infinite value out of the output, so a wavefront must not multiply the V rows of its
+// neighbour's positions.  It has them in one step, the one its own last position ends in, and takes that step's V rows
+// from a copy in LDS with the neighbour's rows cleared.  (Cleared in the fragments, behind a branch in every step or by
+// masks, the registers and clocks cost every step: 1B shape, 2000 ids behind 3000, 10.28 -> 10.47 and 10.57 ms exact,
+// 6.93 -> 7.11 and 7.29 fast; with the copy 10.06 -> 10.05 and 6.86 -> 6.93.)
 //
 // What bounds it: a step of 32 positions is 512 MFMA clocks and about as many of the vector units (sixteen v_exp_f32 are
 // 256 of them), and one wavefront does them one after the other, so what counts is wavefronts per SIMD: the stages are
@@ -1009,9 +1014,11 @@ struct AttentionShape {
     static constexpr int kRowBytes = 2 * kHs, kPieces = kHs / 8;
     static constexpr int kHalfBytes = kStep * kRowBytes, kStageBytes = 2 * kHalfBytes;  // K rows, then V rows
     static constexpr int kLoads = kStageBytes / 1024 / kR;                              // requests per wavefront and step
-    static constexpr int kStages = kHs == 64 && kP == 2 ? 3 : 2;  // 2 x 2: 48 / 64 KiB, at least two workgroups to a compute unit
+    static constexpr int kStages = kHs == 64 && kP == 2 ? 3 : 2;  // 2 x 2: 52 / 72 KiB, at least two workgroups to a compute unit
     static constexpr int kMergeBytes = (kP - 1) * kR * (kHs / 2 + 2) * 64 * 4;
-    static constexpr int kLdsBytes = kP * kStages * kStageBytes > kMergeBytes ? kP * kStages * kStageBytes : kMergeBytes;
+    static constexpr int kOwnValues = kP * kStages * kStageBytes;  // behind the stages: V rows of a step, for each row of wavefronts but the last
+    static constexpr int kStepBytes = kOwnValues + (kR - 1) * kHalfBytes;
+    static constexpr int kLdsBytes = kStepBytes > kMergeBytes ? kStepBytes : kMergeBytes;
     static_assert(kLdsBytes <= 160 * 1024, "LDS of a workgroup");
 };
 
@@ -1139,7 +1146,7 @@ __global__ __launch_bounds__(64 * kR * kP, 2) void k_attention_mfma(const float*
 #pragma unroll
         for (int dt = 0; dt < kDTiles; ++dt) {
             const int piece = 4 * dt + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
-            v_at[dt] = kHalfBytes + row * kRowBytes + 16 * (piece ^ (kHs == 64 ? 4 * ((row >> 1) & 1) : 4 * (row & 3))) + 8 * (lane & 1);
+            v_at[dt] = row * kRowBytes + 16 * (piece ^ (kHs == 64 ? 4 * ((row >> 1) & 1) : 4 * (row & 3))) + 8 * (lane & 1);
         }
     }
 
@@ -1153,6 +1160,19 @@ __global__ __launch_bounds__(64 * kR * kP, 2) void k_attention_mfma(const float*
         if (turn + kStages - 1 < turns) request(turn + kStages - 1);
         if (p0 >= wave_limit) continue;
         const char* stage = stages + (turn % kStages) * kStageBytes;
+        const char* values = stage + kHalfBytes;
+        if constexpr (kR > 1) {
+            if (p0 + kStep > wave_limit && wave_limit < limit) {  // (uniform; one wavefront of its row, one step)
+                char* own = att_lds + Shape::kOwnValues + wr * kHalfBytes;
+#pragma unroll
+                for (int i = 0; i < kLoadsPerHalf; ++i) {
+                    uintx4 v = *reinterpret_cast<const uintx4*>(values + 1024 * i + 16 * lane);
+                    if (p0 + i * kRowsPerLoad + lane / kPieces >= wave_limit) v = uintx4{0u, 0u, 0u, 0u};
+                    *reinterpret_cast<uintx4*>(own + 1024 * i + 16 * lane) = v;
+                }
+                values = own;
+            }
+        }
         floatx16 st;
 #pragma unroll
         for (int e = 0; e < 16; ++e) st[e] = 0.0f;
@@ -1213,7 +1233,7 @@ __global__ __launch_bounds__(64 * kR * kP, 2) void k_attention_mfma(const float*
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
                     vf.part[j] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                        (__attribute__((address_space(3))) short4_t*)(stage + v_at[dt] + (16 * s2 + 8 * j) * kRowBytes));
+                        (__attribute__((address_space(3))) short4_t*)(values + v_at[dt] + (16 * s2 + 8 * j) * kRowBytes));
                 o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf.whole, ph, o[dt], 0, 0, 0);
                 if constexpr (kLo) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf.whole, pl, o[dt], 0, 0, 0);
             }

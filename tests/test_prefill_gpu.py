@@ -574,3 +574,44 @@ def test_attention_keeps_the_queries_remainders(head_size, n):
     print(f"head size {head_size}, {n} ids: scores of {largest / np.sqrt(head_size):.0f} differ by {off:.1e}, bound {bound:.1e}", flush=True)
     assert off <= bound
     m.close()
+
+
+@pytest.mark.parametrize("fast", [False, True])
+@pytest.mark.parametrize("name,start,n,at", [("hs64_gqa4", 0, 40, 12), ("hs64_gqa4", 0, 520, 12), ("hs64_gqa4", 300, 40, 39), ("hs64", 5, 289, 40),
+                                             ("hs64", 5, 545, 40), ("hs128", 33, 513, 50)])
+def test_an_infinite_value_stays_with_the_positions_that_attend_to_it(name, start, n, at, fast, test_options):
+    """One prompt id whose value vectors overflow binary16 in the first layer: the second layer's cache entries of the
+    positions before it, as far as other wavefronts of the attention work on them (32 / gqa tokens each), against those with
+    the one-wavefront-per-token attention, which reads no later position.  Every workgroup shape, heads of 64 and 128."""
+    shape = MANY_HEADS[name]
+    m = Model(shape)
+    m.load_synthetic(6)
+    emb, wv = synth_tensor(shape, capi.T_TOKEN_EMBEDDING, 6), synth_tensor(shape, capi.T_WV, 6)
+    emb[:, 0] = 0.0
+    emb[7] = 0.0
+    emb[7, 0] = 1.0
+    wv[0, :, 0] = np.float16(60000.0).view(np.uint16)
+    m.upload(capi.T_TOKEN_EMBEDDING, emb)
+    m.upload(capi.T_WV, wv)
+    m.tie_classifier()
+    ids = capi.synth_token_ids(start + n, 9, shape.vocab_size)
+    ids[ids == 7] = 8
+    ids[start + at] = 7
+    m.set_prefill_mode(capi.PREFILL_FAST if fast else capi.PREFILL_EXACT)
+    per_wavefront = 32 // (shape.n_heads // shape.n_kv_heads)
+    upto = start + at // per_wavefront * per_wavefront
+    got = []
+    for matrix_cores in (1, 0):
+        test_options(capi.OPT_PREFILL_MFMA_ATTENTION, matrix_cores)
+        if start:
+            m.prefill(ids[:start], 0)
+        m.prefill(ids[start:], start)
+        k, v, _, _ = caches(m, shape, start + n)
+        assert np.isinf(v[0, :, start + at]).all() and np.isfinite(v[0, :, :start + at]).all()
+        got.append((k[1, :, :upto], v[1, :, :upto]))
+    # (the fast mode's attention rounds queries and weights to binary16 on the matrix cores only)
+    own, share = (2.0 ** -9, 2.0 ** -11) if not fast else (0.0, 2.0 ** -6)
+    for x, y in zip(*got):
+        assert np.isfinite(x).all()
+        assert np.all(np.abs(x - y) <= np.maximum(np.abs(y) * own, np.abs(y).max() * share))
+    m.close()
