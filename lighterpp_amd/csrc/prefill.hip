@@ -972,7 +972,7 @@ __global__ __launch_bounds__(256) void k_attention(const float* __restrict__ q, 
 // A wavefront owns 32 query rows = (32 / gqa) consecutive tokens x the gqa query heads of one KV head, and walks the
 // context in steps of 32 positions.  A workgroup is kR x kP such wavefronts: kR take neighbouring rows and share every
 // step's K and V rows, kP take the steps in turn and merge their running (maximum, sum, output) at the end.  2 x 2 where
-// that makes workgroups enough; a batch of few rows takes 1 x 8 (heads of 128: 1 x 4, for want of LDS).  Per step:
+// that makes workgroups enough; a batch of few rows takes 1 x 8 or 1 x 4 (heads of 128: 1 x 4, for want of LDS).  Per step:
 //   S^T[pos][row] = sum_d K[pos][d] Q[row][d]     A = K rows, B = Q (head + remainder, in registers for the whole walk)
 //   online softmax: in the result a LANE holds one query row (its column) and 16 of the 32 positions, the lane 32 further
 //                   on the other 16 -- maximum and rescaling are per lane, with one exchange between the two halves of
@@ -1703,11 +1703,19 @@ lpp_status launch_attention_as(const lpp_model* m, const float* q, pf::half_t* h
     LPP_CHECK_LAUNCH("k_attention_mfma");
     return LPP_OK;
 }
-// Up to a tile of 32 rows per compute unit the longest walk is what counts, and eight wavefronts share it.
+// Up to a tile of 32 rows per compute unit the longest walk is what counts, and eight wavefronts share it (heads of 128:
+// four).  Up to two tiles, heads of 64: 2 x 2 would leave up to half of the compute units without a workgroup and walk the
+// context in halves, 1 x 8 would be a second round of workgroups for most of them; 1 x 4 it is.  1B shape, exact mode,
+// 257 ids behind 0 / 3000 / 7000, 1 x 8: 2.15 / 2.55 / 3.06 ms, 2 x 2: 2.10 / 2.67 / 3.42, 1 x 4: 2.09 / 2.46 / 2.91; 512 ids
+// behind 7000: 3.71, 4.02, 3.62.  Above, the rows two wavefronts share count for more: 1024 ids, fast mode, behind 0: 2 x 2
+// 3.13, 1 x 4 3.16; 640 ids behind 7000, exact, is the other way round (5.43, 5.12).  Heads of 128: 2 x 2 is the
+// faster one throughout (six layers of the 8B shape's width, 257 ids behind 14000: 2.30 against 2.39; 1024: 4.30 against 4.86).
 template <int kHs, bool kLo>
 lpp_status launch_attention(const lpp_model* m, const float* q, pf::half_t* hi, pf::half_t* lo, int layer, int pos0, int n, hipStream_t s) {
     const int tokens = 32 / m->gqa, tiles = (n + tokens - 1) / tokens * m->cfg.n_kv_heads;
     if (tiles <= compute_units()) return launch_attention_as<kHs, kLo, 1, kHs == 64 ? 8 : 4>(m, q, hi, lo, layer, pos0, n, s);
+    if constexpr (kHs == 64)
+        if (tiles <= 2 * compute_units()) return launch_attention_as<kHs, kLo, 1, 4>(m, q, hi, lo, layer, pos0, n, s);
     return launch_attention_as<kHs, kLo, 2, 2>(m, q, hi, lo, layer, pos0, n, s);
 }
 lpp_status attention(const lpp_model* m, const float* q, pf::half_t* hi, pf::half_t* lo, int layer, int pos0, int n, bool remainders,
