@@ -494,7 +494,9 @@ enum lpp_test_option {
     LPP_OPT_PREFILL_MFMA_ATTENTION = 9, /* [1] matrix-core attention; 0: one wavefront per token and KV head            */
     LPP_OPT_DECODE_CALIBRATE = 10,      /* [1] LPP_PATH_PERSISTENT: before a model's first token, trace two tokens and deal the
                                                hidden units out by how fast each XCD got through the gate/up phase; 0: evenly  */
-    LPP_OPT_COUNT = 11
+    LPP_OPT_PREFILL_ROOM = 11,          /* [0] n > 0: device memory is reported to have room for the buffers of batches of up to
+                                               n tokens only; n < 0: the same, but it shows when they are allocated          */
+    LPP_OPT_COUNT = 12
 };
 lpp_status lpp_set_test_option(int option, int value);
 lpp_status lpp_get_test_option(int option, int *value);

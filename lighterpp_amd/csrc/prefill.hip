@@ -1484,32 +1484,68 @@ size_t partial_floats(const lpp_model* m, int t_pad) {
     return !fused && pair > most ? pair : most;
 }
 
-lpp_status ensure_scratch(lpp_model* m, int t_pad) {
-    const size_t room = partial_floats(m, t_pad);
-    if (m->pf_cap >= t_pad && m->pf_room >= room) return LPP_OK;
-    prefill_release(m);
+struct ScratchLayout {
+    size_t offset[kBufAll];
+    size_t total;
+    size_t room;  // floats of kBufPartials
+};
+ScratchLayout scratch_layout(const lpp_model* m, int t_pad) {
     const lpp_config& c = m->cfg;
     const size_t t = static_cast<size_t>(t_pad);
+    ScratchLayout s = {};
+    s.room = partial_floats(m, t_pad);
     const size_t bytes[kBufAll] = {t * sizeof(int),
                                    t * c.dim * sizeof(float),
                                    t * c.dim * sizeof(float),
                                    t * m->kv_dim * sizeof(float),
                                    t * m->kv_dim * sizeof(float),
-                                   room * sizeof(float),
+                                   s.room * sizeof(float),
                                    t * c.dim * sizeof(pf::half_t),
                                    t * c.dim * sizeof(pf::half_t),
                                    // the feed-forward activations, written while hi/lo are still being read
                                    t * c.hidden_dim * sizeof(pf::half_t),
                                    t * c.hidden_dim * sizeof(pf::half_t)};
-    size_t offset[kBufAll], total = 0;
     for (int i = 0; i < kBufAll; ++i) {
-        offset[i] = total;
-        total += (bytes[i] + 255) / 256 * 256;
+        s.offset[i] = s.total;
+        s.total += (bytes[i] + 255) / 256 * 256;
     }
-    LPP_TRY(lpp_malloc(&m->pf_buf[kBufAll], total));
-    for (int i = 0; i < kBufAll; ++i) m->pf_buf[i] = static_cast<char*>(m->pf_buf[kBufAll]) + offset[i];
+    return s;
+}
+
+bool scratch_held(const lpp_model* m, const ScratchLayout& s, int t_pad) { return m->pf_cap >= t_pad && m->pf_room >= s.room; }
+
+// Whether device memory has room for the buffers of t_pad tokens in the place of those the model holds: asked before those
+// are given up, so that a model that lives with the smaller batch keeps its buffers from call to call.
+bool scratch_fits(const lpp_model* m, int t_pad) {
+    const ScratchLayout s = scratch_layout(m, t_pad);
+    const int forced = test_option(LPP_OPT_PREFILL_ROOM);
+    if (forced > 0 && t_pad > forced) return false;
+    if (scratch_held(m, s, t_pad)) return true;
+    size_t free_bytes = 0, all_bytes = 0;
+    if (hipMemGetInfo(&free_bytes, &all_bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;  // (the allocation will say)
+    }
+    const size_t held = m->pf_cap > 0 ? scratch_layout(m, m->pf_cap).total : 0;
+    return s.total <= free_bytes + held;
+}
+
+// `quiet`: an allocation that fails leaves lpp_last_error as it is (the caller has another way to go).
+lpp_status ensure_scratch(lpp_model* m, int t_pad, bool quiet = false) {
+    const ScratchLayout s = scratch_layout(m, t_pad);
+    if (scratch_held(m, s, t_pad)) return LPP_OK;
+    prefill_release(m);
+    const int forced = test_option(LPP_OPT_PREFILL_ROOM);
+    hipError_t e = hipErrorOutOfMemory;
+    if (forced >= 0 || t_pad <= -forced) e = hipMalloc(&m->pf_buf[kBufAll], s.total);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        m->pf_buf[kBufAll] = nullptr;
+        return quiet ? LPP_ERR_OOM : fail(LPP_ERR_OOM, "prefill buffers: hipMalloc(%zu) failed: %s", s.total, hipGetErrorString(e));
+    }
+    for (int i = 0; i < kBufAll; ++i) m->pf_buf[i] = static_cast<char*>(m->pf_buf[kBufAll]) + s.offset[i];
     m->pf_cap = t_pad;
-    m->pf_room = room;
+    m->pf_room = s.room;
     return LPP_OK;
 }
 
@@ -1856,7 +1892,8 @@ lpp_status lpp_prefill(lpp_model* m, const int* tokens, int n_tokens, int start_
     // 2048 takes 8.6 ms, of 640 3.7, of 1280 or 1408 6.0 or 6.5, so 2600 ids are better cut 2048 + 552 than into halves.)
     int each = n_tokens < pf::kChunk ? n_tokens : pf::kChunk;
     if (each > pf::kSmallChunk) {
-        const lpp_status st = ensure_scratch(m, padded_tokens(each));
+        const int t_pad = padded_tokens(each);
+        const lpp_status st = scratch_fits(m, t_pad) ? ensure_scratch(m, t_pad, true) : LPP_ERR_OOM;
         if (st == LPP_ERR_OOM) each = pf::kSmallChunk;
         else if (st != LPP_OK) return st;
     }

@@ -616,3 +616,43 @@ def test_an_infinite_value_stays_with_the_positions_that_attend_to_it(name, star
         assert np.isfinite(x).all()
         assert np.all(np.abs(x - y) <= np.maximum(np.abs(y) * own, np.abs(y).max() * share))
     m.close()
+
+
+@pytest.mark.parametrize("room", [512, -512])
+def test_prefill_where_memory_has_no_room_for_the_longest_batch(lib, room, test_options):
+    """Device memory reported as too small for the buffers of more than 512 tokens, ahead of the allocation or by it: the same
+    cache as from calls of 512 ids, bit for bit, twice in a row (the second call finds the buffers of the first), and
+    lpp_last_error as it was before a call that succeeded.  Then with room: one batch again."""
+    shape = Shape(256, 512, 2, 4, 2, 1024, 2600, 10000.0, fp16=True, tied=True)
+    a, b, c = Model(shape), Model(shape), Model(shape)
+    for m in (a, b, c):
+        m.load_synthetic(19)
+    n = 1300
+    ids, more = capi.synth_token_ids(n, 20, shape.vocab_size), capi.synth_token_ids(n, 21, shape.vocab_size)
+    for at in range(0, n, 512):
+        b.prefill(ids[at:at + 512], at)
+    c.prefill(ids, 0)
+    c.prefill(more, n)
+    assert lib.lpp_prefill(a.handle, None, 1, 0) == capi.LPP_ERR_INVALID_ARG
+    said = lib.lpp_last_error()
+    test_options(capi.OPT_PREFILL_ROOM, room)
+    a.prefill(ids, 0)
+    ka, va, kf, vf = caches(a, shape, n)
+    kb, vb, _, _ = caches(b, shape, n)
+    assert np.array_equal(ka, kb) and np.array_equal(va, vb)
+    assert not kf[:, :, n:, :].any() and not vf[:, :, n:, :].any(), "slots beyond the prompt were written"
+    for at in range(0, n, 512):
+        b.prefill(more[at:at + 512], n + at)
+    a.prefill(more, n)
+    ka, va, _, _ = caches(a, shape, 2 * n)
+    kb, vb, _, _ = caches(b, shape, 2 * n)
+    assert np.array_equal(ka, kb) and np.array_equal(va, vb)
+    assert lib.lpp_last_error() == said
+    test_options(capi.OPT_PREFILL_ROOM, 0)
+    a.prefill(ids, 0)
+    a.prefill(more, n)
+    ka, va, _, _ = caches(a, shape, 2 * n)
+    kc, vc, _, _ = caches(c, shape, 2 * n)
+    assert np.array_equal(ka, kc) and np.array_equal(va, vc)
+    for m in (a, b, c):
+        m.close()
