@@ -1512,29 +1512,36 @@ ScratchLayout scratch_layout(const lpp_model* m, int t_pad) {
     return s;
 }
 
-bool scratch_held(const lpp_model* m, const ScratchLayout& s, int t_pad) { return m->pf_cap >= t_pad && m->pf_room >= s.room; }
+// Tokens the buffers are made for where t_pad are needed: whole steps of 128 up to 512, of 512 beyond, so that prompts
+// that grow from call to call seldom cost an allocation and the device-wide wait for the buffers given up.
+int scratch_tokens(int t_pad) {
+    const int step = t_pad <= pf::kSmallChunk ? pf::kTileTokens : pf::kSmallChunk;
+    return (t_pad + step - 1) / step * step;
+}
+
+bool scratch_held(const lpp_model* m, int t_pad) { return m->pf_cap >= t_pad && m->pf_room >= partial_floats(m, t_pad); }
 
 // Whether device memory has room for the buffers of t_pad tokens in the place of those the model holds: asked before those
 // are given up, so that a model that lives with the smaller batch keeps its buffers from call to call.
 bool scratch_fits(const lpp_model* m, int t_pad) {
-    const ScratchLayout s = scratch_layout(m, t_pad);
     const int forced = test_option(LPP_OPT_PREFILL_ROOM);
     if (forced > 0 && t_pad > forced) return false;
-    if (scratch_held(m, s, t_pad)) return true;
+    if (scratch_held(m, t_pad)) return true;
     size_t free_bytes = 0, all_bytes = 0;
     if (hipMemGetInfo(&free_bytes, &all_bytes) != hipSuccess) {
         (void)hipGetLastError();
         return true;  // (the allocation will say)
     }
     const size_t held = m->pf_cap > 0 ? scratch_layout(m, m->pf_cap).total : 0;
-    return s.total <= free_bytes + held;
+    return scratch_layout(m, scratch_tokens(t_pad)).total <= free_bytes + held;
 }
 
 // `quiet`: an allocation that fails leaves lpp_last_error as it is (the caller has another way to go).
 lpp_status ensure_scratch(lpp_model* m, int t_pad, bool quiet = false) {
-    const ScratchLayout s = scratch_layout(m, t_pad);
-    if (scratch_held(m, s, t_pad)) return LPP_OK;
+    if (scratch_held(m, t_pad)) return LPP_OK;
     prefill_release(m);
+    const int tokens = scratch_tokens(t_pad);
+    const ScratchLayout s = scratch_layout(m, tokens);
     const int forced = test_option(LPP_OPT_PREFILL_ROOM);
     hipError_t e = hipErrorOutOfMemory;
     if (forced >= 0 || t_pad <= -forced) e = hipMalloc(&m->pf_buf[kBufAll], s.total);
@@ -1544,7 +1551,7 @@ lpp_status ensure_scratch(lpp_model* m, int t_pad, bool quiet = false) {
         return quiet ? LPP_ERR_OOM : fail(LPP_ERR_OOM, "prefill buffers: hipMalloc(%zu) failed: %s", s.total, hipGetErrorString(e));
     }
     for (int i = 0; i < kBufAll; ++i) m->pf_buf[i] = static_cast<char*>(m->pf_buf[kBufAll]) + s.offset[i];
-    m->pf_cap = t_pad;
+    m->pf_cap = tokens;
     m->pf_room = s.room;
     return LPP_OK;
 }

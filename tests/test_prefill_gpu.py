@@ -656,3 +656,24 @@ def test_prefill_where_memory_has_no_room_for_the_longest_batch(lib, room, test_
     assert np.array_equal(ka, kc) and np.array_equal(va, vc)
     for m in (a, b, c):
         m.close()
+
+
+def test_prompts_that_grow_keep_the_buffers(lib):
+    """Prompts of 20, 50, 90, 128 ids, then of 600, 700, 1000: device memory in use moves with the first of either only."""
+    import ctypes as C
+    hip = C.CDLL("libamdhip64.so")  # (the runtime the library is linked against)
+
+    def free_bytes():
+        free, total = C.c_size_t(0), C.c_size_t(0)
+        assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    m = Model(Shape(2048, 5632, 2, 32, 4, 1024, 1024, 10000.0, fp16=True, tied=True))
+    m.load_synthetic(22)
+    for lengths in ((20, 50, 90, 128), (600, 700, 1000)):
+        seen = []
+        for n in lengths:
+            m.prefill(capi.synth_token_ids(n, 23, 1024), 0)
+            seen.append(free_bytes())
+        assert len(set(seen)) == 1, seen
+    m.close()
