@@ -1395,10 +1395,6 @@ lpp_status launch_few_as(const pf::PipeJob& job, hipStream_t s) {
     LPP_CHECK_LAUNCH("k_gemm_few");
     return LPP_OK;
 }
-template <int kFi, int kTj, int kMode>
-lpp_status launch_few(const pf::PipeJob& job, hipStream_t s) {
-    return job.xl != nullptr ? launch_few_as<kFi, kTj, kMode, true>(job, s) : launch_few_as<kFi, kTj, kMode, false>(job, s);
-}
 
 // How a product is laid out on the device: what a workgroup's tile is and in how many ranges K is cut.
 struct Plan {
@@ -1426,16 +1422,20 @@ int padded_tokens(int n) {
 // of workgroups that does not fill the device counts almost whole; no launch is faster than its weights at 3.9 TB/s;
 // every partial product of a cut K is written (2.5 TB/s, in many short runs) and read (5 TB/s) once more.  The constants
 // are a fit to 1100 timed launches (ten weight matrices of the TinyLlama, 1B and 8B shapes, 32 to 2048 tokens, both
-// modes, every tile below): 14 % rms, and the launch picked is 2.2 % slower than the fastest one on average.
+// modes, every tile of the list): 14 % rms, and the launch picked is 2.2 % slower than the fastest one on average.
 //
 // `max_splits`: ranges K may be cut into.  `row_step`: every matrix is a whole number of row_step rows.  `pair`: W1 and W3
 // side by side in a tile (total_n counts both).
 Plan plan_gemm(int total_n, int K, int t_pad, int max_splits, bool lo, int row_step, bool pair) {
+    // `exact`, `fast`: the modes in which the model picks the tile at 256 compute units, n to 300000 and K to 32768 (one of
+    // 32 x 128, timed for the fit as well, in neither).  launch_plan has the kernels of this list.
     static constexpr struct {
         bool few;
         int fi, tj;
-    } kTiles[] = {{true, 1, 1}, {true, 1, 2}, {true, 1, 3}, {true, 1, 4}, {true, 2, 1}, {true, 2, 2}, {true, 2, 3}, {true, 2, 4},
-                  {true, 4, 1}, {true, 4, 2}, {false, 2, 2}, {false, 4, 2}};
+        bool exact, fast;
+    } kTiles[] = {{true, 1, 1, true, true}, {true, 1, 2, false, true}, {true, 1, 3, false, true}, {true, 2, 1, true, true},
+                  {true, 2, 2, true, true}, {true, 2, 3, true, true},  {true, 2, 4, false, true}, {true, 4, 1, true, false},
+                  {true, 4, 2, true, false}, {false, 2, 2, true, true}, {false, 4, 2, true, true}};
     Plan best = {false, 2, 2, 1};
     const bool wide_allowed = row_step % 256 == 0 && test_option(LPP_OPT_PREFILL_WIDE_TILES) != 0;
     if (t_pad > 256) {
@@ -1451,6 +1451,7 @@ Plan plan_gemm(int total_n, int K, int t_pad, int max_splits, bool lo, int row_s
     for (const auto& t : kTiles) {
         const Plan p = {t.few, t.fi, t.tj, 1};
         const int rows = p.tile_rows(), tokens = p.tile_tokens();
+        if (!(lo ? t.exact : t.fast)) continue;
         if (row_step % rows != 0 || t_pad % tokens != 0 || (pair && t.fi == 1)) continue;
         if (!t.few && t.fi == 4 && !wide_allowed) continue;
         for (int splits = 1; splits <= max_splits; splits *= 2) {
@@ -1575,24 +1576,20 @@ lpp_status launch_plan(const Plan& p, const pf::PipeJob& job_in, hipStream_t s) 
         if (p.fi == 4) return launch_pipe<4, 2, kMode, 32>(job, s);
         return launch_pipe<2, 2, kMode>(job, s);
     }
-    if (p.fi == 4) return p.tj == 1 ? launch_few<4, 1, kMode>(job, s) : launch_few<4, 2, kMode>(job, s);
-    if (p.fi == 2) {
-        switch (p.tj) {
-            case 1: return launch_few<2, 1, kMode>(job, s);
-            case 2: return launch_few<2, 2, kMode>(job, s);
-            case 3: return launch_few<2, 3, kMode>(job, s);
-            default: return launch_few<2, 4, kMode>(job, s);
-        }
+    const bool lo = job.xl != nullptr;
+    const int tile = 10 * p.fi + p.tj;
+    if (lo && tile == 41) return launch_few_as<4, 1, kMode, true>(job, s);
+    if (lo && tile == 42) return launch_few_as<4, 2, kMode, true>(job, s);
+    if (tile == 21) return lo ? launch_few_as<2, 1, kMode, true>(job, s) : launch_few_as<2, 1, kMode, false>(job, s);
+    if (tile == 22) return lo ? launch_few_as<2, 2, kMode, true>(job, s) : launch_few_as<2, 2, kMode, false>(job, s);
+    if (tile == 23) return lo ? launch_few_as<2, 3, kMode, true>(job, s) : launch_few_as<2, 3, kMode, false>(job, s);
+    if (!lo && tile == 24) return launch_few_as<2, 4, kMode, false>(job, s);
+    if constexpr (kMode != 2) {  // (a pair has as many rows of either matrix in a tile)
+        if (tile == 11) return lo ? launch_few_as<1, 1, kMode, true>(job, s) : launch_few_as<1, 1, kMode, false>(job, s);
+        if (!lo && tile == 12) return launch_few_as<1, 2, kMode, false>(job, s);
+        if (!lo && tile == 13) return launch_few_as<1, 3, kMode, false>(job, s);
     }
-    if constexpr (kMode != 2) {
-        switch (p.tj) {
-            case 1: return launch_few<1, 1, kMode>(job, s);
-            case 2: return launch_few<1, 2, kMode>(job, s);
-            case 3: return launch_few<1, 3, kMode>(job, s);
-            default: return launch_few<1, 4, kMode>(job, s);
-        }
-    }
-    return fail(LPP_ERR_STATE, "prefill GEMM: no kernel for a pair of matrices in one row tile");
+    return fail(LPP_ERR_STATE, "prefill GEMM: no kernel for a tile of %d x %d", p.tile_rows(), p.tile_tokens());
 }
 
 // `partials` (optional, partial_floats long): room for the partial products of a split K.  A product
@@ -1972,17 +1969,12 @@ namespace {
 int g_setup_state[kMaxDevices] = {};
 char g_setup_message[kMaxDevices][256] = {};
 
-// (every tile plan_gemm may give whole tiles of 128 tokens)
+// (every tile of k_gemm_few that plan_gemm may give the exact mode for 128 or 256 tokens)
 template <int kMode>
 lpp_status size_few_for() {
     LPP_TRY((size_few<1, 1, kMode, true>()));
-    LPP_TRY((size_few<1, 2, kMode, true>()));
-    LPP_TRY((size_few<1, 3, kMode, true>()));
-    LPP_TRY((size_few<1, 4, kMode, true>()));
     LPP_TRY((size_few<2, 1, kMode, true>()));
     LPP_TRY((size_few<2, 2, kMode, true>()));
-    LPP_TRY((size_few<2, 3, kMode, true>()));
-    LPP_TRY((size_few<2, 4, kMode, true>()));
     LPP_TRY((size_few<4, 1, kMode, true>()));
     return size_few<4, 2, kMode, true>();
 }
