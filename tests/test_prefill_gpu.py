@@ -441,6 +441,41 @@ def test_attention_on_the_matrix_cores_against_the_vector_kernel(name, start, n,
     m.close()
 
 
+FAST_SHAPES = {
+    "tinyllama": Shape(2048, 5632, 2, 32, 4, 1024, 2112, 10000.0, fp16=True, tied=True),
+    "wide": Shape(4096, 8192, 2, 32, 8, 1024, 160, 10000.0, fp16=True, tied=True),
+    **MANY_HEADS,
+}
+
+
+@pytest.mark.parametrize("name,start,n", [*(("tinyllama", 0, n) for n in (1, 33, 65, 96, 97, 128, 129, 257, 385, 640, 2011, 2048)), ("tinyllama", 95, 1100),
+                                          ("wide", 0, 64), ("wide", 0, 96), ("wide", 0, 97), ("wide", 0, 128), ("hs64", 95, 256),
+                                          ("hs64", 95, 257), ("hs64", 95, 513), ("hs128", 33, 512), ("hs128", 33, 513), ("hs64_gqa4", 64, 520)])
+def test_fast_mode_against_the_exact_one(name, start, n):
+    """The kernels without remainders: every token tile and weight tile they have, token tiles in bands (640 ids and more), every
+    workgroup shape of the attention, behind a context and without.  The second layer's cache entries against the exact
+    mode's.  Between them are the roundings of six inputs (norm, query, weights, attention's output, norm, SwiGLU) and of
+    layer 1's norm to binary16, 2^-11 each at most: the 2-norm of the difference is held to 2^-9 of the result's, every entry to
+    2^-6 of the largest."""
+    shape = FAST_SHAPES[name]
+    m = Model(shape)
+    m.load_synthetic(12)
+    ids = capi.synth_token_ids(start + n, 13, shape.vocab_size)
+    if start:
+        m.prefill(ids[:start], 0)
+    m.prefill(ids[start:], start)
+    k0, v0, _, _ = caches(m, shape, start + n)
+    m.set_prefill_mode(capi.PREFILL_FAST)
+    m.prefill(ids[start:], start)
+    k, v, kf, vf = caches(m, shape, start + n)
+    assert not kf[:, :, start + n:, :].any() and not vf[:, :, start + n:, :].any(), "slots beyond the prompt were written"
+    for what, x, y in (("K", k[1], k0[1]), ("V", v[1], v0[1])):
+        rel, most = np.linalg.norm(x - y) / np.linalg.norm(y), np.max(np.abs(x - y)) / np.abs(y).max()
+        print(f"{name} {n} ids behind {start}, {what}: {rel:.1e} in the 2-norm, {most:.1e} of the largest entry", flush=True)
+        assert rel <= 2.0 ** -9 and most <= 2.0 ** -6
+    m.close()
+
+
 @pytest.mark.parametrize("n", [2048, 2049, 2500])
 def test_prompts_around_the_longest_batch(n):
     """One batch of 2048, and one with a rest behind it: the same cache as in calls of 500 ids, to one binary16 step."""
@@ -461,11 +496,11 @@ def test_prompts_around_the_longest_batch(n):
     b.close()
 
 
-def test_prefill_of_a_long_prompt_at_full_size():
-    """Llama-3.2-1B shape with the long-context cache: 1500 prompt ids in one batch (twelve
-    token tiles); caches and the next step against prefill by decode."""
+@pytest.mark.parametrize("n", [1500, 4400])
+def test_prefill_of_a_long_prompt_at_full_size(n):
+    """Llama-3.2-1B shape with the long-context cache: 1500 prompt ids in one batch (twelve token tiles), 4400 in three (2048, 2048,
+    304), the later ones attending to the earlier ones' cache entries; caches and the next step against prefill by decode."""
     shape = CONFIGS["c4_llama32_1b_longctx_fp16"]
-    n = 1500
     prompt = capi.synth_token_ids(n, 14, shape.vocab_size)
     a = Model(shape)
     a.load_synthetic(1)
@@ -494,7 +529,7 @@ def test_prefill_of_a_long_prompt_at_full_size():
 
 
 @pytest.mark.parametrize("head_size", [64, 128])
-@pytest.mark.parametrize("n", [46, 2200])  # a walk shared by eight (four) wavefronts, and 64 rows to a workgroup
+@pytest.mark.parametrize("n", [46, 700, 1100])  # heads of 64: a walk shared by eight wavefronts, by four, and 64 rows to a workgroup
 def test_attention_keeps_the_queries_remainders(head_size, n):
     """Two positions whose scores are equal in exact arithmetic, with values +1 and -1: the attention's output is
     tanh((score_0 - score_1) / 2) of the scores as computed, zero but for their error.  Queries are small and keys large, so
@@ -509,7 +544,9 @@ def test_attention_keeps_the_queries_remainders(head_size, n):
     and remainder that is head_size / 2 roundings of 2^-24 S, and a few more for the scale and the reference, for either of the
     pair.  (Measured: 0; with log2(e) / sqrt(head_size) multiplied into the query before the split, 5 and 3 times the bound.)"""
     quarter = head_size // 4
-    dim, heads, kv_heads, vocab = 4 * head_size, 4, 2, 64
+    kv_heads, vocab = 8, 64
+    heads = 2 * kv_heads
+    dim = heads * head_size
     kv = kv_heads * head_size
     shape = Shape(dim, 128, 2, heads, kv_heads, vocab, n + 8, 1e30, fp16=True, tied=True)
     rng = np.random.default_rng(head_size)
@@ -517,8 +554,7 @@ def test_attention_keeps_the_queries_remainders(head_size, n):
     emb = np.zeros((vocab, dim), F)
     for t in range(queries + 2):
         emb[t, 4 * t:4 * t + 4] = 1024.0
-    if dim == 512:  # (four more that nothing reads: the root of the mean square is 128 in either dim)
-        emb[:queries + 2, 448:452] = 1024.0
+    emb[:queries + 2, 192:192 + dim // 64 - 4] = 1024.0  # (nothing reads these: the root of the mean square is 128 in either dim)
     xn = 8.0
     gain = np.ones((2, dim), F)
     gain[0, 8:4 * (queries + 2)] = 2.0 ** -13
@@ -547,8 +583,8 @@ def test_attention_keeps_the_queries_remainders(head_size, n):
             for t in range(queries):
                 wq[0, rows, 4 * (t + 2)] = top[t]
                 wq[0, rows, 4 * (t + 2) + 1] = rest[t]
-        wo[0, dim - 4 + h, h * head_size] = 64.0
-        wk[1, half + h, dim - 4 + h] = 128.0
+        wo[0, dim - heads + h, h * head_size] = 64.0
+        wk[1, half + h, dim - heads + h] = 128.0
     m = Model(shape)
     w = {t: np.zeros(shape.tensor_shape(t), np.uint16) for t in MATRIX_TENSORS if t != capi.T_WCLS}
     w[capi.T_WQ], w[capi.T_WK], w[capi.T_WV], w[capi.T_WO] = (a.view(np.uint16) for a in (wq, wk, wv, wo))
