@@ -197,8 +197,10 @@ lpp_status run_loop(lpp_model* m, const int* prompt, int n_prompt, int steps, fl
     int pos = 0;
     int n_out = 0;
     // 1. prefill, main.cpp:163-180.  Batched: the cache entries of all but the last prompt id in one
-    //    pass per 512 ids; what the decode steps would have sampled is what the reference drops.
-    //    (a batch costs about as much as five decode steps at the 1B shape: short prompts stay with decode)
+    //    pass per 2048 ids; what the decode steps would have sampled is what the reference drops.
+    //    (The line lies where a batch cost five decode steps and a margin.  A batch of up to 32 ids now costs one and a half to
+    //    two -- TinyLlama shape 1.23 ms, of 0.61 a step, 1B 0.90 of 0.60, 8B 4.04 of 2.85 -- so that three ids would pay;
+    //    prompts below the line keep the decode loop's own bits, as they always have.)
     constexpr int kShortestBatchedPrompt = 8;
     if (batched && n_prompt - 1 >= kShortestBatchedPrompt && lpp_prefill_supported(m) == LPP_OK) {
         for (int i = 0; i < n_prompt - 1; ++i) push(prompt[i]);
