@@ -147,6 +147,13 @@ struct Tagged {
     unsigned spin_limit;
     int trace_stride;  // timeline: 0 = workgroup 0 only; else every workgroup writes its own block of this many words
     const int* gu_first;  // [workgroups + 1] first hidden unit of each workgroup (gu_unit0)
+    // given >= 0: the step reads this id, not the record's, and nobody wants what it would sample: it ends with the last
+    // layer's k and v rows (as a batched prefill does), delivers no token and leaves the record alone.  1B shape:
+    // classifier, sampler and the rest of the last layer are 116 of a step's 564 us, TinyLlama's 49 of 590.
+    // (The two stay last: placed among the step's other values they moved the arguments behind them to other
+    // alignments, and every token of the 1B shape took 4.7 us longer.)
+    int given;
+    int stop;  // nonzero: an id that ends a sequence is not read: the launch, queued before that id was known, does nothing
 };
 
 // Rows of each matrix one workgroup owns (a contiguous block), and LDS sizes.
@@ -364,7 +371,7 @@ __host__ __device__ inline int slices_used(int d, int chunk_cols) {
     return (d + width - 1) / width;
 }
 
-template <bool kF16>
+template <bool kF16, bool kGiven>
 __device__ __forceinline__ void gemv_role(const DecodeArgs& a, Control& ctl, const uint4* __restrict__ steps, int j,
                                           const float* xs, float* results, bool trace_on) {
     constexpr int kPer = WTraits<kF16>::kPerLoad;
@@ -379,6 +386,13 @@ __device__ __forceinline__ void gemv_role(const DecodeArgs& a, Control& ctl, con
 
     uintx4 batch_a = list[lane];               // entries of the steps being requested now, one per lane
     uintx4 batch_b = list[kStepBatch + lane];  // the batch after it, requested a whole batch ahead
+    // (a step that samples nothing ends with the last layer's q, k and v: entries of later phases become terminating ones,
+    // a batch at a time, when its turn comes -- it is in by then)
+    auto end_behind = [&](uintx4& batch) {
+        if constexpr (kGiven)
+            if (((batch[2] >> kStepPhaseShift) & kStepPhaseMask) > n_phases - 5u) batch[2] = 0u;
+    };
+    end_behind(batch_a);
     uintx4 w[kDepth][kStepLoads];
     unsigned meta[kDepth];  // StepEntry::meta of the step held in w[k]
     unsigned cols[kDepth];  // StepEntry::cols
@@ -545,9 +559,11 @@ __device__ __forceinline__ void gemv_role(const DecodeArgs& a, Control& ctl, con
     int next_batch = 2;
     int first_round = 1;  // the priming requests were round 0 of the first batch
     while (more) {
+        if (first_round == 0) end_behind(batch_a);
         for (int r = first_round; r < kRoundsPerBatch && more; ++r) run_round(batch_a, r * kDepth);
         first_round = 0;
         batch_a = list[next_batch * kStepBatch + lane];
+        end_behind(batch_b);
         for (int r = 0; r < kRoundsPerBatch && more; ++r) run_round(batch_b, r * kDepth);
         batch_b = list[(next_batch + 1) * kStepBatch + lane];
         next_batch += 2;
@@ -952,7 +968,8 @@ __device__ __forceinline__ int block_rows(int total, int block, int wg) {
 template <int kHs>
 __device__ __forceinline__ void xcd_att_prefetch(const Ctx& c, const Io& io, const Lds& l, int layer);
 
-template <bool kXcd>
+// (kGiven: the instance for steps that sample nothing, Tagged::given)
+template <bool kXcd, bool kGiven>
 __device__ __forceinline__ void io_qkv(Ctx& c, Io& io, const Lds& l, int layer) {
 #pragma clang fp contract(off)
     const DecodeArgs& a = c.a;
@@ -979,7 +996,7 @@ __device__ __forceinline__ void io_qkv(Ctx& c, Io& io, const Lds& l, int layer) 
     // hand-over steps away.  (Requested a layer ahead, during the gate/up phase, the same bytes make that phase,
     // which is bound by bandwidth, longer by more than they take here.)
     if constexpr (kXcd) {
-        if (c.t.xa_chunk > 0) {
+        if (c.t.xa_chunk > 0 && !(kGiven && layer == a.n_layers - 1)) {
             if (hs == 64) xcd_att_prefetch<64>(c, io, l, layer);
             else xcd_att_prefetch<128>(c, io, l, layer);
         }
@@ -2502,7 +2519,7 @@ __device__ __forceinline__ void io_classify_sample(Ctx& c, Io& io, const Lds& l)
     ++c.phase_index;
 }
 
-template <bool kF16, bool kXcd>
+template <bool kXcd, bool kGiven>
 __device__ __forceinline__ void io_role(Ctx& c, Io& io, const Lds& l) {
     const DecodeArgs& a = c.a;
     // The thread index is made opaque before every phase: per-thread addresses are then formed
@@ -2511,7 +2528,8 @@ __device__ __forceinline__ void io_role(Ctx& c, Io& io, const Lds& l) {
     auto fresh = [&]() { io.it = exchange_thread_index(io.iw); };
     for (int layer = 0; layer < a.n_layers; ++layer) {
         fresh();
-        io_qkv<kXcd>(c, io, l, layer);
+        io_qkv<kXcd, kGiven>(c, io, l, layer);
+        if (kGiven && layer == a.n_layers - 1) break;
         fresh();
         io_attention<kXcd>(c, io, l, layer);
         fresh();
@@ -2524,7 +2542,7 @@ __device__ __forceinline__ void io_role(Ctx& c, Io& io, const Lds& l) {
                 c.t.share_hidden, c.seq(layer, kGateUp), c.seq(layer, kDown));
     }
     fresh();
-    io_classify_sample(c, io, l);
+    if constexpr (!kGiven) io_classify_sample(c, io, l);
     if (io.it == 0 && lds_peek(&c.ctl.error) != 0u) report_error(a.step, 2);
 }
 
@@ -2533,8 +2551,10 @@ __device__ __forceinline__ void io_role(Ctx& c, Io& io, const Lds& l) {
 // ---------------------------------------------------------------------------
 
 // (kXcd: with the item that splits a context over an XCD, att_xcd_item.  A second instance of the kernel rather than
-// a branch in the one: merely compiled in, that item's registers cost every other plan 5 us per token at the 1B shape.)
-template <bool kF16, bool kXcd>
+// a branch in the one: merely compiled in, that item's registers cost every other plan 5 us per token at the 1B shape.
+// kGiven: a prompt's step that samples nothing, an instance for the same reason: its checks as run-time ones cost the
+// others 4 us per token.)
+template <bool kF16, bool kXcd, bool kGiven>
 __global__ __launch_bounds__(kThreads) void k_decode_dataflow(DecodeArgs a, Tagged t, Blocks b,
                                                               const uint4* __restrict__ row_lists, int row_list_stride) {
     extern __shared__ __align__(16) float lds[];
@@ -2557,6 +2577,7 @@ __global__ __launch_bounds__(kThreads) void k_decode_dataflow(DecodeArgs a, Tagg
                 __hip_atomic_fetch_max(&a.step->error, 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
+        if (t.stop != 0 && ends_sequence(a.step->token)) number = -1;
         numbered = number;
     }
     const int dim_pad = (a.dim + 7) & ~7;
@@ -2582,13 +2603,14 @@ __global__ __launch_bounds__(kThreads) void k_decode_dataflow(DecodeArgs a, Tagg
         reinterpret_cast<unsigned*>(&ctl)[i] = 0u;
     __syncthreads();  // the only workgroup-wide barrier: the two kinds of wavefronts part ways here
     const int wg = __builtin_amdgcn_readfirstlane(numbered);
+    if (wg < 0) return;
     const int wave = wave_index();
     if (wave < kGemvWaves) {
-        gemv_role<kF16>(a, ctl, row_lists + static_cast<size_t>(wg * kGemvWaves + wave) * row_list_stride, wave, l.xs,
+        gemv_role<kF16, kGiven>(a, ctl, row_lists + static_cast<size_t>(wg * kGemvWaves + wave) * row_list_stride, wave, l.xs,
                         l.results, (wg == 0 || t.trace_stride > 0) && wave == 0 && a.trace != nullptr);
     } else {
         // (kept inside the vocabulary whatever a launch that gave up left in the record: it indexes the embedding)
-        const int token_in = min(max(__builtin_amdgcn_readfirstlane(a.step->token), 0), a.vocab - 1);
+        const int token_in = kGiven ? t.given : min(max(__builtin_amdgcn_readfirstlane(a.step->token), 0), a.vocab - 1);
         unsigned long long* my_trace = nullptr;
         if (a.trace != nullptr && (wg == 0 || t.trace_stride > 0)) my_trace = a.trace + static_cast<size_t>(wg) * t.trace_stride;
         const int n_xcc = t.n_xcc > 1 ? t.n_xcc : 1;
@@ -2597,7 +2619,7 @@ __global__ __launch_bounds__(kThreads) void k_decode_dataflow(DecodeArgs a, Tagg
               gu_unit0(t.gu_first, wg), gu_units(t.gu_first, wg)};
         Io io{static_cast<int>(threadIdx.x) - kGemvWaves * kWave, wave - kGemvWaves, 0u, 0, a.step};
         if (c.trace && io.it == 0) c.trace[kTraceMarks * phases_per_token(a.n_layers)] = wall_clock64();
-        io_role<kF16, kXcd>(c, io, l);
+        io_role<kXcd, kGiven>(c, io, l);
     }
 }
 
@@ -2871,6 +2893,8 @@ df::Tagged tagged_of(const lpp_model* m, bool generating, int lane_item_cap) {
         }
     }
     t.history_len = m->df_history_len;
+    t.given = m->df_given;
+    t.stop = m->df_stop;
     t.temperature = m->df_temperature;
     t.penalty = m->df_penalty;
     // model.cpp:291: one draw per step; a generate call brings them as an array (absent: zeros)
@@ -3121,16 +3145,16 @@ static lpp_status launch_impl(lpp_model* m, const ph::DecodeArgs& a, hipStream_t
         LPP_REQUIRE(m->head_size <= df::kMaxHeadPad, "persistent decode: head_size %d exceeds %d", m->head_size,
                     df::kMaxHeadPad);
         const size_t lds_most = kLdsLimit;  // (every launch brings its own size, up to what a compute unit has)
-        if (hipFuncSetAttribute(reinterpret_cast<const void*>(&df::k_decode_dataflow<kF16, false>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_most)) != hipSuccess ||
-            hipFuncSetAttribute(reinterpret_cast<const void*>(&df::k_decode_dataflow<kF16, true>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_most)) != hipSuccess)
-            return fail(LPP_ERR_UNSUPPORTED, "persistent decode needs %zu bytes of LDS per workgroup", lds_most);
-        int per_cu = 0, per_cu_xcd = 0;
-        LPP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, df::k_decode_dataflow<kF16, false>, df::kThreads, lds_most));
-        LPP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_xcd, df::k_decode_dataflow<kF16, true>, df::kThreads, lds_most));
-        if (per_cu < 1 || per_cu_xcd < 1)
-            return fail(LPP_ERR_UNSUPPORTED, "persistent decode kernel does not fit a compute unit (LDS %zu bytes)", lds_most);
+        for (const auto kernel : {&df::k_decode_dataflow<kF16, false, false>, &df::k_decode_dataflow<kF16, true, false>,
+                                  &df::k_decode_dataflow<kF16, false, true>, &df::k_decode_dataflow<kF16, true, true>}) {
+            if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    static_cast<int>(lds_most)) != hipSuccess)
+                return fail(LPP_ERR_UNSUPPORTED, "persistent decode needs %zu bytes of LDS per workgroup", lds_most);
+            int per_cu = 0;
+            LPP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, df::kThreads, lds_most));
+            if (per_cu < 1)
+                return fail(LPP_ERR_UNSUPPORTED, "persistent decode kernel does not fit a compute unit (LDS %zu bytes)", lds_most);
+        }
         m->persist_grid = p.grid;
     }
     bool moved = false;  // a weight tensor changed its address: both lists are stale
@@ -3160,16 +3184,17 @@ static lpp_status launch_impl(lpp_model* m, const ph::DecodeArgs& a, hipStream_t
     if (tagged.n_xcc > 1 && take_forced_ticket_failure()) tagged.ticket_base -= static_cast<unsigned>(m->persist_grid / tagged.n_xcc);
     LPP_REQUIRE(p.lds_bytes <= kLdsLimit, "persistent decode: %zu bytes of LDS per workgroup", p.lds_bytes);
     tagged.gu_first = m->df_gu_first[which];
-    if (xa.chunk > 0)
-        hipLaunchKernelGGL((df::k_decode_dataflow<kF16, true>), dim3(m->persist_grid), dim3(df::kThreads), p.lds_bytes, s, a,
-                           tagged, p.blocks, static_cast<const uint4*>(m->df_rows[which]), m->df_row_stride[which]);
-    else
-        hipLaunchKernelGGL((df::k_decode_dataflow<kF16, false>), dim3(m->persist_grid), dim3(df::kThreads), p.lds_bytes, s, a,
-                           tagged, p.blocks, static_cast<const uint4*>(m->df_rows[which]), m->df_row_stride[which]);
+    const bool given = m->df_given >= 0;
+    const auto kernel = xa.chunk > 0 ? (given ? &df::k_decode_dataflow<kF16, true, true> : &df::k_decode_dataflow<kF16, true, false>)
+                                     : (given ? &df::k_decode_dataflow<kF16, false, true> : &df::k_decode_dataflow<kF16, false, false>);
+    hipLaunchKernelGGL(kernel, dim3(m->persist_grid), dim3(df::kThreads), p.lds_bytes, s, a, tagged, p.blocks,
+                       static_cast<const uint4*>(m->df_rows[which]), m->df_row_stride[which]);
     LPP_CHECK_LAUNCH("k_decode_dataflow");
     m->df_base += df::phases_per_token(m->cfg.n_layers);
     if (tagged.n_xcc > 1) m->df_ticket_base += static_cast<unsigned>(m->persist_grid / tagged.n_xcc);  // one ticket per workgroup
-    if (!m->df_freeze) {  // what finish_token does to the device's record
+    if (given) {
+        m->df_pos += 1;
+    } else if (!m->df_freeze) {  // what finish_token does to the device's record
         if (m->df_history_cap > 0 && m->df_history_len < m->df_history_cap) m->df_history_len += 1;
         m->df_pos += 1;
         m->df_step_index += 1;

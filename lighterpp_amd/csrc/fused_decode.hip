@@ -387,6 +387,8 @@ static lpp_status begin_run(lpp_model* m, const StepParams& init, hipStream_t s)
     m->df_penalty = sp.penalty;
     m->df_r = sp.r;
     m->df_uniforms_host = nullptr;
+    m->df_given = -1;
+    m->df_stop = 0;
     LPP_HIP(hipMemcpyAsync(m->step, &sp, sizeof sp, hipMemcpyHostToDevice, s));
     if (m->path == LPP_PATH_PERSISTENT) LPP_TRY(lpp_memset(m->sync_words + 64, 0, 2 * sizeof(unsigned)));
     return LPP_OK;
@@ -429,6 +431,52 @@ lpp_status fused_forward(lpp_model* m, int token, int pos, float temperature, fl
     return LPP_OK;
 }
 
+// main.cpp:196-223: one forward per token, n_steps of them behind begin_run.  The device feeds each sampled id back by
+// itself and writes it to pinned host memory; token i+1 is launched before the host waits for the 4 bytes of token i, so
+// the device never idles on the host.  `until_end`: an id that ends a sequence is the last one; the launch that is queued
+// behind it by then does nothing.  `first_queued`: the first step has been launched already, behind others of the caller's;
+// if it comes to nothing, those may have as well, and *from_the_start tells the caller to launch them all again.
+static lpp_status generate_steps(lpp_model* m, int n_steps, bool until_end, bool first_queued, int* out_tokens, int* delivered,
+                                 bool* from_the_start, hipStream_t s) {
+    int launched = first_queued ? 1 : 0;
+    bool relaunched = false;
+    for (int i = 0; i < n_steps; ++i) {
+        while (launched < n_steps && launched <= i + 1) {
+            m->df_stop = until_end && launched > 0;
+            LPP_TRY(launch_token(m, true, s));
+            ++launched;
+        }
+        if (await_token(m, i, s) != LPP_OK) {
+            // The stream went idle without token i: a persistent launch drained with an error code.  Such a launch
+            // leaves the device's step record as it found it, so the record says where to pick up.
+            if (m->path != LPP_PATH_PERSISTENT) return LPP_ERR_HIP;
+            StepParams rec{};
+            LPP_HIP(hipMemcpy(&rec, m->step, sizeof rec, hipMemcpyDeviceToHost));
+            if (rec.error == 0) return LPP_ERR_HIP;  // (await_token's own message stands)
+            bool again = false;
+            LPP_TRY(dataflow_after_error(m, rec.error, &again));
+            if (!again || relaunched || rec.step_index != i)
+                return fail(LPP_ERR_HIP, "decode kernel: workgroups unevenly spread over the XCDs");
+            if (first_queued && i == 0) {
+                *from_the_start = true;
+                break;
+            }
+            relaunched = true;
+            m->df_pos = rec.pos;
+            m->df_history_len = rec.history_len;
+            m->df_step_index = rec.step_index;
+            launched = i;
+            --i;
+            continue;
+        }
+        out_tokens[i] = m->pinned_tokens[i];
+        *delivered = i + 1;
+        if (until_end && ends_sequence(out_tokens[i])) break;
+    }
+    m->df_stop = 0;
+    return LPP_OK;
+}
+
 lpp_status fused_generate(lpp_model* m, int first_token, int start_pos, int n_steps, float temperature,
                           float penalty, int* history, int* history_len, int history_cap, const float* uniforms,
                           int* out_tokens, lpp_gen_stats* stats) {
@@ -462,40 +510,10 @@ lpp_status fused_generate(lpp_model* m, int first_token, int start_pos, int n_st
     }
     LPP_HIP(hipStreamSynchronize(s));
 
-    // main.cpp:196-223: one forward per token.  The device feeds each sampled id
-    // back by itself and writes it to pinned host memory; token i+1 is launched
-    // before the host waits for the 4 bytes of token i, so the device never idles
-    // on the host.
     LPP_HIP(hipEventRecord(m->ev_a, s));
     const auto t0 = std::chrono::steady_clock::now();
-    int launched = 0;
-    bool relaunched = false;
-    for (int i = 0; i < n_steps; ++i) {
-        while (launched < n_steps && launched <= i + 1) {
-            LPP_TRY(launch_token(m, true, s));
-            ++launched;
-        }
-        if (await_token(m, i, s) != LPP_OK) {
-            // The stream went idle without token i: a persistent launch drained with an error code.  Such a launch
-            // leaves the device's step record as it found it, so the record says where to pick up.
-            if (m->path != LPP_PATH_PERSISTENT) return LPP_ERR_HIP;
-            StepParams rec{};
-            LPP_HIP(hipMemcpy(&rec, m->step, sizeof rec, hipMemcpyDeviceToHost));
-            if (rec.error == 0) return LPP_ERR_HIP;  // (await_token's own message stands)
-            bool again = false;
-            LPP_TRY(dataflow_after_error(m, rec.error, &again));
-            if (!again || relaunched || rec.step_index != i)
-                return fail(LPP_ERR_HIP, "decode kernel: workgroups unevenly spread over the XCDs");
-            relaunched = true;
-            m->df_pos = rec.pos;
-            m->df_history_len = rec.history_len;
-            m->df_step_index = rec.step_index;
-            launched = i;
-            --i;
-            continue;
-        }
-        out_tokens[i] = m->pinned_tokens[i];
-    }
+    int delivered = 0;  // (all of them, or an error)
+    LPP_TRY(generate_steps(m, n_steps, false, false, out_tokens, &delivered, nullptr, s));
     m->df_uniforms_host = nullptr;
     const auto t1 = std::chrono::steady_clock::now();
     LPP_HIP(hipEventRecord(m->ev_b, s));
@@ -526,6 +544,63 @@ lpp_status fused_generate(lpp_model* m, int first_token, int start_pos, int n_st
         stats->kernel_launches = (m->path == LPP_PATH_PERSISTENT) ? n_steps : 0;
     }
     return LPP_OK;
+}
+
+// The steps are queued ahead of their results, the prompt's all at once: lpp_forward per id waits for each one and costs
+// the host 40 us a step (record and window uploaded, token and record read back: 166 us a step at the 15M shape, of
+// which the kernel is 125).  What the prompt's steps would sample is dropped (main.cpp:163-180): they sample nothing.
+lpp_status persistent_run(lpp_model* m, const int* given, int n_given, int pos, int token, int n_steps, float temperature,
+                          float penalty, const int* history, int history_len, int history_cap, const float* uniforms,
+                          int* out_tokens, int* n_out, double* seconds) {
+    *n_out = 0;
+    *seconds = 0.0;
+    for (int t = 0; t < LPP_T_COUNT; ++t)
+        if (!m->w_loaded[t]) return fail(LPP_ERR_STATE, "weight tensor %d has not been uploaded", t);
+    LPP_TRY(require_fused(m));
+    LPP_TRY(calibrate_gateup(m));
+    hipStream_t s = stream();
+    LPP_TRY(ensure_gen_capacity(m, n_steps > 0 ? n_steps : 1));
+    StepParams sp{};
+    sp.token = token;
+    sp.history_len = history_len;
+    sp.history_cap = history_cap;
+    sp.history_next = history_len % history_cap;
+    sp.temperature = temperature;
+    sp.penalty = penalty;
+    for (int attempt = 0;; ++attempt) {
+        sp.pos = pos + n_given;
+        LPP_TRY(begin_run(m, sp, s));
+        if (history_len > 0)
+            LPP_HIP(hipMemcpyAsync(m->history, history, static_cast<size_t>(history_len) * sizeof(int), hipMemcpyHostToDevice, s));
+        for (int i = 0; i < n_steps; ++i) m->pinned_tokens[i] = kNoToken;
+        m->df_uniforms_host = uniforms;
+        m->df_pos = pos;
+        for (int i = 0; i < n_given; ++i) {
+            m->df_given = given[i];
+            LPP_TRY(launch_token(m, true, s));
+        }
+        m->df_given = -1;
+        LPP_HIP(hipEventRecord(m->ev_a, s));
+        if (n_steps > 0) LPP_TRY(launch_token(m, true, s));
+        LPP_HIP(hipEventSynchronize(m->ev_a));
+        const auto t0 = std::chrono::steady_clock::now();
+        bool again = false;
+        const lpp_status st = n_steps > 0 ? generate_steps(m, n_steps, true, true, out_tokens, n_out, &again, s) : LPP_OK;
+        *seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+        m->df_uniforms_host = nullptr;
+        LPP_TRY(st);
+        if (!again) {
+            LPP_HIP(hipStreamSynchronize(s));
+            StepParams rec{};
+            LPP_HIP(hipMemcpy(&rec, m->step, sizeof rec, hipMemcpyDeviceToHost));
+            if (rec.error == 0) return LPP_OK;
+            LPP_TRY(dataflow_after_error(m, rec.error, &again));
+            if (again && *n_out > 0 && ends_sequence(out_tokens[*n_out - 1])) return LPP_OK;  // (the launch behind the last id)
+        }
+        // The first generated step came to nothing, for a reason of its own or because a given one before it gave up (what
+        // is behind such a launch finds the abort flag raised and delivers nothing): all of them again.
+        if (!again || attempt > 0 || *n_out > 0) return fail(LPP_ERR_HIP, "decode kernel: workgroups unevenly spread over the XCDs");
+    }
 }
 
 // ---------------------------------------------------------------------------

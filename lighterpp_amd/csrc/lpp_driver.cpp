@@ -10,6 +10,7 @@
 #include <cerrno>
 #include <chrono>
 #include <cstring>
+#include <vector>
 
 #include "lpp_internal.hpp"
 #include "lpp_model.hpp"
@@ -196,6 +197,19 @@ lpp_status run_loop(lpp_model* m, const int* prompt, int n_prompt, int steps, fl
     };
     int pos = 0;
     int n_out = 0;
+    int token = prompt[n_prompt - 1];
+    int stopped = 0;
+    auto report = [&](double seconds) {
+        if (res == nullptr) return;
+        res->n_tokens = n_out;
+        res->final_pos = pos;
+        res->stopped_by_eos = stopped;
+        res->reported_count = pos - n_prompt;  // main.cpp:229
+        res->history_len = history_len;
+        std::memset(res->history, 0, sizeof res->history);
+        std::memcpy(res->history, history, static_cast<size_t>(history_len) * sizeof(int));
+        res->wall_seconds = seconds;
+    };
     // 1. prefill, main.cpp:163-180.  Batched: the cache entries of all but the last prompt id in one
     //    pass per 2048 ids; what the decode steps would have sampled is what the reference drops.
     //    (The line lies where a batch cost five decode steps and a margin.  A batch of up to 32 ids now costs one and a half to
@@ -207,6 +221,31 @@ lpp_status run_loop(lpp_model* m, const int* prompt, int n_prompt, int steps, fl
         LPP_TRY(lpp_prefill(m, prompt, n_prompt - 1, 0));
         pos = n_prompt - 1;
     }
+    if (m->path == LPP_PATH_PERSISTENT && pos < n_prompt && n_prompt <= steps) {
+        //    By decode steps queued ahead, samples and all: what follows this block, with the same ids and windows.
+        //    (Where nothing is generated the last prompt id's logits stay readable: not here.)
+        const int n_given = n_prompt - 1 - pos;
+        for (int i = pos; i < n_prompt; ++i) push(prompt[i]);
+        std::vector<int> ids(static_cast<size_t>(steps - (n_prompt - 1)));
+        int n_ids = 0;
+        double seconds = 0.0;
+        LPP_TRY(lpp::persistent_run(m, prompt + pos, n_given, pos, token, static_cast<int>(ids.size()), temperature, 1.05f, history,
+                                    history_len, kHistory < cfg.seq_len ? kHistory : cfg.seq_len,
+                                    uniforms ? uniforms + (n_prompt - 1) : nullptr, ids.data(), &n_ids, &seconds));
+        pos = n_prompt - 1;
+        for (int i = 0; i < n_ids; ++i) {
+            push(ids[i]);
+            if (lpp::ends_sequence(ids[i])) {
+                stopped = 1;
+                break;
+            }
+            if (n_out < out_capacity) out_tokens[n_out] = ids[i];
+            ++n_out;
+            ++pos;
+        }
+        report(seconds);
+        return LPP_OK;
+    }
     //    By decode: penalty 1.1, the sampled id is dropped
     for (int i = pos; i < n_prompt - 1; ++i) {
         push(prompt[i]);
@@ -216,34 +255,22 @@ lpp_status run_loop(lpp_model* m, const int* prompt, int n_prompt, int steps, fl
         ++pos;
     }
     // 2. main.cpp:182-190
-    int token = prompt[n_prompt - 1];
     push(token);
     // 3. generation, main.cpp:196-223: penalty 1.05; an end-of-sequence id ends the loop after it
     //    entered the window, before the position advances
     const auto t0 = std::chrono::steady_clock::now();
-    int stopped = 0;
     for (; pos < steps; ++pos) {
         LPP_TRY(lpp_forward(m, token, pos, temperature, topp, 1.05f, history, history_len, uniforms ? uniforms[pos] : 0.0f,
                             &token));
         push(token);
-        if (token == 2 || token == 128001 || token == 128009) {  // main.cpp:211-213
+        if (lpp::ends_sequence(token)) {  // main.cpp:211-213
             stopped = 1;
             break;
         }
         if (n_out < out_capacity) out_tokens[n_out] = token;
         ++n_out;
     }
-    const auto t1 = std::chrono::steady_clock::now();
-    if (res != nullptr) {
-        res->n_tokens = n_out;
-        res->final_pos = pos;
-        res->stopped_by_eos = stopped;
-        res->reported_count = pos - n_prompt;  // main.cpp:229
-        res->history_len = history_len;
-        std::memset(res->history, 0, sizeof res->history);
-        std::memcpy(res->history, history, static_cast<size_t>(history_len) * sizeof(int));
-        res->wall_seconds = std::chrono::duration<double>(t1 - t0).count();  // main.cpp:196, 225-226
-    }
+    report(std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count());  // main.cpp:196, 225-226
     return LPP_OK;
 }
 

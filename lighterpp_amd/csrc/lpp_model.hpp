@@ -68,6 +68,8 @@ struct lpp_model {
     int df_pos = 0, df_history_len = 0, df_history_cap = 0, df_step_index = 0, df_freeze = 0;
     float df_temperature = 0.0f, df_penalty = 1.0f, df_r = 0.0f;
     const float* df_uniforms_host = nullptr; // per-step draws of the generate call in progress (host memory)
+    int df_given = -1;                       // >= 0: the next launch reads this id instead of the record's and samples nothing
+    int df_stop = 0;                         // nonzero: the next launch does nothing if the id it is to read ends a sequence
     unsigned df_base = 0;                    // sequence-number base of the next persistent launch
     int df_trace_stride = 0;                 // timeline words per workgroup when every workgroup is traced (0: workgroup 0 only)
     int persist_grid = 0;                    // workgroups of the persistent kernel (0: not sized yet)
@@ -128,5 +130,13 @@ lpp_status fused_forward(lpp_model* m, int token, int pos, float temperature, fl
 lpp_status fused_generate(lpp_model* m, int first_token, int start_pos, int n_steps, float temperature,
                           float penalty, int* history, int* history_len, int history_cap,
                           const float* uniforms, int* out_tokens, lpp_gen_stats* stats);
+// lpp_run's decode steps on LPP_PATH_PERSISTENT: ids given[0 .. n_given) from position pos on, for their cache entries
+// alone, then up to n_steps generated ones from `token`, until one ends the sequence (it is delivered too).
+// `uniforms`: the first generated step's draw first.  *seconds: from the last given id's end to the last generated one.
+lpp_status persistent_run(lpp_model* m, const int* given, int n_given, int pos, int token, int n_steps, float temperature,
+                          float penalty, const int* history, int history_len, int history_cap, const float* uniforms,
+                          int* out_tokens, int* n_out, double* seconds);
+// Ids that end a sequence (main.cpp:211-213).
+__host__ __device__ inline bool ends_sequence(int token) { return token == 2 || token == 128001 || token == 128009; }
 
 }  // namespace lpp
