@@ -496,7 +496,8 @@ enum lpp_test_option {
                                                hidden units out by how fast each XCD got through the gate/up phase; 0: evenly  */
     LPP_OPT_PREFILL_ROOM = 11,          /* [0] n > 0: device memory is reported to have room for the buffers of batches of up to
                                                n tokens only; n < 0: the same, but it shows when they are allocated          */
-    LPP_OPT_COUNT = 12
+    LPP_OPT_DECODE_RESIDENT = 12,       /* [1] small fp32 models: every layer in the registers of one XCD               */
+    LPP_OPT_COUNT = 13
 };
 lpp_status lpp_set_test_option(int option, int value);
 lpp_status lpp_get_test_option(int option, int *value);

@@ -63,6 +63,7 @@ constexpr int kPollBatch = 8;                      // tagged values one thread r
 constexpr int kItemPositions = 1024;               // a one-head attention work item stays within twice this many positions
 constexpr int kAttScoreFloats = 512;               // half of the sampler's LDS copy of the penalty window
 constexpr int kMaxHeadPad = 128;
+constexpr int kGridCap = 1024;                     // workgroups the statistics table has room for
 constexpr int kShortRounds = 2;                    // cache rows per lane group a one-head work item requests at once
 constexpr int kPacedSteps = 2;                     // next-phase rows a streaming wavefront sends out early after a burst
 constexpr int kMaxAttHeads = 4;                    // query heads of one KV head a work item of att_xcd_item covers at most
@@ -154,6 +155,7 @@ struct Tagged {
     // alignments, and every token of the 1B shape took 4.7 us longer.)
     int given;
     int stop;  // nonzero: an id that ends a sequence is not read: the launch, queued before that id was known, does nothing
+    u64* near_stats;  // [n_xcc][4 * kGridCap] the statistics, a copy to each XCD (gather_values)
 };
 
 // Rows of each matrix one workgroup owns (a contiguous block), and LDS sizes.
@@ -2333,33 +2335,13 @@ __device__ __forceinline__ void io_attention(Ctx& c, Io& io, const Lds& l, int l
 // Classifier + sampler (exchange wavefronts)
 // ---------------------------------------------------------------------------
 
-// Workgroup w owns the contiguous vocabulary rows [w*cls, ...): their logits
-// stay in LDS, the sampler's per-row work happens there, and only three numbers
-// per workgroup (maximum, its lowest index, sum of exponentials) are exchanged.
-// The workgroup whose slice of the CDF contains the draw (or that holds the
-// first maximum, for temperature 0) finishes the token (model.cpp:256-303,
-// main.cpp:200-208).
-__device__ __forceinline__ void io_classify_sample(Ctx& c, Io& io, const Lds& l) {
+// Penalty, temperature and draw over the vocabulary rows r0 .. r0 + n - 1 this workgroup holds the logits lg of, by the
+// exchange wavefronts.  lg lies behind the tables at l.xs (four floats to a workgroup).
+__device__ __forceinline__ void sample_token(Ctx& c, Io& io, const Lds& l, float* lg, int r0, int n) {
     const DecodeArgs& a = c.a;
     Control& ctl = c.ctl;
-    const int vocab = a.vocab, dim = a.dim, wg = c.wg, nwg = c.nwg;
+    const int vocab = a.vocab, wg = c.wg, nwg = c.nwg, r1 = r0 + n;
     const int it = io.it;
-    mark(c, io, 0);
-    const float scale = stage_norm(c, io, l, c.t.x, nullptr, dim, c.seq(a.n_layers - 1, kDown), a.rms_final);
-    mark(c, io, 2);
-    wait_gemv(ctl, 4 * a.n_layers);
-    mark(c, io, 3);
-    const int r0 = min(vocab, wg * c.b.cls);
-    const int n = block_rows(vocab, c.b.cls, wg);
-    const int r1 = r0 + n;
-    float* lg = l.xs + 4 * nwg;  // beside the sampler tables; the streaming wavefronts are done with xs
-    for (int i = it; i < n; i += kIoThreads) {
-        lg[i] = row_result(l.results, i, c.b.ns_dim) * scale;
-        a.logits[r0 + i] = lg[i];  // raw logits stay readable after the token
-    }
-    mark(c, io, 4);
-    ++c.phase_index;
-
     const float temperature = c.temperature, penalty = c.penalty;
     const int history_len = c.history_len;
     if (penalty > 1.0f && history_len > 0) {  // model.cpp:258-270, once per occurrence
@@ -2421,12 +2403,14 @@ __device__ __forceinline__ void io_classify_sample(Ctx& c, Io& io, const Lds& l)
     float* st_sum = l.xs + nwg;      // [nwg]
     float* st_arg = l.xs + 2 * nwg;  // [nwg] (int bits)
     float* st_cum = l.xs + 3 * nwg;  // [nwg] mass before the workgroup
-    poll_values(c.t.stats, nwg * 4, tag, c, io, [&](int i, float v, int, bool) {
+    auto take = [&](int i, float v, int, bool) {
         const int w = i >> 2, f = i & 3;
         if (f == 0) st_max[w] = v;
         else if (f == 1) st_sum[w] = v;
         else if (f == 2) st_arg[w] = v;
-    });
+    };
+    if (c.t.n_xcc > 1) gather_values(c.t.stats, c.t.near_stats, 4 * kGridCap, 4 * c.t.n_xcc, nwg * 4, tag, c, io, take);
+    else poll_values(c.t.stats, nwg * 4, tag, c, io, take);
     io_sync(ctl, io);
     mark(c, io, 2);
     if (temperature == 0.0f) {  // model.cpp:272-283: first maximum wins
@@ -2519,6 +2503,35 @@ __device__ __forceinline__ void io_classify_sample(Ctx& c, Io& io, const Lds& l)
     ++c.phase_index;
 }
 
+// Workgroup w owns the contiguous vocabulary rows [w*cls, ...): their logits
+// stay in LDS, the sampler's per-row work happens there, and only three numbers
+// per workgroup (maximum, its lowest index, sum of exponentials) are exchanged.
+// The workgroup whose slice of the CDF contains the draw (or that holds the
+// first maximum, for temperature 0) finishes the token (model.cpp:256-303,
+// main.cpp:200-208).
+__device__ __forceinline__ void io_classify_sample(Ctx& c, Io& io, const Lds& l) {
+    const DecodeArgs& a = c.a;
+    Control& ctl = c.ctl;
+    const int vocab = a.vocab, dim = a.dim, wg = c.wg, nwg = c.nwg;
+    const int it = io.it;
+    mark(c, io, 0);
+    const float scale = stage_norm(c, io, l, c.t.x, nullptr, dim, c.seq(a.n_layers - 1, kDown), a.rms_final);
+    mark(c, io, 2);
+    wait_gemv(ctl, 4 * a.n_layers);
+    mark(c, io, 3);
+    const int r0 = min(vocab, wg * c.b.cls);
+    const int n = block_rows(vocab, c.b.cls, wg);
+    float* lg = l.xs + 4 * nwg;  // beside the sampler tables; the streaming wavefronts are done with xs
+    for (int i = it; i < n; i += kIoThreads) {
+        lg[i] = row_result(l.results, i, c.b.ns_dim) * scale;
+        a.logits[r0 + i] = lg[i];  // raw logits stay readable after the token
+    }
+    mark(c, io, 4);
+    ++c.phase_index;
+
+    sample_token(c, io, l, lg, r0, n);
+}
+
 template <bool kXcd, bool kGiven>
 __device__ __forceinline__ void io_role(Ctx& c, Io& io, const Lds& l) {
     const DecodeArgs& a = c.a;
@@ -2550,6 +2563,26 @@ __device__ __forceinline__ void io_role(Ctx& c, Io& io, const Lds& l) {
 // The kernel
 // ---------------------------------------------------------------------------
 
+// Workgroups are numbered by where they run: XCD + n_xcc * (the order in which the XCD's workgroups got here).
+// Which rows, attention items and slices a workgroup owns then says which XCD's L2 they pass through, whatever
+// the order in which the hardware handed the workgroups out.  An XCD that does not get its share of the
+// workgroups (they are handed out in turn: it always has) ends the launch with an error.  -1: nothing to do (Tagged::stop).
+__device__ __forceinline__ int workgroup_number(const DecodeArgs& a, const Tagged& t, int nwg) {
+    int number = blockIdx.x;
+    if (t.n_xcc > 1) {
+        const int x = hardware_xcc() % t.n_xcc;
+        const unsigned order = __hip_atomic_fetch_add(t.tickets + x, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - t.ticket_base;
+        if (order < static_cast<unsigned>(nwg / t.n_xcc)) {
+            number = static_cast<int>(order) * t.n_xcc + x;
+        } else {
+            __hip_atomic_store(t.abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_fetch_max(&a.step->error, 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    if (t.stop != 0 && ends_sequence(a.step->token)) number = -1;
+    return number;
+}
+
 // (kXcd: with the item that splits a context over an XCD, att_xcd_item.  A second instance of the kernel rather than
 // a branch in the one: merely compiled in, that item's registers cost every other plan 5 us per token at the 1B shape.
 // kGiven: a prompt's step that samples nothing, an instance for the same reason: its checks as run-time ones cost the
@@ -2561,25 +2594,7 @@ __global__ __launch_bounds__(kThreads) void k_decode_dataflow(DecodeArgs a, Tagg
     __shared__ Control ctl;
     __shared__ int numbered;
     const int nwg = gridDim.x;
-    // Workgroups are numbered by where they run: XCD + n_xcc * (the order in which the XCD's workgroups got here).
-    // Which rows, attention items and slices a workgroup owns then says which XCD's L2 they pass through, whatever
-    // the order in which the hardware handed the workgroups out.  An XCD that does not get its share of the
-    // workgroups (they are handed out in turn: it always has) ends the launch with an error.
-    if (threadIdx.x == 0) {
-        int number = blockIdx.x;
-        if (t.n_xcc > 1) {
-            const int x = hardware_xcc() % t.n_xcc;
-            const unsigned order = __hip_atomic_fetch_add(t.tickets + x, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - t.ticket_base;
-            if (order < static_cast<unsigned>(nwg / t.n_xcc)) {
-                number = static_cast<int>(order) * t.n_xcc + x;
-            } else {
-                __hip_atomic_store(t.abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_fetch_max(&a.step->error, 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-        }
-        if (t.stop != 0 && ends_sequence(a.step->token)) number = -1;
-        numbered = number;
-    }
+    if (threadIdx.x == 0) numbered = workgroup_number(a, t, nwg);
     const int dim_pad = (a.dim + 7) & ~7;
     Lds l;
     l.xraw = lds;
@@ -2622,6 +2637,8 @@ __global__ __launch_bounds__(kThreads) void k_decode_dataflow(DecodeArgs a, Tagg
         io_role<kXcd, kGiven>(c, io, l);
     }
 }
+
+#include "resident_decode.hpp"
 
 // Which XCD each workgroup of a launch of this shape lands on.
 __global__ void k_probe_xcc(int* out) {
@@ -2822,7 +2839,6 @@ Plan plan_for(const lpp_model* m, bool parking, const XcdAttention* xa = nullptr
     return p;
 }
 
-constexpr int kGridCap = 1024;  // workgroups the statistics table has room for
 // Tagged values of one XCD's copy of an n-value vector: whole 128-byte lines.
 size_t near_stride(int n) { return (static_cast<size_t>(n) + 15) / 16 * 16; }
 
@@ -2831,7 +2847,41 @@ size_t tagged_count(const lpp_model* m, int grid_cap) {
     return static_cast<size_t>(c.dim) * 3 + static_cast<size_t>(m->kv_dim) * 2 + c.hidden_dim +
            static_cast<size_t>(c.n_heads) * splits_cap_for(m) * (m->head_size + 2) + 4u * grid_cap +
            32u + static_cast<size_t>(kMaxXcc) * (near_stride(c.hidden_dim) + near_stride(c.dim + 2 * m->kv_dim)) +
-           static_cast<size_t>(kMaxXcc) * kMaxPerXcc * near_stride(m->gqa * (m->head_size + 2));
+           static_cast<size_t>(kMaxXcc) * kMaxPerXcc * near_stride(m->gqa * (m->head_size + 2)) +
+           16u + static_cast<size_t>(kMaxXcc) * (4u * grid_cap + 3 * near_stride(c.dim));
+}
+
+// k_decode_resident's plan: whether the model's layers fit an XCD's registers as that kernel lays them out, and how the
+// rows are shared.  (Where it applies it is the faster one throughout: 15M shape 122 us a token, 58 here.  What
+// does not fit -- a binary16 model of the size has no use here yet, wider rows or more of them need a second pass over
+// the registers -- takes k_decode_dataflow, and so do longer contexts and a traced token.)
+bool resident_plan(const lpp_model* m, const df::Blocks& b, int grid, int npos, df::Resident* rs, size_t* lds_bytes) {
+    const lpp_config& c = m->cfg;
+    const int n_xcc = m->df_xcc, hs = m->head_size;
+    if (test_option(LPP_OPT_DECODE_RESIDENT) == 0 || c.weight_precision != LPP_WEIGHT_FP32) return false;
+    if (n_xcc <= 1 || n_xcc > kMaxXcc || grid % n_xcc != 0 || npos > df::kResPositions) return false;
+    const int row_wgs = grid / n_xcc - c.n_heads;
+    if (row_wgs < 1 || c.dim > df::kResDim || c.hidden_dim > df::kResHidden || c.dim % 4 != 0 || c.hidden_dim % 4 != 0) return false;
+    if (hs > df::kResHead || hs % 8 != 0) return false;
+    auto per = [&](int total) { return (total + row_wgs - 1) / row_wgs; };
+    rs->qkv = (per(c.dim + 2 * m->kv_dim) + 1) & ~1;  // RoPE pairs stay inside one workgroup
+    rs->o = rs->down = per(c.dim);
+    rs->gu = per(c.hidden_dim);
+    constexpr int kSlots = df::kResThreads / df::kResGroup;
+    if (rs->qkv > kSlots || 2 * rs->gu > kSlots || rs->down > df::kResThreads / df::kWave) return false;
+    rs->near_stride = static_cast<int>(near_stride(c.dim));
+    // (the last thing in the allocation, on whole lines: no XCD's slots share one with another's)
+    df::u64* end = static_cast<df::u64*>(m->tagged) + tagged_count(m, df::kGridCap);
+    rs->near = reinterpret_cast<df::u64*>(reinterpret_cast<uintptr_t>(end - static_cast<size_t>(kMaxXcc) * 3 * rs->near_stride) & ~static_cast<uintptr_t>(127));
+    const int fixed = df::kResDim + b.xs_floats + df::kResHidden + 3 * df::kResHead + df::kResPositions + df::kResThreads / df::kWave * df::kResHead;
+    constexpr int kLdsFloats = (160 * 1024 - 2048) / 4;
+    const int window = 2 * df::kAttScoreFloats;  // (the sampler's, in the classifier rows' place)
+    if (fixed + window > kLdsFloats) return false;
+    rs->cls_in_lds = (kLdsFloats - fixed) / c.dim;
+    if (rs->cls_in_lds > b.cls) rs->cls_in_lds = b.cls;
+    const int cls_floats = rs->cls_in_lds * c.dim;
+    *lds_bytes = static_cast<size_t>(fixed + (cls_floats > window ? cls_floats : window)) * sizeof(float);
+    return true;
 }
 
 // Positions a one-head attention item of a head of size 64 can keep on the compute unit (att_lane_item): two 8-KiB
@@ -2858,14 +2908,15 @@ df::Tagged tagged_of(const lpp_model* m, bool generating, int lane_item_cap) {
     t.xb = p;           p += c.dim;
     t.hb = p;           p += c.hidden_dim;
     t.part = p;         p += static_cast<size_t>(c.n_heads) * splits_cap_for(m) * (m->head_size + 2);
-    t.stats = p;        p += 4u * kGridCap;
+    t.stats = p;        p += 4u * df::kGridCap;
     p = reinterpret_cast<df::u64*>((reinterpret_cast<uintptr_t>(p) + 127) & ~static_cast<uintptr_t>(127));
     t.near_hidden_stride = static_cast<int>(near_stride(c.hidden_dim));
     t.near_hb = p;      p += static_cast<size_t>(kMaxXcc) * t.near_hidden_stride;
     t.near_qkv_stride = static_cast<int>(near_stride(c.dim + 2 * m->kv_dim));
     t.near_qkv = p;     p += static_cast<size_t>(kMaxXcc) * t.near_qkv_stride;
     t.near_part_stride = static_cast<int>(near_stride(m->gqa * (m->head_size + 2)));
-    t.near_part = p;
+    t.near_part = p;    p += static_cast<size_t>(kMaxXcc) * kMaxPerXcc * t.near_part_stride;
+    t.near_stats = p;
     t.xa_chunk = t.xa_active = t.xa_ppw = 0;
     t.tickets = m->sync_words + 96;
     t.ticket_base = m->df_ticket_base;
@@ -3051,7 +3102,7 @@ lpp_status build_step_lists(lpp_model* m, const Plan& p, int which) {
 
 }  // namespace
 
-size_t dataflow_tagged_bytes(const lpp_model* m) { return tagged_count(m, kGridCap) * sizeof(df::u64); }
+size_t dataflow_tagged_bytes(const lpp_model* m) { return tagged_count(m, df::kGridCap) * sizeof(df::u64); }
 
 // A streaming wavefront covers one column slice of at most kStepLoads 1-KiB chunks per row, and a
 // row has at most one slice per streaming wavefront: rows beyond 8 x 4 KiB (8192 fp32 or 16384
@@ -3067,6 +3118,19 @@ const char* dataflow_unsupported_reason(const lpp_model* m) {
 }
 
 lpp_status dataflow_take_options(lpp_model* m, hipStream_t s);
+
+// The host's own count of what a launch does to the step record, the sequence numbers and the ticket counters.
+static void launched(lpp_model* m, int n_xcc) {
+    m->df_base += df::phases_per_token(m->cfg.n_layers);
+    if (n_xcc > 1) m->df_ticket_base += static_cast<unsigned>(m->persist_grid / n_xcc);  // one ticket per workgroup
+    if (m->df_given >= 0) {
+        m->df_pos += 1;
+    } else if (!m->df_freeze) {  // what finish_token does to the device's record
+        if (m->df_history_cap > 0 && m->df_history_len < m->df_history_cap) m->df_history_len += 1;
+        m->df_pos += 1;
+        m->df_step_index += 1;
+    }
+}
 
 template <bool kF16>
 static lpp_status launch_impl(lpp_model* m, const ph::DecodeArgs& a, hipStream_t s) {
@@ -3141,7 +3205,7 @@ static lpp_status launch_impl(lpp_model* m, const ph::DecodeArgs& a, hipStream_t
         tagged.base = 0;
     }
     if (m->persist_grid == 0) {
-        LPP_REQUIRE(p.grid <= kGridCap, "persistent decode: %d compute units exceed the statistics table", p.grid);
+        LPP_REQUIRE(p.grid <= df::kGridCap, "persistent decode: %d compute units exceed the statistics table", p.grid);
         LPP_REQUIRE(m->head_size <= df::kMaxHeadPad, "persistent decode: head_size %d exceeds %d", m->head_size,
                     df::kMaxHeadPad);
         const size_t lds_most = kLdsLimit;  // (every launch brings its own size, up to what a compute unit has)
@@ -3155,7 +3219,23 @@ static lpp_status launch_impl(lpp_model* m, const ph::DecodeArgs& a, hipStream_t
             if (per_cu < 1)
                 return fail(LPP_ERR_UNSUPPORTED, "persistent decode kernel does not fit a compute unit (LDS %zu bytes)", lds_most);
         }
+        if constexpr (!kF16)
+            for (const auto kernel : {&df::k_decode_resident<false>, &df::k_decode_resident<true>})
+                LPP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                            static_cast<int>(lds_most)));
         m->persist_grid = p.grid;
+    }
+    if constexpr (!kF16) {
+        df::Resident rs = {};
+        size_t lds_bytes = 0;
+        if (a.trace == nullptr && resident_plan(m, parked_plan.blocks, m->persist_grid, m->df_pos + 1, &rs, &lds_bytes)) {
+            if (take_forced_ticket_failure()) tagged.ticket_base -= static_cast<unsigned>(m->persist_grid / tagged.n_xcc);
+            const auto kernel = m->df_given >= 0 ? &df::k_decode_resident<true> : &df::k_decode_resident<false>;
+            hipLaunchKernelGGL(kernel, dim3(m->persist_grid), dim3(df::kResThreads), lds_bytes, s, a, tagged, parked_plan.blocks, rs);
+            LPP_CHECK_LAUNCH("k_decode_resident");
+            launched(m, tagged.n_xcc);
+            return LPP_OK;
+        }
     }
     bool moved = false;  // a weight tensor changed its address: both lists are stale
     for (int t = 0; t < LPP_T_COUNT && !moved; ++t) moved = m->df_rows_key[t] != m->w[t];
@@ -3190,15 +3270,7 @@ static lpp_status launch_impl(lpp_model* m, const ph::DecodeArgs& a, hipStream_t
     hipLaunchKernelGGL(kernel, dim3(m->persist_grid), dim3(df::kThreads), p.lds_bytes, s, a, tagged, p.blocks,
                        static_cast<const uint4*>(m->df_rows[which]), m->df_row_stride[which]);
     LPP_CHECK_LAUNCH("k_decode_dataflow");
-    m->df_base += df::phases_per_token(m->cfg.n_layers);
-    if (tagged.n_xcc > 1) m->df_ticket_base += static_cast<unsigned>(m->persist_grid / tagged.n_xcc);  // one ticket per workgroup
-    if (given) {
-        m->df_pos += 1;
-    } else if (!m->df_freeze) {  // what finish_token does to the device's record
-        if (m->df_history_cap > 0 && m->df_history_len < m->df_history_cap) m->df_history_len += 1;
-        m->df_pos += 1;
-        m->df_step_index += 1;
-    }
+    launched(m, tagged.n_xcc);
     return LPP_OK;
 }
 

@@ -489,6 +489,64 @@ def test_context_split_over_an_xcd_matches_oracle(name):
     o.close()
 
 
+RESIDENT = {
+    # name: (shape, first positions of the runs).  fp32 models whose layers fit an XCD's registers (dim to 320, hidden to 768).
+    "c1_more_layers_than_xcds": (Shape(288, 768, 10, 6, 6, 1000, 256, 10000.0, fp16=False, tied=True), (0, 62, 250)),
+    "widest_gqa": (Shape(320, 768, 3, 8, 2, 50000, 600, 500000.0, fp16=False, tied=False), (0, 126, 254, 507)),  # classifier rows beyond LDS
+    "hs64_one_kv_head": (Shape(256, 516, 2, 4, 1, 777, 520, 10000.0, fp16=False, tied=True), (0, 254, 510)),
+    "tiny_idle_workgroups": (Shape(32, 44, 9, 4, 2, 300, 64, 10000.0, fp16=False, tied=True), (0, 58)),
+    "one_layer": (Shape(64, 160, 1, 1, 1, 500, 64, 10000.0, fp16=False, tied=False), (0,)),
+}
+
+
+@pytest.mark.parametrize("name", list(RESIDENT))
+def test_layers_resident_in_an_xcd_match_the_oracle(name, test_options):
+    """The persistent path of small fp32 models, a layer to an XCD: logits and greedy ids against the oracle and against
+    the general kernel (taken by the hook, and by itself past 512 positions), NaN bit patterns past the context."""
+    shape, starts = RESIDENT[name]
+    m, o = build(shape, 19)
+    m.set_path(capi.PATH_PERSISTENT)
+    hs, nkv, L = shape.head_size, shape.n_kv_heads, shape.n_layers
+    n = L * nkv * shape.seq_len * hs
+    kfill = capi.synth_normal_f16(n, 901, 1.0).reshape(L, nkv, shape.seq_len, hs)
+    vfill = capi.synth_normal_f16(n, 902, 1.0).reshape(L, nkv, shape.seq_len, hs)
+    for start in starts:
+        k_cpu, v_cpu = kfill.copy(), vfill.copy()
+        k_cpu[:, :, start:, :] = 0
+        v_cpu[:, :, start:, :] = 0
+        o.buf("key_cache")[:] = capi.f16_to_f32(k_cpu.reshape(-1))
+        o.buf("value_cache")[:] = capi.f16_to_f32(v_cpu.reshape(-1))
+        fed, wants, tok = [], [], 5
+        positions = range(start, min(start + 8, shape.seq_len))
+        for pos in positions:
+            fed.append(tok)
+            wants.append(o.forward_logits(tok, pos))
+            tok = int(np.argmax(wants[-1]))
+        caches = []
+        for resident in (1, 0):
+            test_options(capi.OPT_DECODE_RESIDENT, resident)
+            k_gpu, v_gpu = kfill.copy(), vfill.copy()
+            k_gpu[:, :, start:, :] = 0x7e00  # binary16 NaN
+            v_gpu[:, :, start:, :] = 0x7e00
+            m.write_buffer(capi.B_KEY_CACHE, k_gpu)
+            m.write_buffer(capi.B_VALUE_CACHE, v_gpu)
+            for pos, t, want in zip(positions, fed, wants):
+                nxt = m.forward(t, pos, 0.0)
+                got = m.buffer(capi.B_LOGITS)
+                assert np.all(np.isfinite(got)), (start, pos, resident)
+                assert rel_err(got, want) <= LOGIT_TOL, (start, pos, resident)
+                assert nxt == int(np.argmax(want)), (start, pos, resident)
+            kc = m.buffer(capi.B_KEY_CACHE).reshape(k_gpu.shape)
+            assert np.array_equal(kc[:, :, :start], k_gpu[:, :, :start]) and np.all(kc[:, :, positions[-1] + 1:] == 0x7e00)
+            k = m.buffer(capi.B_K).reshape(nkv, hs)  # the run state holds the last layer's
+            assert np.array_equal(kc[L - 1, :, positions[-1]], k.astype(np.float16).view(np.uint16))
+            caches.append(kc.view(np.float16).astype(np.float32)[:, :, list(positions)])
+        # one binary16 step between the two kernels' orders of the same fp32 sums, amplified through the layers
+        assert np.max(np.abs(caches[0] - caches[1])) <= LOGIT_TOL * np.max(np.abs(caches[1]))
+    m.close()
+    o.close()
+
+
 def test_model_argument_errors():
     shape = SMALL_SHAPES["gqa4_fp16"]
     m = Model(shape)
