@@ -2335,6 +2335,14 @@ __device__ __forceinline__ void io_attention(Ctx& c, Io& io, const Lds& l, int l
 // Classifier + sampler (exchange wavefronts)
 // ---------------------------------------------------------------------------
 
+// The window is scanned once per entry: it comes into LDS (the attention score area, idle by then) ahead of the logits,
+// while the last layer is still on its way.
+__device__ __forceinline__ bool window_fits(int history_len) { return history_len <= 2 * kAttScoreFloats; }
+__device__ __forceinline__ void stage_window(const Ctx& c, float* sc, int it, int threads) {
+    if (c.penalty > 1.0f && window_fits(c.history_len))
+        for (int i = it; i < c.history_len; i += threads) reinterpret_cast<int*>(sc)[i] = c.a.history[i];
+}
+
 // Penalty, temperature and draw over the vocabulary rows r0 .. r0 + n - 1 this workgroup holds the logits lg of, by the
 // exchange wavefronts.  lg lies behind the tables at l.xs (four floats to a workgroup).
 __device__ __forceinline__ void sample_token(Ctx& c, Io& io, const Lds& l, float* lg, int r0, int n) {
@@ -2345,18 +2353,29 @@ __device__ __forceinline__ void sample_token(Ctx& c, Io& io, const Lds& l, float
     const float temperature = c.temperature, penalty = c.penalty;
     const int history_len = c.history_len;
     if (penalty > 1.0f && history_len > 0) {  // model.cpp:258-270, once per occurrence
-        // the window is scanned once per entry: bring it into LDS first (the attention score area is idle)
-        int* window = reinterpret_cast<int*>(l.sc);
-        const bool window_fits = history_len <= 2 * kAttScoreFloats;
-        if (window_fits)
-            for (int i = it; i < history_len; i += kIoThreads) window[i] = a.history[i];
-        io_sync(ctl, io);
-        const int* hist = window_fits ? window : a.history;
-        for (int i = it; i < history_len; i += kIoThreads) {
-            const int tok = hist[i];
-            if (tok < r0 || tok >= r1) continue;
-            const int count = smp::owned_count(hist, history_len, i);
-            if (count > 0) lg[tok - r0] = smp::penalise(lg[tok - r0], penalty, count);
+        io_sync(ctl, io);  // (logits and window: another thread's)
+        const int* hist = window_fits(history_len) ? reinterpret_cast<const int*>(l.sc) : a.history;
+        if (history_len <= kWave) {
+            // main.cpp's window of 64: an entry to each lane of one wavefront, one comparison across it per id that lies
+            // in these rows.  (A thread that walks the window for its entry takes a microsecond at 17 entries, and the
+            // whole device waits for the workgroup that has one.)
+            if (io.iw == 0) {
+                const int tok = lane_id() < history_len ? hist[lane_id()] : -1;
+                unsigned long long here = __builtin_amdgcn_ballot_w64(tok >= r0 && tok < r1);
+                while (here != 0ull) {
+                    const int t = __builtin_amdgcn_readlane(tok, __builtin_ctzll(here));
+                    const unsigned long long same = __builtin_amdgcn_ballot_w64(tok == t);
+                    if (lane_id() == 0) lg[t - r0] = smp::penalise(lg[t - r0], penalty, __builtin_popcountll(same));
+                    here &= ~same;
+                }
+            }
+        } else {
+            for (int i = it; i < history_len; i += kIoThreads) {
+                const int tok = hist[i];
+                if (tok < r0 || tok >= r1) continue;
+                const int count = smp::owned_count(hist, history_len, i);
+                if (count > 0) lg[tok - r0] = smp::penalise(lg[tok - r0], penalty, count);
+            }
         }
         io_sync(ctl, io);
     }
@@ -2425,22 +2444,23 @@ __device__ __forceinline__ void sample_token(Ctx& c, Io& io, const Lds& l, float
         }
         io_sync(ctl, io);
     } else {
-        float top = -INFINITY;
-        for (int w = it; w < nwg; w += kIoThreads) top = fmaxf(top, st_max[w]);
-        top = io_max(ctl, io, top);
-        float mass = 0.0f;
-        for (int w = it; w < nwg; w += kIoThreads) {
-            const float mw = (st_max[w] == -INFINITY) ? 0.0f : st_sum[w] * expf(st_max[w] - top);
-            st_cum[w] = mw;
-            mass += mw;
-        }
-        const float total = io_sum(ctl, io, mass);
-        const float r = c.r;
+        // (one wavefront: the numbers of 256 workgroups are four to a lane, and every barrier saved is a third of a microsecond)
         if (io.iw == 0) {
             // Running mass in workgroup order = index order of the CDF (model.cpp:294-301): every
             // lane takes a run of consecutive workgroups, a scan across the lanes gives each run's start.
             const int per_lane = (nwg + kWave - 1) / kWave;
             const int w0 = lane_id() * per_lane, w1 = min(nwg, w0 + per_lane);
+            float top = -INFINITY;
+            for (int w = w0; w < w1; ++w) top = fmaxf(top, st_max[w]);
+            top = wave_max(top);
+            float mass = 0.0f;
+            for (int w = w0; w < w1; ++w) {
+                const float mw = (st_max[w] == -INFINITY) ? 0.0f : st_sum[w] * expf(st_max[w] - top);
+                st_cum[w] = mw;
+                mass += mw;
+            }
+            const float total = wave_sum(mass);
+            const float r = c.r;
             float run = 0.0f;
             for (int w = w0; w < w1; ++w) run += st_cum[w] / total;
             float cum = wave_inclusive_scan(run) - run;
@@ -2451,16 +2471,18 @@ __device__ __forceinline__ void sample_token(Ctx& c, Io& io, const Lds& l, float
                 st_cum[w] = before;
                 if (target == 0x7fffffff && r < cum) target = w;
             }
-#pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) target = min(target, __shfl_xor(target, o));
+            target = wave_min(target);
             if (lane_id() == 0) {
                 ctl.target = target == 0x7fffffff ? -1 : target;
                 ctl.token = vocab - 1;  // model.cpp:302 when no bucket is reached
+                ctl.red[0][0] = top;
+                ctl.red[0][1] = total;
             }
         }
         io_sync(ctl, io);
         if (lds_ld(&ctl.target) == wg) {
             // inside the target workgroup: p_i = e_i * exp(m_w - top) / total, running sum in index order
+            const float top = lds_ld(&ctl.red[0][0]), total = lds_ld(&ctl.red[0][1]), r = c.r;
             const float f = expf(mine.v - top) / total;
             const float before = st_cum[wg];
             const int per_thread = (n + kIoThreads - 1) / kIoThreads;
@@ -2479,8 +2501,7 @@ __device__ __forceinline__ void sample_token(Ctx& c, Io& io, const Lds& l, float
                 run += lg[i] * f;
                 if (found == 0x7fffffff && r < offset + run) found = r0 + i;
             }
-#pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) found = min(found, __shfl_xor(found, o));
+            found = wave_min(found);
             if (lane_id() == 0) ctl.wave_found[io.iw] = found;
             io_sync(ctl, io);
             if (it == 0) {
@@ -2515,6 +2536,7 @@ __device__ __forceinline__ void io_classify_sample(Ctx& c, Io& io, const Lds& l)
     const int vocab = a.vocab, dim = a.dim, wg = c.wg, nwg = c.nwg;
     const int it = io.it;
     mark(c, io, 0);
+    stage_window(c, l.sc, it, kIoThreads);
     const float scale = stage_norm(c, io, l, c.t.x, nullptr, dim, c.seq(a.n_layers - 1, kDown), a.rms_final);
     mark(c, io, 2);
     wait_gemv(ctl, 4 * a.n_layers);
@@ -2875,12 +2897,10 @@ bool resident_plan(const lpp_model* m, const df::Blocks& b, int grid, int npos, 
     rs->near = reinterpret_cast<df::u64*>(reinterpret_cast<uintptr_t>(end - static_cast<size_t>(kMaxXcc) * 3 * rs->near_stride) & ~static_cast<uintptr_t>(127));
     const int fixed = df::kResDim + b.xs_floats + df::kResHidden + 3 * df::kResHead + df::kResPositions + df::kResThreads / df::kWave * df::kResHead;
     constexpr int kLdsFloats = (160 * 1024 - 2048) / 4;
-    const int window = 2 * df::kAttScoreFloats;  // (the sampler's, in the classifier rows' place)
-    if (fixed + window > kLdsFloats) return false;
+    if (fixed > kLdsFloats) return false;
     rs->cls_in_lds = (kLdsFloats - fixed) / c.dim;
     if (rs->cls_in_lds > b.cls) rs->cls_in_lds = b.cls;
-    const int cls_floats = rs->cls_in_lds * c.dim;
-    *lds_bytes = static_cast<size_t>(fixed + (cls_floats > window ? cls_floats : window)) * sizeof(float);
+    *lds_bytes = static_cast<size_t>(fixed + rs->cls_in_lds * c.dim) * sizeof(float);
     return true;
 }
 

@@ -85,26 +85,32 @@ __device__ __forceinline__ ArgMax argmax_better(ArgMax a, ArgMax b) {
     bool take_b = (b.v > a.v) || (b.v == a.v && b.i < a.i);
     return take_b ? b : a;
 }
+__device__ __forceinline__ int wave_min(int v) {
+    v = min(v, dpp_move_i<kDppXor1>(v));
+    v = min(v, dpp_move_i<kDppXor2>(v));
+    v = min(v, dpp_move_i<kDppHalfMirror>(v));
+    v = min(v, dpp_move_i<kDppMirror>(v));
+    return min(min(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+               min(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+}
+// (the value, then the smallest index that has it: lane moves inside the registers, where pairs exchanged through
+// ds_bpermute are twelve trips to the LDS, one after the other)
 __device__ __forceinline__ ArgMax wave_argmax(ArgMax m) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        ArgMax o;
-        o.v = __shfl_xor(m.v, off);
-        o.i = __shfl_xor(m.i, off);
-        m = argmax_better(m, o);
-    }
-    return m;
+    const float top = wave_max(m.v);
+    return ArgMax{top, wave_min(m.v == top ? m.i : 0x7fffffff)};
 }
 
-// Inclusive prefix sum across the wavefront (lane order).
+// Inclusive prefix sum across the wavefront (lane order): inside the rows of 16 by shifts, then the rows before.
 __device__ __forceinline__ float wave_inclusive_scan(float v) {
-    const int lane = lane_id();
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-        float up = __shfl_up(v, off);
-        if (lane >= off) v += up;
-    }
-    return v;
+    v += dpp_move<0x111>(v);  // row_shr by 1, 2, 4, 8: zero comes in
+    v += dpp_move<0x112>(v);
+    v += dpp_move<0x114>(v);
+    v += dpp_move<0x118>(v);
+    const float r0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 15));
+    const float r1 = r0 + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 31));
+    const float r2 = r1 + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 47));
+    const int row = lane_id() >> 4;
+    return v + (row == 0 ? 0.0f : row == 1 ? r0 : row == 2 ? r1 : r2);
 }
 
 __device__ __forceinline__ uintx4 load16(const void* p) {

@@ -418,6 +418,8 @@ __global__ __launch_bounds__(kResThreads) void k_decode_resident(DecodeArgs a, T
     if constexpr (!kGiven) {
         if (!requested) request_classifier();
         const float gain = tid < a.dim ? a.rms_final[tid] : 0.0f;
+        static_assert(2 * kAttScoreFloats <= kResThreads / kWave * kResHead, "the window takes the weighted values' place");
+        stage_window(c, l.part, tid, kResThreads);
         resident_await_turn(c, a.n_layers - 1);
         // In two hops, as gather_values: 256 workgroups that poll the same 18 lines across the fabric get them 2.6 to 3.3 us
         // after they were published.
@@ -461,7 +463,7 @@ __global__ __launch_bounds__(kResThreads) void k_decode_resident(DecodeArgs a, T
         if (wave_index() < kIoWaves) {
             Lds s = {};
             s.xs = l.xs;
-            s.sc = l.cls;  // (the window: the classifier's rows have been read)
+            s.sc = l.part;
             Io io{tid, wave_index(), 0u, 0, a.step};
             sample_token(c, io, s, lg, r0, n_cls);
             if (io.it == 0 && lds_peek(&ctl.error) != 0u) report_error(a.step, 2);
