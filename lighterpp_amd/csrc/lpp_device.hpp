@@ -74,6 +74,24 @@ __device__ __forceinline__ float wave_max(float v) {
     return fmaxf(fmaxf(a, b), fmaxf(c, d));
 }
 
+// v + that of the lane 16 further in each half of the wavefront, then + the other half's: lanes that are equal modulo 16.
+__device__ __forceinline__ float rows_sum(float v) {
+    const unsigned u = __float_as_uint(v);
+    const auto rows = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    const unsigned s = __float_as_uint(__uint_as_float(rows[0]) + __uint_as_float(rows[1]));
+    const auto halves = __builtin_amdgcn_permlane32_swap(s, s, false, false);
+    return __uint_as_float(halves[0]) + __uint_as_float(halves[1]);
+}
+// Sum over the lanes that are equal modulo kGroup (a power of two, at most 16): rotations inside the rows of 16, then the rows.
+template <int kGroup>
+__device__ __forceinline__ float congruent_sum(float v) {
+    if constexpr (kGroup <= 8) v += dpp_move<0x128>(v);  // row_ror by 8, 4, 2, 1
+    if constexpr (kGroup <= 4) v += dpp_move<0x124>(v);
+    if constexpr (kGroup <= 2) v += dpp_move<0x122>(v);
+    if constexpr (kGroup <= 1) v += dpp_move<0x121>(v);
+    return rows_sum(v);
+}
+
 // (value, index) pair ordered as the CPU argmax orders candidates: larger value
 // first, and among equal values the smaller index (model.cpp:275-281 keeps the
 // first maximum because it replaces only on strict >).

@@ -32,6 +32,8 @@ __device__ __forceinline__ float group_sum(float v) {
     return v;
 }
 
+using AnyFloatx4 = float __attribute__((ext_vector_type(4), aligned(4)));  // a 16-byte request at any float's address
+
 // scores: grid (position tiles, kv heads).
 template <int kGroup>
 __global__ __launch_bounds__(kAttThreads) void scores_kernel(float* __restrict__ out,
@@ -39,30 +41,37 @@ __global__ __launch_bounds__(kAttThreads) void scores_kernel(float* __restrict__
                                                              const uint16_t* __restrict__ k_layer,
                                                              int npos, int gqa, int head_size,
                                                              int seq_len) {
-    extern __shared__ __align__(16) float qs[];  // [gqa][hs_pad]
     const int kvh = blockIdx.y;
-    const int hs_pad = kGroup * 8;
-    for (int i = threadIdx.x; i < gqa * hs_pad; i += kAttThreads) {
-        const int qh = i / hs_pad, e = i - qh * hs_pad;
-        qs[i] = (e < head_size) ? q[static_cast<size_t>(kvh * gqa + qh) * head_size + e] : 0.0f;
-    }
-    __syncthreads();
-
-    constexpr int kPosPerBlock = kAttThreads / kGroup;
+    constexpr int kPosPerBlock = kAttThreads / kGroup, kHeads = 4;
     const int sub = static_cast<int>(threadIdx.x) % kGroup;
     const int t = static_cast<int>(blockIdx.x) * kPosPerBlock + static_cast<int>(threadIdx.x) / kGroup;
-    const bool live = (t < npos) && (sub * 8 < head_size);
+    const bool inside = sub * 8 < head_size, live = t < npos && inside;
     uintx4 kb = uintx4{0u, 0u, 0u, 0u};
     if (live) {
         const uint16_t* kp = k_layer + (static_cast<size_t>(kvh) * seq_len + t) * head_size + sub * 8;
         kb = load16(kp);
     }
-    for (int qh = 0; qh < gqa; ++qh) {
-        const float* qv = qs + qh * hs_pad + sub * 8;
-        floatx4 xa = *reinterpret_cast<const floatx4*>(qv);
-        floatx4 xb = *reinterpret_cast<const floatx4*>(qv + 4);
-        float s = group_sum<kGroup>(dot8(kb, xa, xb, 0.0f));
-        if (sub == 0 && t < npos) out[static_cast<size_t>(kvh * gqa + qh) * seq_len + t] = s;
+    // (the lane's part of q straight into registers, four heads requested at a time beside the K row: through LDS it is a round trip and a barrier ahead of everything.  1B shape, 100
+    // positions, in a decode step: 3.28 -> 3.08 us a launch; in requests of 4 bytes 4.0)
+    const float* qv = q + static_cast<size_t>(kvh) * gqa * head_size + (inside ? sub * 8 : 0);
+    for (int h0 = 0; h0 < gqa; h0 += kHeads) {
+        float x[kHeads][8];
+#pragma unroll
+        for (int h = 0; h < kHeads; ++h)
+#pragma unroll
+            for (int e = 0; e < 8; e += 4) {
+                const float* from = qv + static_cast<size_t>(h0 + h < gqa ? h0 + h : h0) * head_size + e;
+                const floatx4 four = *reinterpret_cast<const AnyFloatx4*>(from);
+#pragma unroll
+                for (int z = 0; z < 4; ++z) x[h][e + z] = four[z];
+            }
+#pragma unroll
+        for (int h = 0; h < kHeads; ++h) {
+            if (h0 + h >= gqa) break;
+            const floatx4 xa = {x[h][0], x[h][1], x[h][2], x[h][3]}, xb = {x[h][4], x[h][5], x[h][6], x[h][7]};
+            const float s = group_sum<kGroup>(dot8(kb, xa, xb, 0.0f));
+            if (sub == 0 && t < npos) out[static_cast<size_t>(kvh * gqa + h0 + h) * seq_len + t] = s;
+        }
     }
 }
 
@@ -141,9 +150,40 @@ __global__ __launch_bounds__(kSoftmaxThreads) void softmax_kernel(float* out, co
     for (int t = threadIdx.x; t < npos; t += kSoftmaxThreads) orow[t] = orow[t] / total;
 }
 
+// Rows of up to 512 positions: one wavefront each, eight values to a lane, no barrier.  (32 rows of 16, 100 and 256
+// positions: 3.1 -> 2.4 us a launch, of 512: 3.08 -> 2.64.)
+constexpr int kSoftmaxWave = 8 * kWave;
+__global__ __launch_bounds__(kWave) void softmax_wave_kernel(float* out, const float* x, int npos, int att_stride) {
+    const float* row = x + static_cast<size_t>(blockIdx.x) * att_stride;
+    float* orow = out + static_cast<size_t>(blockIdx.x) * att_stride;
+    float v[8], top = -INFINITY, total = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const int t = static_cast<int>(threadIdx.x) + kWave * k;
+        v[k] = t < npos ? row[t] : -INFINITY;
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) top = fmaxf(top, v[k]);
+    top = wave_max(top);
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+        if (static_cast<int>(threadIdx.x) + kWave * k < npos) {
+            v[k] = expf(v[k] - top);
+            total += v[k];
+        }
+    total = wave_sum(total);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const int t = static_cast<int>(threadIdx.x) + kWave * k;
+        if (t < npos) orow[t] = v[k] / total;
+    }
+}
+
 // aggregation: one workgroup per query head.  Lane groups stride over the
-// positions, each lane keeping 8 output columns; the per-group partial sums
-// are combined through LDS in a fixed order.
+// positions, each lane keeping 8 output columns; the groups of a wavefront meet
+// by lane moves, the wavefronts through LDS, in a fixed order.  (A tree over all
+// groups in LDS has a barrier to each of its seven levels: 1B shape, 100
+// positions, 3.40 us a launch; 3.1 this way, 3.33 with 256 threads that request eight rows each.)
 constexpr int kAggThreads = 1024;
 template <int kGroup>
 __global__ __launch_bounds__(kAggThreads) void aggregate_kernel(float* __restrict__ out,
@@ -151,9 +191,8 @@ __global__ __launch_bounds__(kAggThreads) void aggregate_kernel(float* __restric
                                                                 const float* __restrict__ att,
                                                                 int npos, int head_size, int gqa,
                                                                 int att_stride) {
-    extern __shared__ __align__(16) float part[];  // [ngroups][hs_pad]
-    constexpr int kGroups = kAggThreads / kGroup;
-    const int hs_pad = kGroup * 8;
+    constexpr int kGroups = kAggThreads / kGroup, kWaves = kAggThreads / kWave;
+    __shared__ float part[kWaves][8 * kGroup];  // a wavefront's sums, one row each
     const int h = blockIdx.x;
     const int sub = static_cast<int>(threadIdx.x) % kGroup;
     const int grp = static_cast<int>(threadIdx.x) / kGroup;
@@ -163,22 +202,25 @@ __global__ __launch_bounds__(kAggThreads) void aggregate_kernel(float* __restric
     if (sub * 8 < head_size) {
         for (int t = grp; t < npos; t += kGroups) {
             const float a = ah[t];
-            half8_t vv = as_half8(load16(vh + static_cast<size_t>(t) * head_size + sub * 8));
+            const half8_t vv = as_half8(load16(vh + static_cast<size_t>(t) * head_size + sub * 8));
 #pragma unroll
             for (int e = 0; e < 8; ++e) acc[e] = fmaf(static_cast<float>(vv[e]), a, acc[e]);
         }
     }
 #pragma unroll
-    for (int e = 0; e < 8; ++e) part[grp * hs_pad + sub * 8 + e] = acc[e];
-    __syncthreads();
-    // Tree over groups: halve until one row is left.
-    for (int width = kGroups / 2; width >= 1; width >>= 1) {
-        for (int i = threadIdx.x; i < width * hs_pad; i += kAggThreads)
-            part[i] += part[i + width * hs_pad];
-        __syncthreads();
+    for (int e = 0; e < 8; ++e) acc[e] = congruent_sum<kGroup>(acc[e]);
+    if (lane_id() < kGroup) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) part[wave_index()][sub * 8 + e] = acc[e];
     }
-    for (int e = threadIdx.x; e < head_size; e += kAggThreads)
-        out[static_cast<size_t>(h) * head_size + e] = part[e];
+    __syncthreads();
+    const int e = static_cast<int>(threadIdx.x);
+    if (e < head_size) {
+        float s = part[0][e];
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) s += part[w][e];
+        out[static_cast<size_t>(h) * head_size + e] = s;
+    }
 }
 
 // Long contexts: several workgroups per query head, each over a contiguous run of positions, so that the launch has
@@ -233,12 +275,10 @@ __global__ __launch_bounds__(kAggSplitThreads) void aggregate_split_kernel(float
             }
         }
     }
-    // The groups of a wavefront meet by lane exchange (group g with g ^ 1, then ^ 2, ...), the wavefronts through LDS,
+    // The groups of a wavefront meet by lane moves, the wavefronts through LDS,
     // added in wavefront order: always the same order, so a call repeats bit for bit.
 #pragma unroll
-    for (int off = kGroup; off < kWave; off <<= 1)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[e] += __shfl_xor(acc[e], off);
+    for (int e = 0; e < 8; ++e) acc[e] = congruent_sum<kGroup>(acc[e]);
     const int wave = static_cast<int>(threadIdx.x) / kWave;
     if (lane_id() < kGroup) {
 #pragma unroll
@@ -349,10 +389,10 @@ lpp_status lpp_multihead_gemv(float* d_out, const float* d_q, const lpp_half* d_
     }
     const int per_block = kAttThreads / g;
     const dim3 grid((npos + per_block - 1) / per_block, n_kv_heads);
-    const size_t lds = static_cast<size_t>(gqa) * g * 8 * sizeof(float);
-    LPP_REQUIRE(lds <= 65536, "lpp_multihead_gemv: %d query heads per KV head do not fit in LDS", gqa);
-#define LPP_SCORES(G)                                                                              \
-    hipLaunchKernelGGL((scores_kernel<G>), grid, dim3(kAttThreads), lds, stream(), d_out, d_q,     \
+    LPP_REQUIRE(static_cast<size_t>(gqa) * g * 8 * sizeof(float) <= 65536,
+                "lpp_multihead_gemv: %d query heads per KV head are more than 64 KiB of q", gqa);
+#define LPP_SCORES(G)                                                                             \
+    hipLaunchKernelGGL((scores_kernel<G>), grid, dim3(kAttThreads), 0, stream(), d_out, d_q,     \
                        k_layer, npos, gqa, head_size, seq_len)
     switch (g) {
         case 1: LPP_SCORES(1); break;
@@ -386,7 +426,9 @@ lpp_status lpp_softmax_multihead(float* d_out, const float* d_x, int n_heads, in
 #define LPP_SOFTMAX(KEPT)                                                                                    \
     hipLaunchKernelGGL((softmax_kernel<KEPT>), dim3(n_heads), dim3(kSoftmaxThreads), 0, stream(), d_out, d_x, \
                        seq_len, att_stride)
-    if (seq_len <= kSoftmaxThreads) LPP_SOFTMAX(1);
+    if (seq_len <= kSoftmaxWave)
+        hipLaunchKernelGGL(softmax_wave_kernel, dim3(n_heads), dim3(kWave), 0, stream(), d_out, d_x, seq_len, att_stride);
+    else if (seq_len <= kSoftmaxThreads) LPP_SOFTMAX(1);
     else if (seq_len <= 4 * kSoftmaxThreads) LPP_SOFTMAX(4);
     else if (seq_len <= 16 * kSoftmaxThreads) LPP_SOFTMAX(16);
     else LPP_SOFTMAX(0);
@@ -436,9 +478,8 @@ lpp_status lpp_aggregation_multihead(float* d_out, const lpp_half* d_v, const fl
         LPP_CHECK_LAUNCH("aggregate_split_kernel");
         return LPP_OK;
     }
-    const size_t lds = static_cast<size_t>(kAggThreads) * 8 * sizeof(float);  // 32 KiB
 #define LPP_AGG(G)                                                                                  \
-    hipLaunchKernelGGL((aggregate_kernel<G>), dim3(n_heads), dim3(kAggThreads), lds, stream(), d_out, \
+    hipLaunchKernelGGL((aggregate_kernel<G>), dim3(n_heads), dim3(kAggThreads), 0, stream(), d_out, \
                        d_v, d_att, seq_len, head_size, gqa_factor, att_stride)
     switch (g) {
         case 1: LPP_AGG(1); break;

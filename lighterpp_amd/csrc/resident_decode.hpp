@@ -85,16 +85,6 @@ struct ResidentLds {
     float* cls;    // [cls_in_lds][dim]
 };
 
-// v + that of the lane 16 further round in each half of the wavefront, then + the other half's.
-__device__ __forceinline__ float rows_sum(float v) {
-    const unsigned u = __float_as_uint(v);
-    const auto rows = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-    const unsigned s = __float_as_uint(__uint_as_float(rows[0]) + __uint_as_float(rows[1]));
-    const auto halves = __builtin_amdgcn_permlane32_swap(s, s, false, false);
-    return __uint_as_float(halves[0]) + __uint_as_float(halves[1]);
-}
-constexpr int kDppRowRor8 = 0x128;
-
 // One query head: its context in registers before q arrives, a lane per quarter of a K row and a lane per 8 dimensions
 // of a V row (model.cpp:186-198, softmax ops.cpp:56-75; the current position's k and v rounded as the cache holds them).
 __device__ __forceinline__ void resident_attention(Ctx& c, const ResidentLds& l, const Resident& rs, int layer, int h) {
@@ -187,10 +177,7 @@ __device__ __forceinline__ void resident_attention(Ctx& c, const ResidentLds& l,
     }
     // (the eight lanes of a wavefront that hold the same dimensions)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        out[e] += dpp_move<kDppRowRor8>(out[e]);
-        out[e] = rows_sum(out[e]);
-    }
+    for (int e = 0; e < 8; ++e) out[e] = congruent_sum<8>(out[e]);
     if (lane < 8) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) l.part[wave * kResHead + 8 * lane + e] = out[e];

@@ -389,6 +389,48 @@ def test_aggregation_multihead(lib, nh, gqa, hs, seq, n):
         assert np.all(np.abs(got[h] - exact) <= 0.01 * np.abs(exact) + 1e-4)
 
 
+# (rows that can be read 16 bytes at a time have a kernel each for up to 2048, 4096 and 8192 values; all others the general one)
+@pytest.mark.parametrize("n", [4, 2044, 2046, 2048, 2052, 4096, 4100, 8188, 8192, 8196])
+def test_rmsnorm_around_the_rows_of_each_kernel(lib, n):
+    """Each of the three addresses in turn at 16 bytes and off it; the word behind the row stays as it was.  Bound: the sum of
+    squares of n terms errs by at most (n / 512 + 16) ulp in the order that a workgroup takes, its root by half of that."""
+    rng = np.random.default_rng(n)
+    xs, g = rng.standard_normal(n).astype(F), (1 + 0.1 * rng.standard_normal(n)).astype(F)
+    exact = xs * g / np.sqrt(np.mean(xs.astype(np.float64) ** 2) + 1e-5)
+    for off in [(0, 0, 0), (1, 0, 0), (0, 1, 0), (0, 0, 1)]:
+        dx, dg, dout = (DB.from_numpy(np.concatenate([np.full(o, 3, F), a, np.full(1, 3, F)])) for o, a in zip(off, (xs, g, xs)))
+        capi.check(lib.lpp_rmsnorm(dout.at(4 * off[2]), dx.at(4 * off[0]), dg.at(4 * off[1]), n))
+        got = dout.to_numpy(F)
+        assert np.allclose(got[off[2]:-1], exact, rtol=(n / 1024 + 12) * np.finfo(F).eps, atol=0), off
+        assert got[-1] == 3 and (off[2] == 0 or got[0] == 3)
+
+
+@pytest.mark.parametrize("nh,nkv,hs,npos", [(8, 2, 64, 65), (9, 3, 48, 100), (5, 1, 128, 33), (16, 2, 8, 511), (12, 2, 40, 512)])
+def test_scores_and_softmax_around_a_wavefront(lib, nh, nkv, hs, npos):
+    """q at 16 bytes and off it (heads per K/V head that are no multiple of the four read at a time), then the
+    softmax of 1, npos, 512 and 513 positions (one wavefront up to 512) in rows whose rest stays as it was."""
+    seq = 520
+    rng = np.random.default_rng(nh * hs)
+    q, k16 = rng.standard_normal((nh, hs)).astype(F), rng.standard_normal((1, nkv, seq, hs)).astype(np.float16)
+    k64 = np.repeat(k16[0, :, :npos].astype(np.float64), nh // nkv, axis=0)
+    exact = np.einsum("he,hte->ht", q.astype(np.float64), k64)
+    bound = (hs + 8) * np.finfo(F).eps * np.einsum("he,hte->ht", np.abs(q).astype(np.float64), np.abs(k64))
+    dk = DB.from_numpy(k16.view(np.uint16))
+    for off in (0, 1):
+        dq, dout = DB.from_numpy(np.concatenate([np.zeros(off, F), q.ravel()])), DB.from_numpy(np.full((nh, seq), 7, F))
+        capi.check(lib.lpp_multihead_gemv(dout.ptr, dq.at(4 * off), dk.ptr, 0, npos - 1, nh, nkv, hs, seq))
+        got = dout.to_numpy(F).reshape(nh, seq)
+        assert np.all(np.abs(got[:, :npos] - exact) <= bound) and np.all(got[:, npos:] == 7)
+    x = (4 * rng.standard_normal((nh, seq))).astype(F)
+    for n in (1, npos, 512, 513):
+        d = DB.from_numpy(x)
+        capi.check(lib.lpp_softmax_multihead(d.ptr, d.ptr, nh, n, seq))
+        got = d.to_numpy(F).reshape(nh, seq)
+        p = np.exp(x[:, :n].astype(np.float64) - x[:, :n].max(1, keepdims=True))
+        assert np.allclose(got[:, :n], p / p.sum(1, keepdims=True), rtol=3e-6, atol=1e-12)
+        assert np.array_equal(bits(got[:, n:]), bits(x[:, n:]))
+
+
 # ---- sampler -----------------------------------------------------------------------------------
 
 def sample_gpu(lib, logits, temperature, penalty, history, r, topp=0.9):
