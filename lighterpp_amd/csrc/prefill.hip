@@ -184,48 +184,43 @@ __global__ __launch_bounds__(256) void k_norm_split_wide(float* __restrict__ x, 
 }
 
 // RoPE on q and k of token t (ops.cpp:34-54), q kept in fp32, k and v written to the
-// caches as binary16 at position pos0 + t (model.cpp:171-176).  With `splits` > 1, qs/ks/vs are the
+// caches as binary16 at position pos0 + t (model.cpp:171-176).  With kSplits > 1, qs/ks/vs are the
 // first of that many partial products, split_stride floats apart, and are summed in order here;
-// q receives the rotated sum either way.
-__global__ __launch_bounds__(256) void k_rope_scatter(float* __restrict__ q, const float* __restrict__ qs,
-                                                      const float* __restrict__ ks, const float* __restrict__ vs,
-                                                      const float2* __restrict__ rope, uint16_t* __restrict__ key_cache,
-                                                      uint16_t* __restrict__ value_cache, int layer, int pos0, int dim,
-                                                      int kv_dim, int hs, int seq_len, int splits, size_t split_stride) {
+// q receives the rotated sum either way.  Grid (workgroups to a row of q, k and v, tokens): a thread has
+// two pairs (16-byte loads and stores; dim, kv_dim and the head size are multiples of 4) and requests
+// all its parts before it uses the first, one round trip to memory.
+template <int kSplits>
+__global__ __launch_bounds__(256) void k_rope_scatter(float* q, const float* qs, const float* __restrict__ ks,
+                                                      const float* __restrict__ vs, const float2* __restrict__ rope,
+                                                      uint16_t* __restrict__ key_cache, uint16_t* __restrict__ value_cache,
+                                                      int layer, int pos0, int dim, int kv_dim, int hs, int seq_len,
+                                                      size_t split_stride) {
 #pragma clang fp contract(off)
-    const int t = blockIdx.x;
-    const int pos = pos0 + t;
-    const float2* cs_row = rope + static_cast<size_t>(pos) * (hs / 2);
-    // (two pairs per thread: 16-byte loads and stores; dim, kv_dim and the head size are multiples of 4)
-    auto summed = [&](const float* first, size_t at) {
-        floatx4 v = *reinterpret_cast<const floatx4*>(first + at);
-        for (int z = 1; z < splits; ++z) {
-            const floatx4 a = *reinterpret_cast<const floatx4*>(first + z * split_stride + at);
-            v = floatx4{v[0] + a[0], v[1] + a[1], v[2] + a[2], v[3] + a[3]};
-        }
-        return v;
-    };
-    for (int i = 4 * threadIdx.x; i < dim; i += 4 * blockDim.x) {
-        const size_t at = static_cast<size_t>(t) * dim + i;
-        const floatx4 cs = *reinterpret_cast<const floatx4*>(cs_row + ((i % hs) >> 1));  // (cos, sin) of two pairs
-        const floatx4 v = summed(qs, at);
-        *reinterpret_cast<floatx4*>(q + at) =
-            floatx4{v[0] * cs[0] - v[1] * cs[1], v[0] * cs[1] + v[1] * cs[0], v[2] * cs[2] - v[3] * cs[3], v[2] * cs[3] + v[3] * cs[2]};
+    const int t = blockIdx.y, pos = pos0 + t;
+    const int column = 4 * static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
+    if (column >= dim + 2 * kv_dim) return;
+    const bool is_q = column < dim, is_v = column >= dim + kv_dim;
+    const int i = is_q ? column : (is_v ? column - dim - kv_dim : column - dim);
+    const size_t at = static_cast<size_t>(t) * (is_q ? dim : kv_dim) + i;
+    const float* from = (is_q ? qs : (is_v ? vs : ks)) + at;
+    const int head = i / hs, within = i - head * hs;
+    floatx4 part[kSplits];
+#pragma unroll
+    for (int z = 0; z < kSplits; ++z) part[z] = *reinterpret_cast<const floatx4*>(from + z * split_stride);
+    const floatx4 cs = *reinterpret_cast<const floatx4*>(rope + static_cast<size_t>(pos) * (hs / 2) + (within >> 1));  // (cos, sin) of two pairs
+    floatx4 v = part[0];
+#pragma unroll
+    for (int z = 1; z < kSplits; ++z) v = floatx4{v[0] + part[z][0], v[1] + part[z][1], v[2] + part[z][2], v[3] + part[z][3]};
+    if (!is_v) v = floatx4{v[0] * cs[0] - v[1] * cs[1], v[0] * cs[1] + v[1] * cs[0], v[2] * cs[2] - v[3] * cs[3], v[2] * cs[3] + v[3] * cs[2]};
+    if (is_q) {
+        *reinterpret_cast<floatx4*>(q + at) = v;
+        return;
     }
-    for (int i = 4 * threadIdx.x; i < kv_dim; i += 4 * blockDim.x) {
-        const size_t at = static_cast<size_t>(t) * kv_dim + i;
-        const floatx4 kk = summed(ks, at), vv = summed(vs, at);
-        const floatx4 cs = *reinterpret_cast<const floatx4*>(cs_row + ((i % hs) >> 1));
-        const int head = i / hs, within = i - head * hs;
-        const size_t dst = static_cast<size_t>(layer) * kv_dim * seq_len + static_cast<size_t>(head) * seq_len * hs +
-                           static_cast<size_t>(pos) * hs + within;
-        typedef uint16_t ushort4_t __attribute__((ext_vector_type(4)));
-        *reinterpret_cast<ushort4_t*>(key_cache + dst) =
-            ushort4_t{f32_to_f16_bits(kk[0] * cs[0] - kk[1] * cs[1]), f32_to_f16_bits(kk[0] * cs[1] + kk[1] * cs[0]),
-                      f32_to_f16_bits(kk[2] * cs[2] - kk[3] * cs[3]), f32_to_f16_bits(kk[2] * cs[3] + kk[3] * cs[2])};
-        *reinterpret_cast<ushort4_t*>(value_cache + dst) =
-            ushort4_t{f32_to_f16_bits(vv[0]), f32_to_f16_bits(vv[1]), f32_to_f16_bits(vv[2]), f32_to_f16_bits(vv[3])};
-    }
+    typedef uint16_t ushort4_t __attribute__((ext_vector_type(4)));
+    uint16_t* cache = is_v ? value_cache : key_cache;
+    *reinterpret_cast<ushort4_t*>(cache + static_cast<size_t>(layer) * kv_dim * seq_len + static_cast<size_t>(head) * seq_len * hs +
+                                  static_cast<size_t>(pos) * hs + within) =
+        ushort4_t{f32_to_f16_bits(v[0]), f32_to_f16_bits(v[1]), f32_to_f16_bits(v[2]), f32_to_f16_bits(v[3])};
 }
 
 // (hi, lo)[t][u] = (g * sigmoid(g)) * up (ops.cpp:78-87); rows t >= n_tokens are zero.
@@ -1708,6 +1703,19 @@ lpp_status norm_split(float* x, const float* gain, pf::half_t* hi, pf::half_t* l
     return LPP_OK;
 }
 
+// (gemm() cuts K into 1, 2, 4 or 8 ranges)
+lpp_status rope_scatter(const lpp_model* m, float* q, const float* qs, const float* ks, const float* vs, int layer, int pos0, int n,
+                        int q_dim, int splits, size_t split_stride, hipStream_t s) {
+    const auto kernel = splits == 1   ? &pf::k_rope_scatter<1>
+                        : splits == 2 ? &pf::k_rope_scatter<2>
+                        : splits == 4 ? &pf::k_rope_scatter<4>
+                                      : &pf::k_rope_scatter<8>;
+    hipLaunchKernelGGL(kernel, dim3((q_dim + 2 * m->kv_dim + 1023) / 1024, n), dim3(256), 0, s, q, qs, ks, vs, m->rope, m->key_cache,
+                       m->value_cache, layer, pos0, q_dim, m->kv_dim, m->head_size, m->cfg.seq_len, split_stride);
+    LPP_CHECK_LAUNCH("k_rope_scatter");
+    return LPP_OK;
+}
+
 // (hi, lo)[t][u] = SwiGLU(W1 x[t], W3 x[t])[u] in one launch: the gate and the up projection of a
 // feature share a workgroup, and the activation is applied to the accumulators.
 lpp_status gate_up_swiglu(const void* w1, const void* w3, int hidden, const pf::half_t* xh, const pf::half_t* xl, int K, int t_pad,
@@ -1818,9 +1826,7 @@ lpp_status prefill_chunk(lpp_model* m, const int* tokens, int n, int pos0) {
         const float* qs = qkv_split > 1 ? partials : q;
         const float* ks = qkv_split > 1 ? partials + static_cast<size_t>(t_pad) * q_dim : k;
         const float* vs = qkv_split > 1 ? partials + static_cast<size_t>(t_pad) * (q_dim + kv) : v;
-        hipLaunchKernelGGL(pf::k_rope_scatter, dim3(n), dim3(256), 0, s, q, qs, ks, vs, m->rope, m->key_cache, m->value_cache, l,
-                           pos0, q_dim, kv, hs, c.seq_len, qkv_split, qkv_stride);
-        LPP_CHECK_LAUNCH("k_rope_scatter");
+        LPP_TRY(rope_scatter(m, q, qs, ks, vs, l, pos0, n, q_dim, qkv_split, qkv_stride, s));
         if (last_layer) break;
         // (rows n .. t_pad of hi/lo are still the zeros k_norm_split wrote: the attention writes rows < n only)
         const bool matrix_cores = 32 % m->gqa == 0 && test_option(LPP_OPT_PREFILL_MFMA_ATTENTION) != 0;
