@@ -18,6 +18,7 @@
 // operation order (ops.cpp:20-87).
 #include <cmath>
 #include <cstdlib>
+#include <type_traits>
 
 #include "lpp_device.hpp"
 #include "lpp_internal.hpp"
@@ -380,6 +381,7 @@ struct PipeJob {
     half_t* out_hi;                          // kMode 2: [tokens][out_ld]
     half_t* out_lo;
     int out_ld;
+    int live, each;  // k_gemm_pipe, kRagged: tokens there are, tokens to a tile (a multiple of 32)
 };
 
 constexpr int kPipeTripK = 64;  // columns per trip of the narrow tiles; K must be a multiple
@@ -414,7 +416,7 @@ __device__ __forceinline__ void swiglu_split4(half4_pf_t& hi, half4_pf_t& lo, co
     }
 }
 
-template <int kFi, int kTj, int kMode, int kTripK, bool kLo>
+template <int kFi, int kTj, int kMode, int kTripK, bool kLo, bool kRagged>
 __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
     typedef PipeShape<kFi, kTj, kTripK, kLo> Shape;
     constexpr int kRowsA = Shape::kRowsA, kRowsB = Shape::kRowsB, kStages = Shape::kStages, kLoads = Shape::kLoads;
@@ -444,8 +446,9 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
     const int r = lane & 31, g = lane >> 5;
     const int wf = wave & 1, wt = wave >> 1;
     constexpr int kFeaturesPerTile = kMode == 2 ? 32 * kFi : 64 * kFi;
-    const int f_base = tile_x * kFeaturesPerTile, t_base = token_tile * kRowsB;
+    const int f_base = tile_x * kFeaturesPerTile, t_base = token_tile * (kRagged ? job.each : kRowsB);
 
+    auto row_of = [&](int row) { return kRagged && row >= job.each ? job.each - 1 : row; };  // (a row past the tile's: any, nobody multiplies it)
     // what each lane requests: request q of this wavefront fills 1 KiB = rows (64 / kPieces) (wave + 4 q) .. of a stage
     const char* src[kLoads];
 #pragma unroll
@@ -463,22 +466,28 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
                 from = w + static_cast<size_t>(f_base + row) * K;
             }
         } else if (!kLo || row < kRowsA + kRowsB) {
-            from = job.xh + static_cast<size_t>(t_base + row - kRowsA) * K;
+            from = job.xh + static_cast<size_t>(t_base + row_of(row - kRowsA)) * K;
         } else {
-            from = job.xl + static_cast<size_t>(t_base + row - kRowsA - kRowsB) * K;
+            from = job.xl + static_cast<size_t>(t_base + row_of(row - kRowsA - kRowsB)) * K;
         }
         src[q] = reinterpret_cast<const char*>(from + k_first) + 16 * piece;
     }
     const unsigned lds_base = static_cast<unsigned>(reinterpret_cast<uintptr_t>(
         (__attribute__((address_space(3))) char*)pipe_lds));
     const int trips = job.k_len / kTripK;
-    auto request = [&](int trip) {
+    // (tile_columns: columns of 32 tokens that the tile has; where a request is of eight rows, those of the others are not made)
+    constexpr int kWeightLoads = kRowsA / (64 / kPieces) / 4, kColumnLoads = kPieces == 8 ? 1 : 0, kTileColumns = 2 * kTj;
+    auto made = [&](int q, int tile_columns) { return kColumnLoads == 0 || q < kWeightLoads || (q - kWeightLoads) % kTileColumns < tile_columns; };
+    auto request = [&](int trip, auto tile_columns) {
         const unsigned at = __builtin_amdgcn_readfirstlane(lds_base + (trip % kStages) * kStageBytes + wave * 1024);
         const int column = __builtin_amdgcn_readfirstlane(trip * kRowBytes);
 #pragma unroll
         for (int q = 0; q < kLoads; ++q)
-            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off\n" ::"v"(src[q] + column), "s"(at + q * 4096)
-                         : "memory");
+            if (made(q, tile_columns)) {
+                const char* from = src[q] + column;
+                const unsigned to = at + q * 4096;
+                asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off\n" ::"v"(from), "s"(to) : "memory");
+            }
     };
     // where each lane reads its fragments: row r of an MFMA tile, pieces 2 s + g of k-step s
     int a_off[kSteps], b_off[kSteps];
@@ -500,72 +509,100 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
     struct Frags {
         half8_t a[kFi], bh[kTj], bl[kTj];
     };
-    auto read = [&](Frags& f, int trip, int s) {
+    auto read = [&](Frags& f, int trip, int s, auto columns) {
+        if (columns == 0) return;
         const char* stage = pipe_lds + (trip % kStages) * kStageBytes;
 #pragma unroll
         for (int i = 0; i < kFi; ++i) f.a[i] = *reinterpret_cast<const half8_t*>(stage + a_off[s] + i * 32 * kRowBytes);
 #pragma unroll
-        for (int j = 0; j < kTj; ++j) {
+        for (int j = 0; j < columns; ++j) {
             f.bh[j] = *reinterpret_cast<const half8_t*>(stage + b_off[s] + j * 32 * kRowBytes);
             if constexpr (kLo) f.bl[j] = *reinterpret_cast<const half8_t*>(stage + b_off[s] + (kRowsB + j * 32) * kRowBytes);
         }
     };
     // (one half of a k-step's MFMAs: the weight tiles [kFi / 2 * half, kFi / 2 * (half + 1)))
-    auto multiply_half = [&](const Frags& f, int half) {
+    auto multiply_half = [&](const Frags& f, int half, auto columns) {
 #pragma unroll
         for (int i = kFi / 2 * half; i < kFi / 2 * (half + 1); ++i)
 #pragma unroll
-            for (int j = 0; j < kTj; ++j) {
+            for (int j = 0; j < columns; ++j) {
                 acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.a[i], f.bh[j], acc[i][j], 0, 0, 0);
                 if constexpr (kLo) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.a[i], f.bl[j], acc[i][j], 0, 0, 0);
             }
     };
     // (requesting wavefronts) wait until the requests of `trip` have landed: those of later trips, at
     // most kStages - 2 of them, may be in flight
-    auto landed = [&](int trip, int trips) {
+    auto landed = [&](int trip, int trips, auto tile_columns) {
+        constexpr int kMade = kLoads - kColumnLoads * (kLo ? 2 : 1) * (kTileColumns - decltype(tile_columns)::value);
         const int later = trips - 1 - trip;
-        if (kStages > 2 && later >= kStages - 2) wait_requests<(kStages - 2) * kLoads>();
+        if (kStages > 2 && later >= kStages - 2) wait_requests<(kStages - 2) * kMade>();
         else wait_requests<0>();
     };
     // One barrier per trip, inside the last k-step of the trip before: the requesting wavefronts
     // arrive when the trip's data has landed, the multiplying ones when they hold the last
     // fragments of the trip before in registers, which frees that trip's stage for the requests of
     // trip t + kStages.
-    if (requester) {
+    const int tile_end = kRagged ? min(job.live, t_base + job.each) : t_base + kRowsB;
+    auto feed = [&](auto tile_columns) {
 #pragma unroll
         for (int t = 0; t < kStages - 1; ++t)
-            if (t < trips) request(t);
-        landed(0, trips);
+            if (__builtin_expect(t < trips, 1)) request(t, tile_columns);
+        landed(0, trips, tile_columns);
         __syncthreads();
-        if (kStages - 1 < trips) request(kStages - 1);
+        if (__builtin_expect(kStages - 1 < trips, 1)) request(kStages - 1, tile_columns);
         for (int t = 0; t < trips; ++t) {
-            landed(t + 1, trips);
+            landed(t + 1, trips, tile_columns);
             __syncthreads();
-            if (t + kStages < trips) request(t + kStages);
+            if (t + kStages < trips) request(t + kStages, tile_columns);
+        }
+    };
+    if (requester) {
+        if constexpr (kRagged && kColumnLoads != 0) {
+            static_assert(kTileColumns == 4, "columns of a tile");
+            const int tile_columns = __builtin_amdgcn_readfirstlane((tile_end - t_base + 31) / 32);
+            if (tile_columns >= 4) feed(std::integral_constant<int, 4>{});
+            else if (tile_columns == 3) feed(std::integral_constant<int, 3>{});
+            else if (tile_columns == 2) feed(std::integral_constant<int, 2>{});
+            else feed(std::integral_constant<int, 1>{});
+        } else {
+            feed(std::integral_constant<int, kTileColumns>{});
         }
         return;
     }
-    Frags frags[2];
-    __syncthreads();
-    read(frags[0], 0, 0);
     // The fragments of a k-step are read from LDS behind the first half of the MFMAs of the k-step
     // before and are waited for by the k-step after: the wait the compiler places is for every
     // read in flight, so none may be in flight that has not had half a k-step to arrive.
-    for (int t = 0; t < trips; ++t) {
+    auto walk = [&](auto columns) {
+        Frags frags[2];
+        __syncthreads();
+        read(frags[0], 0, 0, columns);
+        for (int t = 0; t < trips; ++t) {
 #pragma unroll
-        for (int s = 0; s < kSteps; ++s) {
-            const Frags& cur = frags[s & 1];
-            Frags& next = frags[(s + 1) & 1];
-            const bool last = s == kSteps - 1;
-            multiply_half(cur, 0);
-            __builtin_amdgcn_sched_barrier(0);
-            // (after the last trip this reads a stage nobody uses: one path through the loop)
-            if (last) __syncthreads();
-            read(next, last ? t + 1 : t, last ? 0 : s + 1);
-            __builtin_amdgcn_sched_barrier(0);
-            multiply_half(cur, 1);
-            __builtin_amdgcn_sched_barrier(0);
+            for (int s = 0; s < kSteps; ++s) {
+                const Frags& cur = frags[s & 1];
+                Frags& next = frags[(s + 1) & 1];
+                const bool last = s == kSteps - 1;
+                multiply_half(cur, 0, columns);
+                __builtin_amdgcn_sched_barrier(0);
+                // (after the last trip this reads a stage nobody uses: one path through the loop)
+                if (last) __syncthreads();
+                read(next, last ? t + 1 : t, last ? 0 : s + 1, columns);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply_half(cur, 1, columns);
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
+    };
+    // kRagged: columns of 32 tokens that are not the tile's, or past the last token, are neither multiplied nor stored.
+    int columns = kTj;
+    if constexpr (kRagged) {
+        static_assert(kTj == 2, "columns of a wavefront: 0, 1 or 2");
+        columns = __builtin_amdgcn_readfirstlane(max(0, min(kTj, (tile_end - t_base - wt * 32 * kTj + 31) / 32)));
+        if (columns == 2) walk(std::integral_constant<int, 2>{});
+        else if (columns == 1) walk(std::integral_constant<int, 1>{});
+        else walk(std::integral_constant<int, 0>{});
+    } else {
+        walk(std::integral_constant<int, kTj>{});
     }
     // D[m][n]: a lane holds column n = lane % 32 (a token) and rows m = 8 (e / 4) + 4 (lane / 32) + e % 4 (features):
     // stored from there, an instruction would write 16 or 32 bytes to each of 32 rows of the output.  Every 32 x 32
@@ -585,6 +622,7 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
         half_t* tile = reinterpret_cast<half_t*>(room);
 #pragma unroll
         for (int j = 0; j < kTj; ++j) {
+            if (kRagged && j >= columns) break;
             half4_t h[kPairs][4], l[kPairs][4];
 #pragma unroll
             for (int i = 0; i < kPairs; ++i)
@@ -622,6 +660,7 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
         for (int i = 0; i < kFi; ++i)
 #pragma unroll
             for (int j = 0; j < kTj; ++j) {
+                if (kRagged && j >= columns) break;
 #pragma unroll
                 for (int e4 = 0; e4 < 4; ++e4)
                     *reinterpret_cast<floatx4*>(tile + r * kPitch + 8 * e4 + 4 * g) =
@@ -1354,10 +1393,10 @@ lpp_status size_lds(const void* kernel, int bytes, bool (&sized)[64]) {
     }
     return LPP_OK;
 }
-template <int kFi, int kTj, int kMode, int kTripK, bool kLo = true>
+template <int kFi, int kTj, int kMode, int kTripK, bool kLo = true, bool kRagged = false>
 lpp_status size_pipe() {
     static bool sized[64] = {};
-    return size_lds(reinterpret_cast<const void*>(&pf::k_gemm_pipe<kFi, kTj, kMode, kTripK, kLo>),
+    return size_lds(reinterpret_cast<const void*>(&pf::k_gemm_pipe<kFi, kTj, kMode, kTripK, kLo, kRagged>),
                     pf::PipeShape<kFi, kTj, kTripK, kLo>::kLdsBytes, sized);
 }
 template <int kFi, int kTj, int kMode, bool kLo>
@@ -1366,19 +1405,34 @@ lpp_status size_few() {
     return size_lds(reinterpret_cast<const void*>(&pf::k_gemm_few<kFi, kTj, kMode, kLo>), pf::FewShape<kFi, kTj, kLo>::kLdsBytes, sized);
 }
 
-template <int kFi, int kTj, int kMode, int kTripK, bool kLo>
+template <int kFi, int kTj, int kMode, int kTripK, bool kLo, bool kRagged>
 lpp_status launch_pipe_as(const pf::PipeJob& job, hipStream_t s) {
     typedef pf::PipeShape<kFi, kTj, kTripK, kLo> Shape;
-    LPP_TRY((size_pipe<kFi, kTj, kMode, kTripK, kLo>()));
+    LPP_TRY((size_pipe<kFi, kTj, kMode, kTripK, kLo, kRagged>()));
     const int per_die = (job.groups + 7) / 8;
-    hipLaunchKernelGGL((pf::k_gemm_pipe<kFi, kTj, kMode, kTripK, kLo>), dim3(per_die * 8 * job.token_tiles), dim3(512), Shape::kLdsBytes, s, job);
+    hipLaunchKernelGGL((pf::k_gemm_pipe<kFi, kTj, kMode, kTripK, kLo, kRagged>), dim3(per_die * 8 * job.token_tiles), dim3(512), Shape::kLdsBytes, s,
+                       job);
     LPP_CHECK_LAUNCH("k_gemm_pipe");
     return LPP_OK;
 }
 // (a job without a remainder array takes the kernels that neither fetch nor multiply one)
+//
+// Tokens are padded to 128.  In the exact mode the device's power is what limits the products of a full tile, and columns of
+// 32 that hold no token take as much of it: where they are a twelfth of all or more, the kernels that leave them out are
+// the faster ones (1B shape, 300 ids, 2 of 12: 2.14 -> 2.06 ms, 200, 1 of 8: 1.68 -> 1.66; of 450 ids, 1 of 16, 2.472 ->
+// 2.495).  The tokens are dealt out evenly where that makes every tile narrower: 150 ids as 96 + 54, 1.585 -> 1.495 ms; 8B
+// shape 7.73 -> 7.05.  In the fast mode only that pays: 150 ids 1.417 -> 1.280, 257 ids 1.721 -> 1.625, but 200 ids, cut
+// 128 + 72 either way, 1.454 -> 1.463.
 template <int kFi, int kTj, int kMode, int kTripK = pf::kPipeTripK>
-lpp_status launch_pipe(const pf::PipeJob& job, hipStream_t s) {
-    return job.xl != nullptr ? launch_pipe_as<kFi, kTj, kMode, kTripK, true>(job, s) : launch_pipe_as<kFi, kTj, kMode, kTripK, false>(job, s);
+lpp_status launch_pipe(const pf::PipeJob& job_in, hipStream_t s) {
+    pf::PipeJob job = job_in;
+    const int columns = (job.live + 31) / 32, all = 2 * kTj * job.token_tiles;
+    job.each = 32 * ((columns + job.token_tiles - 1) / job.token_tiles);
+    if (job.xl != nullptr ? 12 * (all - columns) >= all : job.each < 64 * kTj)
+        return job.xl != nullptr ? launch_pipe_as<kFi, kTj, kMode, kTripK, true, true>(job, s)
+                                 : launch_pipe_as<kFi, kTj, kMode, kTripK, false, true>(job, s);
+    return job.xl != nullptr ? launch_pipe_as<kFi, kTj, kMode, kTripK, true, false>(job, s)
+                             : launch_pipe_as<kFi, kTj, kMode, kTripK, false, false>(job, s);
 }
 
 template <int kFi, int kTj, int kMode, bool kLo>
@@ -1597,7 +1651,7 @@ lpp_status launch_plan(const Plan& p, const pf::PipeJob& job_in, hipStream_t s) 
 // without it they are added to y here, in order.
 lpp_status gemm(const Product* prods, int count, const pf::half_t* xh, const pf::half_t* xl, int K, int t_pad, bool accumulate,
                 hipStream_t s, float* partials = nullptr, size_t partial_floats = 0, int* left_split = nullptr,
-                bool remainder = true) {
+                bool remainder = true, int live = 0x7fffffff) {
     LPP_REQUIRE(count >= 1 && count <= 3 && t_pad > 0 && t_pad % 32 == 0 && K % 32 == 0, "prefill GEMM: %d products, K %d, T %d",
                 count, K, t_pad);
     if (left_split != nullptr) *left_split = 1;
@@ -1637,6 +1691,7 @@ lpp_status gemm(const Product* prods, int count, const pf::half_t* xh, const pf:
         job.split_stride = stride;
         job.feature_tiles = feature_tiles;
         job.token_tiles = token_tiles;
+        job.live = live < t_pad ? live : t_pad;
         job.groups = feature_tiles * splits;
         const bool add_in_kernel = accumulate && splits == 1;
         if (add_in_kernel) LPP_TRY(launch_plan<1>(plan, job, s));
@@ -1720,7 +1775,7 @@ lpp_status rope_scatter(const lpp_model* m, float* q, const float* qs, const flo
 // (hi, lo)[t][u] = SwiGLU(W1 x[t], W3 x[t])[u] in one launch: the gate and the up projection of a
 // feature share a workgroup, and the activation is applied to the accumulators.
 lpp_status gate_up_swiglu(const void* w1, const void* w3, int hidden, const pf::half_t* xh, const pf::half_t* xl, int K, int t_pad,
-                          pf::half_t* out_hi, pf::half_t* out_lo, hipStream_t s, bool remainder) {
+                          pf::half_t* out_hi, pf::half_t* out_lo, hipStream_t s, bool remainder, int live) {
     pf::PipeJob job = {};
     job.w[0] = static_cast<const pf::half_t*>(w1);
     job.w[1] = static_cast<const pf::half_t*>(w3);
@@ -1734,6 +1789,7 @@ lpp_status gate_up_swiglu(const void* w1, const void* w3, int hidden, const pf::
     const Plan plan = plan_gemm(2 * hidden, K, t_pad, 1, remainder, hidden % 128 == 0 ? 256 : 128, true);
     job.feature_tiles = 2 * hidden / plan.tile_rows();  // half of a tile's rows from either matrix
     job.token_tiles = t_pad / plan.tile_tokens();
+    job.live = live;
     job.groups = job.feature_tiles;
     job.out_hi = out_hi;
     job.out_lo = out_lo;
@@ -1822,7 +1878,7 @@ lpp_status prefill_chunk(lpp_model* m, const int* tokens, int n, int pos0) {
                                 {layer_of(LPP_T_WV, l, kv, dim), v, kv}};
         const int q_dim = last_layer ? 0 : dim;
         int qkv_split = 1;
-        LPP_TRY(gemm(qkv + (last_layer ? 1 : 0), last_layer ? 2 : 3, hi, lo, dim, t_pad, false, s, partials, room, &qkv_split, exact));
+        LPP_TRY(gemm(qkv + (last_layer ? 1 : 0), last_layer ? 2 : 3, hi, lo, dim, t_pad, false, s, partials, room, &qkv_split, exact, n));
         const size_t qkv_stride = static_cast<size_t>(t_pad) * (q_dim + 2 * kv);
         const float* qs = qkv_split > 1 ? partials : q;
         const float* ks = qkv_split > 1 ? partials + static_cast<size_t>(t_pad) * q_dim : k;
@@ -1842,22 +1898,22 @@ lpp_status prefill_chunk(lpp_model* m, const int* tokens, int n, int pos0) {
                                m->value_cache, hi, lo, l, pos0, dim, kv, hs, m->gqa, c.seq_len, n);
         LPP_CHECK_LAUNCH("k_attention");
         const Product wo = {layer_of(LPP_T_WO, l, dim, dim), x, dim};
-        LPP_TRY(gemm(&wo, 1, hi, lo, dim, t_pad, true, s, partials, room, &pending, exact));
+        LPP_TRY(gemm(&wo, 1, hi, lo, dim, t_pad, true, s, partials, room, &pending, exact, n));
         // feed-forward block, model.cpp:221-226
         LPP_TRY(norm_split(x, static_cast<const float*>(m->w[LPP_T_RMS_FFN]) + static_cast<size_t>(l) * dim, hi, lo, dim, n, t_pad, partials,
                            pending > 1 ? pending : 0, static_cast<size_t>(t_pad) * dim, s, !lean));
         if (fused_ffn) {
             LPP_TRY(gate_up_swiglu(layer_of(LPP_T_W1, l, hidden, dim), layer_of(LPP_T_W3, l, hidden, dim), hidden, hi, lo, dim, t_pad,
-                                   hi2, lo2, s, exact));
+                                   hi2, lo2, s, exact, n));
         } else {
             float *gate = partials, *up = partials + static_cast<size_t>(t_pad) * hidden;
             const Product gate_up[2] = {{layer_of(LPP_T_W1, l, hidden, dim), gate, hidden}, {layer_of(LPP_T_W3, l, hidden, dim), up, hidden}};
-            LPP_TRY(gemm(gate_up, 2, hi, lo, dim, t_pad, false, s, nullptr, 0, nullptr, exact));
+            LPP_TRY(gemm(gate_up, 2, hi, lo, dim, t_pad, false, s, nullptr, 0, nullptr, exact, n));
             hipLaunchKernelGGL(pf::k_swiglu_split, dim3((hidden + 255) / 256, t_pad), dim3(256), 0, s, gate, up, hi2, lo2, hidden, n);
             LPP_CHECK_LAUNCH("k_swiglu_split");
         }
         const Product w2 = {layer_of(LPP_T_W2, l, dim, hidden), x, dim};
-        LPP_TRY(gemm(&w2, 1, hi2, lo2, hidden, t_pad, true, s, partials, room, &pending, exact));
+        LPP_TRY(gemm(&w2, 1, hi2, lo2, hidden, t_pad, true, s, partials, room, &pending, exact, n));
     }
     LPP_HIP(hipStreamSynchronize(s));
     return LPP_OK;

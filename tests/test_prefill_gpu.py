@@ -410,6 +410,27 @@ def test_small_batches_around_the_edges_of_the_token_tiles(n, test_options):
     m.close()
 
 
+@pytest.mark.parametrize("fast", [False, True])
+@pytest.mark.parametrize("hidden,n", [*((5632, n) for n in (129, 160, 161, 192, 193, 224, 257, 288, 289, 320, 352, 416, 417, 448, 640, 704)), (128, 150), (256, 300)])
+def test_tokens_that_leave_columns_of_the_last_tiles_empty(hidden, n, fast):
+    """A prompt's first n ids against the same prompt filled up to whole tiles of 128 tokens, whose every column is
+    multiplied: what the first n leave behind depends on nothing behind them, and both sum in the same order.  Bound: one
+    binary16 step, or 2^-11 of the largest entry.  The buffers hold another, longer prompt's rows before; K of one trip too."""
+    shape = Shape(2048, hidden, 2, 32, 4, 1024, 1152, 10000.0, fp16=True, tied=True)
+    m = Model(shape)
+    m.load_synthetic(3)
+    m.set_prefill_mode(capi.PREFILL_FAST if fast else capi.PREFILL_EXACT)
+    whole = capi.synth_token_ids((n + 127) // 128 * 128, 5, shape.vocab_size)
+    m.prefill(whole, 0)
+    k0, v0, _, _ = caches(m, shape, n)
+    m.prefill(capi.synth_token_ids(1150, 9, shape.vocab_size), 0)
+    m.prefill(whole[:n], 0)
+    k, v, _, _ = caches(m, shape, n)
+    for x, y in ((k, k0), (v, v0)):
+        assert np.all(np.abs(x - y) <= np.maximum(np.abs(y) * 2.0 ** -9, np.abs(y).max() * 2.0 ** -11))
+    m.close()
+
+
 MANY_HEADS = {  # heads of 64: the attention's workgroup shapes change behind 256 and 512 ids (GQA 4: 512 and 1024); of 128: behind 512
     "hs64": Shape(2048, 256, 2, 32, 32, 512, 640, 10000.0, fp16=True, tied=True),
     "hs128": Shape(2048, 256, 2, 16, 16, 512, 640, 10000.0, fp16=True, tied=True),
