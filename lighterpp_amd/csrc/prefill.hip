@@ -1452,6 +1452,10 @@ struct Plan {
     int splits;
     int tile_rows() const { return (few ? 32 : 64) * fi; }
     int tile_tokens() const { return (few ? 32 : 64) * tj; }
+    // Tiles of k_gemm_few that hold a token (150 ids, Wo in tiles of 64: three of four; 1B shape 1.466 -> 1.455 ms);
+    // k_gemm_pipe deals the tokens out (launch_pipe).  The plan itself goes by t_pad: by the tokens it would take Wo of 130 to
+    // 160 ids for k_gemm_pipe's tile of 96, 1.5 % faster there and 2.4 % slower at 192.
+    int token_tiles(int t_pad, int live) const { return few ? (live + tile_tokens() - 1) / tile_tokens() : t_pad / tile_tokens(); }
 };
 
 // Rows the activations of n tokens are padded to: whole tiles of 128 tokens, or of 32 up to that many.
@@ -1668,8 +1672,9 @@ lpp_status gemm(const Product* prods, int count, const pf::half_t* xh, const pf:
         const size_t stride = static_cast<size_t>(t_pad) * total_n;
         int most = 1;
         while (partials != nullptr && (count == 1 || left_split != nullptr) && most < 8 && stride * 2 * most <= partial_floats) most *= 2;
+        live = live < t_pad ? live : t_pad;
         const Plan plan = plan_gemm(total_n, K, t_pad, most, remainder, step, false);
-        const int tile = plan.tile_rows(), feature_tiles = total_n / tile, token_tiles = t_pad / plan.tile_tokens(), splits = plan.splits;
+        const int tile = plan.tile_rows(), feature_tiles = total_n / tile, token_tiles = plan.token_tiles(t_pad, live), splits = plan.splits;
         pf::PipeJob job = {};
         int at = 0;
         size_t before = 0;
@@ -1691,7 +1696,7 @@ lpp_status gemm(const Product* prods, int count, const pf::half_t* xh, const pf:
         job.split_stride = stride;
         job.feature_tiles = feature_tiles;
         job.token_tiles = token_tiles;
-        job.live = live < t_pad ? live : t_pad;
+        job.live = live;
         job.groups = feature_tiles * splits;
         const bool add_in_kernel = accumulate && splits == 1;
         if (add_in_kernel) LPP_TRY(launch_plan<1>(plan, job, s));
@@ -1788,7 +1793,7 @@ lpp_status gate_up_swiglu(const void* w1, const void* w3, int hidden, const pf::
     job.k_len = K;
     const Plan plan = plan_gemm(2 * hidden, K, t_pad, 1, remainder, hidden % 128 == 0 ? 256 : 128, true);
     job.feature_tiles = 2 * hidden / plan.tile_rows();  // half of a tile's rows from either matrix
-    job.token_tiles = t_pad / plan.tile_tokens();
+    job.token_tiles = plan.token_tiles(t_pad, live);
     job.live = live;
     job.groups = job.feature_tiles;
     job.out_hi = out_hi;
