@@ -45,12 +45,12 @@ HBM_PEAK_GBS = 8000.0
 # (with a note) from the moment the file changes until the two runs are repeated
 # (profiles/persistent_decode_<workload>_pmc_hbm_traffic.txt give the commands, one file per configuration).
 KERNEL_SOURCES = {"k_decode_dataflow": ROOT / "lighterpp_amd" / "csrc" / "dataflow_decode.hip"}
-_MEASURED_SOURCE = "139941b0656e525d92eaab49db8b02a6e9f394abcff588ca3524e4c9bfb94717"
+_MEASURED_SOURCE = "76b7236c174f724f83b7831177b526cabf7e99ef3859eb7d0b2e8c4653ccf089"
 MEASURED_HBM_BYTES_PER_LAUNCH = {
-    ("c2_tinyllama_1b_fp16", "k_decode_dataflow"): (2.1260e9, _MEASURED_SOURCE),
-    ("c3_llama32_1b_fp16", "k_decode_dataflow"): (2.5143e9, _MEASURED_SOURCE),
-    ("c4_llama32_1b_longctx_fp16", "k_decode_dataflow"): (2.8007e9, _MEASURED_SOURCE),
-    ("c5_llama3_8b_fp16", "k_decode_dataflow"): (1.5185e10, _MEASURED_SOURCE),
+    ("c2_tinyllama_1b_fp16", "k_decode_dataflow"): (2.1262e9, _MEASURED_SOURCE),
+    ("c3_llama32_1b_fp16", "k_decode_dataflow"): (2.5144e9, _MEASURED_SOURCE),
+    ("c4_llama32_1b_longctx_fp16", "k_decode_dataflow"): (2.8001e9, _MEASURED_SOURCE),
+    ("c5_llama3_8b_fp16", "k_decode_dataflow"): (1.5187e10, _MEASURED_SOURCE),
 }
 
 

@@ -12,7 +12,7 @@
 // of the device, wait in LDS by the time the last layer is done.
 //
 // What bounds it: latency.  Per layer five hand-overs of 0.8 to 1.2 us (four inside an XCD, one across) and the barriers
-// and reductions between them.  15M shape, a token: 122 us before, 58 now: about 7 a layer, 8 the sampler.
+// and reductions between them.  15M shape, a token: 122 us before, 58 now: about 7 a layer, 6 the sampler.
 //
 // Every value is formed by exactly one workgroup; sums run over a lane's elements in order, then across the lanes.
 
