@@ -1279,7 +1279,12 @@ __global__ __launch_bounds__(64 * kR * kP, 2) void k_attention_mfma(const float*
     if (!seen) top = -INFINITY;
     // The wavefronts of a row meet in LDS, lane for lane: each leaves its (maximum, sum, output), and each adds up its share of
     // the output's pieces of four values in the order of the wavefronts (one wavefront for all of them, the others gone:
-    // 1B shape, 32 ids: 7.2 us a launch, 6.15 this way; 8B, 150 ids: 9.8 and 9.2).  Those past the context's last step have left nothing and are not read.
+    // 1B shape, 32 ids: 7.2 us a launch, 6.15 this way; 8B, 150 ids: 9.8 and 9.2).  Those past the context's last step have
+    // left nothing and are not read.
+    // Of the first two parts one is rounded with its weight on its own and the other added by a fused multiply-add.  Which one
+    // is written out and stays as it is, the second part for the sums and the outputs of heads of 64, the first for the
+    // outputs of heads of 128: the weights of the fast mode are no powers of two, and the other choice moves last bits of
+    // outputs, which the binary16 inputs of the products behind them turn into 8e-4 of the cache (1B shape, 2011 ids).
     __syncthreads();  // (the stages are free)
     constexpr int kFours = kHs / 8, kPart = Shape::kPartFloats;  // pieces of four values, floats of a wavefront's part
     const int parts = steps < kP ? steps : kP;
@@ -1294,7 +1299,7 @@ __global__ __launch_bounds__(64 * kR * kP, 2) void k_attention_mfma(const float*
                 floatx4{o[four >> 2][4 * (four & 3)], o[four >> 2][4 * (four & 3) + 1], o[four >> 2][4 * (four & 3) + 2], o[four >> 2][4 * (four & 3) + 3]};
     }
     __syncthreads();
-    float weight[kP], all_top = -INFINITY, total = 0.0f;
+    float weight[kP], all_top = -INFINITY, total;
 #pragma unroll
     for (int w = 0; w < kP; ++w) {
         weight[w] = w < parts ? merge[w * kPart + lane] : -INFINITY;
@@ -1302,21 +1307,27 @@ __global__ __launch_bounds__(64 * kR * kP, 2) void k_attention_mfma(const float*
     }
     if (all_top == -INFINITY) all_top = 0.0f;  // (a row past the last token)
 #pragma unroll
-    for (int w = 0; w < kP; ++w) {
-        weight[w] = __builtin_amdgcn_exp2f(weight[w] - all_top);
-        if (w < parts) total = fmaf(merge[w * kPart + 64 + lane], weight[w], total);
-    }
+    for (int w = 0; w < kP; ++w) weight[w] = __builtin_amdgcn_exp2f(weight[w] - all_top);
+    auto sum_of = [&](int w) { return w < parts ? merge[w * kPart + 64 + lane] : 0.0f; };
+    total = fmaf(sum_of(0), weight[0], sum_of(1) * weight[1]);
+#pragma unroll
+    for (int w = 2; w < kP; ++w) total = fmaf(sum_of(w), weight[w], total);
     if (!valid) return;
     const size_t base = static_cast<size_t>(my_tok) * dim + (kvh * gqa + my_head) * kHs;
     const float inv_sum = 1.0f / total;
 #pragma unroll
     for (int f = 0; f < kFours / kP; ++f) {
         const int four = wp + kP * f;
-        floatx4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+        auto part_of = [&](int w) { return *reinterpret_cast<const floatx4*>(merge + w * kPart + 128 + 256 * four + 4 * lane); };
+        const floatx4 first = part_of(0), second = parts > 1 ? part_of(1) : floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        floatx4 v;
 #pragma unroll
-        for (int w = 0; w < kP; ++w) {
+        for (int u = 0; u < 4; ++u)
+            v[u] = kHs == 64 ? fmaf(first[u], weight[0], second[u] * weight[1]) : fmaf(second[u], weight[1], first[u] * weight[0]);
+#pragma unroll
+        for (int w = 2; w < kP; ++w) {
             if (w >= parts) break;
-            const floatx4 a = *reinterpret_cast<const floatx4*>(merge + w * kPart + 128 + 256 * four + 4 * lane);
+            const floatx4 a = part_of(w);
 #pragma unroll
             for (int u = 0; u < 4; ++u) v[u] = fmaf(a[u], weight[w], v[u]);
         }

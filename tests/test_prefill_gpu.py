@@ -675,6 +675,52 @@ def test_an_infinite_value_stays_with_the_positions_that_attend_to_it(name, star
     m.close()
 
 
+@pytest.mark.parametrize("n", [8, 300, 600])
+def test_the_merge_of_two_wavefronts_rounds_the_second_part_with_its_weight(n):
+    """Fast mode, heads of 64, each workgroup shape of the attention: the second wavefront's part is rounded with its weight, the
+    first one's is added to that (fused, as its weight need not be 1).  A cached context of two steps: the first scores 0 and its values sum to -(t w) as
+    fp32 rounds it, the second scores below 0 and has the sum t and the weight w, so that the output is 0 and not what is left
+    of t w behind the rounding (one rounding of the whole would leave it).  w is exp2 of the hardware, within 4 units in
+    the last place: dimension 4 + j of a head tries the j-th neighbour of the exact value."""
+    shape = Shape(2048, 128, 2, 32, 32, 64, 768, 500000.0, fp16=True, tied=True)
+    nh, hs, L, dim, start = shape.n_heads, shape.head_size, shape.n_layers, shape.dim, 64
+    w = {t: np.zeros(shape.tensor_shape(t), np.float16 if t in MATRIX_TENSORS else F) for t in range(capi.T_WCLS)}
+    x = np.zeros((nh, hs), F)
+    x[:, 32:48] = 2.0  # mean square 1; nothing where the attention's candidates are added
+    w[capi.T_TOKEN_EMBEDDING][:] = x.ravel()
+    for t in (capi.T_RMS_ATT, capi.T_RMS_FFN, capi.T_RMS_FINAL):
+        w[t][:] = 1.0
+    w[capi.T_WQ][0, np.arange(nh) * hs + 62, 32] = 2.0  # q of every head: 4 in the pair that RoPE turns least, exact in binary16
+    w[capi.T_WO][0] = np.eye(dim) * 4096.0
+    w[capi.T_WV][1] = np.eye(dim)
+    m = Model(shape)
+    for t, a in w.items():
+        m.upload(t, a.view(np.uint16) if a.dtype == np.float16 else a)
+    m.tie_classifier()
+    m.set_prefill_mode(capi.PREFILL_FAST)
+    k, v = (np.zeros((L, nh, shape.seq_len, hs), np.float16) for _ in range(2))
+    scale = F(F(1.44269504088896341) / np.sqrt(F(hs)))
+    for h in range(nh):
+        k[0, h, 32:64, 62] = -(40 + h) / 32.0
+        t = (5, 7, 11, 13)[h % 4] * 2.0 ** 11
+        v[0, h, 32, :9] = t
+        weight = F(np.exp2(np.float64(F(4.0) * F(k[0, h, 32, 62]) * scale)))
+        for j in range(-4, 5):
+            rest = F(t) * (weight.view(np.int32) + np.int32(j)).view(F)
+            for row in range(3):  # 24 bits as three binary16 values
+                v[0, h, row, 4 + j] = -rest
+                rest = rest + F(v[0, h, row, 4 + j])
+            assert rest == 0
+    m.write_buffer(capi.B_KEY_CACHE, k.view(np.uint16))
+    m.write_buffer(capi.B_VALUE_CACHE, v.view(np.uint16))
+    m.prefill(np.arange(n) % shape.vocab_size, start)
+    # (tokens behind position 95 have a third step, which the second wavefront of two may have rescaled its part for)
+    out = caches(m, shape, min(start + n, 96))[1][1, :, start:, :9]
+    zeros = (out == 0).sum(axis=2)
+    assert np.all((zeros == 1) | (zeros == 2))  # (two neighbours of w may round t w alike)
+    m.close()
+
+
 @pytest.mark.parametrize("room", [512, -512])
 def test_prefill_where_memory_has_no_room_for_the_longest_batch(lib, room, test_options):
     """Device memory reported as too small for the buffers of more than 512 tokens, ahead of the allocation or by it: the same
