@@ -336,7 +336,8 @@ typedef struct lpp_run_result {
     int reported_count;  /* "Tokens generated" as main.cpp:229 counts: final_pos - n_prompt */
     int history_len;     /* the penalty window as the loop left it                        */
     int history[64];
-    double wall_seconds; /* steady_clock around the generation loop (main.cpp:196-226)    */
+    double wall_seconds; /* of the generation loop, its first step included (main.cpp:196-226): steady_clock, or
+                          * the device's clock where the steps are queued ahead (LPP_PATH_PERSISTENT) */
 } lpp_run_result;
 
 /* The driver loop of main.cpp:139-232 without text: prefill by decode of

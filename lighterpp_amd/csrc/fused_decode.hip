@@ -547,8 +547,10 @@ lpp_status fused_generate(lpp_model* m, int first_token, int start_pos, int n_st
 }
 
 // The steps are queued ahead of their results, the prompt's all at once: lpp_forward per id waits for each one and costs
-// the host 40 us a step (record and window uploaded, token and record read back: 166 us a step at the 15M shape, of
-// which the kernel is 125).  What the prompt's steps would sample is dropped (main.cpp:163-180): they sample nothing.
+// the host 40 us a step (record and window uploaded, token and record read back: at the 15M shape 166 us a step with a kernel
+// of 125, which is 58 by now).  What the prompt's steps would sample is dropped (main.cpp:163-180): they sample nothing.
+// The first generated step runs before the host could take the time at which it starts, so the time of the loop is the
+// device's: from behind the last given step to behind the last generated one.
 lpp_status persistent_run(lpp_model* m, const int* given, int n_given, int pos, int token, int n_steps, float temperature,
                           float penalty, const int* history, int history_len, int history_cap, const float* uniforms,
                           int* out_tokens, int* n_out, double* seconds) {
@@ -583,14 +585,16 @@ lpp_status persistent_run(lpp_model* m, const int* given, int n_given, int pos, 
         LPP_HIP(hipEventRecord(m->ev_a, s));
         if (n_steps > 0) LPP_TRY(launch_token(m, true, s));
         LPP_HIP(hipEventSynchronize(m->ev_a));
-        const auto t0 = std::chrono::steady_clock::now();
         bool again = false;
         const lpp_status st = n_steps > 0 ? generate_steps(m, n_steps, true, true, out_tokens, n_out, &again, s) : LPP_OK;
-        *seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
         m->df_uniforms_host = nullptr;
         LPP_TRY(st);
         if (!again) {
-            LPP_HIP(hipStreamSynchronize(s));
+            LPP_HIP(hipEventRecord(m->ev_b, s));
+            LPP_HIP(hipEventSynchronize(m->ev_b));
+            float ms = 0.0f;
+            LPP_HIP(hipEventElapsedTime(&ms, m->ev_a, m->ev_b));
+            *seconds = 1e-3 * ms;
             StepParams rec{};
             LPP_HIP(hipMemcpy(&rec, m->step, sizeof rec, hipMemcpyDeviceToHost));
             if (rec.error == 0) return LPP_OK;

@@ -132,7 +132,7 @@ lpp_status fused_generate(lpp_model* m, int first_token, int start_pos, int n_st
                           const float* uniforms, int* out_tokens, lpp_gen_stats* stats);
 // lpp_run's decode steps on LPP_PATH_PERSISTENT: ids given[0 .. n_given) from position pos on, for their cache entries
 // alone, then up to n_steps generated ones from `token`, until one ends the sequence (it is delivered too).
-// `uniforms`: the first generated step's draw first.  *seconds: from the last given id's end to the last generated one.
+// `uniforms`: the first generated step's draw first.  *seconds: from the last given id's end to the last generated one's.
 lpp_status persistent_run(lpp_model* m, const int* given, int n_given, int pos, int token, int n_steps, float temperature,
                           float penalty, const int* history, int history_len, int history_cap, const float* uniforms,
                           int* out_tokens, int* n_out, double* seconds);

@@ -202,6 +202,23 @@ def test_run_leaves_what_single_steps_leave(name, fail, test_options):
     b.close()
 
 
+@pytest.mark.parametrize("batched", [False, True])
+def test_the_time_of_a_reply_of_one_id_is_a_step(batched):
+    """wall_seconds holds the whole first generated step, which is launched behind the prompt's before the host can look at
+    the clock: never less than a step in a row of them takes on the device (5 % for the clocks)."""
+    shape = Shape(288, 768, 6, 6, 6, 32000, 256, 10000.0, fp16=False, tied=True) if not batched else \
+        Shape(256, 512, 2, 4, 2, 2048, 160, 500000.0, fp16=True, tied=True)
+    m = Model(shape)
+    m.load_synthetic(3)
+    m.set_path(capi.PATH_PERSISTENT)
+    prompt = capi.synth_token_ids(16, 4, shape.vocab_size)
+    step = min(m.generate(int(prompt[-1]), 15, 16)[2].device_ms / 16e3 for _ in range(5))
+    walls = [m.run(prompt, len(prompt), 0.0, batched_prefill=batched)[1].wall_seconds for _ in range(8)]
+    print(f"a step {step * 1e6:.1f} us, a reply of one id {[round(w * 1e6, 1) for w in walls]} us", flush=True)
+    assert min(walls) >= 0.95 * step
+    m.close()
+
+
 def test_run_fp16_model_persistent():
     shape = Shape(256, 512, 3, 8, 2, 2048, 160, 500000.0, fp16=True, tied=True)
     m = Model(shape)
