@@ -51,8 +51,9 @@ __global__ __launch_bounds__(kAttThreads) void scores_kernel(float* __restrict__
         const uint16_t* kp = k_layer + (static_cast<size_t>(kvh) * seq_len + t) * head_size + sub * 8;
         kb = load16(kp);
     }
-    // (the lane's part of q straight into registers, four heads requested at a time beside the K row: through LDS it is a round trip and a barrier ahead of everything.  1B shape, 100
-    // positions, in a decode step: 3.28 -> 3.08 us a launch; in requests of 4 bytes 4.0)
+    // (the lane's part of q straight into registers, four heads requested at a time beside the K row: through LDS it is a round
+    // trip and a barrier ahead of everything.  1B shape, 100 positions, in a decode step: 3.28 -> 3.08 us a launch; in
+    // requests of 4 bytes 4.0.  A lane past the head's end has zeros: its K row is zero, and an infinite q would make NaN of it)
     const float* qv = q + static_cast<size_t>(kvh) * gqa * head_size + (inside ? sub * 8 : 0);
     for (int h0 = 0; h0 < gqa; h0 += kHeads) {
         float x[kHeads][8];
@@ -63,7 +64,7 @@ __global__ __launch_bounds__(kAttThreads) void scores_kernel(float* __restrict__
                 const float* from = qv + static_cast<size_t>(h0 + h < gqa ? h0 + h : h0) * head_size + e;
                 const floatx4 four = *reinterpret_cast<const AnyFloatx4*>(from);
 #pragma unroll
-                for (int z = 0; z < 4; ++z) x[h][e + z] = four[z];
+                for (int z = 0; z < 4; ++z) x[h][e + z] = inside ? four[z] : 0.0f;
             }
 #pragma unroll
         for (int h = 0; h < kHeads; ++h) {

@@ -431,6 +431,23 @@ def test_scores_and_softmax_around_a_wavefront(lib, nh, nkv, hs, npos):
         assert np.array_equal(bits(got[:, n:]), bits(x[:, n:]))
 
 
+@pytest.mark.parametrize("hs", [8, 24, 40, 48, 64, 80, 128])
+@pytest.mark.parametrize("at", [0, 7])
+def test_scores_of_an_infinite_q(lib, hs, at):
+    """An infinite value among a head's first eight gives infinite scores of the sign of its K entry, also where the head does
+    not fill the lanes that share it; the heads beside it stay finite."""
+    nh, nkv, seq, npos = 4, 2, 48, 33
+    rng = np.random.default_rng(hs + at)
+    q, k16 = rng.standard_normal((nh, hs)).astype(F), rng.standard_normal((1, nkv, seq, hs)).astype(np.float16)
+    q[1, at], q[2, at] = np.inf, -np.inf
+    dq, dk, dout = DB.from_numpy(q), DB.from_numpy(k16.view(np.uint16)), DB.from_numpy(np.full((nh, seq), 7, F))
+    capi.check(lib.lpp_multihead_gemv(dout.ptr, dq.ptr, dk.ptr, 0, npos - 1, nh, nkv, hs, seq))
+    got = dout.to_numpy(F).reshape(nh, seq)[:, :npos]
+    assert np.array_equal(got[1], np.copysign(np.inf, k16[0, 0, :npos, at].astype(F)))
+    assert np.array_equal(got[2], np.copysign(np.inf, -k16[0, 1, :npos, at].astype(F)))
+    assert np.isfinite(got[[0, 3]]).all()
+
+
 # ---- sampler -----------------------------------------------------------------------------------
 
 def sample_gpu(lib, logits, temperature, penalty, history, r, topp=0.9):
