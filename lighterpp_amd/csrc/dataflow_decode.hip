@@ -3139,6 +3139,47 @@ const char* dataflow_unsupported_reason(const lpp_model* m) {
 
 lpp_status dataflow_take_options(lpp_model* m, hipStream_t s);
 
+// How workgroups are numbered by XCD on this device (lpp_model::df_xcc), found out once.
+static lpp_status number_by_xcc(lpp_model* m, hipStream_t s) {
+    if (m->df_xcc != 0) return LPP_OK;
+    // Workgroups are handed to the XCDs in turn.  The per-XCD hand-overs rely on every XCD getting an equal share
+    // of them, so it is measured, not assumed: anything but workgroup w on XCD (first + w) % n switches them off.
+    m->df_xcc = 1;
+    if (test_option(LPP_OPT_DECODE_XCD_HANDOVERS) != 0) {
+        const int grid = compute_units();
+        void* d = nullptr;
+        LPP_TRY(lpp_malloc(&d, static_cast<size_t>(grid) * sizeof(int)));
+        hipLaunchKernelGGL(df::k_probe_xcc, dim3(grid), dim3(df::kThreads), 0, s, static_cast<int*>(d));
+        std::vector<int> where(grid);
+        const hipError_t e = hipMemcpyAsync(where.data(), d, where.size() * sizeof(int), hipMemcpyDeviceToHost, s);
+        const hipError_t e2 = hipStreamSynchronize(s);
+        lpp_free(d);
+        LPP_HIP(e);
+        LPP_HIP(e2);
+        int n = 0;
+        for (int x : where) n = x + 1 > n ? x + 1 : n;
+        bool in_turn = n > 1 && n <= kMaxXcc && grid % n == 0;
+        for (int w = 0; w < grid && in_turn; ++w) in_turn = where[w] == (where[0] + w) % n;
+        if (in_turn) m->df_xcc = n;
+    }
+    return LPP_OK;
+}
+
+// Positions below *reach are k_decode_resident's, all others k_decode_dataflow's.
+lpp_status dataflow_resident_reach(lpp_model* m, hipStream_t s, int* reach) {
+    LPP_TRY(dataflow_take_options(m, s));
+    LPP_TRY(number_by_xcc(m, s));
+    if (m->df_resident_reach < 0) {
+        df::Resident rs = {};
+        size_t lds_bytes = 0;
+        const bool fits = m->cfg.weight_precision == LPP_WEIGHT_FP32 && dataflow_unsupported_reason(m) == nullptr &&
+                          resident_plan(m, plan_for(m, false).blocks, compute_units(), 1, &rs, &lds_bytes);
+        m->df_resident_reach = fits ? df::kResPositions : 0;
+    }
+    *reach = m->df_resident_reach;
+    return LPP_OK;
+}
+
 // The host's own count of what a launch does to the step record, the sequence numbers and the ticket counters.
 static void launched(lpp_model* m, int n_xcc) {
     m->df_base += df::phases_per_token(m->cfg.n_layers);
@@ -3156,28 +3197,7 @@ template <bool kF16>
 static lpp_status launch_impl(lpp_model* m, const ph::DecodeArgs& a, hipStream_t s) {
     if (const char* why = dataflow_unsupported_reason(m)) return fail(LPP_ERR_UNSUPPORTED, "%s", why);
     LPP_TRY(dataflow_take_options(m, s));
-    if (m->df_xcc == 0) {
-        // Workgroups are handed to the XCDs in turn.  The per-XCD hand-overs rely on every XCD getting an equal share
-        // of them, so it is measured, not assumed: anything but workgroup w on XCD (first + w) % n switches them off.
-        m->df_xcc = 1;
-        if (test_option(LPP_OPT_DECODE_XCD_HANDOVERS) != 0) {
-            const int grid = compute_units();
-            void* d = nullptr;
-            LPP_TRY(lpp_malloc(&d, static_cast<size_t>(grid) * sizeof(int)));
-            hipLaunchKernelGGL(df::k_probe_xcc, dim3(grid), dim3(df::kThreads), 0, s, static_cast<int*>(d));
-            std::vector<int> where(grid);
-            const hipError_t e = hipMemcpyAsync(where.data(), d, where.size() * sizeof(int), hipMemcpyDeviceToHost, s);
-            const hipError_t e2 = hipStreamSynchronize(s);
-            lpp_free(d);
-            LPP_HIP(e);
-            LPP_HIP(e2);
-            int n = 0;
-            for (int x : where) n = x + 1 > n ? x + 1 : n;
-            bool in_turn = n > 1 && n <= kMaxXcc && grid % n == 0;
-            for (int w = 0; w < grid && in_turn; ++w) in_turn = where[w] == (where[0] + w) % n;
-            if (in_turn) m->df_xcc = n;
-        }
-    }
+    LPP_TRY(number_by_xcc(m, s));
     // Two plans: with parked gate/up rows while only the first n_heads workgroups hold an attention item
     // (one split per head), without them at longer contexts.  Each has its own step lists.
     const bool parking_allowed = test_option(LPP_OPT_DECODE_PARKING) != 0;
@@ -3311,6 +3331,7 @@ lpp_status dataflow_forget_plans(lpp_model* m, hipStream_t s, int df_xcc) {
         m->df_calibrated = false;
     }
     m->df_xcc = df_xcc;
+    m->df_resident_reach = -1;
     m->persist_grid = 0;
     m->df_ticket_base = 0;
     if (m->sync_words != nullptr) LPP_TRY(lpp_memset(m->sync_words + 96, 0, kMaxXcc * sizeof(unsigned)));

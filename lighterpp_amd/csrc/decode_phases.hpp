@@ -873,5 +873,6 @@ lpp_status dataflow_forget_lists(lpp_model* m, hipStream_t s);
 void dataflow_partition_classes(const lpp_model* m, int* item_workgroups, int* n_xcc);
 lpp_status dataflow_after_error(lpp_model* m, int code, bool* relaunch);
 lpp_status dataflow_take_options(lpp_model* m, hipStream_t s);
+lpp_status dataflow_resident_reach(lpp_model* m, hipStream_t s, int* reach);
 
 }  // namespace lpp

@@ -21,7 +21,8 @@
 #include "decode_phases.hpp"
 
 // (defined with the timeline code at the end of the file)
-static lpp_status calibrate_gateup(lpp_model* m);
+static lpp_status calibrate_gateup(lpp_model* m, int positions);
+constexpr int kTraced = 0x7fffffff;  // (for its `positions`: whatever the position, a traced token is k_decode_dataflow's)
 
 namespace lpp {
 namespace {
@@ -397,7 +398,7 @@ static lpp_status begin_run(lpp_model* m, const StepParams& init, hipStream_t s)
 lpp_status fused_forward(lpp_model* m, int token, int pos, float temperature, float penalty, const int* history,
                          int history_len, float r, int* next_token) {
     LPP_TRY(require_fused(m));
-    LPP_TRY(calibrate_gateup(m));
+    LPP_TRY(calibrate_gateup(m, pos + 1));
     hipStream_t s = stream();
     const bool use_history = penalty > 1.0f && history != nullptr && history_len > 0;
     if (use_history)
@@ -482,7 +483,7 @@ lpp_status fused_generate(lpp_model* m, int first_token, int start_pos, int n_st
                           int* out_tokens, lpp_gen_stats* stats) {
     LPP_TRY(require_fused(m));
     if (n_steps == 0) return LPP_OK;
-    LPP_TRY(calibrate_gateup(m));
+    LPP_TRY(calibrate_gateup(m, start_pos + n_steps));
     hipStream_t s = stream();
     LPP_TRY(ensure_gen_capacity(m, n_steps));
     StepParams sp{};
@@ -559,7 +560,7 @@ lpp_status persistent_run(lpp_model* m, const int* given, int n_given, int pos, 
     for (int t = 0; t < LPP_T_COUNT; ++t)
         if (!m->w_loaded[t]) return fail(LPP_ERR_STATE, "weight tensor %d has not been uploaded", t);
     LPP_TRY(require_fused(m));
-    LPP_TRY(calibrate_gateup(m));
+    LPP_TRY(calibrate_gateup(m, pos + n_given + n_steps));
     hipStream_t s = stream();
     LPP_TRY(ensure_gen_capacity(m, n_steps > 0 ? n_steps : 1));
     StepParams sp{};
@@ -726,7 +727,7 @@ extern "C" lpp_status lpp_profile_kernels(lpp_model* m, int pos, int reps, lpp_k
         if (!m->w_loaded[t]) return fail(LPP_ERR_STATE, "weight tensor %d has not been uploaded", t);
     if (m->path == LPP_PATH_OPS) return ops_profile(m, pos, reps, out, capacity, count);
     if (!m->fused_ok) return fail(LPP_ERR_UNSUPPORTED, "fused path unavailable: %s", m->fused_why);
-    LPP_TRY(calibrate_gateup(m));
+    LPP_TRY(calibrate_gateup(m, pos + 1));
     StepParams sp{};
     sp.pos = pos;
     sp.temperature = 0.8f;
@@ -800,17 +801,21 @@ static lpp_status trace_impl(lpp_model* m, int pos, unsigned long long* out, int
 
 // The gate/up phase moves two thirds of a layer's bytes and ends when its slowest workgroup publishes.  How fast
 // a workgroup gets through it depends on the XCD it runs on (the same XCDs finish late layer after layer, up to 2 us
-// of a 31 us phase at the 8B shape) and on whether it holds an attention item.  Before a model's first token on the
-// persistent path, two tokens are therefore traced at position 256 (a few hundred positions of context, whatever
+// of a 31 us phase at the 8B shape) and on whether it holds an attention item.  Before a model's first token that
+// k_decode_dataflow decodes, two tokens are therefore traced at position 256 (a few hundred positions of context, whatever
 // the cache holds there: what a short run sees on average) and the hidden units dealt out anew: a class of
 // workgroups (those of one XCD that hold no attention item) that published d later than the median of a phase that
-// took T gets 1 - d / T of its share, and so does the rest of its XCD.  Results do not change (a hidden unit's value does not depend on who forms it); the cache rows the
-// traced tokens write at that position are put back.
-static lpp_status calibrate_gateup(lpp_model* m) {
+// took T gets 1 - d / T of its share, and so does the rest of its XCD.  Results do not change (a hidden unit's value
+// does not depend on who forms it); the cache rows the traced tokens write at that position are put back.
+// `positions`: the caller is about to decode positions below it; where all of them are k_decode_resident's, nothing is done yet.
+static lpp_status calibrate_gateup(lpp_model* m, int positions) {
     using namespace lpp;
     if (m->path != LPP_PATH_PERSISTENT) return LPP_OK;
     LPP_TRY(dataflow_take_options(m, stream()));  // (a changed test option drops the calibration with the plans)
     if (m->df_calibrated) return LPP_OK;
+    int reach = 0;
+    if (positions != kTraced) LPP_TRY(dataflow_resident_reach(m, stream(), &reach));
+    if (positions <= reach) return LPP_OK;
     m->df_calibrated = true;
     if (test_option(LPP_OPT_DECODE_CALIBRATE) == 0) return LPP_OK;
     for (int t = 0; t < LPP_T_COUNT; ++t)
@@ -899,7 +904,7 @@ extern "C" lpp_status lpp_trace_token(lpp_model* m, int pos, unsigned long long*
     if (m != nullptr && m->fused_ok) {  // (the timeline is that of the partition the decode loop runs with)
         const int saved_path = m->path;
         m->path = LPP_PATH_PERSISTENT;
-        const lpp_status st = calibrate_gateup(m);
+        const lpp_status st = calibrate_gateup(m, kTraced);
         m->path = saved_path;
         LPP_TRY(st);
     }
@@ -912,7 +917,7 @@ extern "C" lpp_status lpp_trace_token_all(lpp_model* m, int pos, unsigned long l
     if (m != nullptr && m->fused_ok) {
         const int saved_path = m->path;
         m->path = LPP_PATH_PERSISTENT;
-        const lpp_status st = calibrate_gateup(m);
+        const lpp_status st = calibrate_gateup(m, kTraced);
         m->path = saved_path;
         LPP_TRY(st);
     }

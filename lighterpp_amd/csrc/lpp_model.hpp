@@ -71,6 +71,7 @@ struct lpp_model {
     int df_given = -1;                       // >= 0: the next launch reads this id instead of the record's and samples nothing
     int df_stop = 0;                         // nonzero: the next launch does nothing if the id it is to read ends a sequence
     unsigned df_base = 0;                    // sequence-number base of the next persistent launch
+    int df_resident_reach = -1;              // positions below it are k_decode_resident's (-1: not worked out yet)
     int df_trace_stride = 0;                 // timeline words per workgroup when every workgroup is traced (0: workgroup 0 only)
     int persist_grid = 0;                    // workgroups of the persistent kernel (0: not sized yet)
     unsigned df_ticket_base = 0;             // what the per-XCD workgroup counters read before the next persistent launch

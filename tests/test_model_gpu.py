@@ -547,6 +547,47 @@ def test_layers_resident_in_an_xcd_match_the_oracle(name, test_options):
     o.close()
 
 
+def test_a_resident_model_launches_the_general_kernel_only_where_it_needs_it(test_options):
+    """A new small fp32 model's first calls are as many launches as tokens: the two traced tokens (three launches each) that deal
+    out the general kernel's hidden units come with the first call that leaves the first 512 positions.  Counted by the hook
+    that counts launches down to a failing one."""
+    shape = Shape(288, 768, 3, 6, 6, 1000, 600, 10000.0, fp16=False, tied=True)
+    launches = 0
+
+    def check(expect):
+        nonlocal launches
+        launches += expect
+        assert capi.get_test_option(capi.OPT_DECODE_FAIL_TICKETS) == 1000 - launches
+
+    for first in ("forward", "generate", "run", "profile"):
+        m = Model(shape)
+        m.load_synthetic(3)
+        m.set_path(capi.PATH_PERSISTENT)
+        test_options(capi.OPT_DECODE_FAIL_TICKETS, 1000)
+        launches = 0
+        if first == "forward":
+            m.forward(5, 511)
+            check(1)
+        elif first == "generate":
+            m.generate(5, 500, 12)
+            check(12)
+        elif first == "run":
+            m.run([5, 6, 7], 10, 0.0)
+            check(10)
+        else:
+            m.profile_kernels(20, reps=4)
+            check(4)
+        if first == "run":
+            m.generate(5, 500, 13)
+            check(13 + 6)
+        else:
+            m.forward(5, 512)
+            check(1 + 6)
+        m.generate(5, 510, 4)
+        check(4)
+        m.close()
+
+
 def test_model_argument_errors():
     shape = SMALL_SHAPES["gqa4_fp16"]
     m = Model(shape)
