@@ -2714,6 +2714,7 @@ std::vector<int> gateup_table(const lpp_model* m, const df::Blocks& b, int grid,
 }
 
 constexpr int kMaxXcc = 8;
+constexpr size_t kLdsLimit = 160 * 1024 - 2048;  // of a compute unit's LDS, the rest is for the kernels' static part
 constexpr int kMaxPerXcc = 32;  // workgroups of one XCD the XCD-wide attention split is laid out for
 
 // The split of a KV head's context over the workgroups of its XCD (att_xcd_item) at npos positions, for a plan whose
@@ -2874,14 +2875,18 @@ size_t tagged_count(const lpp_model* m, int grid_cap) {
 }
 
 // k_decode_resident's plan: whether the model's layers fit an XCD's registers as that kernel lays them out, and how the
-// rows are shared.  (Where it applies it is the faster one throughout: 15M shape 122 us a token, 58 here.  What
-// does not fit -- a binary16 model of the size has no use here yet, wider rows or more of them need a second pass over
-// the registers -- takes k_decode_dataflow, and so do longer contexts and a traced token.)
-bool resident_plan(const lpp_model* m, const df::Blocks& b, int grid, int npos, df::Resident* rs, size_t* lds_bytes) {
+// rows are shared.  Where it applies it is the faster one.  Both kernels, us a token at position 0 / 448 (k_decode_dataflow
+// second): dim 288, hidden 768, 6 layers, vocabulary 32000, 56.8 / 57.5 at 190 against 118.5 / 122.2; 320, 768, 6, 8 heads,
+// 60.0 / 66.1 against 120 / 135, with a vocabulary of 128256, whose rows no longer fit LDS, 73.1 / 78.8 against 140 / 154, one
+// such layer 38.3 / 38.2 against 60.1 / 62.3; 256, 516, 2, 25.4 / 27.0 against 46.8 / 53.6; 128, 384, 24, 160 / 184 against
+// 441 / 501; 32, 44, 9, 67.7 / 76.6 against 170 / 198, one such layer 18.2 / 19.2 against 31.2 / 34.8.
+// What does not fit -- a binary16 model of the size has no use here yet, wider rows or more of them need a second pass over
+// the registers -- takes k_decode_dataflow, and so do longer contexts (dataflow_resident_reach) and a traced token.
+bool resident_plan(const lpp_model* m, const df::Blocks& b, int grid, df::Resident* rs, size_t* lds_bytes) {
     const lpp_config& c = m->cfg;
     const int n_xcc = m->df_xcc, hs = m->head_size;
     if (test_option(LPP_OPT_DECODE_RESIDENT) == 0 || c.weight_precision != LPP_WEIGHT_FP32) return false;
-    if (n_xcc <= 1 || n_xcc > kMaxXcc || grid % n_xcc != 0 || npos > df::kResPositions) return false;
+    if (n_xcc <= 1 || n_xcc > kMaxXcc || grid % n_xcc != 0) return false;
     const int row_wgs = grid / n_xcc - c.n_heads;
     if (row_wgs < 1 || c.dim > df::kResDim || c.hidden_dim > df::kResHidden || c.dim % 4 != 0 || c.hidden_dim % 4 != 0) return false;
     if (hs > df::kResHead || hs % 8 != 0) return false;
@@ -2896,7 +2901,7 @@ bool resident_plan(const lpp_model* m, const df::Blocks& b, int grid, int npos, 
     df::u64* end = static_cast<df::u64*>(m->tagged) + tagged_count(m, df::kGridCap);
     rs->near = reinterpret_cast<df::u64*>(reinterpret_cast<uintptr_t>(end - static_cast<size_t>(kMaxXcc) * 3 * rs->near_stride) & ~static_cast<uintptr_t>(127));
     const int fixed = df::kResDim + b.xs_floats + df::kResHidden + 3 * df::kResHead + df::kResPositions + df::kResThreads / df::kWave * df::kResHead;
-    constexpr int kLdsFloats = (160 * 1024 - 2048) / 4;
+    constexpr int kLdsFloats = kLdsLimit / sizeof(float);
     if (fixed > kLdsFloats) return false;
     rs->cls_in_lds = (kLdsFloats - fixed) / c.dim;
     if (rs->cls_in_lds > b.cls) rs->cls_in_lds = b.cls;
@@ -3172,8 +3177,17 @@ lpp_status dataflow_resident_reach(lpp_model* m, hipStream_t s, int* reach) {
     if (m->df_resident_reach < 0) {
         df::Resident rs = {};
         size_t lds_bytes = 0;
-        const bool fits = m->cfg.weight_precision == LPP_WEIGHT_FP32 && dataflow_unsupported_reason(m) == nullptr &&
-                          resident_plan(m, plan_for(m, false).blocks, compute_units(), 1, &rs, &lds_bytes);
+        bool fits = m->cfg.weight_precision == LPP_WEIGHT_FP32 && dataflow_unsupported_reason(m) == nullptr &&
+                    resident_plan(m, plan_for(m, false).blocks, compute_units(), &rs, &lds_bytes);
+        // (all workgroups of a launch must be resident at once: one that would not fit a compute unit is not launched)
+        if (fits)
+            for (const auto kernel : {&df::k_decode_resident<false>, &df::k_decode_resident<true>}) {
+                int per_cu = 0;
+                LPP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                            static_cast<int>(kLdsLimit)));  // (every launch brings its own size)
+                LPP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, df::kResThreads, lds_bytes));
+                fits = fits && per_cu >= 1;
+            }
         m->df_resident_reach = fits ? df::kResPositions : 0;
     }
     *reach = m->df_resident_reach;
@@ -3209,7 +3223,6 @@ static lpp_status launch_impl(lpp_model* m, const ph::DecodeArgs& a, hipStream_t
     // workgroups of its XCD, if the shape allows and the rows fit LDS.  That plan parks gate/up rows as well, fewer
     // of them (its merge areas hold four heads), and has step lists of its own (without parking it shares those of
     // the plan without).
-    constexpr size_t kLdsLimit = 160 * 1024 - 2048;
     Plan xcd_plan = plan_for(m, false);
     XcdAttention xa = {};
     {
@@ -3259,16 +3272,14 @@ static lpp_status launch_impl(lpp_model* m, const ph::DecodeArgs& a, hipStream_t
             if (per_cu < 1)
                 return fail(LPP_ERR_UNSUPPORTED, "persistent decode kernel does not fit a compute unit (LDS %zu bytes)", lds_most);
         }
-        if constexpr (!kF16)
-            for (const auto kernel : {&df::k_decode_resident<false>, &df::k_decode_resident<true>})
-                LPP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                            static_cast<int>(lds_most)));
         m->persist_grid = p.grid;
     }
     if constexpr (!kF16) {
         df::Resident rs = {};
         size_t lds_bytes = 0;
-        if (a.trace == nullptr && resident_plan(m, parked_plan.blocks, m->persist_grid, m->df_pos + 1, &rs, &lds_bytes)) {
+        int reach = 0;
+        if (a.trace == nullptr) LPP_TRY(dataflow_resident_reach(m, s, &reach));
+        if (m->df_pos < reach && resident_plan(m, parked_plan.blocks, m->persist_grid, &rs, &lds_bytes)) {
             if (take_forced_ticket_failure()) tagged.ticket_base -= static_cast<unsigned>(m->persist_grid / tagged.n_xcc);
             const auto kernel = m->df_given >= 0 ? &df::k_decode_resident<true> : &df::k_decode_resident<false>;
             hipLaunchKernelGGL(kernel, dim3(m->persist_grid), dim3(df::kResThreads), lds_bytes, s, a, tagged, parked_plan.blocks, rs);
