@@ -2890,6 +2890,8 @@ bool resident_plan(const lpp_model* m, const df::Blocks& b, int grid, df::Reside
     const int row_wgs = grid / n_xcc - c.n_heads;
     if (row_wgs < 1 || c.dim > df::kResDim || c.hidden_dim > df::kResHidden || c.dim % 4 != 0 || c.hidden_dim % 4 != 0) return false;
     if (hs > df::kResHead || hs % 8 != 0) return false;
+    // (a workgroup's logits lie behind the sampler's tables, four floats to a workgroup, in the area that x is still read from)
+    if (4 * grid < df::kResDim) return false;
     auto per = [&](int total) { return (total + row_wgs - 1) / row_wgs; };
     rs->qkv = (per(c.dim + 2 * m->kv_dim) + 1) & ~1;  // RoPE pairs stay inside one workgroup
     rs->o = rs->down = per(c.dim);
