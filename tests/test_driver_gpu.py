@@ -134,9 +134,13 @@ def test_run_with_temperature_and_long_prompt(path):
     m.close()
 
 QUEUED = {
-    "mha_fp32": Shape(288, 768, 3, 6, 6, 1000, 96, 10000.0, fp16=False, tied=True),
-    "gqa4_8kv": Shape(2048, 1024, 2, 32, 8, 500, 640, 500000.0, fp16=True, tied=True),   # parked rows, one-pass item
-    "hs128_8kv": Shape(1024, 512, 1, 8, 8, 3000, 300, 10000.0, fp16=True, tied=True),     # context split from 96 positions on
+    # name: (shape, prompt ids, steps, the earliest generated step that ends the sequence)
+    "mha_fp32": (Shape(288, 768, 3, 6, 6, 1000, 96, 10000.0, fp16=False, tied=True), 7, 40, 9),          # a layer to an XCD
+    "mha_fp32_general": (Shape(288, 768, 3, 6, 6, 1000, 96, 10000.0, fp16=False, tied=True), 7, 40, 9),  # (that kernel off)
+    "mha_fp32_past_512": (Shape(288, 768, 2, 6, 6, 1000, 640, 10000.0, fp16=False, tied=True), 516, 560, 9),  # one kernel, then the other
+    "fp32_sliced": (Shape(1536, 2304, 2, 12, 4, 600, 96, 10000.0, fp16=False, tied=True), 7, 40, 9),     # rows of several slices
+    "gqa4_8kv": (Shape(2048, 1024, 2, 32, 8, 500, 640, 500000.0, fp16=True, tied=True), 7, 40, 9),       # parked rows, one-pass item
+    "hs128_8kv": (Shape(1024, 512, 1, 8, 8, 3000, 300, 10000.0, fp16=True, tied=True), 130, 170, 2),      # context split from 96 positions on
 }
 
 
@@ -146,9 +150,9 @@ def test_run_leaves_what_single_steps_leave(name, fail, test_options):
     """lpp_run on the persistent path queues its steps ahead (the prompt's end with their k and v rows, a launch behind an
     id that ends the sequence does nothing): ids, cache and last logits are those of one lpp_forward per id, bit for
     bit, also where the sequence ends early; where a launch fails its ticket check, to the rounding of the plan that follows."""
-    shape = QUEUED[name]
+    shape, n_prompt, steps, end_at = QUEUED[name]
     w = weights(shape, 5)
-    n_prompt, steps, end_at = (130, 170, 2) if name == "hs128_8kv" else (7, 40, 9)
+    test_options(capi.OPT_DECODE_RESIDENT, int(name != "mha_fp32_general"))
     prompt = [int(t) if t not in EOS else 3 for t in capi.synth_token_ids(n_prompt, 4, shape.vocab_size)]
 
     def loaded():
@@ -166,6 +170,8 @@ def test_run_leaves_what_single_steps_leave(name, fail, test_options):
     last = next(int(t) for i, t in enumerate(ids) if i >= end_at and t not in prompt and t not in ids[:i])
     w[capi.T_TOKEN_EMBEDDING][[2, last]] = w[capi.T_TOKEN_EMBEDDING][[last, 2]]
     a, b = loaded(), loaded()
+    for m in (a, b):  # (the launches that deal out the hidden units come with it: none of those is the one that fails)
+        m.forward(3, shape.seq_len - 1, 0.0)
     if fail:
         test_options(capi.OPT_DECODE_FAIL_TICKETS, n_prompt - 2 if fail == 3 else n_prompt + 3)
     ids, res = a.run(prompt, steps, 0.0)

@@ -161,6 +161,38 @@ def test_generate_sampled_matches_oracle(path):
     o.close()
 
 
+@pytest.mark.parametrize("cap", [63, 65, 100, 1100])
+@pytest.mark.parametrize("name", ["fp32_layer_to_an_xcd", "fp16"])
+def test_a_penalty_window_longer_than_a_wavefront(name, cap):
+    """The persistent path's sampler takes a window of up to 64 entries an entry to a lane, longer ones by threads that walk it,
+    in LDS up to 1024 entries: windows that start one short of their capacity and slide, every id in them several times."""
+    shape = (Shape(288, 768, 2, 6, 6, 1000, 1200, 10000.0, fp16=False, tied=True) if name != "fp16" else
+             Shape(256, 512, 2, 8, 2, 1000, 1200, 500000.0, fp16=True, tied=True))
+    m, o = build(shape, 17)
+    m.set_path(capi.PATH_PERSISTENT)
+    steps, tok = 24, 42
+    draws = capi.synth_uniform_f32(steps, 99)
+    hist = [int(t) % (cap // 3) for t in capi.synth_token_ids(cap - 1, 5, shape.vocab_size)]
+    for temperature in (0.8, 0.0):
+        toks, after, _ = m.generate(tok, 0, steps, temperature=temperature, penalty=1.3, history=hist, history_cap=cap, uniforms=draws)
+        window, fed, agree = list(hist), tok, 0
+        for i in range(steps):
+            o.forward_logits(fed, i)
+            if temperature == 0.0:
+                want, z = ob.orc_sample(o.buf("logits"), 0.0, 1.0, 1.3, window, 0.0)
+                gap = float(z[want] - z[toks[i]]) / float(np.max(np.abs(z)))
+            else:
+                want, lo, hi = ob.orc_sample_cdf(o.buf("logits"), temperature, 1.3, window, float(draws[i]))
+                gap = min(abs(float(draws[i]) - lo), abs(float(draws[i]) - hi))
+            agree += int(want == toks[i])
+            assert want == toks[i] or gap < LOGIT_TOL, (temperature, i, gap)
+            fed = int(toks[i])
+            window = (window + [fed])[-cap:]
+        assert agree >= steps - 1 and after == window
+    m.close()
+    o.close()
+
+
 def test_generate_paths_agree_and_window_wraps():
     """Fused generate == operator-path generate token for token (greedy, penalty on,
     window of 5 so that it wraps many times)."""
