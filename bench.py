@@ -325,6 +325,8 @@ def main() -> int:
                         mean_handover_cost_us=round(summary["mean_handover_cost_us"], 2),
                         note="every workgroup writes eight time marks per phase: the traced token is slower than "
                              "an untraced one (avg_launch_us), the proportions are what this is for")
+        if roofline["kernel"] != "k_decode_dataflow":
+            timeline["note"] = "of k_decode_dataflow, which has the marks: this model's own tokens are " + roofline["kernel"] + "'s"
 
     parity = None
     if args.parity_steps > 0:

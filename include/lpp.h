@@ -432,6 +432,9 @@ lpp_status lpp_profile_kernels(lpp_model *m, int pos, int reps, lpp_kernel_time 
  * finished.  Attention (first work item): 0 entered, 5 q/k/v received, 1 = 6 = 2
  * shared through LDS, 7 context walked, 3 lane groups and wavefronts merged,
  * 4 published.
+ * The marks are those of k_decode_dataflow: a traced token runs in it also where the
+ * model's own tokens are k_decode_resident's (small fp32 models, up to 512 positions;
+ * lpp_profile_kernels names the kernel).
  * *count = marks * phases, *marks_per_phase = marks. */
 lpp_status lpp_trace_token(lpp_model *m, int pos, unsigned long long *out, int capacity, int *count,
                            int *marks_per_phase);

@@ -671,7 +671,9 @@ lpp_status profile_impl(lpp_model* m, int pos, int reps, lpp_kernel_time* out, i
         LPP_HIP(hipEventSynchronize(m->ev_b));
         float total = 0.0f;
         LPP_HIP(hipEventElapsedTime(&total, m->ev_a, m->ev_b));
-        add("k_decode_dataflow", 1, static_cast<double>(total) / reps, token_bytes);
+        int reach = 0;
+        LPP_TRY(dataflow_resident_reach(m, s, &reach));
+        add(pos < reach ? "k_decode_resident" : "k_decode_dataflow", 1, static_cast<double>(total) / reps, token_bytes);
         *count = n < capacity ? n : capacity;
         return LPP_OK;
     }

@@ -620,6 +620,17 @@ def test_a_resident_model_launches_the_general_kernel_only_where_it_needs_it(tes
         m.close()
 
 
+def test_profile_names_the_kernel_that_decodes(test_options):
+    """lpp_profile_kernels on the persistent path: a small fp32 model's tokens are k_decode_resident's up to 512 positions."""
+    m = Model(Shape(288, 768, 2, 6, 6, 1000, 600, 10000.0, fp16=False, tied=True))
+    m.load_synthetic(3)
+    m.set_path(capi.PATH_PERSISTENT)
+    for resident, pos, want in [(1, 0, "k_decode_resident"), (1, 511, "k_decode_resident"), (1, 512, "k_decode_dataflow"), (0, 0, "k_decode_dataflow")]:
+        test_options(capi.OPT_DECODE_RESIDENT, resident)
+        assert [row[0] for row in m.profile_kernels(pos, reps=2)] == [want], (resident, pos)
+    m.close()
+
+
 def test_model_argument_errors():
     shape = SMALL_SHAPES["gqa4_fp16"]
     m = Model(shape)
