@@ -40,11 +40,12 @@ sys.path.insert(0, str(ROOT / "tests"))
 
 HBM_PEAK_GBS = 8000.0
 # (config, kernel) -> (HBM bytes fetched + written per launch from rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, SHA-256 of
-# the kernel's source file when the two counter runs were made).  Hardware counters cannot be read in-process, so
-# the figure is a constant; it is quoted only while the kernel's source is the one that was measured, and is null
-# (with a note) from the moment the file changes until the two runs are repeated
+# the files that hold the kernel's device code when the two counter runs were made).  Hardware counters cannot be read in-process, so
+# the figure is a constant; it is quoted only while the kernel's code is the one that was measured, and is null
+# (with a note) from the moment a file changes until the two runs are repeated
 # (profiles/persistent_decode_<workload>_pmc_hbm_traffic.txt give the commands, one file per configuration).
-KERNEL_SOURCES = {"k_decode_dataflow": ROOT / "lighterpp_amd" / "csrc" / "dataflow_decode.hip"}
+_CSRC = ROOT / "lighterpp_amd" / "csrc"
+KERNEL_SOURCES = {"k_decode_dataflow": [_CSRC / f for f in ("dataflow_decode.hip", "decode_phases.hpp", "lpp_device.hpp", "sampler.hpp")]}
 _MEASURED_SOURCE = "76b7236c174f724f83b7831177b526cabf7e99ef3859eb7d0b2e8c4653ccf089"
 MEASURED_HBM_BYTES_PER_LAUNCH = {
     ("c2_tinyllama_1b_fp16", "k_decode_dataflow"): (2.1262e9, _MEASURED_SOURCE),
@@ -54,16 +55,24 @@ MEASURED_HBM_BYTES_PER_LAUNCH = {
 }
 
 
+def source_digest(kernel: str):
+    """SHA-256 over the kernel's files, or None if one is not there."""
+    import hashlib
+    files = KERNEL_SOURCES.get(kernel, [])
+    if not files or not all(f.exists() for f in files):
+        return None
+    return hashlib.sha256(b"".join(f.read_bytes() for f in files)).hexdigest()
+
+
 def measured_traffic(config: str, kernel: str):
     """(bytes per launch or None, note or None) for the dominant kernel."""
-    import hashlib
     entry = MEASURED_HBM_BYTES_PER_LAUNCH.get((config, kernel))
     if entry is None:
         return None, "no counter run for this configuration"
-    src = KERNEL_SOURCES.get(kernel)
-    if src is None or not src.exists():
+    digest = source_digest(kernel)
+    if digest is None:
         return None, "kernel source not found: counter figure not quoted"
-    if hashlib.sha256(src.read_bytes()).hexdigest() != entry[1]:
+    if digest != entry[1]:
         return None, "kernel source changed since the counter runs: repeat them"
     return entry[0], None
 

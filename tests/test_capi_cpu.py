@@ -149,3 +149,29 @@ def test_bytes_per_token_matches_published_plan():
     assert abs(avg(CONFIGS["c5_llama3_8b_fp16"], 32, 1024) - 15.082) < 2e-2
     assert CONFIGS["c3_llama32_1b_fp16"].matrix_params() == 1_235_746_816 or \
         abs(CONFIGS["c3_llama32_1b_fp16"].matrix_params() / 1e6 - 1235.7) < 0.1
+
+
+def test_counter_figures_are_quoted_for_the_measured_device_code_only(tmp_path, monkeypatch):
+    """bench.py's HBM bytes per launch are constants of counter runs: null as soon as one of the files with the kernel's device
+    code, headers included, is another."""
+    import sys
+    from pathlib import Path
+    monkeypatch.syspath_prepend(str(Path(__file__).resolve().parents[1]))
+    monkeypatch.setattr(sys, "argv", ["bench.py"])
+    import bench
+    csrc = Path(bench.__file__).parent / "lighterpp_amd" / "csrc"
+    names = ("dataflow_decode.hip", "decode_phases.hpp", "lpp_device.hpp", "sampler.hpp")
+    for config, kernel in bench.MEASURED_HBM_BYTES_PER_LAUNCH:
+        assert [f.name for f in bench.KERNEL_SOURCES[kernel]] == list(names)
+        copies = [tmp_path / n for n in names]
+        for f in copies:
+            f.write_bytes((csrc / f.name).read_bytes())
+        monkeypatch.setitem(bench.KERNEL_SOURCES, kernel, copies)
+        monkeypatch.setitem(bench.MEASURED_HBM_BYTES_PER_LAUNCH, (config, kernel), (1.0, bench.source_digest(kernel)))
+        assert bench.measured_traffic(config, kernel) == (1.0, None)
+        for f in copies:
+            kept = f.read_bytes()
+            f.write_bytes(kept + b" ")
+            assert bench.measured_traffic(config, kernel)[0] is None
+            f.write_bytes(kept)
+        monkeypatch.setitem(bench.KERNEL_SOURCES, kernel, [csrc / n for n in names])
