@@ -35,42 +35,55 @@ __device__ __forceinline__ float group_sum(float v) {
 using AnyFloatx4 = float __attribute__((ext_vector_type(4), aligned(4)));  // a 16-byte request at any float's address
 
 // scores: grid (position tiles, kv heads).
-template <int kGroup>
+// kStaged: q through LDS, read once by a workgroup, instead of straight into each lane's registers, eight 16-byte requests beside
+// the K row's one.  Same products in the same order.  Through LDS it is a round trip and a barrier ahead of everything, which is
+// what a launch of few workgroups consists of (1B shape, 100 positions, in a decode step: 3.28 us a launch, 3.08 from registers;
+// in requests of 4 bytes 4.0); with several workgroups to a compute unit the requests for q are what its L1 is busy with
+// (lpp_multihead_gemv has both sides' times).
+template <int kGroup, bool kStaged>
 __global__ __launch_bounds__(kAttThreads) void scores_kernel(float* __restrict__ out,
                                                              const float* __restrict__ q,
                                                              const uint16_t* __restrict__ k_layer,
                                                              int npos, int gqa, int head_size,
                                                              int seq_len) {
+    extern __shared__ __align__(16) float qs[];  // kStaged: [gqa][hs_pad], zeros past the head's end
     const int kvh = blockIdx.y;
-    constexpr int kPosPerBlock = kAttThreads / kGroup, kHeads = 4;
+    constexpr int kPosPerBlock = kAttThreads / kGroup, kHeads = kStaged ? 1 : 4, kPad = kGroup * 8;
     const int sub = static_cast<int>(threadIdx.x) % kGroup;
     const int t = static_cast<int>(blockIdx.x) * kPosPerBlock + static_cast<int>(threadIdx.x) / kGroup;
     const bool inside = sub * 8 < head_size, live = t < npos && inside;
+    if constexpr (kStaged) {
+        for (int i = threadIdx.x; i < gqa * kPad; i += kAttThreads) {
+            const int h = i / kPad, e = i - h * kPad;
+            qs[i] = e < head_size ? q[static_cast<size_t>(kvh * gqa + h) * head_size + e] : 0.0f;
+        }
+        __syncthreads();
+    }
     uintx4 kb = uintx4{0u, 0u, 0u, 0u};
     if (live) {
         const uint16_t* kp = k_layer + (static_cast<size_t>(kvh) * seq_len + t) * head_size + sub * 8;
         kb = load16(kp);
     }
-    // (the lane's part of q straight into registers, four heads requested at a time beside the K row: through LDS it is a round
-    // trip and a barrier ahead of everything.  1B shape, 100 positions, in a decode step: 3.28 -> 3.08 us a launch; in
-    // requests of 4 bytes 4.0.  A lane past the head's end has zeros: its K row is zero, and an infinite q would make NaN of it)
+    // (a lane past the head's end has zeros of q: its K row is zero, and an infinite q would make NaN of it)
     const float* qv = q + static_cast<size_t>(kvh) * gqa * head_size + (inside ? sub * 8 : 0);
     for (int h0 = 0; h0 < gqa; h0 += kHeads) {
-        float x[kHeads][8];
+        floatx4 x[kHeads][2];
 #pragma unroll
         for (int h = 0; h < kHeads; ++h)
 #pragma unroll
-            for (int e = 0; e < 8; e += 4) {
-                const float* from = qv + static_cast<size_t>(h0 + h < gqa ? h0 + h : h0) * head_size + e;
-                const floatx4 four = *reinterpret_cast<const AnyFloatx4*>(from);
-#pragma unroll
-                for (int z = 0; z < 4; ++z) x[h][e + z] = inside ? four[z] : 0.0f;
+            for (int j = 0; j < 2; ++j) {
+                if constexpr (kStaged) {
+                    x[h][j] = *reinterpret_cast<const floatx4*>(qs + (h0 + h) * kPad + sub * 8 + 4 * j);
+                } else {
+                    const float* from = qv + static_cast<size_t>(h0 + h < gqa ? h0 + h : h0) * head_size + 4 * j;
+                    const floatx4 four = *reinterpret_cast<const AnyFloatx4*>(from);
+                    x[h][j] = inside ? four : floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+                }
             }
 #pragma unroll
         for (int h = 0; h < kHeads; ++h) {
             if (h0 + h >= gqa) break;
-            const floatx4 xa = {x[h][0], x[h][1], x[h][2], x[h][3]}, xb = {x[h][4], x[h][5], x[h][6], x[h][7]};
-            const float s = group_sum<kGroup>(dot8(kb, xa, xb, 0.0f));
+            const float s = group_sum<kGroup>(dot8(kb, x[h][0], x[h][1], 0.0f));
             if (sub == 0 && t < npos) out[static_cast<size_t>(kvh * gqa + h0 + h) * seq_len + t] = s;
         }
     }
@@ -390,11 +403,18 @@ lpp_status lpp_multihead_gemv(float* d_out, const float* d_q, const lpp_half* d_
     }
     const int per_block = kAttThreads / g;
     const dim3 grid((npos + per_block - 1) / per_block, n_kv_heads);
-    LPP_REQUIRE(static_cast<size_t>(gqa) * g * 8 * sizeof(float) <= 65536,
-                "lpp_multihead_gemv: %d query heads per KV head are more than 64 KiB of q", gqa);
-#define LPP_SCORES(G)                                                                             \
-    hipLaunchKernelGGL((scores_kernel<G>), grid, dim3(kAttThreads), 0, stream(), d_out, d_q,     \
-                       k_layer, npos, gqa, head_size, seq_len)
+    const size_t lds = static_cast<size_t>(gqa) * g * 8 * sizeof(float);
+    LPP_REQUIRE(lds <= 65536, "lpp_multihead_gemv: %d query heads per KV head are more than 64 KiB of q", gqa);
+    // q from registers while every workgroup has a compute unit to itself, through LDS beyond.  us a launch, registers / LDS:
+    // 32 heads of 64 on 8 KV heads 2.52 / 2.76 at 513 positions (136 workgroups), 2.84 / 2.72 at 1200 (304), 4.84 / 3.48 at
+    // 8192; on 32 KV heads 2.20 / 2.28 at 100 (128), 2.54 / 2.28 at 300 (320), 11.8 / 6.8 at 8192; 32 heads of 128 on 8 2.60 /
+    // 2.92 at 512 (256), 3.28 / 3.04 at 1200 (600).  Heads of 8 have whole positions to a lane and are slower from registers
+    // throughout (2.34 / 2.14 at 100, 8 workgroups).
+    const bool staged = g == 1 || static_cast<long long>(grid.x) * grid.y > compute_units();
+#define LPP_SCORES(G)                                                                                      \
+    hipLaunchKernelGGL((staged ? &scores_kernel<G, true> : &scores_kernel<G, G == 1>), grid,               \
+                       dim3(kAttThreads), staged ? lds : 0, stream(), d_out, d_q, k_layer, npos, gqa,      \
+                       head_size, seq_len)
     switch (g) {
         case 1: LPP_SCORES(1); break;
         case 2: LPP_SCORES(2); break;
