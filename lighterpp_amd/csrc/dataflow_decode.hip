@@ -132,7 +132,8 @@ struct Tagged {
     unsigned hs_magic;     // floor(2^32 / head_size) + 1: x / head_size == __umulhi(x, hs_magic) for x < 2^25
     int att_splits;        // context splits per query head at this position (worked out on the host: the search
     int att_group_splits;  // is a few dozen integer divisions); > 0: items cover two heads of a KV head, this many splits
-    float inv_sqrt_head;   // 1 / sqrt(head_size), formed on the host (on the device it would sit in a vector register all token long)
+    // 1 / sqrt(head_size), formed on the host (on the device it would sit in a vector register all token long)
+    float inv_sqrt_head;
     int lane_item_cap;     // contexts up to this many positions take the one-pass item of a head of size 64 (att_lane_item)
     // A KV head's context split over the workgroups of its XCD (att_xcd_item): xa_chunk > 0 switches it on.
     int xa_chunk;          // positions per workgroup (a multiple of 8, at most 8 * 64)
@@ -167,7 +168,8 @@ struct Blocks {
     int gu_split;   // context: they park nothing and own fewer units instead)
     int park_rows;  // gate/up rows a workgroup from gu_split on keeps in LDS instead of streaming them (even; 0: none)
     int park_floats;
-    int qkv_by_xcc; // > 0: the stacked [Wq; Wk; Wv] rows are dealt out per XCD, this many KV heads (with their query heads) to each
+    // > 0: the stacked [Wq; Wk; Wv] rows are dealt out per XCD, this many KV heads (with their query heads) to each
+    int qkv_by_xcc;
     int xa_cu_shift;  // att_xcd_item: log2 of the workgroups that share a KV head
     int xa_opc;       // att_xcd_item: attention outputs each of them combines
     int kv_floats;    // LDS behind the parked rows for what the K and V rows of a workgroup's share of a context need beyond them
@@ -787,7 +789,8 @@ __device__ __forceinline__ int hardware_xcc() {
 // A long vector every workgroup needs in full (the SwiGLU output), fetched in two hops.  Polled
 // directly, each of the 256 compute units pulls the whole vector across the fabric between the
 // XCDs, again for every attempt that comes too early: two megabytes per XCD and attempt at 8192
-// values.  Here the workgroups of an XCD share that work: workgroup r of the XCD polls slice r of the vector (device scope, as before) and stores it,
+// values.  Here the workgroups of an XCD share that work: workgroup r of the XCD polls slice r of the vector (device scope,
+// as before) and stores it,
 // tags included, into a copy of the vector that belongs to its XCD; every workgroup then polls that
 // copy.  Those stores stay in the XCD's own L2 (plain stores; a device-scope store would write
 // through and drop the line), and the polls are non-temporal loads, which the compute unit's L1
@@ -934,7 +937,8 @@ __device__ __forceinline__ float stage_norm(Ctx& c, Io& io, const Lds& l, const 
     signal_received(c.ctl);
     signal_staged(c.ctl);
     ss = io_sum(c.ctl, io, ss);
-    ss /= c.b.dim_as_float;  // n, converted on the host: here the conversion's result would be kept in (and spilled from) a vector register
+    // n, converted on the host: here the conversion's result would be kept in (and spilled from) a vector register
+    ss /= c.b.dim_as_float;
     ss += 1e-5f;
     return 1.0f / sqrtf(ss);
 }
@@ -1606,7 +1610,8 @@ __device__ __forceinline__ void att_lane_item(Ctx& c, Io& io, const Lds& l, int 
                 qa[i] = *reinterpret_cast<const floatx4*>(l.qkv + 8 * (4 * r + i));
                 qb[i] = *reinterpret_cast<const floatx4*>(l.qkv + 8 * (4 * r + i) + 4);
             }
-            __builtin_amdgcn_sched_barrier(0);  // (left alone, the scheduler pairs every read with its use: one LDS round trip per piece)
+            // (left alone, the scheduler pairs every read with its use: one LDS round trip per piece)
+            __builtin_amdgcn_sched_barrier(0);
             float part[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) part[i] = dot8(kbits[i], qa[i], qb[i], 0.0f);
@@ -1873,7 +1878,8 @@ __device__ __forceinline__ void att_xcd_item(Ctx& c, Io& io, const Lds& l, int l
             const int hd = lane & 3, p0 = lane & ~3;
             floatx4 acc_head = floatx4{0.0f, 0.0f, 0.0f, 0.0f}, acc_rest = acc_head;
             if (x.count > 0) {  // (uniform)
-                const int my = w0 + (lane < x.count ? lane : 0);  // (lanes past the wavefront's positions read its first row; their scores are dropped)
+                // (lanes past the wavefront's positions read its first row; their scores are dropped)
+                const int my = w0 + (lane < x.count ? lane : 0);
                 const char* q_head = reinterpret_cast<const char*>(l.qkv + kMaxAttHeads * kMaxHeadPad) + hd * (kHs * 2);
                 const char* q_rest = q_head + kMaxAttHeads * kHs * 2;
 #pragma unroll
@@ -1952,7 +1958,8 @@ __device__ __forceinline__ void att_xcd_item(Ctx& c, Io& io, const Lds& l, int l
                         for (int j = 0; j < kG; ++j) {
                             if (j * kWave < n) {  // (uniform)
                                 const int p = j * kWave + lane;
-                                const int my = first + (p < n ? p : 0);  // (lanes past the part read its first row; their scores are dropped)
+                                // (lanes past the part read its first row; their scores are dropped)
+                                const int my = first + (p < n ? p : 0);
                                 uintx4 kbits[4];
 #pragma unroll
                                 for (int i = 0; i < 4; ++i) kbits[i] = *reinterpret_cast<const uintx4*>(kbase + (4 * r + i) * chunk * 16 + my * 16);

@@ -208,7 +208,8 @@ __global__ __launch_bounds__(256) void k_rope_scatter(float* q, const float* qs,
     floatx4 part[kSplits];
 #pragma unroll
     for (int z = 0; z < kSplits; ++z) part[z] = *reinterpret_cast<const floatx4*>(from + z * split_stride);
-    const floatx4 cs = *reinterpret_cast<const floatx4*>(rope + static_cast<size_t>(pos) * (hs / 2) + (within >> 1));  // (cos, sin) of two pairs
+    // (cos, sin) of two pairs
+    const floatx4 cs = *reinterpret_cast<const floatx4*>(rope + static_cast<size_t>(pos) * (hs / 2) + (within >> 1));
     floatx4 v = part[0];
 #pragma unroll
     for (int z = 1; z < kSplits; ++z) v = floatx4{v[0] + part[z][0], v[1] + part[z][1], v[2] + part[z][2], v[3] + part[z][3]};
@@ -448,7 +449,8 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
     constexpr int kFeaturesPerTile = kMode == 2 ? 32 * kFi : 64 * kFi;
     const int f_base = tile_x * kFeaturesPerTile, t_base = token_tile * (kRagged ? job.each : kRowsB);
 
-    auto row_of = [&](int row) { return kRagged && row >= job.each ? job.each - 1 : row; };  // (a row past the tile's: any, nobody multiplies it)
+    // (a row past the tile's: any, nobody multiplies it)
+    auto row_of = [&](int row) { return kRagged && row >= job.each ? job.each - 1 : row; };
     // what each lane requests: request q of this wavefront fills 1 KiB = rows (64 / kPieces) (wave + 4 q) .. of a stage
     const char* src[kLoads];
 #pragma unroll
@@ -635,7 +637,8 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
                 }
             const size_t at = static_cast<size_t>(t_base + wt * 32 * kTj + 32 * j) * job.out_ld + f_base + wf * kWide + 8 * part;
 #pragma unroll
-            for (int which_half = 0; which_half < (kLo ? 2 : 1); ++which_half) {  // (without kLo the next GEMM reads no remainders either)
+            // (without kLo the next GEMM reads no remainders either)
+            for (int which_half = 0; which_half < (kLo ? 2 : 1); ++which_half) {
 #pragma unroll
                 for (int i = 0; i < kPairs; ++i)
 #pragma unroll
@@ -1051,7 +1054,8 @@ struct AttentionShape {
     static constexpr int kPartFloats = (kHs / 2 + 2) * 64;  // a wavefront's maximum, sum and output
     static constexpr int kMergeBytes = kP * kR * kPartFloats * 4;
     static_assert(kP > 1 && kHs / 8 % kP == 0, "the output's pieces are shared out among the wavefronts of a row");
-    static constexpr int kOwnValues = kP * kStages * kStageBytes;  // behind the stages: V rows of a step, for each row of wavefronts but the last
+    // behind the stages: V rows of a step, for each row of wavefronts but the last
+    static constexpr int kOwnValues = kP * kStages * kStageBytes;
     static constexpr int kStepBytes = kOwnValues + (kR - 1) * kHalfBytes;
     static constexpr int kLdsBytes = kStepBytes > kMergeBytes ? kStepBytes : kMergeBytes;
     static_assert(kLdsBytes <= 160 * 1024, "LDS of a workgroup");
@@ -1105,7 +1109,8 @@ __global__ __launch_bounds__(64 * kR * kP, 2) void k_attention_mfma(const float*
     const int tile = static_cast<int>(gridDim.y) - 1 - order;
     const int first_token = tile * kR * tokens_per_wave;                                         // of the workgroup
     const int t0 = first_token + wr * tokens_per_wave;                                           // of the wavefront
-    auto end_of = [&](int token) { return pos0 + (token < n_tokens ? token : n_tokens); };       // positions below which `token`s before attend
+    // positions below which `token`s before attend
+    auto end_of = [&](int token) { return pos0 + (token < n_tokens ? token : n_tokens); };
     const int limit = end_of(first_token + kR * tokens_per_wave);                // the workgroup reads [0, limit)
     const int wave_limit = t0 < n_tokens ? end_of(t0 + tokens_per_wave) : 0;     // the wavefront attends to [0, wave_limit)
     const int my_tok = t0 + r / gqa, my_head = r % gqa;
