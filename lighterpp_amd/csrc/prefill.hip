@@ -5,7 +5,7 @@
 // a time and dropping what the sampler returns (src/main.cpp:163-180), which reads
 // every weight once per prompt token.  Here the prompt's tokens go through each
 // layer together, so the matrix products are GEMMs on the matrix cores
-// (v_mfma_f32_32x32x16_f16) and every weight is read once per chunk of up to 2048
+// (v_mfma_f32_16x16x32_f16 and 32x32x16) and every weight is read once per chunk of up to 2048
 // tokens.  What a prefill leaves behind is exactly what the decode loop reads
 // later: K and V of the prompt positions, rounded to binary16 as the cache store
 // rounds them (model.cpp:171-176, kernels.cuh:34).  The classifier and the sampler
@@ -345,16 +345,19 @@ __global__ __launch_bounds__(256) void k_gemm(const half_t* __restrict__ w, cons
 // a SIMD runs one of each kind.
 //
 // The four multiplying wavefronts (2 x 2) own a tile of 64 kFi features x 64 kTj tokens; a wavefront
-// owns 32 kFi x 32 kTj of it (kFi x kTj MFMA tiles: the weight side is the longer one, because the
+// owns 32 kFi x 32 kTj of it (2 kFi x 2 kTj MFMA tiles of 16 x 16: the weight side is the longer one, because the
 // activations come twice, as head and remainder, and every fragment is read from LDS once per
-// wavefront that uses it).  A trip covers kTripK columns (64 = a whole cache line per row and
+// wavefront that uses it).  What bounds a full tile is the device's power, so the products are
+// v_mfma_f32_16x16x32_f16, remainder right behind head in the same accumulator: 32 x 32 x 16 needs a lower clock for the same
+// work (the exact mode's W1+W3, 512 ids: 1B shape 69 -> 63 us, 8B 252 -> 224; of 2048 ids of the 1B shape 260 -> 236, W2 127 ->
+// 112; the fast mode, half of it data, 2 to 5 %).  A trip covers kTripK columns (64 = a whole cache line per row and
 // trip, or 32 where 64 would leave room for two stages only): the rows of the three operand
 // tiles lie one after the other in a stage of LDS, and a requesting wavefront fills 1 KiB of it
 // with one global_load_lds_dwordx4 (lane i -> 16 bytes at M0 + 16 i): no registers are staged
 // and nothing waits for the data but the s_waitcnt ahead of the trip that multiplies it.  As
 // many stages as 160 KiB hold, five at most.
 //
-// LDS banks: a fragment read takes 16 bytes per lane from 32 consecutive rows; with rows of 128
+// LDS banks: a fragment read takes 16 bytes per lane from 16 consecutive rows; with rows of 128
 // (64) bytes every second (fourth) row starts in the same bank, so the 16-byte pieces of row r
 // are stored in the order piece ^ ((r >> 1) & 7) (piece ^ ((r >> 2) & 3)): 16 consecutive lanes then
 // cover all 64 banks once.  The permutation is applied on the way in, by the address each lane
@@ -364,8 +367,8 @@ __global__ __launch_bounds__(256) void k_gemm(const half_t* __restrict__ w, cons
 // wait for all outstanding requests (they may alias), which is the pipeline's whole depth.
 //
 // kMode 0 stores the tile, 1 adds it to y, 2 is the feed-forward pair: the tile's weight rows are
-// 32 kFi features of W1 (the wavefront's first kFi / 2 MFMA tiles) and the same features of W3
-// (its last kFi / 2), and what is stored is (g * sigmoid(g)) * up (ops.cpp:78-87), split into
+// 32 kFi features of W1 (the wavefront's first kFi MFMA tiles) and the same features of W3
+// (its last kFi), and what is stored is (g * sigmoid(g)) * up (ops.cpp:78-87), split into
 // binary16 head and remainder as the next product wants it.
 struct PipeJob {
     const half_t* w[3];
@@ -417,12 +420,90 @@ __device__ __forceinline__ void swiglu_split4(half4_pf_t& hi, half4_pf_t& lo, co
     }
 }
 
+// A wavefront's sums on their way out.  D[m][n]: a lane holds column n = lane % 16 (a token) and rows m = 4 (lane / 16) + e
+// (features): stored from there, an instruction would write 16 bytes or 8 to each of 16 rows of the output.  The tiles
+// therefore pass through LDS, [token][feature], and leave as whole lines, eight lanes to a token's row.  `room`: kLeaveBytes that are the
+// wavefront's own; its LDS accesses are served in order, so no barrier is needed between a tile's writes, its reads and
+// the next tile's writes.  t0: the wavefront's first token, f_base: the workgroup's first feature, wf: the wavefront's
+// place along the features; only the first live_tiles token tiles are stored.
+constexpr int kLeaveBytes = 32 * 36 * 4;
+template <int kMode, bool kLo, int kI, int kJ>
+__device__ __forceinline__ void leave(const floatx4 (&acc)[kI][kJ], char* room, const PipeJob& job, int which, int split, int t0, int live_tiles,
+                                      int f_base, int wf) {
+    const int lane = lane_id();
+    if constexpr (kMode == 2) {
+        static_assert(kI % 2 == 0, "a wavefront's gate and up tiles: as many of each");
+        constexpr int kPairs = kI / 2, kWide = 16 * kPairs;  // features of the wavefront's output
+        constexpr int kPitch = kWide + 8;                    // binary16 per token row of the transposed tile, padding included
+        constexpr int kLanes = kWide / 8, kRowsAtOnce = 64 / kLanes;
+        static_assert(16 * kPitch * 2 <= kLeaveBytes, "room");
+        const int part = lane % kLanes, row_of = lane / kLanes;
+        half_t* tile = reinterpret_cast<half_t*>(room);
+#pragma unroll
+        for (int j = 0; j < kJ; ++j) {
+            if (j >= live_tiles) break;
+            half4_pf_t h[kPairs], l[kPairs];
+#pragma unroll
+            for (int i = 0; i < kPairs; ++i) {
+                const float gate[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+                const float up[4] = {acc[i + kPairs][j][0], acc[i + kPairs][j][1], acc[i + kPairs][j][2], acc[i + kPairs][j][3]};
+                swiglu_split4(h[i], l[i], gate, up);
+            }
+            const size_t at = static_cast<size_t>(t0 + 16 * j) * job.out_ld + f_base + wf * kWide + 8 * part;
+            // (without kLo the next GEMM reads no remainders either)
+#pragma unroll
+            for (int which_half = 0; which_half < (kLo ? 2 : 1); ++which_half) {
+#pragma unroll
+                for (int i = 0; i < kPairs; ++i)
+                    *reinterpret_cast<half4_pf_t*>(tile + (lane & 15) * kPitch + 16 * i + 4 * (lane >> 4)) = which_half == 0 ? h[i] : l[i];
+                half_t* out = which_half == 0 ? job.out_hi : job.out_lo;
+#pragma unroll
+                for (int pass = 0; pass < 16 / kRowsAtOnce; ++pass) {
+                    const int n = kRowsAtOnce * pass + row_of;
+                    *reinterpret_cast<half8_t*>(out + at + static_cast<size_t>(n) * job.out_ld) =
+                        *reinterpret_cast<const half8_t*>(tile + n * kPitch + 8 * part);
+                }
+            }
+        }
+    } else {
+        constexpr int kPitch = 36;  // floats per token row of the transposed tile: 32 features + padding
+        const int part8 = lane & 7, row8 = lane >> 3;
+        float* tile = reinterpret_cast<float*>(room);
+        float* __restrict__ y = (which == 2 ? job.y[2] : (which == 1 ? job.y[1] : job.y[0])) + static_cast<size_t>(split) * job.split_stride;
+        const int ldy = which == 2 ? job.ldy[2] : (which == 1 ? job.ldy[1] : job.ldy[0]);
+#pragma unroll
+        for (int j = 0; j < kJ; j += 2) {
+            if (j >= live_tiles) break;
+#pragma unroll
+            for (int i = 0; i < kI; i += 2) {
+#pragma unroll
+                for (int jj = 0; jj < 2; ++jj)
+#pragma unroll
+                    for (int ii = 0; ii < 2; ++ii)
+                        *reinterpret_cast<floatx4*>(tile + (16 * jj + (lane & 15)) * kPitch + 16 * ii + 4 * (lane >> 4)) = acc[i + ii][j + jj];
+                float* first = y + static_cast<size_t>(t0 + 16 * j) * ldy + f_base + wf * 16 * kI + 16 * i + 4 * part8;
+#pragma unroll
+                for (int pass = 0; pass < 4; ++pass) {
+                    const int n = 8 * pass + row8;
+                    floatx4* out = reinterpret_cast<floatx4*>(first + static_cast<size_t>(n) * ldy);
+                    floatx4 v = *reinterpret_cast<const floatx4*>(tile + n * kPitch + 4 * part8);
+                    if constexpr (kMode == 1) {
+                        const floatx4 old = *out;
+                        v = floatx4{old[0] + v[0], old[1] + v[1], old[2] + v[2], old[3] + v[3]};
+                    }
+                    *out = v;
+                }
+            }
+        }
+    }
+}
+
 template <int kFi, int kTj, int kMode, int kTripK, bool kLo, bool kRagged>
 __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
     typedef PipeShape<kFi, kTj, kTripK, kLo> Shape;
     constexpr int kRowsA = Shape::kRowsA, kRowsB = Shape::kRowsB, kStages = Shape::kStages, kLoads = Shape::kLoads;
     constexpr int kStageBytes = Shape::kStageBytes, kRowBytes = Shape::kRowBytes;
-    constexpr int kSteps = kTripK / 16;      // k-steps per trip
+    constexpr int kSteps = kTripK / 32;      // k-steps per trip
     constexpr int kPieces = kTripK / 8;      // 16-byte pieces of a row
     constexpr int kSwizzleShift = kPieces == 8 ? 1 : 2;
     extern __shared__ __align__(1024) char pipe_lds[];
@@ -444,7 +525,6 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
     const int tile_x = tile_all - (which == 2 ? job.first_tile[2] : (which == 1 ? job.first_tile[1] : 0));
     const half_t* __restrict__ w = which == 2 ? job.w[2] : (which == 1 ? job.w[1] : job.w[0]);
     const int K = job.K, k_first = split * job.k_len;
-    const int r = lane & 31, g = lane >> 5;
     const int wf = wave & 1, wt = wave >> 1;
     constexpr int kFeaturesPerTile = kMode == 2 ? 32 * kFi : 64 * kFi;
     const int f_base = tile_x * kFeaturesPerTile, t_base = token_tile * (kRagged ? job.each : kRowsB);
@@ -491,46 +571,43 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
                 asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off\n" ::"v"(from), "s"(to) : "memory");
             }
     };
-    // where each lane reads its fragments: row r of an MFMA tile, pieces 2 s + g of k-step s
+    // where each lane reads its fragments: row lane % 16 of an MFMA tile, piece 4 s + lane / 16 of k-step s
     int a_off[kSteps], b_off[kSteps];
 #pragma unroll
     for (int s = 0; s < kSteps; ++s) {
-        const int piece = (2 * s + g) ^ ((r >> kSwizzleShift) & (kPieces - 1));
-        a_off[s] = (wf * 32 * kFi + r) * kRowBytes + 16 * piece;
-        b_off[s] = (kRowsA + wt * 32 * kTj + r) * kRowBytes + 16 * piece;
+        const int row = lane & 15, piece = (4 * s + (lane >> 4)) ^ ((row >> kSwizzleShift) & (kPieces - 1));
+        a_off[s] = (wf * 32 * kFi + row) * kRowBytes + 16 * piece;
+        b_off[s] = (kRowsA + wt * 32 * kTj + row) * kRowBytes + 16 * piece;
     }
 
-    floatx16 acc[kFi][kTj];
+    constexpr int kI = 2 * kFi, kJ = 2 * kTj;  // MFMA tiles of the wavefront
+    floatx4 acc[kI][kJ];
 #pragma unroll
-    for (int i = 0; i < kFi; ++i)
+    for (int i = 0; i < kI; ++i)
 #pragma unroll
-        for (int j = 0; j < kTj; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+        for (int j = 0; j < kJ; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 
-    struct Frags {
-        half8_t a[kFi], bh[kTj], bl[kTj];
+    struct Tokens {
+        half8_t h[kJ], l[kJ];
     };
-    auto read = [&](Frags& f, int trip, int s, auto columns) {
-        if (columns == 0) return;
+    half8_t a[kI];
+    auto read_tokens = [&](Tokens& f, int trip, int s, int j) {
         const char* stage = pipe_lds + (trip % kStages) * kStageBytes;
-#pragma unroll
-        for (int i = 0; i < kFi; ++i) f.a[i] = *reinterpret_cast<const half8_t*>(stage + a_off[s] + i * 32 * kRowBytes);
-#pragma unroll
-        for (int j = 0; j < columns; ++j) {
-            f.bh[j] = *reinterpret_cast<const half8_t*>(stage + b_off[s] + j * 32 * kRowBytes);
-            if constexpr (kLo) f.bl[j] = *reinterpret_cast<const half8_t*>(stage + b_off[s] + (kRowsB + j * 32) * kRowBytes);
-        }
+        f.h[j] = *reinterpret_cast<const half8_t*>(stage + b_off[s] + j * 16 * kRowBytes);
+        if constexpr (kLo) f.l[j] = *reinterpret_cast<const half8_t*>(stage + b_off[s] + (kRowsB + j * 16) * kRowBytes);
     };
-    // (one half of a k-step's MFMAs: the weight tiles [kFi / 2 * half, kFi / 2 * (half + 1)))
-    auto multiply_half = [&](const Frags& f, int half, auto columns) {
+    auto read_weights = [&](int trip, int s, int i) {
+        const char* stage = pipe_lds + (trip % kStages) * kStageBytes;
+        a[i] = *reinterpret_cast<const half8_t*>(stage + a_off[s] + i * 16 * kRowBytes);
+    };
+    // (one weight tile's MFMAs of a k-step)
+    auto multiply_row = [&](const Tokens& f, int i, auto columns) {
 #pragma unroll
-        for (int i = kFi / 2 * half; i < kFi / 2 * (half + 1); ++i)
-#pragma unroll
-            for (int j = 0; j < columns; ++j) {
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.a[i], f.bh[j], acc[i][j], 0, 0, 0);
-                if constexpr (kLo) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.a[i], f.bl[j], acc[i][j], 0, 0, 0);
-            }
+        for (int j = 0; j < 2 * columns; ++j) {
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], f.h[j], acc[i][j], 0, 0, 0);
+            if constexpr (kLo) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], f.l[j], acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
     };
     // (requesting wavefronts) wait until the requests of `trip` have landed: those of later trips, at
     // most kStages - 2 of them, may be in flight
@@ -571,28 +648,54 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
         }
         return;
     }
-    // The fragments of a k-step are read from LDS behind the first half of the MFMAs of the k-step
-    // before and are waited for by the k-step after: the wait the compiler places is for every
-    // read in flight, so none may be in flight that has not had half a k-step to arrive.
+    // The weight tiles of a k-step are multiplied one after the other, and each one's registers take the next k-step's
+    // fragment as soon as it is done; the tokens' fragments are in two sets.  The next trip's barrier is behind the first
+    // quarter of the last k-step: by then every read of this trip has long been served.
     auto walk = [&](auto columns) {
-        Frags frags[2];
+        Tokens tokens[2];
         __syncthreads();
-        read(frags[0], 0, 0, columns);
-        for (int t = 0; t < trips; ++t) {
+        if (columns != 0) {
 #pragma unroll
-            for (int s = 0; s < kSteps; ++s) {
-                const Frags& cur = frags[s & 1];
-                Frags& next = frags[(s + 1) & 1];
-                const bool last = s == kSteps - 1;
-                multiply_half(cur, 0, columns);
-                __builtin_amdgcn_sched_barrier(0);
-                // (after the last trip this reads a stage nobody uses: one path through the loop)
-                if (last) __syncthreads();
-                read(next, last ? t + 1 : t, last ? 0 : s + 1, columns);
-                __builtin_amdgcn_sched_barrier(0);
-                multiply_half(cur, 1, columns);
-                __builtin_amdgcn_sched_barrier(0);
+            for (int j = 0; j < 2 * columns; ++j) read_tokens(tokens[0], 0, 0, j);
+#pragma unroll
+            for (int i = 0; i < kI; ++i) read_weights(0, 0, i);
+        }
+        constexpr int kMeet = kI / 4 - 1;
+        auto step = [&](const Tokens& cur, Tokens& next, int t, auto s) {
+            constexpr bool last = decltype(s)::value == kSteps - 1;
+            constexpr int s_next = last ? 0 : decltype(s)::value + 1;
+            // (after the last trip this reads a stage nobody uses: one path through the loop)
+            const int t_next = last ? t + 1 : t;
+#pragma unroll
+            for (int i = 0; i < kI; ++i) {
+                multiply_row(cur, i, columns);
+                if constexpr (last)
+                    if (i == kMeet) {
+                        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                        __syncthreads();
+                    }
+                if (i >= kMeet && columns != 0) {
+#pragma unroll
+                    for (int k = i == kMeet ? 0 : i; k <= i; ++k) read_weights(t_next, s_next, k);
+                    if (i < kMeet + 2)
+#pragma unroll
+                        for (int j = (i - kMeet) * columns; j < (i - kMeet + 1) * columns; ++j) read_tokens(next, t_next, s_next, j);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
+        };
+        if constexpr (kSteps == 2) {
+            for (int t = 0; t < trips; ++t) {
+                step(tokens[0], tokens[1], t, std::integral_constant<int, 0>{});
+                step(tokens[1], tokens[0], t, std::integral_constant<int, 1>{});
+            }
+        } else {
+            int t = 0;
+            for (; t + 1 < trips; t += 2) {
+                step(tokens[0], tokens[1], t, std::integral_constant<int, 0>{});
+                step(tokens[1], tokens[0], t + 1, std::integral_constant<int, 0>{});
+            }
+            if (t < trips) step(tokens[0], tokens[1], t, std::integral_constant<int, 0>{});
         }
     };
     // kRagged: columns of 32 tokens that are not the tile's, or past the last token, are neither multiplied nor stored.
@@ -606,82 +709,10 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
     } else {
         walk(std::integral_constant<int, kTj>{});
     }
-    // D[m][n]: a lane holds column n = lane % 32 (a token) and rows m = 8 (e / 4) + 4 (lane / 32) + e % 4 (features):
-    // stored from there, an instruction would write 16 or 32 bytes to each of 32 rows of the output.  Every 32 x 32
-    // tile therefore passes through LDS, [token][feature], and leaves as whole 128-byte lines, eight lanes to a
-    // token's row.  The room is the wavefront's quarter of a stage that neither the last trip nor the read past
-    // it uses; a wavefront's LDS accesses are served in order, so no barrier is needed between a tile's writes, its
-    // reads and the next tile's writes.
-    static_assert(kStages >= 3 && kStageBytes / 4 >= 32 * 144, "room for a transposed tile per wavefront");
+    // (room: the wavefront's quarter of a stage that neither the last trip nor the read past it uses)
+    static_assert(kStages >= 3 && kStageBytes / 4 >= kLeaveBytes, "room for a transposed tile per wavefront");
     char* room = pipe_lds + ((trips + 1) % kStages) * kStageBytes + wave * (kStageBytes / 4);
-    if constexpr (kMode == 2) {
-        static_assert(kFi % 2 == 0, "a wavefront's gate and up tiles: as many of each");
-        typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-        constexpr int kPairs = kFi / 2, kWide = 32 * kPairs;  // features of the wavefront's output
-        constexpr int kPitch = kWide + 8;                     // binary16 per token row of the transposed tile, padding included
-        constexpr int kLanes = kWide / 8, kRowsAtOnce = 64 / kLanes;
-        const int part = lane % kLanes, row_of = lane / kLanes;
-        half_t* tile = reinterpret_cast<half_t*>(room);
-#pragma unroll
-        for (int j = 0; j < kTj; ++j) {
-            if (kRagged && j >= columns) break;
-            half4_t h[kPairs][4], l[kPairs][4];
-#pragma unroll
-            for (int i = 0; i < kPairs; ++i)
-#pragma unroll
-                for (int e4 = 0; e4 < 4; ++e4) {
-                    const float gate[4] = {acc[i][j][4 * e4], acc[i][j][4 * e4 + 1], acc[i][j][4 * e4 + 2], acc[i][j][4 * e4 + 3]};
-                    const float up[4] = {acc[i + kPairs][j][4 * e4], acc[i + kPairs][j][4 * e4 + 1], acc[i + kPairs][j][4 * e4 + 2],
-                                         acc[i + kPairs][j][4 * e4 + 3]};
-                    swiglu_split4(h[i][e4], l[i][e4], gate, up);
-                }
-            const size_t at = static_cast<size_t>(t_base + wt * 32 * kTj + 32 * j) * job.out_ld + f_base + wf * kWide + 8 * part;
-#pragma unroll
-            // (without kLo the next GEMM reads no remainders either)
-            for (int which_half = 0; which_half < (kLo ? 2 : 1); ++which_half) {
-#pragma unroll
-                for (int i = 0; i < kPairs; ++i)
-#pragma unroll
-                    for (int e4 = 0; e4 < 4; ++e4)
-                        *reinterpret_cast<half4_t*>(tile + r * kPitch + 32 * i + 8 * e4 + 4 * g) = which_half == 0 ? h[i][e4] : l[i][e4];
-                half_t* out = which_half == 0 ? job.out_hi : job.out_lo;
-#pragma unroll
-                for (int pass = 0; pass < 32 / kRowsAtOnce; ++pass) {
-                    const int n = kRowsAtOnce * pass + row_of;
-                    *reinterpret_cast<half8_t*>(out + at + static_cast<size_t>(n) * job.out_ld) =
-                        *reinterpret_cast<const half8_t*>(tile + n * kPitch + 8 * part);
-                }
-            }
-        }
-    } else {
-        const int row8 = lane >> 3, part8 = lane & 7;
-        constexpr int kPitch = 36;  // floats per token row of the transposed tile: 32 features + padding
-        float* tile = reinterpret_cast<float*>(room);
-        float* __restrict__ y = (which == 2 ? job.y[2] : (which == 1 ? job.y[1] : job.y[0])) + static_cast<size_t>(split) * job.split_stride;
-        const int ldy = which == 2 ? job.ldy[2] : (which == 1 ? job.ldy[1] : job.ldy[0]);
-#pragma unroll
-        for (int i = 0; i < kFi; ++i)
-#pragma unroll
-            for (int j = 0; j < kTj; ++j) {
-                if (kRagged && j >= columns) break;
-#pragma unroll
-                for (int e4 = 0; e4 < 4; ++e4)
-                    *reinterpret_cast<floatx4*>(tile + r * kPitch + 8 * e4 + 4 * g) =
-                        floatx4{acc[i][j][4 * e4], acc[i][j][4 * e4 + 1], acc[i][j][4 * e4 + 2], acc[i][j][4 * e4 + 3]};
-                float* first = y + static_cast<size_t>(t_base + wt * 32 * kTj + 32 * j) * ldy + f_base + wf * 32 * kFi + 32 * i + 4 * part8;
-#pragma unroll
-                for (int pass = 0; pass < 4; ++pass) {
-                    const int n = 8 * pass + row8;
-                    floatx4* out = reinterpret_cast<floatx4*>(first + static_cast<size_t>(n) * ldy);
-                    floatx4 v = *reinterpret_cast<const floatx4*>(tile + n * kPitch + 4 * part8);
-                    if constexpr (kMode == 1) {
-                        const floatx4 old = *out;
-                        v = floatx4{old[0] + v[0], old[1] + v[1], old[2] + v[2], old[3] + v[3]};
-                    }
-                    *out = v;
-                }
-            }
-    }
+    leave<kMode, kLo>(acc, room, job, which, split, t_base + wt * 32 * kTj, kRagged ? 2 * columns : kJ, f_base, wf);
 }
 
 // The same product for a batch of few tokens, where the weights are the traffic and the tiles above would leave most
