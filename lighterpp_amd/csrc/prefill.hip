@@ -385,7 +385,8 @@ struct PipeJob {
     half_t* out_hi;                          // kMode 2: [tokens][out_ld]
     half_t* out_lo;
     int out_ld;
-    int live, each;  // k_gemm_pipe, kRagged: tokens there are, tokens to a tile (a multiple of 32)
+    int live, each;  // tokens there are; k_gemm_pipe, kRagged: tokens to a tile (a multiple of 32)
+    int rows;        // k_gemm_block: rows of x and of the output, a multiple of 32
 };
 
 constexpr int kPipeTripK = 64;  // columns per trip of the narrow tiles; K must be a multiple
@@ -713,6 +714,156 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
     static_assert(kStages >= 3 && kStageBytes / 4 >= kLeaveBytes, "room for a transposed tile per wavefront");
     char* room = pipe_lds + ((trips + 1) % kStages) * kStageBytes + wave * (kStageBytes / 4);
     leave<kMode, kLo>(acc, room, job, which, split, t_base + wt * 32 * kTj, kRagged ? 2 * columns : kJ, f_base, wf);
+}
+
+// The same product in blocks of 256 features x 256 tokens, for batches that make enough of them.
+//
+// Eight wavefronts, two to a SIMD, all of them multiply: each owns 128 features x 64 tokens.  The two of a SIMD take turns,
+// one barrier apart: while one multiplies a trip of 32 columns, the other reads its fragments of the trip from LDS and sends
+// for a later one, so the matrix cores are busy but for the barriers (4650 clocks for 4096 clocks of MFMAs) and a
+// wavefront that a request holds up holds nobody else.  A trip's rows are 64 bytes, in the order of k_gemm_pipe's narrow trips;
+// kStages trips are in LDS at once.
+//
+// What bounds it is the device's power, not its clocks: the loop of the exact mode runs at 1.7 GHz, and what makes it
+// faster is less energy to a product.  That is why a block is as large as the registers allow (a third fewer bytes
+// from L2 and from LDS than 256 x 128), and why the products are v_mfma_f32_16x16x32_f16, head and remainder one after the
+// other into the same accumulator: of the same block, W1+W3 of 2048 ids of the 1B shape takes 233 us in products of 32 x 32 x 16,
+// 213 in 16 x 16 x 32, and 204 with the accumulator kept from head to remainder (266 in k_gemm_pipe's tiles of 256 x 128);
+// without the remainders 134, 126 (and 160).  Fed from registers alone, with neither requests nor reads, the same loop takes
+// 168 us.
+constexpr int kBlock = 256;  // features and tokens of a block
+template <bool kLo>
+struct BlockShape {
+    static constexpr int kTripK = 32, kRowBytes = 2 * kTripK;
+    static constexpr int kRows = (kLo ? 3 : 2) * kBlock;
+    static constexpr int kStageBytes = kRows * kRowBytes;
+    static constexpr int kStages = (160 * 1024) / kStageBytes;
+    static constexpr int kLoads = kRows / 128;  // requests of 1 KiB per wavefront and stage
+    static constexpr int kLdsBytes = kStages * kStageBytes;
+    static_assert(kStages >= 3, "stages of a workgroup");
+};
+
+template <int kMode, bool kLo>
+__global__ __launch_bounds__(512, 2) void k_gemm_block(PipeJob job) {
+    typedef BlockShape<kLo> Shape;
+    constexpr int kStages = Shape::kStages, kLoads = Shape::kLoads, kStageBytes = Shape::kStageBytes, kRowBytes = Shape::kRowBytes;
+    constexpr int kWaveF = 128, kI = kWaveF / 16, kJ = 4;
+    extern __shared__ __align__(1024) char block_lds[];
+    const int lane = lane_id();
+    const int wave = __builtin_amdgcn_readfirstlane(wave_index());
+    // (workgroups that share a weight tile on one die, job.band token tiles at a time: as in k_gemm_pipe)
+    const int id = static_cast<int>(blockIdx.x), die = id & 7, within = id >> 3;
+    const int per_band = ((job.groups + 7) >> 3) * job.band, band = within / per_band, in_band = within - band * per_band;
+    const int group = (in_band / job.band) * 8 + die;
+    if (group >= job.groups) return;
+    const int token_tile = band * job.band + in_band % job.band;
+    const int tile_all = group % job.feature_tiles, split = group / job.feature_tiles;
+    const int which = tile_all >= job.first_tile[2] ? 2 : (tile_all >= job.first_tile[1] ? 1 : 0);
+    const int tile_x = tile_all - (which == 2 ? job.first_tile[2] : (which == 1 ? job.first_tile[1] : 0));
+    const half_t* __restrict__ w = which == 2 ? job.w[2] : (which == 1 ? job.w[1] : job.w[0]);
+    const int K = job.K, k_first = split * job.k_len;
+    const int wf = wave & 1, wt = wave >> 1;
+    const bool second = wave >= 4;  // (wavefronts w and w + 4 share a SIMD)
+    const int f_base = tile_x * (kMode == 2 ? kBlock / 2 : kBlock), t_base = token_tile * kBlock;
+
+    // Request q of this wavefront fills 1 KiB of a stage: 16 rows from 16 (wave + 8 q) on, four lanes to a row's 64 bytes.  The
+    // lanes' offsets from the first row are the same for all of them.  Token rows past the buffer's are its last ones again.
+    const unsigned lane_off = static_cast<unsigned>(lane >> 2) * static_cast<unsigned>(2 * K) + 16u * ((lane & 3) ^ (lane >> 4));
+    const char* base[kLoads];
+#pragma unroll
+    for (int q = 0; q < kLoads; ++q) {
+        const int row = 16 * (wave + 8 * q);
+        const half_t* from;
+        if (row < kBlock) {
+            if constexpr (kMode == 2) {
+                const int owner = row / kWaveF, rem = row % kWaveF;
+                from = (rem >= kWaveF / 2 ? job.w[1] : job.w[0]) + static_cast<size_t>(f_base + owner * (kWaveF / 2) + rem % (kWaveF / 2)) * K;
+            } else {
+                from = w + static_cast<size_t>(f_base + row) * K;
+            }
+        } else {
+            from = (kLo && row >= 2 * kBlock ? job.xl : job.xh) + static_cast<size_t>(min(t_base + row % kBlock, job.rows - 16)) * K;
+        }
+        base[q] = reinterpret_cast<const char*>(from + k_first);
+    }
+    const unsigned lds_base = static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)block_lds));
+    const int trips = job.k_len / Shape::kTripK;
+    auto request = [&](int trip, int slot) {
+        const unsigned at = __builtin_amdgcn_readfirstlane(lds_base + slot * kStageBytes + wave * 1024);
+        const unsigned off = lane_off + static_cast<unsigned>(trip) * kRowBytes;
+        // (s_nop 4: the scalar address may have been written by a vector instruction just before)
+#pragma unroll
+        for (int q = 0; q < kLoads; ++q)
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %0, %1\n" ::"v"(off), "s"(base[q]), "s"(at + q * 8192) : "memory");
+    };
+    // `trip` has landed: of this wavefront's requests those of the kStages - 2 trips behind it may be out
+    auto landed = [&](int trip) {
+        if (trips - 1 - trip >= kStages - 2) wait_requests<(kStages - 2) * kLoads>();
+        else wait_requests<0>();
+    };
+    auto meet = [] {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    // fragments: row lane % 16 of a 16-row tile, the 16-byte piece lane / 16 of the trip's 64 bytes
+    const int read_off = (lane & 15) * kRowBytes + 16 * ((lane >> 4) ^ ((lane >> 2) & 3));
+    floatx4 acc[kI][kJ];
+#pragma unroll
+    for (int i = 0; i < kI; ++i)
+#pragma unroll
+        for (int j = 0; j < kJ; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    half8_t a[kI], bh[kJ], bl[kJ];
+    auto read = [&](int slot) {
+        const char* rows_a = block_lds + slot * kStageBytes + wf * kWaveF * kRowBytes + read_off;
+        const char* rows_b = block_lds + slot * kStageBytes + (kBlock + wt * 64) * kRowBytes + read_off;
+#pragma unroll
+        for (int j = 0; j < kJ; ++j) {
+            bh[j] = *reinterpret_cast<const half8_t*>(rows_b + 16 * j * kRowBytes);
+            if constexpr (kLo) bl[j] = *reinterpret_cast<const half8_t*>(rows_b + (kBlock + 16 * j) * kRowBytes);
+        }
+#pragma unroll
+        for (int i = 0; i < kI; ++i) a[i] = *reinterpret_cast<const half8_t*>(rows_a + 16 * i * kRowBytes);
+    };
+    auto multiply = [&]() {
+#pragma unroll
+        for (int j = 0; j < kJ; ++j)
+#pragma unroll
+            for (int i = 0; i < kI; ++i) {
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], bh[j], acc[i][j], 0, 0, 0);
+                if constexpr (kLo) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], bl[j], acc[i][j], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);  // (in this order)
+            }
+    };
+    // A trip is read by the first group in one turn and by the second in the next; what is sent for into its stage, behind the
+    // second one's turn, has kStages - 1 trips less a turn to arrive.  It must have before the first group's read of it: every
+    // wavefront waits for its own requests ahead of the barrier before that.
+#pragma unroll
+    for (int t = 0; t < kStages - 1; ++t)
+        if (t < trips) request(t, t);
+    landed(0);
+    meet();
+    if (second) meet();
+    int slot = 0, into = kStages - 1;
+    const bool idle = t_base + 64 * wt >= job.live;  // (none of this wavefront's tokens is one: it only sends for rows)
+    for (int t = 0; t < trips; ++t) {
+        if (!idle) read(slot);
+        if (t + kStages - 1 < trips) request(t + kStages - 1, into);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (second) landed(t + 1);
+        meet();
+        if (!idle) multiply();
+        if (!second) landed(t + 1);
+        meet();
+        into = slot;
+        slot = slot + 1 == kStages ? 0 : slot + 1;
+    }
+    if (!second) meet();
+    if (idle) return;
+    // (the stages are free)
+    static_assert(Shape::kLdsBytes >= 8 * kLeaveBytes, "room for a transposed tile per wavefront");
+    leave<kMode, kLo>(acc, block_lds + wave * kLeaveBytes, job, which, split, t_base + 64 * wt, min(kJ, (job.rows - t_base - 64 * wt) / 16), f_base, wf);
 }
 
 // The same product for a batch of few tokens, where the weights are the traffic and the tiles above would leave most
@@ -1482,6 +1633,20 @@ lpp_status launch_pipe(const pf::PipeJob& job_in, hipStream_t s) {
                              : launch_pipe_as<kFi, kTj, kMode, kTripK, false, false>(job, s);
 }
 
+template <int kMode, bool kLo>
+lpp_status size_block() {
+    static bool sized[64] = {};
+    return size_lds(reinterpret_cast<const void*>(&pf::k_gemm_block<kMode, kLo>), pf::BlockShape<kLo>::kLdsBytes, sized);
+}
+template <int kMode, bool kLo>
+lpp_status launch_block(pf::PipeJob job, hipStream_t s) {
+    LPP_TRY((size_block<kMode, kLo>()));
+    job.band = job.token_tiles;
+    hipLaunchKernelGGL((pf::k_gemm_block<kMode, kLo>), dim3((job.groups + 7) / 8 * 8 * job.token_tiles), dim3(512), pf::BlockShape<kLo>::kLdsBytes, s, job);
+    LPP_CHECK_LAUNCH("k_gemm_block");
+    return LPP_OK;
+}
+
 template <int kFi, int kTj, int kMode, bool kLo>
 lpp_status launch_few_as(const pf::PipeJob& job, hipStream_t s) {
     constexpr int kLds = pf::FewShape<kFi, kTj, kLo>::kLdsBytes;
@@ -1495,14 +1660,15 @@ lpp_status launch_few_as(const pf::PipeJob& job, hipStream_t s) {
 // How a product is laid out on the device: what a workgroup's tile is and in how many ranges K is cut.
 struct Plan {
     bool few;          // k_gemm_few (rows = 32 fi, tokens = 32 tj), otherwise k_gemm_pipe (rows = 64 fi, tokens = 64 tj)
-    int fi, tj;
+    int fi, tj;        // ({false, 4, 4}: k_gemm_block)
     int splits;
+    bool block() const { return !few && tj == 4; }
     int tile_rows() const { return (few ? 32 : 64) * fi; }
     int tile_tokens() const { return (few ? 32 : 64) * tj; }
     // Tiles of k_gemm_few that hold a token (150 ids, Wo in tiles of 64: three of four; 1B shape 1.466 -> 1.455 ms);
     // k_gemm_pipe deals the tokens out (launch_pipe).  The plan itself goes by t_pad: by the tokens it would take Wo of 130 to
     // 160 ids for k_gemm_pipe's tile of 96, 1.5 % faster there and 2.4 % slower at 192.
-    int token_tiles(int t_pad, int live) const { return few ? (live + tile_tokens() - 1) / tile_tokens() : t_pad / tile_tokens(); }
+    int token_tiles(int t_pad, int live) const { return ((few ? live : t_pad) + tile_tokens() - 1) / tile_tokens(); }
 };
 
 // Rows the activations of n tokens are padded to: whole tiles of 128 tokens, or of 32 up to that many.
@@ -1517,6 +1683,15 @@ int padded_tokens(int n) {
 // wider tile being a third more bytes from L2 and not twice as many (8B shape, 1280 ids: 38.2 -> 36.9 ms, 1792: 51.0 ->
 // 49.4).  In the fast mode it is half as many again, and the narrow tiles' rounds stay the faster ones.
 //
+// k_gemm_block where its blocks, in one range of K or several, should take less: what pays for fewer bytes to a product is
+// filling the device, so the two are compared by their rounds of workgroups.  A round is a launch's share that does not
+// depend on K, and K columns; a last round of a few workgroups still costs a third to two thirds of a full one.  The
+// constants are a fit to 860 timed launches (TinyLlama, 1B and 8B shapes, 384 to 2048 tokens; 3 to 5 % rms, of the tiles
+// of 128 x 128 7 to 9), partial products are written and read at 3 TB/s, and a block is taken where it gains 3 %.  W1+W3,
+// exact / fast mode, tiles against blocks: 1B shape 1024 ids 127 / 81 and 118 / 67 us, 1280 ids (a quarter of a second
+// round) 163 / 108 and 187 / 113, 2048 ids 236 / 156 and 217 / 127; 8B 512 ids 224 / 152 and 196 / 122, 1024 ids 426 / 280
+// and 369 / 224, W2 of 1024 ids 205 / 137 and, K in four ranges, 177 / 109.
+//
 // Up to 256 tokens the choice is made by what a launch of each would take.  A workgroup of k_gemm_few is paced by its
 // bytes from L2 into LDS (57 bytes a nanosecond), one of k_gemm_pipe by its bytes (88) and its MFMA clocks; a last round
 // of workgroups that does not fill the device counts almost whole; no launch is faster than its weights at 3.9 TB/s;
@@ -1526,6 +1701,19 @@ int padded_tokens(int n) {
 //
 // `max_splits`: ranges K may be cut into.  `row_step`: every matrix is a whole number of row_step rows.  `pair`: W1 and W3
 // side by side in a tile (total_n counts both).
+float planned_us(const Plan& p, int total_n, int K, int t_pad, bool lo, bool pair) {
+    struct Cost {
+        float launch, column, round, pair_round, rest;  // us, ns a column, us (the pair's: with SwiGLU), a last round's share at least
+    };
+    static constexpr Cost kCosts[3][2] = {{{0.6f, 8.8f, 6.5f, 6.5f, 0.29f}, {0.0f, 13.5f, 8.0f, 8.0f, 0.33f}},       // 128 x 128
+                                          {{1.7f, 17.7f, 1.0f, 2.4f, 0.60f}, {1.7f, 24.8f, 8.0f, 9.7f, 0.52f}},      // 256 x 128
+                                          {{0.0f, 26.2f, 12.4f, 10.3f, 0.60f}, {0.0f, 42.4f, 12.8f, 19.4f, 0.65f}}}; // blocks
+    const Cost& c = kCosts[p.block() ? 2 : (p.fi == 4 ? 1 : 0)][lo ? 1 : 0];
+    const int wgs = total_n / p.tile_rows() * p.token_tiles(t_pad, t_pad) * p.splits, left = wgs % compute_units();
+    const float rounds = wgs / compute_units() + (left > 0 ? c.rest + (1.0f - c.rest) * left / compute_units() : 0.0f);
+    const float partials = p.splits > 1 ? 4.0f * p.splits * t_pad * total_n / 3e6f : 0.0f;
+    return c.launch + rounds * (1e-3f * c.column * K / p.splits + (pair ? c.pair_round : c.round)) + partials;
+}
 Plan plan_gemm(int total_n, int K, int t_pad, int max_splits, bool lo, int row_step, bool pair) {
     // `exact`, `fast`: the modes in which the model picks the tile at 256 compute units, n to 300000 and K to 32768 (one of
     // 32 x 128, timed for the fit as well, in neither).  launch_plan has the kernels of this list.
@@ -1545,6 +1733,18 @@ Plan plan_gemm(int total_n, int K, int t_pad, int max_splits, bool lo, int row_s
         while (2 * best.splits <= max_splits && total_n / best.tile_rows() * token_tiles * best.splits * 2 <= compute_units() &&
                K % (64 * 2 * best.splits) == 0 && K / (2 * best.splits) >= 512)
             best.splits *= 2;
+        if (!wide_allowed) return best;
+        const Plan tiles = best;
+        float best_us = 0.97f * planned_us(tiles, total_n, K, t_pad, lo, pair);
+        for (int splits = 1; splits <= max_splits; splits *= 2) {
+            const Plan block = {false, 4, 4, splits};
+            if (K % (64 * splits) != 0 || (splits > 1 && (K / splits < 512 || total_n / 256 * block.token_tiles(t_pad, t_pad) * splits > compute_units()))) break;
+            const float us = planned_us(block, total_n, K, t_pad, lo, pair);
+            if (us < best_us) {
+                best_us = us;
+                best = block;
+            }
+        }
         return best;
     }
     float best_us = 1e30f;
@@ -1575,11 +1775,11 @@ Plan plan_gemm(int total_n, int K, int t_pad, int max_splits, bool lo, int row_s
 
 // Floats of kBufPartials that chunks of up to t_pad tokens need: the partial products of the GEMM before (read by the
 // kernel that follows it, so one area does for all of a layer's) -- at most eight of 256 tokens, or one tile of 128 x 128 per
-// compute unit (plan_gemm) -- or the gate and up projections where those are not fused.
+// compute unit, beyond 512 tokens one block of 256 x 256 (plan_gemm) -- or the gate and up projections where those are not fused.
 size_t partial_floats(const lpp_model* m, int t_pad) {
     const size_t t = static_cast<size_t>(t_pad), few = t < 256 ? t : 256;
     size_t most = 8 * few * (m->cfg.dim + 2 * m->kv_dim);
-    const size_t tiles = static_cast<size_t>(compute_units()) * 128 * 128, pair = 2 * t * m->cfg.hidden_dim;
+    const size_t tiles = static_cast<size_t>(compute_units()) * (t > static_cast<size_t>(pf::kSmallChunk) ? 256 * 256 : 128 * 128), pair = 2 * t * m->cfg.hidden_dim;
     if (t > 256 && tiles > most) most = tiles;
     const bool fused = test_option(LPP_OPT_PREFILL_STAGED_GEMM) != 0 && test_option(LPP_OPT_PREFILL_FUSED_FFN) != 0;
     return !fused && pair > most ? pair : most;
@@ -1674,6 +1874,7 @@ template <int kMode>
 lpp_status launch_plan(const Plan& p, const pf::PipeJob& job_in, hipStream_t s) {
     pf::PipeJob job = job_in;
     job.band = band_of(job.token_tiles, job.xl != nullptr);
+    if (p.block()) return job.xl != nullptr ? launch_block<kMode, true>(job, s) : launch_block<kMode, false>(job, s);
     if (!p.few) {
         if (p.fi == 4) return launch_pipe<4, 2, kMode, 32>(job, s);
         return launch_pipe<2, 2, kMode>(job, s);
@@ -1744,6 +1945,7 @@ lpp_status gemm(const Product* prods, int count, const pf::half_t* xh, const pf:
         job.feature_tiles = feature_tiles;
         job.token_tiles = token_tiles;
         job.live = live;
+        job.rows = t_pad;
         job.groups = feature_tiles * splits;
         const bool add_in_kernel = accumulate && splits == 1;
         if (add_in_kernel) LPP_TRY(launch_plan<1>(plan, job, s));
@@ -1842,6 +2044,7 @@ lpp_status gate_up_swiglu(const void* w1, const void* w3, int hidden, const pf::
     job.feature_tiles = 2 * hidden / plan.tile_rows();  // half of a tile's rows from either matrix
     job.token_tiles = plan.token_tiles(t_pad, live);
     job.live = live;
+    job.rows = t_pad;
     job.groups = job.feature_tiles;
     job.out_hi = out_hi;
     job.out_lo = out_lo;
@@ -2100,6 +2303,8 @@ lpp_status run_scratch_setup() {
     LPP_TRY((size_pipe<4, 2, 1, 32>()));
     LPP_TRY((size_pipe<2, 2, 0, pf::kPipeTripK>()));
     LPP_TRY((size_pipe<2, 2, 1, pf::kPipeTripK>()));
+    LPP_TRY((size_block<0, true>()));
+    LPP_TRY((size_block<1, true>()));
     LPP_TRY((size_few_for<0>()));
     LPP_TRY((size_few_for<1>()));
     void* p = nullptr;

@@ -66,6 +66,52 @@ def test_gemm_against_float64(lib, n, k, t, accumulate):
         assert not got[0].any()
 
 
+@pytest.mark.parametrize("n,k,t", [(16384, 64, 1024), (16384, 128, 640), (16384, 320, 896), (32768, 64, 384), (12288, 192, 1280)])
+@pytest.mark.parametrize("accumulate", [0, 1])
+def test_gemm_in_blocks_adds_in_the_order_of_the_tiles(lib, n, k, t, accumulate, test_options):
+    """Products wide enough for blocks of 256 x 256, with fewer trips than the stages hold and more, and a last block
+    half or a quarter of whose tokens are there: the same bits as the tiles of 128 x 128, and near the float64 product."""
+    rng = np.random.default_rng(n + k + t)
+    w = (rng.standard_normal((n, k)) * 0.02).astype(np.float16)
+    x = rng.standard_normal((t, k)).astype(F)
+    y0 = rng.standard_normal((t, n)).astype(F)
+    dw, dx = DB.from_numpy(w.view(np.uint16)), DB.from_numpy(x)
+    got = []
+    for wide in (1, 0):
+        test_options(capi.OPT_PREFILL_WIDE_TILES, wide)
+        dy = DB.from_numpy(y0)
+        capi.check(lib.lpp_prefill_gemm(dy.ptr, dw.ptr, dx.ptr, n, k, t, accumulate))
+        got.append(dy.to_numpy(F, t * n).reshape(t, n))
+    assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+    rows = rng.integers(0, t, 24)
+    want = x[rows].astype(np.float64) @ w.astype(np.float64).T + (y0[rows] if accumulate else 0.0)
+    assert np.max(np.abs(got[0][rows] - want)) <= 1e-5 * np.max(np.abs(want))
+
+
+@pytest.mark.parametrize("fast", [False, True])
+@pytest.mark.parametrize("n", [512, 769, 1000])
+def test_prefill_in_blocks_against_tiles(n, fast, test_options):
+    """8B width, where W1+W3 go in blocks of 256 x 256 and, of the longer prompts, W2 too, its K in four ranges.  Against the tiles:
+    the exact mode to one binary16 step, the fast one to what rounding an input to binary16 costs (2^-9 in the 2-norm)."""
+    shape = Shape(4096, 14336, 2, 32, 8, 512, 1024, 500000.0, fp16=True, tied=True)
+    m = Model(shape)
+    m.load_synthetic(21)
+    m.set_prefill_mode(capi.PREFILL_FAST if fast else capi.PREFILL_EXACT)
+    ids = capi.synth_token_ids(n, 22, shape.vocab_size)
+    m.prefill(ids, 0)
+    k, v, _, _ = caches(m, shape, n)
+    test_options(capi.OPT_PREFILL_WIDE_TILES, 0)
+    m.prefill(ids, 0)
+    k0, v0, kf, vf = caches(m, shape, n)
+    assert not kf[:, :, n:, :].any() and not vf[:, :, n:, :].any(), "slots beyond the prompt were written"
+    for x, y in ((k, k0), (v, v0)):
+        if fast:
+            assert np.linalg.norm(x - y) <= 2.0 ** -9 * np.linalg.norm(y)
+        else:
+            assert np.all(np.abs(x - y) <= np.maximum(np.abs(y) * 2.0 ** -9, np.abs(y).max() * 2.0 ** -11))
+    m.close()
+
+
 def test_gemm_rejects_ragged_shapes(lib):
     d = DB(1 << 20)
     for n, k, t in [(100, 32, 128), (128, 48, 128), (128, 32, 100), (128, 32, 0)]:
