@@ -1232,7 +1232,7 @@ struct AttentionShape {
     static constexpr int kRowBytes = 2 * kHs, kPieces = kHs / 8;
     static constexpr int kHalfBytes = kStep * kRowBytes, kStageBytes = 2 * kHalfBytes;  // K rows, then V rows
     static constexpr int kLoads = kStageBytes / 1024 / kR;                              // requests per wavefront and step
-    static constexpr int kStages = kHs == 64 && kP == 2 ? 3 : 2;  // 2 x 2: 52 / 72 KiB, at least two workgroups to a compute unit
+    static constexpr int kStages = 2;  // 2 x 2: 52 / 72 KiB, at least two workgroups to a compute unit
     static constexpr int kPartFloats = (kHs / 2 + 2) * 64;  // a wavefront's maximum, sum and output
     static constexpr int kMergeBytes = kP * kR * kPartFloats * 4;
     static_assert(kP > 1 && kHs / 8 % kP == 0, "the output's pieces are shared out among the wavefronts of a row");
