@@ -477,6 +477,27 @@ def test_tokens_that_leave_columns_of_the_last_tiles_empty(hidden, n, fast):
     m.close()
 
 
+@pytest.mark.parametrize("fast", [False, True])
+@pytest.mark.parametrize("n", [7, 8, 9, 16, 17, 24, 25, 39, 40, 57, 72, 73, 88, 104, 105, 120, 121, 150])
+def test_token_rows_that_are_not_requested(n, fast):
+    """k_gemm_few sends for token rows in eights, and not for eights without a token: a prompt's first n ids against the
+    same prompt filled up to whole tiles, every row of which is requested.  Same order of sums, so the bound is one
+    binary16 step, or 2^-11 of the largest entry.  A longer prompt has been through the buffers and the compute units' LDS."""
+    shape = Shape(2048, 5632, 2, 32, 4, 1024, 320, 10000.0, fp16=True, tied=True)
+    m = Model(shape)
+    m.load_synthetic(3)
+    m.set_prefill_mode(capi.PREFILL_FAST if fast else capi.PREFILL_EXACT)
+    whole = capi.synth_token_ids((n + 31) // 32 * 32 if n <= 128 else 256, 5, shape.vocab_size)
+    m.prefill(whole, 0)
+    k0, v0, _, _ = caches(m, shape, n)
+    m.prefill(capi.synth_token_ids(256, 9, shape.vocab_size), 0)
+    m.prefill(whole[:n], 0)
+    k, v, _, _ = caches(m, shape, n)
+    for x, y in ((k, k0), (v, v0)):
+        assert np.all(np.abs(x - y) <= np.maximum(np.abs(y) * 2.0 ** -9, np.abs(y).max() * 2.0 ** -11))
+    m.close()
+
+
 MANY_HEADS = {  # heads of 64: the attention's workgroup shapes change behind 256 and 512 ids (GQA 4: 512 and 1024); of 128: behind 512
     "hs64": Shape(2048, 256, 2, 32, 32, 512, 640, 10000.0, fp16=True, tied=True),
     "hs128": Shape(2048, 256, 2, 16, 16, 512, 640, 10000.0, fp16=True, tied=True),
