@@ -1669,7 +1669,7 @@ lpp_status launch_block(pf::PipeJob job, hipStream_t s) {
 }
 
 template <int kFi, int kTj, int kMode, bool kLo, bool kRagged>
-lpp_status launch_few_of(const pf::PipeJob& job, hipStream_t s) {
+lpp_status launch_few_as(const pf::PipeJob& job, hipStream_t s) {
     constexpr int kLds = pf::FewShape<kFi, kTj, kLo>::kLdsBytes;
     LPP_TRY((size_few<kFi, kTj, kMode, kLo, kRagged>()));
     const int per_die = (job.groups + 7) / 8;
@@ -1681,10 +1681,11 @@ lpp_status launch_few_of(const pf::PipeJob& job, hipStream_t s) {
 // ids of the TinyLlama shape 1.69 -> 1.73 ms: the kernel has a loop for every number of requests, and starts with cold
 // instructions), so it has its own; exact mode, before and with it: TinyLlama 10 ids 1.16 -> 1.06 ms, 22 1.16 -> 1.10, 72
 // 1.50 -> 1.42; 1B 24 ids 0.92 -> 0.87; 8B 10 ids 4.18 -> 3.60, 40 4.67 -> 4.19.
-template <int kFi, int kTj, int kMode, bool kLo>
-lpp_status launch_few_as(const pf::PipeJob& job, hipStream_t s) {
-    return job.live <= 32 * kTj * job.token_tiles - 8 ? launch_few_of<kFi, kTj, kMode, kLo, true>(job, s)
-                                                      : launch_few_of<kFi, kTj, kMode, kLo, false>(job, s);
+template <int kFi, int kTj, int kMode>
+lpp_status launch_few(const pf::PipeJob& job, hipStream_t s) {
+    const bool ragged = job.live <= 32 * kTj * job.token_tiles - 8;
+    if (job.xl != nullptr) return ragged ? launch_few_as<kFi, kTj, kMode, true, true>(job, s) : launch_few_as<kFi, kTj, kMode, true, false>(job, s);
+    return ragged ? launch_few_as<kFi, kTj, kMode, false, true>(job, s) : launch_few_as<kFi, kTj, kMode, false, false>(job, s);
 }
 
 // How a product is laid out on the device: what a workgroup's tile is and in how many ranges K is cut.
@@ -1701,9 +1702,10 @@ struct Plan {
     int token_tiles(int t_pad, int live) const { return ((few ? live : t_pad) + tile_tokens() - 1) / tile_tokens(); }
 };
 
-// Rows the activations of n tokens are padded to: whole tiles of 128 tokens, or of 32 up to that many.
+// Rows the activations of n tokens are padded to: whole tiles of 128 tokens, or of 32 up to 64 (up to 96, k_gemm_pipe, whose
+// tiles need rows of 128, was out of reach of 65 to 96 ids: 8B shape, 96 ids 5.75 ms, 128 ids 5.25).
 int padded_tokens(int n) {
-    const int unit = n <= 128 && test_option(LPP_OPT_PREFILL_STAGED_GEMM) != 0 ? 32 : pf::kTileTokens;
+    const int unit = n <= 64 && test_option(LPP_OPT_PREFILL_STAGED_GEMM) != 0 ? 32 : pf::kTileTokens;
     return (n + unit - 1) / unit * unit;
 }
 
@@ -1722,12 +1724,18 @@ int padded_tokens(int n) {
 // round) 163 / 108 and 187 / 113, 2048 ids 236 / 156 and 217 / 127; 8B 512 ids 224 / 152 and 196 / 122, 1024 ids 426 / 280
 // and 369 / 224, W2 of 1024 ids 205 / 137 and, K in four ranges, 177 / 109.
 //
-// Up to 256 tokens the choice is made by what a launch of each would take.  A workgroup of k_gemm_few is paced by its
-// bytes from L2 into LDS (57 bytes a nanosecond), one of k_gemm_pipe by its bytes (88) and its MFMA clocks; a last round
-// of workgroups that does not fill the device counts almost whole; no launch is faster than its weights at 3.9 TB/s;
-// every partial product of a cut K is written (2.5 TB/s, in many short runs) and read (5 TB/s) once more.  The constants
-// are a fit to 1100 timed launches (ten weight matrices of the TinyLlama, 1B and 8B shapes, 32 to 2048 tokens, both
-// modes, every tile of the list): 14 % rms, and the launch picked is 2.2 % slower than the fastest one on average.
+// Up to 256 tokens the choice is made by what a launch of each would take.  A workgroup is paced by its bytes from L2 into
+// LDS, one of k_gemm_pipe by its MFMA clocks where they take longer; a
+// last round of workgroups that does not fill the device counts almost whole; k_gemm_few's sums meet in LDS, a tile of 32 x 32
+// at a time; every partial product of a cut K is written, in many short runs, and read once more.  No launch is faster than
+// its weights, and of two that are bound by them the one with less to do is taken.  The constants are a fit to 10000 timed
+// prefills (TinyLlama, 1B and 8B shapes, 10 to 256 ids, both modes, every tile of the list for each of the four products in
+// turn): up to 128 tokens a prefill is 0.3 % slower on average than with that product's fastest launch.  In the exact mode
+// beyond 128 tokens the constants are an earlier fit's, which makes the better choices there (256 ids of the TinyLlama shape
+// 2.03 ms, 2.06 by the newer one).  Tiles of 256 rows have rows of 64 bytes in a stage, requests of half lines: L2 gives 70
+// bytes a nanosecond to a compute unit that way and 100 in whole lines.
+// Exact mode, by the earlier fit and so: 8B shape 10 ids 3.54 -> 3.35 ms, 40 4.21 -> 3.95, 90 5.76 -> 4.66; 1B 100 ids 1.27 -> 1.21;
+// fast mode: 8B 48 ids 4.34 -> 3.58, 120 5.02 -> 4.39, 1B 200 1.44 -> 1.28, TinyLlama 220 1.84 -> 1.67.
 //
 // `max_splits`: ranges K may be cut into.  `row_step`: every matrix is a whole number of row_step rows.  `pair`: W1 and W3
 // side by side in a tile (total_n counts both).
@@ -1744,16 +1752,13 @@ float planned_us(const Plan& p, int total_n, int K, int t_pad, bool lo, bool pai
     const float partials = p.splits > 1 ? 4.0f * p.splits * t_pad * total_n / 3e6f : 0.0f;
     return c.launch + rounds * (1e-3f * c.column * K / p.splits + (pair ? c.pair_round : c.round)) + partials;
 }
-Plan plan_gemm(int total_n, int K, int t_pad, int max_splits, bool lo, int row_step, bool pair) {
-    // `exact`, `fast`: the modes in which the model picks the tile at 256 compute units, n to 300000 and K to 32768 (one of
-    // 32 x 128, timed for the fit as well, in neither).  launch_plan has the kernels of this list.
+Plan plan_gemm(int total_n, int K, int t_pad, int live, int max_splits, bool lo, int row_step, bool pair) {
+    // (launch_plan has the kernels of this list)
     static constexpr struct {
         bool few;
         int fi, tj;
-        bool exact, fast;
-    } kTiles[] = {{true, 1, 1, true, true}, {true, 1, 2, false, true}, {true, 1, 3, false, true}, {true, 2, 1, true, true},
-                  {true, 2, 2, true, true}, {true, 2, 3, true, true},  {true, 2, 4, false, true}, {true, 4, 1, true, false},
-                  {true, 4, 2, true, false}, {false, 2, 2, true, true}, {false, 4, 2, true, true}};
+    } kTiles[] = {{true, 1, 1}, {true, 1, 2}, {true, 1, 3}, {true, 2, 1}, {true, 2, 2}, {true, 2, 3}, {true, 2, 4}, {true, 4, 1},
+                  {true, 4, 2}, {false, 2, 2}, {false, 4, 2}};
     Plan best = {false, 2, 2, 1};
     const bool wide_allowed = row_step % 256 == 0 && test_option(LPP_OPT_PREFILL_WIDE_TILES) != 0;
     if (t_pad > 256) {
@@ -1777,22 +1782,35 @@ Plan plan_gemm(int total_n, int K, int t_pad, int max_splits, bool lo, int row_s
         }
         return best;
     }
+    struct Rates {
+        float few, pipe, wide, clocks;        // bytes and MFMA clocks a us (wide: of tiles of 256 rows)
+        float launch_few, launch_pipe, sums;  // us; of k_gemm_few's sums, a tile of 32 x 32
+        float round;                          // what a round of workgroups costs whatever there is of it
+        float weights, written, read;         // bytes a us: of weights, of partial products
+    };
+    static constexpr Rates kUpTo128 = {109e3f, 107e3f, 107e3f, 4.7e3f, 1.9f, 2.4f, 0.355f, 0.8f, 10.7e6f, 3.45e6f, 13.5e6f},
+                           kExact = {57e3f, 88e3f, 88e3f, 5.7e6f, 1.9f, 1.9f, 0.0f, 0.87f, 3.9e6f, 2.5e6f, 5e6f},
+                           kFast = {80e3f, 88e3f, 70e3f, 4.7e3f, 1.9f, 1.9f, 0.355f, 0.8f, 10.7e6f, 3.45e6f, 13.5e6f};
+    const Rates& c = t_pad <= 128 ? kUpTo128 : (lo ? kExact : kFast);
+    // A prompt and the same prompt filled up to 32, or beyond 128 tokens to 128, are summed alike: tokens count as whole columns
+    // of those, but for a pair beyond 128, where k_gemm_pipe is the faster one throughout and sums the same in either tile.
+    const int counted = t_pad > 128 && !pair ? t_pad : (min(live, t_pad) + 31) / 32 * 32, columns = counted / 32;
     float best_us = 1e30f;
     for (const auto& t : kTiles) {
         const Plan p = {t.few, t.fi, t.tj, 1};
-        const int rows = p.tile_rows(), tokens = p.tile_tokens();
-        if (!(lo ? t.exact : t.fast)) continue;
-        if (row_step % rows != 0 || t_pad % tokens != 0 || (pair && t.fi == 1)) continue;
+        const int rows = p.tile_rows(), tokens = p.tile_tokens(), token_tiles = p.token_tiles(t_pad, counted);
+        if (row_step % rows != 0 || token_tiles * tokens > t_pad || (pair && t.few && (t.fi == 1 || t_pad > 128))) continue;
         if (!t.few && t.fi == 4 && !wide_allowed) continue;
+        const int sent = min(tokens, 32 * ((columns + token_tiles - 1) / token_tiles));
         for (int splits = 1; splits <= max_splits; splits *= 2) {
             if (splits > 1 && (K % (64 * splits) != 0 || K / splits < 512)) continue;
-            const int wgs = total_n / rows * (t_pad / tokens) * splits;
-            const int rounds = (wgs + compute_units() - 1) / compute_units();
+            const int wgs = total_n / rows * token_tiles * splits, rounds = (wgs + compute_units() - 1) / compute_units();
             const float k = static_cast<float>(K) / splits, copies = lo ? 2.0f : 1.0f;
-            const float bytes = k * 2.0f * (rows + copies * tokens), clocks = k * copies * rows * tokens / 1024.0f;
-            const float busy = t.few ? bytes / 57e3f : bytes / 88e3f + clocks / 5.7e6f;
-            float us = (t.few || t_pad > 128 ? 1.9f : 2.9f) + fmaxf(fmaxf(1.0f, 0.87f * rounds + 0.13f * wgs / compute_units()) * busy, 2.0f * total_n * K / 3.9e6f);
-            if (splits > 1) us += 4.0f * t_pad * total_n * (splits / 2.5e6f + (splits - 1) / 5e6f);
+            const float bytes = k * 2.0f * (rows + copies * sent), clocks = k * copies * rows * sent / 1024.0f;
+            const float turns = fmaxf(1.0f, c.round * rounds + (1.0f - c.round) * wgs / compute_units());
+            const float busy = turns * (t.few ? bytes / c.few : fmaxf(bytes / (t.fi == 4 ? c.wide : c.pipe), clocks / c.clocks)), weights = 2.0f * total_n * K / c.weights;
+            float us = (t.few ? c.launch_few + c.sums * t.fi * t.tj * rounds : c.launch_pipe) + fmaxf(busy, weights) + 0.01f * fminf(busy, weights);
+            if (splits > 1) us += 4.0f * counted * total_n * (splits / c.written + (splits - 1) / c.read);
             if (us < best_us) {
                 best_us = us;
                 best = p;
@@ -1909,18 +1927,22 @@ lpp_status launch_plan(const Plan& p, const pf::PipeJob& job_in, hipStream_t s) 
         if (p.fi == 4) return launch_pipe<4, 2, kMode, 32>(job, s);
         return launch_pipe<2, 2, kMode>(job, s);
     }
-    const bool lo = job.xl != nullptr;
-    const int tile = 10 * p.fi + p.tj;
-    if (lo && tile == 41) return launch_few_as<4, 1, kMode, true>(job, s);
-    if (lo && tile == 42) return launch_few_as<4, 2, kMode, true>(job, s);
-    if (tile == 21) return lo ? launch_few_as<2, 1, kMode, true>(job, s) : launch_few_as<2, 1, kMode, false>(job, s);
-    if (tile == 22) return lo ? launch_few_as<2, 2, kMode, true>(job, s) : launch_few_as<2, 2, kMode, false>(job, s);
-    if (tile == 23) return lo ? launch_few_as<2, 3, kMode, true>(job, s) : launch_few_as<2, 3, kMode, false>(job, s);
-    if (!lo && tile == 24) return launch_few_as<2, 4, kMode, false>(job, s);
+    switch (10 * p.fi + p.tj) {
+        case 21: return launch_few<2, 1, kMode>(job, s);
+        case 22: return launch_few<2, 2, kMode>(job, s);
+        case 23: return launch_few<2, 3, kMode>(job, s);
+        case 24: return launch_few<2, 4, kMode>(job, s);
+        case 41: return launch_few<4, 1, kMode>(job, s);
+        case 42: return launch_few<4, 2, kMode>(job, s);
+        default: break;
+    }
     if constexpr (kMode != 2) {  // (a pair has as many rows of either matrix in a tile)
-        if (tile == 11) return lo ? launch_few_as<1, 1, kMode, true>(job, s) : launch_few_as<1, 1, kMode, false>(job, s);
-        if (!lo && tile == 12) return launch_few_as<1, 2, kMode, false>(job, s);
-        if (!lo && tile == 13) return launch_few_as<1, 3, kMode, false>(job, s);
+        switch (10 * p.fi + p.tj) {
+            case 11: return launch_few<1, 1, kMode>(job, s);
+            case 12: return launch_few<1, 2, kMode>(job, s);
+            case 13: return launch_few<1, 3, kMode>(job, s);
+            default: break;
+        }
     }
     return fail(LPP_ERR_STATE, "prefill GEMM: no kernel for a tile of %d x %d", p.tile_rows(), p.tile_tokens());
 }
@@ -1951,7 +1973,7 @@ lpp_status gemm(const Product* prods, int count, const pf::half_t* xh, const pf:
         int most = 1;
         while (partials != nullptr && (count == 1 || left_split != nullptr) && most < 8 && stride * 2 * most <= partial_floats) most *= 2;
         live = live < t_pad ? live : t_pad;
-        const Plan plan = plan_gemm(total_n, K, t_pad, most, remainder, step, false);
+        const Plan plan = plan_gemm(total_n, K, t_pad, live, most, remainder, step, false);
         const int tile = plan.tile_rows(), feature_tiles = total_n / tile, token_tiles = plan.token_tiles(t_pad, live), splits = plan.splits;
         pf::PipeJob job = {};
         int at = 0;
@@ -2070,7 +2092,7 @@ lpp_status gate_up_swiglu(const void* w1, const void* w3, int hidden, const pf::
     job.xl = remainder ? xl : nullptr;
     job.K = K;
     job.k_len = K;
-    const Plan plan = plan_gemm(2 * hidden, K, t_pad, 1, remainder, hidden % 128 == 0 ? 256 : 128, true);
+    const Plan plan = plan_gemm(2 * hidden, K, t_pad, live, 1, remainder, hidden % 128 == 0 ? 256 : 128, true);
     job.feature_tiles = 2 * hidden / plan.tile_rows();  // half of a tile's rows from either matrix
     job.token_tiles = plan.token_tiles(t_pad, live);
     job.live = live;
@@ -2322,8 +2344,10 @@ char g_setup_message[kMaxDevices][256] = {};
 template <int kMode>
 lpp_status size_few_for() {
     LPP_TRY((size_few<1, 1, kMode, true>()));
+    LPP_TRY((size_few<1, 2, kMode, true>()));
     LPP_TRY((size_few<2, 1, kMode, true>()));
     LPP_TRY((size_few<2, 2, kMode, true>()));
+    LPP_TRY((size_few<2, 4, kMode, true>()));
     LPP_TRY((size_few<4, 1, kMode, true>()));
     return size_few<4, 2, kMode, true>();
 }
