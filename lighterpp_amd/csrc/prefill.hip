@@ -1709,20 +1709,17 @@ int padded_tokens(int n) {
     return (n + unit - 1) / unit * unit;
 }
 
-// More than 256 tokens: k_gemm_pipe, 256 rows a tile where that leaves no compute unit without a workgroup (always for
-// a pair), otherwise 128 and K in as many ranges as the device takes at once.  In the exact mode also 256 where tiles of
-// 128 rows are more than the device takes at once: a second round of them costs more than compute units left idle, the
-// wider tile being a third more bytes from L2 and not twice as many (8B shape, 1280 ids: 38.2 -> 36.9 ms, 1792: 51.0 ->
-// 49.4).  In the fast mode it is half as many again, and the narrow tiles' rounds stay the faster ones.
-//
-// k_gemm_block where its blocks, in one range of K or several, should take less: what pays for fewer bytes to a product is
-// filling the device, so the two are compared by their rounds of workgroups.  A round is a launch's share that does not
-// depend on K, and K columns; a last round of a few workgroups still costs a third to two thirds of a full one.  The
-// constants are a fit to 860 timed launches (TinyLlama, 1B and 8B shapes, 384 to 2048 tokens; 3 to 5 % rms, of the tiles
-// of 128 x 128 7 to 9), partial products are written and read at 3 TB/s, and a block is taken where it gains 3 %.  W1+W3,
-// exact / fast mode, tiles against blocks: 1B shape 1024 ids 127 / 81 and 118 / 67 us, 1280 ids (a quarter of a second
-// round) 163 / 108 and 187 / 113, 2048 ids 236 / 156 and 217 / 127; 8B 512 ids 224 / 152 and 196 / 122, 1024 ids 426 / 280
-// and 369 / 224, W2 of 1024 ids 205 / 137 and, K in four ranges, 177 / 109.
+// More than 256 tokens: k_gemm_pipe's tiles of 128 or 256 rows or k_gemm_block, K in one range or several, by the rounds of
+// workgroups a launch of each makes.  A larger tile has fewer bytes to a product, a smaller one, or more ranges, fills the
+// device better.  A round costs a launch's share that does not depend on K, and K columns; a last round of a few workgroups
+// costs two thirds of a full one or more, and no launch less than one; partial products are written and read at 2.8 TB/s.
+// The constants are a fit to 4100 timed prefills (TinyLlama, 1B and 8B shapes, 300 to 2036 ids, both modes, each tile and cut
+// for each of the four products in turn): a prefill is within 1 % of what that product's fastest launch makes it, and faster
+// than by rules that cut K only while all ranges fit the device at once: exact / fast mode, 8B shape 370 ids 11.9 / 8.51 -> 10.7 /
+// 8.15 ms, 600 18.6 / 14.0 -> 17.1 / 12.3, 750 20.4 / 15.2 -> 19.6 / 14.1; 1B 1140 5.21 / 3.86 -> 4.91 / 3.63; TinyLlama 1530 7.53 ->
+// 7.17, 1140 in the fast mode 4.18 -> 3.99.
+// W1+W3, tiles against blocks: 1B shape 1024 ids 127 / 81 and 118 / 67 us, 1280 ids (a quarter of a second round) 163 / 108
+// and 187 / 113, 2048 ids 236 / 156 and 217 / 127; 8B 512 ids 224 / 152 and 196 / 122, 1024 ids 426 / 280 and 369 / 224.
 //
 // Up to 256 tokens the choice is made by what a launch of each would take.  A workgroup is paced by its bytes from L2 into
 // LDS, one of k_gemm_pipe by its MFMA clocks where they take longer; a
@@ -1743,13 +1740,13 @@ float planned_us(const Plan& p, int total_n, int K, int t_pad, bool lo, bool pai
     struct Cost {
         float launch, column, round, pair_round, rest;  // us, ns a column, us (the pair's: with SwiGLU), a last round's share at least
     };
-    static constexpr Cost kCosts[3][2] = {{{0.6f, 8.8f, 6.5f, 6.5f, 0.29f}, {0.0f, 13.5f, 8.0f, 8.0f, 0.33f}},       // 128 x 128
-                                          {{1.7f, 17.7f, 1.0f, 2.4f, 0.60f}, {1.7f, 24.8f, 8.0f, 9.7f, 0.52f}},      // 256 x 128
-                                          {{0.0f, 26.2f, 12.4f, 10.3f, 0.60f}, {0.0f, 42.4f, 12.8f, 19.4f, 0.65f}}}; // blocks
+    static constexpr Cost kCosts[3][2] = {{{4.9f, 7.4f, 4.7f, 4.9f, 0.67f}, {1.8f, 12.9f, 8.4f, 8.8f, 1.00f}},      // 128 x 128
+                                          {{6.3f, 16.2f, 7.6f, 1.2f, 0.83f}, {16.4f, 23.5f, 9.6f, 7.5f, 0.94f}},    // 256 x 128
+                                          {{0.0f, 20.5f, 5.8f, 18.4f, 1.00f}, {3.8f, 39.4f, 14.0f, 13.7f, 0.96f}}}; // blocks
     const Cost& c = kCosts[p.block() ? 2 : (p.fi == 4 ? 1 : 0)][lo ? 1 : 0];
     const int wgs = total_n / p.tile_rows() * p.token_tiles(t_pad, t_pad) * p.splits, left = wgs % compute_units();
-    const float rounds = wgs / compute_units() + (left > 0 ? c.rest + (1.0f - c.rest) * left / compute_units() : 0.0f);
-    const float partials = p.splits > 1 ? 4.0f * p.splits * t_pad * total_n / 3e6f : 0.0f;
+    const float rounds = fmaxf(1.0f, wgs / compute_units() + (left > 0 ? c.rest + (1.0f - c.rest) * left / compute_units() : 0.0f));
+    const float partials = p.splits > 1 ? 4.0f * p.splits * t_pad * total_n / 2.8e6f : 0.0f;
     return c.launch + rounds * (1e-3f * c.column * K / p.splits + (pair ? c.pair_round : c.round)) + partials;
 }
 Plan plan_gemm(int total_n, int K, int t_pad, int live, int max_splits, bool lo, int row_step, bool pair) {
@@ -1762,24 +1759,25 @@ Plan plan_gemm(int total_n, int K, int t_pad, int live, int max_splits, bool lo,
     Plan best = {false, 2, 2, 1};
     const bool wide_allowed = row_step % 256 == 0 && test_option(LPP_OPT_PREFILL_WIDE_TILES) != 0;
     if (t_pad > 256) {
-        const int token_tiles = t_pad / 128;
-        const bool wide = total_n / 256 * token_tiles >= compute_units() || (lo && total_n / 128 * token_tiles > compute_units());
-        if (pair || (wide_allowed && wide)) best.fi = 4;
-        while (2 * best.splits <= max_splits && total_n / best.tile_rows() * token_tiles * best.splits * 2 <= compute_units() &&
-               K % (64 * 2 * best.splits) == 0 && K / (2 * best.splits) >= 512)
-            best.splits *= 2;
-        if (!wide_allowed) return best;
-        const Plan tiles = best;
-        float best_us = 0.97f * planned_us(tiles, total_n, K, t_pad, lo, pair);
-        for (int splits = 1; splits <= max_splits; splits *= 2) {
-            const Plan block = {false, 4, 4, splits};
-            if (K % (64 * splits) != 0 || (splits > 1 && (K / splits < 512 || total_n / 256 * block.token_tiles(t_pad, t_pad) * splits > compute_units()))) break;
-            const float us = planned_us(block, total_n, K, t_pad, lo, pair);
-            if (us < best_us) {
-                best_us = us;
-                best = block;
-            }
+        if (!wide_allowed) {
+            const int token_tiles = t_pad / 128;
+            if (pair) best.fi = 4;
+            while (2 * best.splits <= max_splits && total_n / best.tile_rows() * token_tiles * best.splits * 2 <= compute_units() &&
+                   K % (64 * 2 * best.splits) == 0 && K / (2 * best.splits) >= 512)
+                best.splits *= 2;
+            return best;
         }
+        float best_us = 1e30f;
+        for (const auto& t : {Plan{false, 2, 2, 1}, Plan{false, 4, 2, 1}, Plan{false, 4, 4, 1}})
+            for (int splits = 1; splits <= max_splits; splits *= 2) {
+                if (splits > 1 && (K % (64 * splits) != 0 || K / splits < 512)) break;
+                const Plan p = {t.few, t.fi, t.tj, splits};
+                const float us = planned_us(p, total_n, K, t_pad, lo, pair);
+                if (us < best_us) {
+                    best_us = us;
+                    best = p;
+                }
+            }
         return best;
     }
     struct Rates {
