@@ -42,7 +42,6 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
-#include <unordered_map>
 #include <vector>
 
 #include "decode_phases.hpp"
@@ -3001,7 +3000,6 @@ lpp_status build_step_lists(lpp_model* m, const Plan& p, int which) {
     const int L = c.n_layers, dim = c.dim, hidden = c.hidden_dim, kv = m->kv_dim;
     const size_t wb = c.weight_precision == LPP_WEIGHT_FP16 ? 2 : 4;
     const int chunk_cols = static_cast<int>(1024 / wb);
-    const size_t rb_dim = static_cast<size_t>(dim) * wb, rb_hidden = static_cast<size_t>(hidden) * wb;
     const int n_xcc = m->df_xcc > 1 ? m->df_xcc : 1;
     auto base = [&](int t) { return reinterpret_cast<unsigned long long>(m->w[t]); };
     auto block_rows = [](int total, int block, int wg) {
@@ -3035,13 +3033,29 @@ lpp_status build_step_lists(lpp_model* m, const Plan& p, int which) {
     LPP_REQUIRE(b.results_floats <= static_cast<int>(df::kStepSlotMask) + 1 && dim < 65536 && hidden < 65536,
                 "persistent decode: shape too large for the step lists");
     std::vector<df::StepEntry> host(static_cast<size_t>(p.grid) * df::kGemvWaves * stride);
-    // columns of every matrix row the lists (and the parked rows) account for, keyed by the row's first byte
-    std::unordered_map<unsigned long long, int> covered;
+    // Columns of every matrix row that the lists (and the parked rows) account for, counted by row number: 3.7 million steps at
+    // the 8B shape, three lists (in a hash table by address a model's first token took 2.35 s there, 0.31 so; 1B shape 0.31 and 0.047).
+    const size_t layers = static_cast<size_t>(L);
+    const struct { int tensor; size_t rows; int cols; } all[] = {
+        {LPP_T_WQ, layers * dim, dim},    {LPP_T_WK, layers * kv, dim},     {LPP_T_WV, layers * kv, dim},  {LPP_T_WO, layers * dim, dim},
+        {LPP_T_W1, layers * hidden, dim}, {LPP_T_W3, layers * hidden, dim}, {LPP_T_W2, layers * dim, hidden},
+        {LPP_T_WCLS, static_cast<size_t>(c.vocab_size), dim}};
+    std::vector<int> covered[LPP_T_COUNT];
+    for (const auto& t : all) covered[t.tensor].assign(t.rows, 0);
+    struct Row {
+        int tensor;
+        size_t row;
+    };
+    bool outside = false;
+    auto cover = [&](const Row& at, int columns) {
+        if (at.row < covered[at.tensor].size()) covered[at.tensor][at.row] += columns;
+        else outside = true;
+    };
     for (int wg = 0; wg < p.grid; ++wg)
         for (int j = 0; j < df::kGemvWaves; ++j) {
             df::StepEntry* out = host.data() + (static_cast<size_t>(wg) * df::kGemvWaves + j) * stride;
             int n = 0;
-            auto phase_rows = [&](int phase, int nrows, int d, auto row_address) {
+            auto phase_rows = [&](int phase, int nrows, int d, auto row_of) {
                 const int nslices = df::slice_count(d, chunk_cols), width = df::slice_width(d, chunk_cols);
                 const int slice = j % nslices, rank = j / nslices, share = df::kGemvWaves / nslices;
                 const int begin = slice * width;
@@ -3056,11 +3070,12 @@ lpp_status build_step_lists(lpp_model* m, const Plan& p, int which) {
                 for (int i = 0; i * share < nrows; ++i) {
                     const int r = i * share + (rank + i) % share;
                     if (r >= nrows) continue;
-                    out[n].ptr = row_address(r) + static_cast<size_t>(begin) * wb;
+                    const Row at = row_of(r);
+                    out[n].ptr = base(at.tensor) + (at.row * d + begin) * wb;
                     out[n].meta = static_cast<unsigned>(r * df::slices_used(d, chunk_cols) + slice) |
                                   (static_cast<unsigned>(phase) << df::kStepPhaseShift) | df::kStepValid;
                     out[n].cols = static_cast<unsigned>(begin) | (static_cast<unsigned>(exist) << 16);
-                    covered[row_address(r)] += exist;
+                    cover(at, exist);
                     ++n;
                 }
                 if (n > first) out[n - 1].meta |= df::kStepLastRow;
@@ -3068,23 +3083,22 @@ lpp_status build_step_lists(lpp_model* m, const Plan& p, int which) {
             for (int l = 0; l < L; ++l) {
                 phase_rows(4 * l + df::kGQkv, df::qkv_rows(b, dim, kv, m->head_size, m->gqa, wg, wg / n_xcc), dim, [&](int r) {
                     const int g = df::qkv_row(b, dim, kv, m->head_size, m->gqa, wg, wg % n_xcc, wg / n_xcc, r);
-                    if (g < dim) return base(LPP_T_WQ) + (static_cast<size_t>(l) * dim + g) * rb_dim;
-                    if (g < dim + kv) return base(LPP_T_WK) + (static_cast<size_t>(l) * kv + (g - dim)) * rb_dim;
-                    return base(LPP_T_WV) + (static_cast<size_t>(l) * kv + (g - dim - kv)) * rb_dim;
+                    if (g < dim) return Row{LPP_T_WQ, static_cast<size_t>(l) * dim + g};
+                    if (g < dim + kv) return Row{LPP_T_WK, static_cast<size_t>(l) * kv + (g - dim)};
+                    return Row{LPP_T_WV, static_cast<size_t>(l) * kv + (g - dim - kv)};
                 });
                 phase_rows(4 * l + df::kGO, block_rows(dim, b.o, wg), dim,
-                           [&](int r) { return base(LPP_T_WO) + (static_cast<size_t>(l) * dim + wg * b.o + r) * rb_dim; });
+                           [&](int r) { return Row{LPP_T_WO, static_cast<size_t>(l) * dim + wg * b.o + r}; });
                 // local row 2u = gate row of hidden unit u, 2u + 1 = its up row
                 phase_rows(4 * l + df::kGGateUp, gu_streamed(wg), dim, [&](int r) {
-                    return base((r & 1) ? LPP_T_W3 : LPP_T_W1) +
-                           (static_cast<size_t>(l) * hidden + df::gu_unit0(p.gu_first.data(), wg) + (r >> 1)) * rb_dim;
+                    return Row{(r & 1) ? LPP_T_W3 : LPP_T_W1, static_cast<size_t>(l) * hidden + df::gu_unit0(p.gu_first.data(), wg) + (r >> 1)};
                 });
                 phase_rows(4 * l + df::kGDown, block_rows(dim, b.down, wg), hidden, [&](int r) {
-                    return base(LPP_T_W2) + (static_cast<size_t>(l) * dim + wg * b.down + r) * rb_hidden;
+                    return Row{LPP_T_W2, static_cast<size_t>(l) * dim + wg * b.down + r};
                 });
             }
             phase_rows(4 * L, block_rows(c.vocab_size, b.cls, wg), dim,
-                       [&](int r) { return base(LPP_T_WCLS) + (static_cast<size_t>(wg) * b.cls + r) * rb_dim; });
+                       [&](int r) { return Row{LPP_T_WCLS, static_cast<size_t>(wg) * b.cls + r}; });
             for (; n < stride; ++n) {
                 out[n].ptr = base(LPP_T_WCLS);
                 out[n].meta = 0;
@@ -3096,28 +3110,14 @@ lpp_status build_step_lists(lpp_model* m, const Plan& p, int which) {
         const int units = df::gu_units(p.gu_first.data(), wg), parked = df::gu_parked_rows(b, wg, units);
         for (int l = 0; l < L; ++l)
             for (int r = 2 * units - parked; r < 2 * units; ++r)
-                covered[base((r & 1) ? LPP_T_W3 : LPP_T_W1) + (static_cast<size_t>(l) * hidden + df::gu_unit0(p.gu_first.data(), wg) + (r >> 1)) * rb_dim] += dim;
+                cover(Row{(r & 1) ? LPP_T_W3 : LPP_T_W1, static_cast<size_t>(l) * hidden + df::gu_unit0(p.gu_first.data(), wg) + (r >> 1)}, dim);
     }
-    {
-        const struct { int tensor; size_t rows; int cols; } all[] = {
-            {LPP_T_WQ, static_cast<size_t>(L) * dim, dim},       {LPP_T_WK, static_cast<size_t>(L) * kv, dim},
-            {LPP_T_WV, static_cast<size_t>(L) * kv, dim},        {LPP_T_WO, static_cast<size_t>(L) * dim, dim},
-            {LPP_T_W1, static_cast<size_t>(L) * hidden, dim},    {LPP_T_W3, static_cast<size_t>(L) * hidden, dim},
-            {LPP_T_W2, static_cast<size_t>(L) * dim, hidden},    {LPP_T_WCLS, static_cast<size_t>(c.vocab_size), dim}};
-        size_t expected = 0;
-        for (const auto& t : all) {
-            expected += t.rows;
-            for (size_t r = 0; r < t.rows; ++r) {
-                const auto it = covered.find(base(t.tensor) + r * static_cast<size_t>(t.cols) * wb);
-                if (it == covered.end() || it->second != t.cols)
-                    return fail(LPP_ERR_STATE, "persistent decode: step lists cover %d of %d columns of row %zu of tensor %d",
-                                it == covered.end() ? 0 : it->second, t.cols, r, t.tensor);
-            }
-        }
-        // (a tied classifier shares no rows with the other matrices: it is its own binary16 copy)
-        if (covered.size() != expected) return fail(LPP_ERR_STATE, "persistent decode: step lists name %zu rows, the model has %zu",
-                                                    covered.size(), expected);
-    }
+    if (outside) return fail(LPP_ERR_STATE, "persistent decode: step lists name a row that the model does not have");
+    for (const auto& t : all)
+        for (size_t r = 0; r < t.rows; ++r)
+            if (covered[t.tensor][r] != t.cols)
+                return fail(LPP_ERR_STATE, "persistent decode: step lists cover %d of %d columns of row %zu of tensor %d", covered[t.tensor][r],
+                            t.cols, r, t.tensor);
     lpp_free(m->df_rows[which]);
     m->df_rows[which] = nullptr;
     lpp_free(m->df_gu_first[which]);
