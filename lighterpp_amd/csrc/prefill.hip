@@ -350,16 +350,19 @@ __global__ __launch_bounds__(256) void k_gemm(const half_t* __restrict__ w, cons
 // wavefront that uses it).  What bounds a full tile is the device's power, so the products are
 // v_mfma_f32_16x16x32_f16, remainder right behind head in the same accumulator: 32 x 32 x 16 needs a lower clock for the same
 // work (the exact mode's W1+W3, 512 ids: 1B shape 69 -> 63 us, 8B 252 -> 224; of 2048 ids of the 1B shape 260 -> 236, W2 127 ->
-// 112; the fast mode, half of it data, 2 to 5 %).  A trip covers kTripK columns (64 = a whole cache line per row and
-// trip, or 32 where 64 would leave room for two stages only): the rows of the three operand
+// 112; the fast mode, half of it data, 2 to 5 %).  A trip covers 64 columns, a whole cache line of every row: L2 gives a compute
+// unit 100 bytes a nanosecond in requests of whole lines and 70 in halves of lines.  The rows of the three operand
 // tiles lie one after the other in a stage of LDS, and a requesting wavefront fills 1 KiB of it
 // with one global_load_lds_dwordx4 (lane i -> 16 bytes at M0 + 16 i): no registers are staged
 // and nothing waits for the data but the s_waitcnt ahead of the trip that multiplies it.  As
-// many stages as 160 KiB hold, five at most.
+// many stages as 160 KiB hold, five at most.  Of 256 x 128 tiles in the exact mode a stage would be 64 KiB, two of them too few:
+// there a trip's weight rows and its token rows are halves of 32 KiB that come and go by themselves, five of them; the weights
+// have two trips to arrive in, the tokens one.  (W1+W3 of 512 ids of the 1B shape, with trips of 32 columns in five stages
+// and so: exact mode 67.9 -> 63.3 us, a prefill 2.33 -> 2.27 ms; fast mode, in three whole stages, 1.87 -> 1.76.)
 //
 // LDS banks: a fragment read takes 16 bytes per lane from 16 consecutive rows; with rows of 128
-// (64) bytes every second (fourth) row starts in the same bank, so the 16-byte pieces of row r
-// are stored in the order piece ^ ((r >> 1) & 7) (piece ^ ((r >> 2) & 3)): 16 consecutive lanes then
+// bytes every second row starts in the same bank, so the 16-byte pieces of row r
+// are stored in the order piece ^ ((r >> 1) & 7): 16 consecutive lanes then
 // cover all 64 banks once.  The permutation is applied on the way in, by the address each lane
 // requests.
 //
@@ -389,17 +392,19 @@ struct PipeJob {
     int rows;        // k_gemm_block: rows of x and of the output, a multiple of 32
 };
 
-constexpr int kPipeTripK = 64;  // columns per trip of the narrow tiles; K must be a multiple
+constexpr int kPipeTripK = 64;  // columns per trip; K must be a multiple
 
 // (kLo: the activations' remainder tile travels and is multiplied too; without it a stage is a third smaller)
-template <int kFi, int kTj, int kTripK, bool kLo = true>
+template <int kFi, int kTj, bool kLo = true>
 struct PipeShape {
-    static constexpr int kRowBytes = 2 * kTripK;
+    static constexpr int kRowBytes = 2 * kPipeTripK;
     static constexpr int kRowsA = 64 * kFi, kRowsB = 64 * kTj, kRows = kRowsA + (kLo ? 2 : 1) * kRowsB;
     static constexpr int kStageBytes = kRows * kRowBytes;
+    // (where a trip's rows of weights and of tokens are 32 KiB each, they come and go by themselves: five such halves)
+    static constexpr bool kHalves = kStageBytes == 65536 && kRowsA == kRows / 2;
     static constexpr int kStages = (160 * 1024) / kStageBytes > 5 ? 5 : (160 * 1024) / kStageBytes;
     static constexpr int kLoads = kStageBytes / 4096;  // requests of 1 KiB per wavefront and stage
-    static constexpr int kLdsBytes = kStages * kStageBytes;
+    static constexpr int kLdsBytes = kHalves ? 5 * 32768 : kStages * kStageBytes;
 };
 
 template <int kCount>
@@ -499,14 +504,14 @@ __device__ __forceinline__ void leave(const floatx4 (&acc)[kI][kJ], char* room, 
     }
 }
 
-template <int kFi, int kTj, int kMode, int kTripK, bool kLo, bool kRagged>
+template <int kFi, int kTj, int kMode, bool kLo, bool kRagged>
 __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
-    typedef PipeShape<kFi, kTj, kTripK, kLo> Shape;
+    typedef PipeShape<kFi, kTj, kLo> Shape;
     constexpr int kRowsA = Shape::kRowsA, kRowsB = Shape::kRowsB, kStages = Shape::kStages, kLoads = Shape::kLoads;
     constexpr int kStageBytes = Shape::kStageBytes, kRowBytes = Shape::kRowBytes;
-    constexpr int kSteps = kTripK / 32;      // k-steps per trip
-    constexpr int kPieces = kTripK / 8;      // 16-byte pieces of a row
-    constexpr int kSwizzleShift = kPieces == 8 ? 1 : 2;
+    constexpr bool kHalves = Shape::kHalves;
+    constexpr int kSteps = kPipeTripK / 32;  // k-steps per trip
+    constexpr int kPieces = kPipeTripK / 8;  // 16-byte pieces of a row
     extern __shared__ __align__(1024) char pipe_lds[];
     const int lane = lane_id();
     const int wave_of_8 = __builtin_amdgcn_readfirstlane(wave_index());
@@ -537,7 +542,7 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
 #pragma unroll
     for (int q = 0; q < kLoads; ++q) {
         const int row = (64 / kPieces) * (wave + 4 * q) + lane / kPieces;
-        const int piece = (lane % kPieces) ^ ((row >> kSwizzleShift) & (kPieces - 1));
+        const int piece = (lane % kPieces) ^ ((row >> 1) & (kPieces - 1));
         const half_t* from;
         if (row < kRowsA) {
             if constexpr (kMode == 2) {
@@ -557,10 +562,10 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
     }
     const unsigned lds_base = static_cast<unsigned>(reinterpret_cast<uintptr_t>(
         (__attribute__((address_space(3))) char*)pipe_lds));
-    const int trips = job.k_len / kTripK;
-    // (tile_columns: columns of 32 tokens that the tile has; where a request is of eight rows, those of the others are not made)
-    constexpr int kWeightLoads = kRowsA / (64 / kPieces) / 4, kColumnLoads = kPieces == 8 ? 1 : 0, kTileColumns = 2 * kTj;
-    auto made = [&](int q, int tile_columns) { return kColumnLoads == 0 || q < kWeightLoads || (q - kWeightLoads) % kTileColumns < tile_columns; };
+    const int trips = job.k_len / kPipeTripK;
+    // (tile_columns: columns of 32 tokens that the tile has; the requests of the others are not made)
+    constexpr int kWeightLoads = kRowsA / (64 / kPieces) / 4, kTileColumns = 2 * kTj;
+    auto made = [&](int q, int tile_columns) { return q < kWeightLoads || (q - kWeightLoads) % kTileColumns < tile_columns; };
     auto request = [&](int trip, auto tile_columns) {
         const unsigned at = __builtin_amdgcn_readfirstlane(lds_base + (trip % kStages) * kStageBytes + wave * 1024);
         const int column = __builtin_amdgcn_readfirstlane(trip * kRowBytes);
@@ -572,13 +577,25 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
                 asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off\n" ::"v"(from), "s"(to) : "memory");
             }
     };
+    // kHalves: half u is the weight rows of trip u / 2 (even) or its token rows
+    auto request_half = [&](int u, auto odd, auto tile_columns) {
+        const unsigned at = __builtin_amdgcn_readfirstlane(lds_base + (u % 5) * 32768 + wave * 1024);
+        const int column = __builtin_amdgcn_readfirstlane((u >> 1) * kRowBytes);
+#pragma unroll
+        for (int q = odd * kWeightLoads; q < (odd ? kLoads : kWeightLoads); ++q)
+            if (made(q, tile_columns)) {
+                const char* from = src[q] + column;
+                const unsigned to = at + (q - odd * kWeightLoads) * 4096;
+                asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off\n" ::"v"(from), "s"(to) : "memory");
+            }
+    };
     // where each lane reads its fragments: row lane % 16 of an MFMA tile, piece 4 s + lane / 16 of k-step s
     int a_off[kSteps], b_off[kSteps];
 #pragma unroll
     for (int s = 0; s < kSteps; ++s) {
-        const int row = lane & 15, piece = (4 * s + (lane >> 4)) ^ ((row >> kSwizzleShift) & (kPieces - 1));
+        const int row = lane & 15, piece = (4 * s + (lane >> 4)) ^ ((row >> 1) & (kPieces - 1));
         a_off[s] = (wf * 32 * kFi + row) * kRowBytes + 16 * piece;
-        b_off[s] = (kRowsA + wt * 32 * kTj + row) * kRowBytes + 16 * piece;
+        b_off[s] = ((kHalves ? 0 : kRowsA) + wt * 32 * kTj + row) * kRowBytes + 16 * piece;
     }
 
     constexpr int kI = 2 * kFi, kJ = 2 * kTj;  // MFMA tiles of the wavefront
@@ -593,12 +610,12 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
     };
     half8_t a[kI];
     auto read_tokens = [&](Tokens& f, int trip, int s, int j) {
-        const char* stage = pipe_lds + (trip % kStages) * kStageBytes;
+        const char* stage = pipe_lds + (kHalves ? (2 * trip + 1) % 5 * 32768 : (trip % kStages) * kStageBytes);
         f.h[j] = *reinterpret_cast<const half8_t*>(stage + b_off[s] + j * 16 * kRowBytes);
         if constexpr (kLo) f.l[j] = *reinterpret_cast<const half8_t*>(stage + b_off[s] + (kRowsB + j * 16) * kRowBytes);
     };
     auto read_weights = [&](int trip, int s, int i) {
-        const char* stage = pipe_lds + (trip % kStages) * kStageBytes;
+        const char* stage = pipe_lds + (kHalves ? 2 * trip % 5 * 32768 : (trip % kStages) * kStageBytes);
         a[i] = *reinterpret_cast<const half8_t*>(stage + a_off[s] + i * 16 * kRowBytes);
     };
     // (one weight tile's MFMAs of a k-step)
@@ -613,7 +630,7 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
     // (requesting wavefronts) wait until the requests of `trip` have landed: those of later trips, at
     // most kStages - 2 of them, may be in flight
     auto landed = [&](int trip, int trips, auto tile_columns) {
-        constexpr int kMade = kLoads - kColumnLoads * (kLo ? 2 : 1) * (kTileColumns - decltype(tile_columns)::value);
+        constexpr int kMade = kLoads - (kLo ? 2 : 1) * (kTileColumns - decltype(tile_columns)::value);
         const int later = trips - 1 - trip;
         if (kStages > 2 && later >= kStages - 2) wait_requests<(kStages - 2) * kMade>();
         else wait_requests<0>();
@@ -624,6 +641,35 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
     // trip t + kStages.
     const int tile_end = kRagged ? min(job.live, t_base + job.each) : t_base + kRowsB;
     auto feed = [&](auto tile_columns) {
+        if constexpr (kHalves) {
+            // Weights, which may come from memory, have two trips to arrive in, tokens, which are in L2, one.
+            constexpr int kTokenLoads = (kLo ? 2 : 1) * decltype(tile_columns)::value;
+            constexpr std::integral_constant<int, 0> weights{};
+            constexpr std::integral_constant<int, 1> tokens{};
+            request_half(0, weights, tile_columns);
+            request_half(1, tokens, tile_columns);
+            if (trips > 1) {
+                request_half(2, weights, tile_columns);
+                request_half(3, tokens, tile_columns);
+            }
+            if (trips > 2) {
+                request_half(4, weights, tile_columns);
+                wait_requests<2 * kWeightLoads + kTokenLoads>();
+            } else if (trips > 1) {
+                wait_requests<kWeightLoads + kTokenLoads>();
+            } else {
+                wait_requests<0>();
+            }
+            __syncthreads();
+            for (int t = 0; t < trips; ++t) {
+                if (t + 2 < trips) wait_requests<kWeightLoads>();  // (those of trip t + 2)
+                else wait_requests<0>();
+                __syncthreads();
+                if (t + 2 < trips) request_half(2 * t + 5, tokens, tile_columns);
+                if (t + 3 < trips) request_half(2 * t + 6, weights, tile_columns);
+            }
+            return;
+        }
 #pragma unroll
         for (int t = 0; t < kStages - 1; ++t)
             if (__builtin_expect(t < trips, 1)) request(t, tile_columns);
@@ -637,7 +683,7 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
         }
     };
     if (requester) {
-        if constexpr (kRagged && kColumnLoads != 0) {
+        if constexpr (kRagged) {
             static_assert(kTileColumns == 4, "columns of a tile");
             const int tile_columns = __builtin_amdgcn_readfirstlane((tile_end - t_base + 31) / 32);
             if (tile_columns >= 4) feed(std::integral_constant<int, 4>{});
@@ -685,18 +731,10 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
                 }
             }
         };
-        if constexpr (kSteps == 2) {
-            for (int t = 0; t < trips; ++t) {
-                step(tokens[0], tokens[1], t, std::integral_constant<int, 0>{});
-                step(tokens[1], tokens[0], t, std::integral_constant<int, 1>{});
-            }
-        } else {
-            int t = 0;
-            for (; t + 1 < trips; t += 2) {
-                step(tokens[0], tokens[1], t, std::integral_constant<int, 0>{});
-                step(tokens[1], tokens[0], t + 1, std::integral_constant<int, 0>{});
-            }
-            if (t < trips) step(tokens[0], tokens[1], t, std::integral_constant<int, 0>{});
+        static_assert(kSteps == 2, "the tokens' fragments of a trip are in the two sets");
+        for (int t = 0; t < trips; ++t) {
+            step(tokens[0], tokens[1], t, std::integral_constant<int, 0>{});
+            step(tokens[1], tokens[0], t, std::integral_constant<int, 1>{});
         }
     };
     // kRagged: columns of 32 tokens that are not the tile's, or past the last token, are neither multiplied nor stored.
@@ -711,8 +749,8 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
         walk(std::integral_constant<int, kTj>{});
     }
     // (room: the wavefront's quarter of a stage that neither the last trip nor the read past it uses)
-    static_assert(kStages >= 3 && kStageBytes / 4 >= kLeaveBytes, "room for a transposed tile per wavefront");
-    char* room = pipe_lds + ((trips + 1) % kStages) * kStageBytes + wave * (kStageBytes / 4);
+    static_assert(kHalves ? kLeaveBytes <= 8192 : kStages >= 3 && kStageBytes / 4 >= kLeaveBytes, "room for a transposed tile per wavefront");
+    char* room = pipe_lds + (kHalves ? (2 * trips + 2) % 5 * 32768 + wave * 8192 : ((trips + 1) % kStages) * kStageBytes + wave * (kStageBytes / 4));
     leave<kMode, kLo>(acc, room, job, which, split, t_base + wt * 32 * kTj, kRagged ? 2 * columns : kJ, f_base, wf);
 }
 
@@ -721,7 +759,7 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
 // Eight wavefronts, two to a SIMD, all of them multiply: each owns 128 features x 64 tokens.  The two of a SIMD take turns,
 // one barrier apart: while one multiplies a trip of 32 columns, the other reads its fragments of the trip from LDS and sends
 // for a later one, so the matrix cores are busy but for the barriers (4650 clocks for 4096 clocks of MFMAs) and a
-// wavefront that a request holds up holds nobody else.  A trip's rows are 64 bytes, in the order of k_gemm_pipe's narrow trips;
+// wavefront that a request holds up holds nobody else.  A trip's rows are 64 bytes, their pieces in the order piece ^ ((r >> 2) & 3);
 // kStages trips are in LDS at once.
 //
 // What bounds it is the device's power, not its clocks: the loop of the exact mode runs at 1.7 GHz, and what makes it
@@ -1612,11 +1650,11 @@ lpp_status size_lds(const void* kernel, int bytes, bool (&sized)[64]) {
     }
     return LPP_OK;
 }
-template <int kFi, int kTj, int kMode, int kTripK, bool kLo = true, bool kRagged = false>
+template <int kFi, int kTj, int kMode, bool kLo = true, bool kRagged = false>
 lpp_status size_pipe() {
     static bool sized[64] = {};
-    return size_lds(reinterpret_cast<const void*>(&pf::k_gemm_pipe<kFi, kTj, kMode, kTripK, kLo, kRagged>),
-                    pf::PipeShape<kFi, kTj, kTripK, kLo>::kLdsBytes, sized);
+    return size_lds(reinterpret_cast<const void*>(&pf::k_gemm_pipe<kFi, kTj, kMode, kLo, kRagged>),
+                    pf::PipeShape<kFi, kTj, kLo>::kLdsBytes, sized);
 }
 template <int kFi, int kTj, int kMode, bool kLo, bool kRagged = false>
 lpp_status size_few() {
@@ -1624,12 +1662,12 @@ lpp_status size_few() {
     return size_lds(reinterpret_cast<const void*>(&pf::k_gemm_few<kFi, kTj, kMode, kLo, kRagged>), pf::FewShape<kFi, kTj, kLo>::kLdsBytes, sized);
 }
 
-template <int kFi, int kTj, int kMode, int kTripK, bool kLo, bool kRagged>
+template <int kFi, int kTj, int kMode, bool kLo, bool kRagged>
 lpp_status launch_pipe_as(const pf::PipeJob& job, hipStream_t s) {
-    typedef pf::PipeShape<kFi, kTj, kTripK, kLo> Shape;
-    LPP_TRY((size_pipe<kFi, kTj, kMode, kTripK, kLo, kRagged>()));
+    typedef pf::PipeShape<kFi, kTj, kLo> Shape;
+    LPP_TRY((size_pipe<kFi, kTj, kMode, kLo, kRagged>()));
     const int per_die = (job.groups + 7) / 8;
-    hipLaunchKernelGGL((pf::k_gemm_pipe<kFi, kTj, kMode, kTripK, kLo, kRagged>), dim3(per_die * 8 * job.token_tiles), dim3(512), Shape::kLdsBytes, s,
+    hipLaunchKernelGGL((pf::k_gemm_pipe<kFi, kTj, kMode, kLo, kRagged>), dim3(per_die * 8 * job.token_tiles), dim3(512), Shape::kLdsBytes, s,
                        job);
     LPP_CHECK_LAUNCH("k_gemm_pipe");
     return LPP_OK;
@@ -1642,16 +1680,16 @@ lpp_status launch_pipe_as(const pf::PipeJob& job, hipStream_t s) {
 // 2.495).  The tokens are dealt out evenly where that makes every tile narrower: 150 ids as 96 + 54, 1.585 -> 1.495 ms; 8B
 // shape 7.73 -> 7.05.  In the fast mode only that pays: 150 ids 1.417 -> 1.280, 257 ids 1.721 -> 1.625, but 200 ids, cut
 // 128 + 72 either way, 1.454 -> 1.463.
-template <int kFi, int kTj, int kMode, int kTripK = pf::kPipeTripK>
+template <int kFi, int kTj, int kMode>
 lpp_status launch_pipe(const pf::PipeJob& job_in, hipStream_t s) {
     pf::PipeJob job = job_in;
     const int columns = (job.live + 31) / 32, all = 2 * kTj * job.token_tiles;
     job.each = 32 * ((columns + job.token_tiles - 1) / job.token_tiles);
     if (job.xl != nullptr ? 12 * (all - columns) >= all : job.each < 64 * kTj)
-        return job.xl != nullptr ? launch_pipe_as<kFi, kTj, kMode, kTripK, true, true>(job, s)
-                                 : launch_pipe_as<kFi, kTj, kMode, kTripK, false, true>(job, s);
-    return job.xl != nullptr ? launch_pipe_as<kFi, kTj, kMode, kTripK, true, false>(job, s)
-                             : launch_pipe_as<kFi, kTj, kMode, kTripK, false, false>(job, s);
+        return job.xl != nullptr ? launch_pipe_as<kFi, kTj, kMode, true, true>(job, s)
+                                 : launch_pipe_as<kFi, kTj, kMode, false, true>(job, s);
+    return job.xl != nullptr ? launch_pipe_as<kFi, kTj, kMode, true, false>(job, s)
+                             : launch_pipe_as<kFi, kTj, kMode, false, false>(job, s);
 }
 
 template <int kMode, bool kLo>
@@ -1729,8 +1767,7 @@ int padded_tokens(int n) {
 // prefills (TinyLlama, 1B and 8B shapes, 10 to 256 ids, both modes, every tile of the list for each of the four products in
 // turn): up to 128 tokens a prefill is 0.3 % slower on average than with that product's fastest launch.  In the exact mode
 // beyond 128 tokens the constants are an earlier fit's, which makes the better choices there (256 ids of the TinyLlama shape
-// 2.03 ms, 2.06 by the newer one).  Tiles of 256 rows have rows of 64 bytes in a stage, requests of half lines: L2 gives 70
-// bytes a nanosecond to a compute unit that way and 100 in whole lines.
+// 2.03 ms, 2.06 by the newer one).
 // Exact mode, by the earlier fit and so: 8B shape 10 ids 3.54 -> 3.35 ms, 40 4.21 -> 3.95, 90 5.76 -> 4.66; 1B 100 ids 1.27 -> 1.21;
 // fast mode: 8B 48 ids 4.34 -> 3.58, 120 5.02 -> 4.39, 1B 200 1.44 -> 1.28, TinyLlama 220 1.84 -> 1.67.
 //
@@ -1741,7 +1778,7 @@ float planned_us(const Plan& p, int total_n, int K, int t_pad, bool lo, bool pai
         float launch, column, round, pair_round, rest;  // us, ns a column, us (the pair's: with SwiGLU), a last round's share at least
     };
     static constexpr Cost kCosts[3][2] = {{{4.9f, 7.4f, 4.7f, 4.9f, 0.67f}, {1.8f, 12.9f, 8.4f, 8.8f, 1.00f}},      // 128 x 128
-                                          {{6.3f, 16.2f, 7.6f, 1.2f, 0.83f}, {16.4f, 23.5f, 9.6f, 7.5f, 0.94f}},    // 256 x 128
+                                          {{6.3f, 13.0f, 7.6f, 1.2f, 1.00f}, {16.4f, 21.3f, 9.6f, 7.5f, 0.94f}},    // 256 x 128
                                           {{0.0f, 20.5f, 5.8f, 18.4f, 1.00f}, {3.8f, 39.4f, 14.0f, 13.7f, 0.96f}}}; // blocks
     const Cost& c = kCosts[p.block() ? 2 : (p.fi == 4 ? 1 : 0)][lo ? 1 : 0];
     const int wgs = total_n / p.tile_rows() * p.token_tiles(t_pad, t_pad) * p.splits, left = wgs % compute_units();
@@ -1788,7 +1825,7 @@ Plan plan_gemm(int total_n, int K, int t_pad, int live, int max_splits, bool lo,
     };
     static constexpr Rates kUpTo128 = {109e3f, 107e3f, 107e3f, 4.7e3f, 1.9f, 2.4f, 0.355f, 0.8f, 10.7e6f, 3.45e6f, 13.5e6f},
                            kExact = {57e3f, 88e3f, 88e3f, 5.7e6f, 1.9f, 1.9f, 0.0f, 0.87f, 3.9e6f, 2.5e6f, 5e6f},
-                           kFast = {80e3f, 88e3f, 70e3f, 4.7e3f, 1.9f, 1.9f, 0.355f, 0.8f, 10.7e6f, 3.45e6f, 13.5e6f};
+                           kFast = {80e3f, 88e3f, 80e3f, 4.7e3f, 1.9f, 1.9f, 0.355f, 0.8f, 10.7e6f, 3.45e6f, 13.5e6f};
     const Rates& c = t_pad <= 128 ? kUpTo128 : (lo ? kExact : kFast);
     // A prompt and the same prompt filled up to 32, or beyond 128 tokens to 128, are summed alike: tokens count as whole columns
     // of those, but for a pair beyond 128, where k_gemm_pipe is the faster one throughout and sums the same in either tile.
@@ -1922,7 +1959,7 @@ lpp_status launch_plan(const Plan& p, const pf::PipeJob& job_in, hipStream_t s) 
     job.band = band_of(job.token_tiles, job.xl != nullptr);
     if (p.block()) return job.xl != nullptr ? launch_block<kMode, true>(job, s) : launch_block<kMode, false>(job, s);
     if (!p.few) {
-        if (p.fi == 4) return launch_pipe<4, 2, kMode, 32>(job, s);
+        if (p.fi == 4) return launch_pipe<4, 2, kMode>(job, s);
         return launch_pipe<2, 2, kMode>(job, s);
     }
     switch (10 * p.fi + p.tj) {
@@ -2351,10 +2388,10 @@ lpp_status size_few_for() {
 }
 
 lpp_status run_scratch_setup() {
-    LPP_TRY((size_pipe<4, 2, 0, 32>()));
-    LPP_TRY((size_pipe<4, 2, 1, 32>()));
-    LPP_TRY((size_pipe<2, 2, 0, pf::kPipeTripK>()));
-    LPP_TRY((size_pipe<2, 2, 1, pf::kPipeTripK>()));
+    LPP_TRY((size_pipe<4, 2, 0>()));
+    LPP_TRY((size_pipe<4, 2, 1>()));
+    LPP_TRY((size_pipe<2, 2, 0>()));
+    LPP_TRY((size_pipe<2, 2, 1>()));
     LPP_TRY((size_block<0, true>()));
     LPP_TRY((size_block<1, true>()));
     LPP_TRY((size_few_for<0>()));
