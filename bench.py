@@ -46,12 +46,12 @@ HBM_PEAK_GBS = 8000.0
 # (profiles/persistent_decode_<workload>_pmc_hbm_traffic.txt give the commands, one file per configuration).
 _CSRC = ROOT / "lighterpp_amd" / "csrc"
 KERNEL_SOURCES = {"k_decode_dataflow": [_CSRC / f for f in ("dataflow_decode.hip", "decode_phases.hpp", "lpp_device.hpp", "sampler.hpp")]}
-_MEASURED_SOURCE = "39da43a65068c2676c513e14a15d57050e482cd1ea11b3c82ef68c917697957b"
+_MEASURED_SOURCE = "5a279f7465ec85c6d19b97c3abe10a73877a09876be6ce5ed0d5b20351a4e208"
 MEASURED_HBM_BYTES_PER_LAUNCH = {
-    ("c2_tinyllama_1b_fp16", "k_decode_dataflow"): (2.1262e9, _MEASURED_SOURCE),
+    ("c2_tinyllama_1b_fp16", "k_decode_dataflow"): (2.1261e9, _MEASURED_SOURCE),
     ("c3_llama32_1b_fp16", "k_decode_dataflow"): (2.5143e9, _MEASURED_SOURCE),
-    ("c4_llama32_1b_longctx_fp16", "k_decode_dataflow"): (2.8001e9, _MEASURED_SOURCE),
-    ("c5_llama3_8b_fp16", "k_decode_dataflow"): (1.5186e10, _MEASURED_SOURCE),
+    ("c4_llama32_1b_longctx_fp16", "k_decode_dataflow"): (2.8003e9, _MEASURED_SOURCE),
+    ("c5_llama3_8b_fp16", "k_decode_dataflow"): (1.5188e10, _MEASURED_SOURCE),
 }
 
 
