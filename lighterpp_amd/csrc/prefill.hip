@@ -1276,7 +1276,7 @@ __global__ __launch_bounds__(256) void k_attention(const float* __restrict__ q, 
 //
 // What bounds it: a step of 32 positions is 512 MFMA clocks and about as many of the vector units (sixteen v_exp_f32 are
 // 256 of them), and one wavefront does them one after the other, so what counts is wavefronts per SIMD: the stages are
-// kept small enough for two or three workgroups to a compute unit.  (Measured and not better: the next step's scores
+// kept small enough for two to four workgroups to a compute unit.  (Measured and not better: the next step's scores
 // formed between this step's weights in the same wavefront, at twice the stages; more steps in flight; 128 rows to a
 // workgroup; a short batch's context split over several workgroups with a kernel that merges them.)  1B shape, exact
 // mode: 150 ids behind 3000, 34 -> 22 us a layer; 2048 ids behind 2048, 107 us on average.
@@ -1291,7 +1291,9 @@ struct AttentionShape {
     static constexpr int kRowBytes = 2 * kHs, kPieces = kHs / 8;
     static constexpr int kHalfBytes = kStep * kRowBytes, kStageBytes = 2 * kHalfBytes;  // K rows, then V rows
     static constexpr int kLoads = kStageBytes / 1024 / kR;                              // requests per wavefront and step
-    static constexpr int kStages = 2;  // 2 x 2: 52 / 72 KiB, at least two workgroups to a compute unit
+    // 2 x 2: 36 / 72 KiB, four or two workgroups to a compute unit (heads of 64 in three stages, 52 KiB: three of them, and
+    // of 2048 ids' 1024 workgroups a last round with one wavefront to a SIMD; behind 2048 positions 119.5 us, 111.1 so)
+    static constexpr int kStages = 2;
     static constexpr int kPartFloats = (kHs / 2 + 2) * 64;  // a wavefront's maximum, sum and output
     static constexpr int kMergeBytes = kP * kR * kPartFloats * 4;
     static_assert(kP > 1 && kHs / 8 % kP == 0, "the output's pieces are shared out among the wavefronts of a row");
@@ -2299,7 +2301,7 @@ lpp_status lpp_prefill(lpp_model* m, const int* tokens, int n_tokens, int start_
         if (!m->w_loaded[t]) return fail(LPP_ERR_STATE, "weight tensor %d has not been uploaded", t);
     LPP_TRY(lpp_prefill_supported(m));
     // Full chunks and a rest: 2048 tokens are the length that fills the device's rounds best.  (1B shape, exact: one chunk of
-    // 2048 takes 8.6 ms, of 640 3.7, of 1280 or 1408 6.0 or 6.5, so 2600 ids are better cut 2048 + 552 than into halves.)
+    // 2048 takes 7.2 ms, of 600 3.0, of 1270 5.2, so 2600 ids are better cut 2048 + 552 than into halves.)
     int each = n_tokens < pf::kChunk ? n_tokens : pf::kChunk;
     if (each > pf::kSmallChunk) {
         const int t_pad = padded_tokens(each);
