@@ -1755,9 +1755,8 @@ int padded_tokens(int n) {
 // costs two thirds of a full one or more, and no launch less than one; partial products are written and read at 2.8 TB/s.
 // The constants are a fit to 4100 timed prefills (TinyLlama, 1B and 8B shapes, 300 to 2036 ids, both modes, each tile and cut
 // for each of the four products in turn): a prefill is within 1 % of what that product's fastest launch makes it, and faster
-// than by rules that cut K only while all ranges fit the device at once: exact / fast mode, 8B shape 370 ids 11.9 / 8.51 -> 10.7 /
-// 8.15 ms, 600 18.6 / 14.0 -> 17.1 / 12.3, 750 20.4 / 15.2 -> 19.6 / 14.1; 1B 1140 5.21 / 3.86 -> 4.91 / 3.63; TinyLlama 1530 7.53 ->
-// 7.17, 1140 in the fast mode 4.18 -> 3.99.
+// than by rules that cut K only while all ranges fit the device at once: exact mode, 8B shape 370 ids 11.9 -> 10.7 ms,
+// 600 18.6 -> 17.1, 750 20.4 -> 19.6; 1B 1140 5.21 -> 4.91; TinyLlama 1530 7.53 -> 7.17.
 // W1+W3, tiles against blocks: 1B shape 1024 ids 127 / 81 and 118 / 67 us, 1280 ids (a quarter of a second round) 163 / 108
 // and 187 / 113, 2048 ids 236 / 156 and 217 / 127; 8B 512 ids 224 / 152 and 196 / 122, 1024 ids 426 / 280 and 369 / 224.
 //
@@ -1769,9 +1768,8 @@ int padded_tokens(int n) {
 // prefills (TinyLlama, 1B and 8B shapes, 10 to 256 ids, both modes, every tile of the list for each of the four products in
 // turn): up to 128 tokens a prefill is 0.3 % slower on average than with that product's fastest launch.  In the exact mode
 // beyond 128 tokens the constants are an earlier fit's, which makes the better choices there (256 ids of the TinyLlama shape
-// 2.03 ms, 2.06 by the newer one).
-// Exact mode, by the earlier fit and so: 8B shape 10 ids 3.54 -> 3.35 ms, 40 4.21 -> 3.95, 90 5.76 -> 4.66; 1B 100 ids 1.27 -> 1.21;
-// fast mode: 8B 48 ids 4.34 -> 3.58, 120 5.02 -> 4.39, 1B 200 1.44 -> 1.28, TinyLlama 220 1.84 -> 1.67.
+// 2.03 ms, 2.06 by the newer one); the fast mode keeps that fit, and its tiles, so that its sums keep their order.
+// Exact mode, by the earlier fit and so: 8B shape 10 ids 3.54 -> 3.35 ms, 40 4.21 -> 3.95, 90 5.76 -> 4.66; 1B 100 ids 1.27 -> 1.21.
 //
 // `max_splits`: ranges K may be cut into.  `row_step`: every matrix is a whole number of row_step rows.  `pair`: W1 and W3
 // side by side in a tile (total_n counts both).
@@ -1798,18 +1796,20 @@ Plan plan_gemm(int total_n, int K, int t_pad, int live, int max_splits, bool lo,
     Plan best = {false, 2, 2, 1};
     const bool wide_allowed = row_step % 256 == 0 && test_option(LPP_OPT_PREFILL_WIDE_TILES) != 0;
     if (t_pad > 256) {
-        if (!wide_allowed) {
-            const int token_tiles = t_pad / 128;
-            if (pair) best.fi = 4;
-            while (2 * best.splits <= max_splits && total_n / best.tile_rows() * token_tiles * best.splits * 2 <= compute_units() &&
-                   K % (64 * 2 * best.splits) == 0 && K / (2 * best.splits) >= 512)
-                best.splits *= 2;
-            return best;
-        }
+        const int token_tiles = t_pad / 128;
+        const bool wide = total_n / 256 * token_tiles >= compute_units() || (lo && total_n / 128 * token_tiles > compute_units());
+        if (pair || (wide_allowed && wide)) best.fi = 4;
+        while (2 * best.splits <= max_splits && total_n / best.tile_rows() * token_tiles * best.splits * 2 <= compute_units() &&
+               K % (64 * 2 * best.splits) == 0 && K / (2 * best.splits) >= 512)
+            best.splits *= 2;
+        if (!wide_allowed) return best;
+        // (the fast mode's results move by more than its bound when sums are cut elsewhere: there K stays cut as this rule cuts it)
+        const int fast_splits = best.splits;
         float best_us = 1e30f;
         for (const auto& t : {Plan{false, 2, 2, 1}, Plan{false, 4, 2, 1}, Plan{false, 4, 4, 1}})
             for (int splits = 1; splits <= max_splits; splits *= 2) {
                 if (splits > 1 && (K % (64 * splits) != 0 || K / splits < 512)) break;
+                if (!lo && splits != fast_splits) continue;
                 const Plan p = {t.few, t.fi, t.tj, splits};
                 const float us = planned_us(p, total_n, K, t_pad, lo, pair);
                 if (us < best_us) {
@@ -1826,17 +1826,19 @@ Plan plan_gemm(int total_n, int K, int t_pad, int live, int max_splits, bool lo,
         float weights, written, read;         // bytes a us: of weights, of partial products
     };
     static constexpr Rates kUpTo128 = {109e3f, 107e3f, 107e3f, 4.7e3f, 1.9f, 2.4f, 0.355f, 0.8f, 10.7e6f, 3.45e6f, 13.5e6f},
-                           kExact = {57e3f, 88e3f, 88e3f, 5.7e6f, 1.9f, 1.9f, 0.0f, 0.87f, 3.9e6f, 2.5e6f, 5e6f},
-                           kFast = {80e3f, 88e3f, 80e3f, 4.7e3f, 1.9f, 1.9f, 0.355f, 0.8f, 10.7e6f, 3.45e6f, 13.5e6f};
-    const Rates& c = t_pad <= 128 ? kUpTo128 : (lo ? kExact : kFast);
+                           kExact = {57e3f, 88e3f, 88e3f, 5.7e6f, 1.9f, 1.9f, 0.0f, 0.87f, 3.9e6f, 2.5e6f, 5e6f};
+    // (the fast mode keeps the earlier fit and its tiles throughout: its results move by more than its bound when sums are cut elsewhere)
+    const bool earlier = !lo || t_pad > 128;
+    const Rates& c = earlier ? kExact : kUpTo128;
     // A prompt and the same prompt filled up to 32, or beyond 128 tokens to 128, are summed alike: tokens count as whole columns
-    // of those, but for a pair beyond 128, where k_gemm_pipe is the faster one throughout and sums the same in either tile.
-    const int counted = t_pad > 128 && !pair ? t_pad : (min(live, t_pad) + 31) / 32 * 32, columns = counted / 32;
+    // of those.
+    const int counted = t_pad > 128 ? t_pad : (min(live, t_pad) + 31) / 32 * 32, columns = counted / 32;
     float best_us = 1e30f;
     for (const auto& t : kTiles) {
         const Plan p = {t.few, t.fi, t.tj, 1};
         const int rows = p.tile_rows(), tokens = p.tile_tokens(), token_tiles = p.token_tiles(t_pad, counted);
-        if (row_step % rows != 0 || token_tiles * tokens > t_pad || (pair && t.few && (t.fi == 1 || t_pad > 128))) continue;
+        if (row_step % rows != 0 || token_tiles * tokens > t_pad || (pair && t.fi == 1)) continue;
+        if (earlier && (counted % tokens != 0 || t.few && (lo ? t.tj == 4 || (t.fi == 1 && t.tj > 1) : t.fi == 4))) continue;
         if (!t.few && t.fi == 4 && !wide_allowed) continue;
         const int sent = min(tokens, 32 * ((columns + token_tiles - 1) / token_tiles));
         for (int splits = 1; splits <= max_splits; splits *= 2) {
@@ -1846,7 +1848,8 @@ Plan plan_gemm(int total_n, int K, int t_pad, int live, int max_splits, bool lo,
             const float bytes = k * 2.0f * (rows + copies * sent), clocks = k * copies * rows * sent / 1024.0f;
             const float turns = fmaxf(1.0f, c.round * rounds + (1.0f - c.round) * wgs / compute_units());
             const float busy = turns * (t.few ? bytes / c.few : fmaxf(bytes / (t.fi == 4 ? c.wide : c.pipe), clocks / c.clocks)), weights = 2.0f * total_n * K / c.weights;
-            float us = (t.few ? c.launch_few + c.sums * t.fi * t.tj * rounds : c.launch_pipe) + fmaxf(busy, weights) + 0.01f * fminf(busy, weights);
+            float us = (t.few ? c.launch_few + c.sums * t.fi * t.tj * rounds : c.launch_pipe + (earlier && t_pad <= 128 ? 1.0f : 0.0f)) +
+                       fmaxf(busy, weights) + (earlier ? 0.0f : 0.01f * fminf(busy, weights));
             if (splits > 1) us += 4.0f * counted * total_n * (splits / c.written + (splits - 1) / c.read);
             if (us < best_us) {
                 best_us = us;
