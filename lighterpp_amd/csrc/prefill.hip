@@ -1861,14 +1861,19 @@ Plan plan_gemm(int total_n, int K, int t_pad, int live, int max_splits, bool lo,
     return best;
 }
 
+// Floats that the partial products of one GEMM of a batch of t_pad tokens may take: at most eight ranges of 256 tokens, or one
+// tile of 128 x 128 per compute unit, beyond 512 tokens one block of 256 x 256 (plan_gemm).  It goes by the batch alone: by the
+// buffers that earlier calls have left, a batch would be cut, and so summed, differently behind a longer one.
+size_t range_limit(const lpp_model* m, int t_pad) {
+    const size_t few = t_pad < 256 ? t_pad : 256, cut = 8 * few * (m->cfg.dim + 2 * m->kv_dim);
+    const size_t tiles = static_cast<size_t>(compute_units()) * (t_pad > pf::kSmallChunk ? 256 * 256 : 128 * 128);
+    return t_pad > 256 && tiles > cut ? tiles : cut;
+}
+
 // Floats of kBufPartials that chunks of up to t_pad tokens need: the partial products of the GEMM before (read by the
-// kernel that follows it, so one area does for all of a layer's) -- at most eight of 256 tokens, or one tile of 128 x 128 per
-// compute unit, beyond 512 tokens one block of 256 x 256 (plan_gemm) -- or the gate and up projections where those are not fused.
+// kernel that follows it, so one area does for all of a layer's), or the gate and up projections where those are not fused.
 size_t partial_floats(const lpp_model* m, int t_pad) {
-    const size_t t = static_cast<size_t>(t_pad), few = t < 256 ? t : 256;
-    size_t most = 8 * few * (m->cfg.dim + 2 * m->kv_dim);
-    const size_t tiles = static_cast<size_t>(compute_units()) * (t > static_cast<size_t>(pf::kSmallChunk) ? 256 * 256 : 128 * 128), pair = 2 * t * m->cfg.hidden_dim;
-    if (t > 256 && tiles > most) most = tiles;
+    const size_t most = range_limit(m, t_pad), pair = 2 * static_cast<size_t>(t_pad) * m->cfg.hidden_dim;
     const bool fused = test_option(LPP_OPT_PREFILL_STAGED_GEMM) != 0 && test_option(LPP_OPT_PREFILL_FUSED_FFN) != 0;
     return !fused && pair > most ? pair : most;
 }
@@ -1987,14 +1992,14 @@ lpp_status launch_plan(const Plan& p, const pf::PipeJob& job_in, hipStream_t s) 
     return fail(LPP_ERR_STATE, "prefill GEMM: no kernel for a tile of %d x %d", p.tile_rows(), p.tile_tokens());
 }
 
-// `partials` (optional, partial_floats long): room for the partial products of a split K.  A product
+// `partials` (optional): room for the partial products of a split K, `limit` floats of them at most.  A product
 // with too few output tiles for the compute units is cut along K into ranges, each multiplied by
 // its own workgroups into `partials`: range z of matrix i lies at partials + z * t_pad * (n_0 + n_1 +
 // ..) + t_pad * (n_0 + .. + n_(i-1)), rows of n_i floats.  With `left_split` the caller adds the
 // ranges itself (in order, in the kernel that reads the product next) and gets their number there;
 // without it they are added to y here, in order.
 lpp_status gemm(const Product* prods, int count, const pf::half_t* xh, const pf::half_t* xl, int K, int t_pad, bool accumulate,
-                hipStream_t s, float* partials = nullptr, size_t partial_floats = 0, int* left_split = nullptr,
+                hipStream_t s, float* partials = nullptr, size_t limit = 0, int* left_split = nullptr,
                 bool remainder = true, int live = 0x7fffffff) {
     LPP_REQUIRE(count >= 1 && count <= 3 && t_pad > 0 && t_pad % 32 == 0 && K % 32 == 0, "prefill GEMM: %d products, K %d, T %d",
                 count, K, t_pad);
@@ -2011,7 +2016,7 @@ lpp_status gemm(const Product* prods, int count, const pf::half_t* xh, const pf:
     if (staged) {
         const size_t stride = static_cast<size_t>(t_pad) * total_n;
         int most = 1;
-        while (partials != nullptr && (count == 1 || left_split != nullptr) && most < 8 && stride * 2 * most <= partial_floats) most *= 2;
+        while (partials != nullptr && (count == 1 || left_split != nullptr) && most < 8 && stride * 2 * most <= limit) most *= 2;
         live = live < t_pad ? live : t_pad;
         const Plan plan = plan_gemm(total_n, K, t_pad, live, most, remainder, step, false);
         const int tile = plan.tile_rows(), feature_tiles = total_n / tile, token_tiles = plan.token_tiles(t_pad, live), splits = plan.splits;
@@ -2203,7 +2208,8 @@ lpp_status prefill_chunk(lpp_model* m, const int* tokens, int n, int pos0) {
     };
     pf::half_t* hi2 = static_cast<pf::half_t*>(m->pf_buf[kBufHi2]);
     pf::half_t* lo2 = static_cast<pf::half_t*>(m->pf_buf[kBufLo2]);
-    const size_t room = m->pf_room;
+    const size_t limit = range_limit(m, t_pad);
+    LPP_REQUIRE(limit <= m->pf_room, "prefill: %zu floats of partial products, room for %zu", limit, m->pf_room);
     // LPP_PREFILL_EXACT: every product takes the activations as binary16 head + remainder.  LPP_PREFILL_FAST: the head
     // alone, in the staged kernels (what a GEMM sees of its input is then what the reference's own GPU GEMV sees,
     // matmul.cu:85-98; accumulation stays fp32).
@@ -2225,7 +2231,7 @@ lpp_status prefill_chunk(lpp_model* m, const int* tokens, int n, int pos0) {
                                 {layer_of(LPP_T_WV, l, kv, dim), v, kv}};
         const int q_dim = last_layer ? 0 : dim;
         int qkv_split = 1;
-        LPP_TRY(gemm(qkv + (last_layer ? 1 : 0), last_layer ? 2 : 3, hi, lo, dim, t_pad, false, s, partials, room, &qkv_split, exact, n));
+        LPP_TRY(gemm(qkv + (last_layer ? 1 : 0), last_layer ? 2 : 3, hi, lo, dim, t_pad, false, s, partials, limit, &qkv_split, exact, n));
         const size_t qkv_stride = static_cast<size_t>(t_pad) * (q_dim + 2 * kv);
         const float* qs = qkv_split > 1 ? partials : q;
         const float* ks = qkv_split > 1 ? partials + static_cast<size_t>(t_pad) * q_dim : k;
@@ -2245,7 +2251,7 @@ lpp_status prefill_chunk(lpp_model* m, const int* tokens, int n, int pos0) {
                                m->value_cache, hi, lo, l, pos0, dim, kv, hs, m->gqa, c.seq_len, n);
         LPP_CHECK_LAUNCH("k_attention");
         const Product wo = {layer_of(LPP_T_WO, l, dim, dim), x, dim};
-        LPP_TRY(gemm(&wo, 1, hi, lo, dim, t_pad, true, s, partials, room, &pending, exact, n));
+        LPP_TRY(gemm(&wo, 1, hi, lo, dim, t_pad, true, s, partials, limit, &pending, exact, n));
         // feed-forward block, model.cpp:221-226
         LPP_TRY(norm_split(x, static_cast<const float*>(m->w[LPP_T_RMS_FFN]) + static_cast<size_t>(l) * dim, hi, lo, dim, n, t_pad, partials,
                            pending > 1 ? pending : 0, static_cast<size_t>(t_pad) * dim, s, !lean));
@@ -2260,7 +2266,7 @@ lpp_status prefill_chunk(lpp_model* m, const int* tokens, int n, int pos0) {
             LPP_CHECK_LAUNCH("k_swiglu_split");
         }
         const Product w2 = {layer_of(LPP_T_W2, l, dim, hidden), x, dim};
-        LPP_TRY(gemm(&w2, 1, hi2, lo2, hidden, t_pad, true, s, partials, room, &pending, exact, n));
+        LPP_TRY(gemm(&w2, 1, hi2, lo2, hidden, t_pad, true, s, partials, limit, &pending, exact, n));
     }
     LPP_HIP(hipStreamSynchronize(s));
     return LPP_OK;

@@ -828,6 +828,25 @@ def test_prefill_where_memory_has_no_room_for_the_longest_batch(lib, room, test_
         m.close()
 
 
+@pytest.mark.parametrize("fast", [False, True])
+def test_a_batch_repeats_bit_for_bit_behind_a_longer_one(fast):
+    """300 ids, 600, then the same 300, of a shape whose W2 is cheaper in more ranges of K than a batch of 300 may have: the
+    buffers that the longer batch leaves behind must not change how the shorter one is summed.  Bit for bit, twice."""
+    shape = Shape(3072, 12288, 2, 24, 4, 512, 640, 500000.0, fp16=True, tied=True)
+    m = Model(shape)
+    m.load_synthetic(24)
+    m.set_prefill_mode(capi.PREFILL_FAST if fast else capi.PREFILL_EXACT)
+    ids, longer = capi.synth_token_ids(300, 25, shape.vocab_size), capi.synth_token_ids(600, 26, shape.vocab_size)
+    m.prefill(ids, 0)
+    k0, v0, _, _ = caches(m, shape, 300)
+    for _ in range(2):
+        m.prefill(longer, 0)
+        m.prefill(ids, 0)
+        k, v, _, _ = caches(m, shape, 300)
+        assert np.array_equal(k, k0) and np.array_equal(v, v0)
+    m.close()
+
+
 def test_prompts_that_grow_keep_the_buffers(lib):
     """Prompts of 20, 50, 90, 128 ids, then of 600, 700, 1000: device memory in use moves with the first of either only."""
     import ctypes as C
