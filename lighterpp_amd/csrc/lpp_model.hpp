@@ -87,6 +87,7 @@ struct lpp_model {
     void* pf_buf[12] = {};                   // batched prefill: activations of a chunk of tokens (prefill.hip)
     int pf_cap = 0;                          // tokens those buffers hold
     size_t pf_room = 0;                      // floats of the area for partial products
+    int pf_room_key = 0;                     // mode and test options they were counted for
     int pf_mode = 0;                         // LPP_PREFILL_EXACT / LPP_PREFILL_FAST
 
     hipGraphExec_t graph_exec[2] = {nullptr, nullptr};  // [0] without, [1] with uniforms/out arrays

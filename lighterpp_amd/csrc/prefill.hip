@@ -1870,11 +1870,38 @@ size_t range_limit(const lpp_model* m, int t_pad) {
     return t_pad > 256 && tiles > cut ? tiles : cut;
 }
 
+// The plan of a product of total_n rows; its partial products take `limit` floats at most.
+Plan plan_product(int total_n, int K, int t_pad, int live, size_t limit, bool lo, int row_step) {
+    const size_t stride = static_cast<size_t>(t_pad) * total_n;
+    int most = 1;
+    while (most < 8 && stride * 2 * most <= limit) most *= 2;
+    return plan_gemm(total_n, K, t_pad, live, most, lo, row_step, false);
+}
+// The largest tile height that a matrix of n rows is a whole number of.
+int tile_step(int n) { return n % 256 == 0 ? 256 : 128; }
+
 // Floats of kBufPartials that chunks of up to t_pad tokens need: the partial products of the GEMM before (read by the
 // kernel that follows it, so one area does for all of a layer's), or the gate and up projections where those are not fused.
+// Up to 512 tokens that is range_limit.  Beyond, only the exact mode's plans go past it, at some shapes and lengths, so those
+// lengths are asked (the fast mode keeps its cuts within a workgroup a compute unit).
 size_t partial_floats(const lpp_model* m, int t_pad) {
-    const size_t most = range_limit(m, t_pad), pair = 2 * static_cast<size_t>(t_pad) * m->cfg.hidden_dim;
-    const bool fused = test_option(LPP_OPT_PREFILL_STAGED_GEMM) != 0 && test_option(LPP_OPT_PREFILL_FUSED_FFN) != 0;
+    const int dim = m->cfg.dim, kv = m->kv_dim;
+    const size_t pair = 2 * static_cast<size_t>(t_pad) * m->cfg.hidden_dim;
+    const bool staged = test_option(LPP_OPT_PREFILL_STAGED_GEMM) != 0;
+    size_t most = range_limit(m, t_pad < pf::kSmallChunk ? t_pad : pf::kSmallChunk);
+    if (staged && m->pf_mode != LPP_PREFILL_FAST)
+        for (int t = pf::kSmallChunk + pf::kTileTokens; t <= t_pad; t += pf::kTileTokens) {
+            const size_t limit = range_limit(m, t);
+            const int narrow = tile_step(dim) < tile_step(kv) ? tile_step(dim) : tile_step(kv);
+            const struct { int n, k, step; } products[] = {{dim + 2 * kv, dim, narrow}, {2 * kv, dim, tile_step(kv)}, {dim, dim, tile_step(dim)},
+                                                           {dim, m->cfg.hidden_dim, tile_step(dim)}};
+            for (const auto& p : products) {
+                const int splits = plan_product(p.n, p.k, t, t, limit, true, p.step).splits;
+                const size_t floats = splits > 1 ? static_cast<size_t>(splits) * t * p.n : 0;
+                if (floats > most) most = floats;
+            }
+        }
+    const bool fused = staged && test_option(LPP_OPT_PREFILL_FUSED_FFN) != 0;
     return !fused && pair > most ? pair : most;
 }
 
@@ -1883,11 +1910,11 @@ struct ScratchLayout {
     size_t total;
     size_t room;  // floats of kBufPartials
 };
-ScratchLayout scratch_layout(const lpp_model* m, int t_pad) {
+ScratchLayout scratch_layout(const lpp_model* m, int t_pad, size_t room) {
     const lpp_config& c = m->cfg;
     const size_t t = static_cast<size_t>(t_pad);
     ScratchLayout s = {};
-    s.room = partial_floats(m, t_pad);
+    s.room = room;
     const size_t bytes[kBufAll] = {t * sizeof(int),
                                    t * c.dim * sizeof(float),
                                    t * c.dim * sizeof(float),
@@ -1913,7 +1940,15 @@ int scratch_tokens(int t_pad) {
     return (t_pad + step - 1) / step * step;
 }
 
-bool scratch_held(const lpp_model* m, int t_pad) { return m->pf_cap >= t_pad && m->pf_room >= partial_floats(m, t_pad); }
+// What partial_floats goes by besides the tokens: buffers made under the same have room for every batch up to theirs.
+int room_key(const lpp_model* m) {
+    return 1 + (m->pf_mode != LPP_PREFILL_FAST) + 2 * (test_option(LPP_OPT_PREFILL_STAGED_GEMM) != 0) +
+           4 * (test_option(LPP_OPT_PREFILL_FUSED_FFN) != 0) + 8 * (test_option(LPP_OPT_PREFILL_WIDE_TILES) != 0);
+}
+
+bool scratch_held(const lpp_model* m, int t_pad) {
+    return m->pf_cap >= t_pad && (m->pf_room_key == room_key(m) || m->pf_room >= partial_floats(m, t_pad));
+}
 
 // Whether device memory has room for the buffers of t_pad tokens in the place of those the model holds: asked before those
 // are given up, so that a model that lives with the smaller batch keeps its buffers from call to call.
@@ -1926,19 +1961,27 @@ bool scratch_fits(const lpp_model* m, int t_pad) {
         (void)hipGetLastError();
         return true;  // (the allocation will say)
     }
-    const size_t held = m->pf_cap > 0 ? scratch_layout(m, m->pf_cap).total : 0;
-    return scratch_layout(m, scratch_tokens(t_pad)).total <= free_bytes + held;
+    const size_t held = m->pf_cap > 0 ? scratch_layout(m, m->pf_cap, m->pf_room).total : 0;
+    const int tokens = scratch_tokens(t_pad);
+    return scratch_layout(m, tokens, partial_floats(m, tokens)).total <= free_bytes + held;
 }
 
-// `quiet`: an allocation that fails leaves lpp_last_error as it is (the caller has another way to go).
+// `quiet`: an allocation that fails leaves lpp_last_error as it is (the caller has another way to go).  Buffers that are too
+// small are made for as many tokens as they were, or more, so that a model that changes its mode from call to call settles.
 lpp_status ensure_scratch(lpp_model* m, int t_pad, bool quiet = false) {
     if (scratch_held(m, t_pad)) return LPP_OK;
+    const int needed = scratch_tokens(t_pad), before = m->pf_cap;
     prefill_release(m);
-    const int tokens = scratch_tokens(t_pad);
-    const ScratchLayout s = scratch_layout(m, tokens);
     const int forced = test_option(LPP_OPT_PREFILL_ROOM);
+    ScratchLayout s = {};
     hipError_t e = hipErrorOutOfMemory;
-    if (forced >= 0 || t_pad <= -forced) e = hipMalloc(&m->pf_buf[kBufAll], s.total);
+    int tokens = before > needed ? before : needed;
+    for (;; tokens = needed) {
+        s = scratch_layout(m, tokens, partial_floats(m, tokens));
+        if (forced >= 0 || t_pad <= -forced) e = hipMalloc(&m->pf_buf[kBufAll], s.total);
+        if (e == hipSuccess || tokens == needed) break;
+        (void)hipGetLastError();
+    }
     if (e != hipSuccess) {
         (void)hipGetLastError();
         m->pf_buf[kBufAll] = nullptr;
@@ -1947,6 +1990,7 @@ lpp_status ensure_scratch(lpp_model* m, int t_pad, bool quiet = false) {
     for (int i = 0; i < kBufAll; ++i) m->pf_buf[i] = static_cast<char*>(m->pf_buf[kBufAll]) + s.offset[i];
     m->pf_cap = tokens;
     m->pf_room = s.room;
+    m->pf_room_key = room_key(m);
     return LPP_OK;
 }
 
@@ -1992,15 +2036,20 @@ lpp_status launch_plan(const Plan& p, const pf::PipeJob& job_in, hipStream_t s) 
     return fail(LPP_ERR_STATE, "prefill GEMM: no kernel for a tile of %d x %d", p.tile_rows(), p.tile_tokens());
 }
 
-// `partials` (optional): room for the partial products of a split K, `limit` floats of them at most.  A product
+// Where the partial products of a split K go: `room` floats, of which a product may use `limit`.
+struct Partials {
+    float* at = nullptr;
+    size_t limit = 0, room = 0;
+};
+
+// `area` (optional): room for partial products.  A product
 // with too few output tiles for the compute units is cut along K into ranges, each multiplied by
-// its own workgroups into `partials`: range z of matrix i lies at partials + z * t_pad * (n_0 + n_1 +
+// its own workgroups into the area: range z of matrix i lies at area.at + z * t_pad * (n_0 + n_1 +
 // ..) + t_pad * (n_0 + .. + n_(i-1)), rows of n_i floats.  With `left_split` the caller adds the
 // ranges itself (in order, in the kernel that reads the product next) and gets their number there;
 // without it they are added to y here, in order.
 lpp_status gemm(const Product* prods, int count, const pf::half_t* xh, const pf::half_t* xl, int K, int t_pad, bool accumulate,
-                hipStream_t s, float* partials = nullptr, size_t limit = 0, int* left_split = nullptr,
-                bool remainder = true, int live = 0x7fffffff) {
+                hipStream_t s, const Partials& area = {}, int* left_split = nullptr, bool remainder = true, int live = 0x7fffffff) {
     LPP_REQUIRE(count >= 1 && count <= 3 && t_pad > 0 && t_pad % 32 == 0 && K % 32 == 0, "prefill GEMM: %d products, K %d, T %d",
                 count, K, t_pad);
     if (left_split != nullptr) *left_split = 1;
@@ -2009,16 +2058,18 @@ lpp_status gemm(const Product* prods, int count, const pf::half_t* xh, const pf:
     for (int i = 0; i < count; ++i) {
         LPP_REQUIRE(prods[i].n > 0 && prods[i].n % pf::kTileFeatures == 0, "prefill GEMM: n %d", prods[i].n);
         total_n += prods[i].n;
-        if (prods[i].n % 256 != 0) step = 128;
+        if (tile_step(prods[i].n) < step) step = tile_step(prods[i].n);
     }
     const bool staged = K % pf::kPipeTripK == 0 && test_option(LPP_OPT_PREFILL_STAGED_GEMM) != 0;
     LPP_REQUIRE(staged || t_pad % pf::kTileTokens == 0, "prefill GEMM: T %d, K %d", t_pad, K);
     if (staged) {
         const size_t stride = static_cast<size_t>(t_pad) * total_n;
-        int most = 1;
-        while (partials != nullptr && (count == 1 || left_split != nullptr) && most < 8 && stride * 2 * most <= limit) most *= 2;
         live = live < t_pad ? live : t_pad;
-        const Plan plan = plan_gemm(total_n, K, t_pad, live, most, remainder, step, false);
+        float* partials = area.at;
+        const bool may_cut = partials != nullptr && (count == 1 || left_split != nullptr);
+        const Plan plan = plan_product(total_n, K, t_pad, live, may_cut ? area.limit : 0, remainder, step);
+        if (plan.splits > 1 && stride * plan.splits > area.room)
+            return fail(LPP_ERR_STATE, "prefill GEMM: %zu floats of partial products, room for %zu", stride * plan.splits, area.room);
         const int tile = plan.tile_rows(), feature_tiles = total_n / tile, token_tiles = plan.token_tiles(t_pad, live), splits = plan.splits;
         pf::PipeJob job = {};
         int at = 0;
@@ -2196,6 +2247,7 @@ lpp_status prefill_chunk(lpp_model* m, const int* tokens, int n, int pos0) {
     float* k = static_cast<float*>(m->pf_buf[kBufK]);
     float* v = static_cast<float*>(m->pf_buf[kBufV]);
     float* partials = static_cast<float*>(m->pf_buf[kBufPartials]);
+    const Partials area = {partials, range_limit(m, t_pad), m->pf_room};
     pf::half_t* hi = static_cast<pf::half_t*>(m->pf_buf[kBufHi]);
     pf::half_t* lo = static_cast<pf::half_t*>(m->pf_buf[kBufLo]);
     LPP_HIP(hipMemcpyAsync(d_tokens, tokens, static_cast<size_t>(n) * sizeof(int), hipMemcpyHostToDevice, s));
@@ -2208,8 +2260,6 @@ lpp_status prefill_chunk(lpp_model* m, const int* tokens, int n, int pos0) {
     };
     pf::half_t* hi2 = static_cast<pf::half_t*>(m->pf_buf[kBufHi2]);
     pf::half_t* lo2 = static_cast<pf::half_t*>(m->pf_buf[kBufLo2]);
-    const size_t limit = range_limit(m, t_pad);
-    LPP_REQUIRE(limit <= m->pf_room, "prefill: %zu floats of partial products, room for %zu", limit, m->pf_room);
     // LPP_PREFILL_EXACT: every product takes the activations as binary16 head + remainder.  LPP_PREFILL_FAST: the head
     // alone, in the staged kernels (what a GEMM sees of its input is then what the reference's own GPU GEMV sees,
     // matmul.cu:85-98; accumulation stays fp32).
@@ -2231,7 +2281,7 @@ lpp_status prefill_chunk(lpp_model* m, const int* tokens, int n, int pos0) {
                                 {layer_of(LPP_T_WV, l, kv, dim), v, kv}};
         const int q_dim = last_layer ? 0 : dim;
         int qkv_split = 1;
-        LPP_TRY(gemm(qkv + (last_layer ? 1 : 0), last_layer ? 2 : 3, hi, lo, dim, t_pad, false, s, partials, limit, &qkv_split, exact, n));
+        LPP_TRY(gemm(qkv + (last_layer ? 1 : 0), last_layer ? 2 : 3, hi, lo, dim, t_pad, false, s, area, &qkv_split, exact, n));
         const size_t qkv_stride = static_cast<size_t>(t_pad) * (q_dim + 2 * kv);
         const float* qs = qkv_split > 1 ? partials : q;
         const float* ks = qkv_split > 1 ? partials + static_cast<size_t>(t_pad) * q_dim : k;
@@ -2251,7 +2301,7 @@ lpp_status prefill_chunk(lpp_model* m, const int* tokens, int n, int pos0) {
                                m->value_cache, hi, lo, l, pos0, dim, kv, hs, m->gqa, c.seq_len, n);
         LPP_CHECK_LAUNCH("k_attention");
         const Product wo = {layer_of(LPP_T_WO, l, dim, dim), x, dim};
-        LPP_TRY(gemm(&wo, 1, hi, lo, dim, t_pad, true, s, partials, limit, &pending, exact, n));
+        LPP_TRY(gemm(&wo, 1, hi, lo, dim, t_pad, true, s, area, &pending, exact, n));
         // feed-forward block, model.cpp:221-226
         LPP_TRY(norm_split(x, static_cast<const float*>(m->w[LPP_T_RMS_FFN]) + static_cast<size_t>(l) * dim, hi, lo, dim, n, t_pad, partials,
                            pending > 1 ? pending : 0, static_cast<size_t>(t_pad) * dim, s, !lean));
@@ -2261,12 +2311,12 @@ lpp_status prefill_chunk(lpp_model* m, const int* tokens, int n, int pos0) {
         } else {
             float *gate = partials, *up = partials + static_cast<size_t>(t_pad) * hidden;
             const Product gate_up[2] = {{layer_of(LPP_T_W1, l, hidden, dim), gate, hidden}, {layer_of(LPP_T_W3, l, hidden, dim), up, hidden}};
-            LPP_TRY(gemm(gate_up, 2, hi, lo, dim, t_pad, false, s, nullptr, 0, nullptr, exact, n));
+            LPP_TRY(gemm(gate_up, 2, hi, lo, dim, t_pad, false, s, {}, nullptr, exact, n));
             hipLaunchKernelGGL(pf::k_swiglu_split, dim3((hidden + 255) / 256, t_pad), dim3(256), 0, s, gate, up, hi2, lo2, hidden, n);
             LPP_CHECK_LAUNCH("k_swiglu_split");
         }
         const Product w2 = {layer_of(LPP_T_W2, l, dim, hidden), x, dim};
-        LPP_TRY(gemm(&w2, 1, hi2, lo2, hidden, t_pad, true, s, partials, limit, &pending, exact, n));
+        LPP_TRY(gemm(&w2, 1, hi2, lo2, hidden, t_pad, true, s, area, &pending, exact, n));
     }
     LPP_HIP(hipStreamSynchronize(s));
     return LPP_OK;
@@ -2279,6 +2329,7 @@ void prefill_release(lpp_model* m) {
     for (void*& p : m->pf_buf) p = nullptr;
     m->pf_cap = 0;
     m->pf_room = 0;
+    m->pf_room_key = 0;
 }
 
 }  // namespace lpp

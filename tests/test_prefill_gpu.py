@@ -847,22 +847,67 @@ def test_a_batch_repeats_bit_for_bit_behind_a_longer_one(fast):
     m.close()
 
 
-def test_prompts_that_grow_keep_the_buffers(lib):
-    """Prompts of 20, 50, 90, 128 ids, then of 600, 700, 1000: device memory in use moves with the first of either only."""
+def hip_free_bytes():
     import ctypes as C
     hip = C.CDLL("libamdhip64.so")  # (the runtime the library is linked against)
+    free, total = C.c_size_t(0), C.c_size_t(0)
+    assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
 
-    def free_bytes():
-        free, total = C.c_size_t(0), C.c_size_t(0)
-        assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
-        return free.value
 
+@pytest.mark.parametrize("fast", [True, False])
+def test_long_batches_reserve_the_partial_products_they_form(fast):
+    """1000 ids of the TinyLlama width, whose plans beyond 512 tokens stay within a tile of 128 x 128 a compute unit in either mode,
+    then 2000 and, the other mode's turn, 1000 again: device memory grows by the activations and the partial products of 256
+    tokens in eight ranges, and by what an allocation is rounded up to (4 MiB allowed)."""
+    shape = Shape(2048, 5632, 2, 32, 4, 1024, 2048, 10000.0, fp16=True, tied=True)
+    ids = capi.synth_token_ids(2000, 28, shape.vocab_size)
+    with_kernels_loaded = Model(shape)
+    with_kernels_loaded.load_synthetic(27)
+    with_kernels_loaded.prefill(ids[:1000], 0)
+    m = Model(shape)
+    m.load_synthetic(27)
+    with_kernels_loaded.close()
+    before = hip_free_bytes()
+    for n, mode in ((1000, fast), (2000, fast), (1000, not fast)):
+        m.set_prefill_mode(capi.PREFILL_FAST if mode else capi.PREFILL_EXACT)
+        m.prefill(ids[:n], 0)
+        tokens = (n if mode == fast else 2000) // 512 * 512 + 512
+        activations = tokens * (4 + 8 * shape.dim + 8 * shape.kv_dim + 4 * shape.dim + 4 * shape.hidden_dim)
+        partials = 4 * max(8 * 256 * (shape.dim + 2 * shape.kv_dim), 256 * 128 * 128)
+        assert before - hip_free_bytes() <= activations + partials + (4 << 20)
+    m.close()
+
+
+@pytest.mark.parametrize("n", [1280, 2048])
+def test_lengths_that_are_cut_into_more_partial_products_after_others(n):
+    """1B width, exact mode: 1152 to 1408 ids cut W2 into four ranges, which take more room than any other length's.  Behind a
+    batch of the fast mode, whose buffers have no such room, and as the rest of a longer prompt: the caches of a fresh model."""
+    shape = Shape(2048, 8192, 2, 32, 8, 512, 3400, 500000.0, fp16=True, tied=True)
+    a, b = Model(shape), Model(shape)
+    for m in (a, b):
+        m.load_synthetic(29)
+    ids = capi.synth_token_ids(3328, 30, shape.vocab_size)
+    a.set_prefill_mode(capi.PREFILL_FAST)
+    a.prefill(ids[:n], 0)
+    a.set_prefill_mode(capi.PREFILL_EXACT)
+    a.prefill(ids, 0)
+    b.prefill(ids[:2048], 0)
+    b.prefill(ids[2048:], 2048)
+    for x, y in zip(caches(a, shape, 3328)[:2], caches(b, shape, 3328)[:2]):
+        assert np.array_equal(x, y)
+    for m in (a, b):
+        m.close()
+
+
+def test_prompts_that_grow_keep_the_buffers(lib):
+    """Prompts of 20, 50, 90, 128 ids, then of 600, 700, 1000: device memory in use moves with the first of either only."""
     m = Model(Shape(2048, 5632, 2, 32, 4, 1024, 1024, 10000.0, fp16=True, tied=True))
     m.load_synthetic(22)
     for lengths in ((20, 50, 90, 128), (600, 700, 1000)):
         seen = []
         for n in lengths:
             m.prefill(capi.synth_token_ids(n, 23, 1024), 0)
-            seen.append(free_bytes())
+            seen.append(hip_free_bytes())
         assert len(set(seen)) == 1, seen
     m.close()
