@@ -1761,7 +1761,7 @@ int padded_tokens(int n) {
 // and 187 / 113, 2048 ids 236 / 156 and 217 / 127; 8B 512 ids 224 / 152 and 196 / 122, 1024 ids 426 / 280 and 369 / 224.
 //
 // Up to 256 tokens the choice is made by what a launch of each would take.  A workgroup is paced by its bytes from L2 into
-// LDS, one of k_gemm_pipe by its MFMA clocks where they take longer; a
+// LDS, one of k_gemm_pipe, in the exact mode up to 128 tokens, by its MFMA clocks where they take longer; a
 // last round of workgroups that does not fill the device counts almost whole; k_gemm_few's sums meet in LDS, a tile of 32 x 32
 // at a time; every partial product of a cut K is written, in many short runs, and read once more.  No launch is faster than
 // its weights, and of two that are bound by them the one with less to do is taken.  The constants are a fit to 10000 timed
@@ -1820,16 +1820,17 @@ Plan plan_gemm(int total_n, int K, int t_pad, int live, int max_splits, bool lo,
         return best;
     }
     struct Rates {
-        float few, pipe, wide, clocks;        // bytes and MFMA clocks a us (wide: of tiles of 256 rows)
+        float few, pipe, clocks;              // bytes and MFMA clocks a us
         float launch_few, launch_pipe, sums;  // us; of k_gemm_few's sums, a tile of 32 x 32
         float round;                          // what a round of workgroups costs whatever there is of it
         float weights, written, read;         // bytes a us: of weights, of partial products
     };
-    static constexpr Rates kUpTo128 = {109e3f, 107e3f, 107e3f, 4.7e3f, 1.9f, 2.4f, 0.355f, 0.8f, 10.7e6f, 3.45e6f, 13.5e6f},
-                           kExact = {57e3f, 88e3f, 88e3f, 5.7e6f, 1.9f, 1.9f, 0.0f, 0.87f, 3.9e6f, 2.5e6f, 5e6f};
-    // (the fast mode keeps the earlier fit and its tiles throughout: its results move by more than its bound when sums are cut elsewhere)
+    // (kEarlier: by its clocks a tile's products take next to nothing, a thousandth of what they do, and no more than settle which
+    // of two tiles of equal bytes it is.  The order of sums hangs on its choices, so they stay as they are.)
+    static constexpr Rates kUpTo128 = {109e3f, 107e3f, 4.7e3f, 1.9f, 2.4f, 0.355f, 0.8f, 10.7e6f, 3.45e6f, 13.5e6f},
+                           kEarlier = {57e3f, 88e3f, 5.7e6f, 1.9f, 1.9f, 0.0f, 0.87f, 3.9e6f, 2.5e6f, 5e6f};
     const bool earlier = !lo || t_pad > 128;
-    const Rates& c = earlier ? kExact : kUpTo128;
+    const Rates& c = earlier ? kEarlier : kUpTo128;
     // A prompt and the same prompt filled up to 32, or beyond 128 tokens to 128, are summed alike: tokens count as whole columns
     // of those.
     const int counted = t_pad > 128 ? t_pad : (min(live, t_pad) + 31) / 32 * 32, columns = counted / 32;
@@ -1847,7 +1848,8 @@ Plan plan_gemm(int total_n, int K, int t_pad, int live, int max_splits, bool lo,
             const float k = static_cast<float>(K) / splits, copies = lo ? 2.0f : 1.0f;
             const float bytes = k * 2.0f * (rows + copies * sent), clocks = k * copies * rows * sent / 1024.0f;
             const float turns = fmaxf(1.0f, c.round * rounds + (1.0f - c.round) * wgs / compute_units());
-            const float busy = turns * (t.few ? bytes / c.few : fmaxf(bytes / (t.fi == 4 ? c.wide : c.pipe), clocks / c.clocks)), weights = 2.0f * total_n * K / c.weights;
+            const float sends = bytes / (t.few ? c.few : c.pipe), products = t.few ? 0.0f : clocks / c.clocks;
+            const float busy = turns * (earlier ? sends + products : fmaxf(sends, products)), weights = 2.0f * total_n * K / c.weights;
             float us = (t.few ? c.launch_few + c.sums * t.fi * t.tj * rounds : c.launch_pipe + (earlier && t_pad <= 128 ? 1.0f : 0.0f)) +
                        fmaxf(busy, weights) + (earlier ? 0.0f : 0.01f * fminf(busy, weights));
             if (splits > 1) us += 4.0f * counted * total_n * (splits / c.written + (splits - 1) / c.read);
