@@ -1721,11 +1721,10 @@ lpp_status launch_few_as(const pf::PipeJob& job, hipStream_t s) {
 // ids of the TinyLlama shape 1.69 -> 1.73 ms: the kernel has a loop for every number of requests, and starts with cold
 // instructions), so it has its own; exact mode, before and with it: TinyLlama 10 ids 1.16 -> 1.06 ms, 22 1.16 -> 1.10, 72
 // 1.50 -> 1.42; 1B 24 ids 0.92 -> 0.87; 8B 10 ids 4.18 -> 3.60, 40 4.67 -> 4.19.
-template <int kFi, int kTj, int kMode>
+template <int kFi, int kTj, int kMode, bool kLo>
 lpp_status launch_few(const pf::PipeJob& job, hipStream_t s) {
     const bool ragged = job.live <= 32 * kTj * job.token_tiles - 8;
-    if (job.xl != nullptr) return ragged ? launch_few_as<kFi, kTj, kMode, true, true>(job, s) : launch_few_as<kFi, kTj, kMode, true, false>(job, s);
-    return ragged ? launch_few_as<kFi, kTj, kMode, false, true>(job, s) : launch_few_as<kFi, kTj, kMode, false, false>(job, s);
+    return ragged ? launch_few_as<kFi, kTj, kMode, kLo, true>(job, s) : launch_few_as<kFi, kTj, kMode, kLo, false>(job, s);
 }
 
 // How a product is laid out on the device: what a workgroup's tile is and in how many ranges K is cut.
@@ -1787,12 +1786,16 @@ float planned_us(const Plan& p, int total_n, int K, int t_pad, bool lo, bool pai
     return c.launch + rounds * (1e-3f * c.column * K / p.splits + (pair ? c.pair_round : c.round)) + partials;
 }
 Plan plan_gemm(int total_n, int K, int t_pad, int live, int max_splits, bool lo, int row_step, bool pair) {
-    // (launch_plan has the kernels of this list)
+    // `exact`, `fast`: padded tokens up to which a mode may be given the tile.  At 32 to 304 compute units, n to 300000 and K to
+    // 32768 the model would give the exact mode no other; the fast mode's are those of the earlier fit.  launch_plan has the
+    // kernels of this list.
     static constexpr struct {
         bool few;
         int fi, tj;
-    } kTiles[] = {{true, 1, 1}, {true, 1, 2}, {true, 1, 3}, {true, 2, 1}, {true, 2, 2}, {true, 2, 3}, {true, 2, 4}, {true, 4, 1},
-                  {true, 4, 2}, {false, 2, 2}, {false, 4, 2}};
+        int exact, fast;
+    } kTiles[] = {{true, 1, 1, 256, 256}, {true, 1, 2, 0, 256}, {true, 1, 3, 128, 256}, {true, 2, 1, 256, 256},
+                  {true, 2, 2, 256, 256}, {true, 2, 3, 256, 256}, {true, 2, 4, 0, 256},   {true, 4, 1, 256, 0},
+                  {true, 4, 2, 256, 0},   {false, 2, 2, 256, 256}, {false, 4, 2, 256, 256}};
     Plan best = {false, 2, 2, 1};
     const bool wide_allowed = row_step % 256 == 0 && test_option(LPP_OPT_PREFILL_WIDE_TILES) != 0;
     if (t_pad > 256) {
@@ -1839,7 +1842,7 @@ Plan plan_gemm(int total_n, int K, int t_pad, int live, int max_splits, bool lo,
         const Plan p = {t.few, t.fi, t.tj, 1};
         const int rows = p.tile_rows(), tokens = p.tile_tokens(), token_tiles = p.token_tiles(t_pad, counted);
         if (row_step % rows != 0 || token_tiles * tokens > t_pad || (pair && t.fi == 1)) continue;
-        if (earlier && (counted % tokens != 0 || t.few && (lo ? t.tj == 4 || (t.fi == 1 && t.tj > 1) : t.fi == 4))) continue;
+        if (t_pad > (lo ? t.exact : t.fast) || (earlier && counted % tokens != 0)) continue;
         if (!t.few && t.fi == 4 && !wide_allowed) continue;
         const int sent = min(tokens, 32 * ((columns + token_tiles - 1) / token_tiles));
         for (int splits = 1; splits <= max_splits; splits *= 2) {
@@ -2018,22 +2021,18 @@ lpp_status launch_plan(const Plan& p, const pf::PipeJob& job_in, hipStream_t s) 
         if (p.fi == 4) return launch_pipe<4, 2, kMode>(job, s);
         return launch_pipe<2, 2, kMode>(job, s);
     }
-    switch (10 * p.fi + p.tj) {
-        case 21: return launch_few<2, 1, kMode>(job, s);
-        case 22: return launch_few<2, 2, kMode>(job, s);
-        case 23: return launch_few<2, 3, kMode>(job, s);
-        case 24: return launch_few<2, 4, kMode>(job, s);
-        case 41: return launch_few<4, 1, kMode>(job, s);
-        case 42: return launch_few<4, 2, kMode>(job, s);
-        default: break;
-    }
+    const bool lo = job.xl != nullptr;
+    const int tile = 10 * p.fi + p.tj;
+    if (lo && tile == 41) return launch_few<4, 1, kMode, true>(job, s);
+    if (lo && tile == 42) return launch_few<4, 2, kMode, true>(job, s);
+    if (!lo && tile == 24) return launch_few<2, 4, kMode, false>(job, s);
+    if (tile == 21) return lo ? launch_few<2, 1, kMode, true>(job, s) : launch_few<2, 1, kMode, false>(job, s);
+    if (tile == 22) return lo ? launch_few<2, 2, kMode, true>(job, s) : launch_few<2, 2, kMode, false>(job, s);
+    if (tile == 23) return lo ? launch_few<2, 3, kMode, true>(job, s) : launch_few<2, 3, kMode, false>(job, s);
     if constexpr (kMode != 2) {  // (a pair has as many rows of either matrix in a tile)
-        switch (10 * p.fi + p.tj) {
-            case 11: return launch_few<1, 1, kMode>(job, s);
-            case 12: return launch_few<1, 2, kMode>(job, s);
-            case 13: return launch_few<1, 3, kMode>(job, s);
-            default: break;
-        }
+        if (tile == 11) return lo ? launch_few<1, 1, kMode, true>(job, s) : launch_few<1, 1, kMode, false>(job, s);
+        if (!lo && tile == 12) return launch_few<1, 2, kMode, false>(job, s);
+        if (tile == 13) return lo ? launch_few<1, 3, kMode, true>(job, s) : launch_few<1, 3, kMode, false>(job, s);
     }
     return fail(LPP_ERR_STATE, "prefill GEMM: no kernel for a tile of %d x %d", p.tile_rows(), p.tile_tokens());
 }
@@ -2443,10 +2442,8 @@ char g_setup_message[kMaxDevices][256] = {};
 template <int kMode>
 lpp_status size_few_for() {
     LPP_TRY((size_few<1, 1, kMode, true>()));
-    LPP_TRY((size_few<1, 2, kMode, true>()));
     LPP_TRY((size_few<2, 1, kMode, true>()));
     LPP_TRY((size_few<2, 2, kMode, true>()));
-    LPP_TRY((size_few<2, 4, kMode, true>()));
     LPP_TRY((size_few<4, 1, kMode, true>()));
     return size_few<4, 2, kMode, true>();
 }
