@@ -758,17 +758,19 @@ __global__ __launch_bounds__(512) void k_gemm_pipe(PipeJob job) {
 //
 // Eight wavefronts, two to a SIMD, all of them multiply: each owns 128 features x 64 tokens.  The two of a SIMD take turns,
 // one barrier apart: while one multiplies a trip of 32 columns, the other reads its fragments of the trip from LDS and sends
-// for a later one, so the matrix cores are busy but for the barriers (4650 clocks for 4096 clocks of MFMAs) and a
-// wavefront that a request holds up holds nobody else.  A trip's rows are 64 bytes, their pieces in the order piece ^ ((r >> 2) & 3);
-// kStages trips are in LDS at once.
+// for a later one, so the matrix cores are busy but for the barriers (exact mode: 4650 clocks of the loop for 64 columns, 4096
+// of them MFMAs; 72 % of the whole launch's clocks at 2048 ids of the 1B shape) and a wavefront that a request holds up holds
+// nobody else.  A trip's rows are 64 bytes, their pieces in the order piece ^ ((r >> 2) & 3); kStages trips are in LDS at once.
+// (By the counters half of the reads' LDS cycles are bank conflicts in that order, where k_gemm_pipe's rows of 128 bytes have
+// next to none.  LDS is busy for 38 % of the launch, behind the matrix cores.)
 //
-// What bounds it is the device's power, not its clocks: the loop of the exact mode runs at 1.7 GHz, and what makes it
-// faster is less energy to a product.  That is why a block is as large as the registers allow (a third fewer bytes
-// from L2 and from LDS than 256 x 128), and why the products are v_mfma_f32_16x16x32_f16, head and remainder one after the
-// other into the same accumulator: of the same block, W1+W3 of 2048 ids of the 1B shape takes 233 us in products of 32 x 32 x 16,
-// 213 in 16 x 16 x 32, and 204 with the accumulator kept from head to remainder (266 in k_gemm_pipe's tiles of 256 x 128);
-// without the remainders 134, 126 (and 160).  Fed from registers alone, with neither requests nor reads, the same loop takes
-// 168 us.
+// What bounds it is the device's power, not its clocks: the exact mode's launches run at 1.7 to 1.9 GHz, and what makes them
+// faster is less energy to a product.  That is why a block is as large as the registers allow (from L2 a quarter fewer bytes to
+// a product than 256 x 128, without the remainders a third; from LDS as many), and why the products are
+// v_mfma_f32_16x16x32_f16, head and remainder one after the other into the same accumulator: of the same block, W1+W3 of 2048
+// ids of the 1B shape takes 233 us in products of 32 x 32 x 16, 213 in 16 x 16 x 32, and 204 with the accumulator kept from head
+// to remainder (266 in k_gemm_pipe's tiles of 256 x 128); without the remainders 134, 126 (and 160).  Fed from registers alone,
+// with neither requests nor reads, the same loop takes 168 us.
 constexpr int kBlock = 256;  // features and tokens of a block
 template <bool kLo>
 struct BlockShape {
@@ -1736,8 +1738,8 @@ struct Plan {
     int tile_rows() const { return (few ? 32 : 64) * fi; }
     int tile_tokens() const { return (few ? 32 : 64) * tj; }
     // Tiles of k_gemm_few that hold a token (150 ids, Wo in tiles of 64: three of four; 1B shape 1.466 -> 1.455 ms);
-    // k_gemm_pipe deals the tokens out (launch_pipe).  The plan itself goes by t_pad: by the tokens it would take Wo of 130 to
-    // 160 ids for k_gemm_pipe's tile of 96, 1.5 % faster there and 2.4 % slower at 192.
+    // k_gemm_pipe deals the tokens out (launch_pipe).  Beyond 128 tokens the plan itself goes by t_pad: by the tokens it would
+    // take Wo of 130 to 160 ids for k_gemm_pipe's tile of 96, 1.5 % faster there and 2.4 % slower at 192.
     int token_tiles(int t_pad, int live) const { return ((few ? live : t_pad) + tile_tokens() - 1) / tile_tokens(); }
 };
 
@@ -1753,16 +1755,17 @@ int padded_tokens(int n) {
 // device better.  A round costs a launch's share that does not depend on K, and K columns; a last round of a few workgroups
 // costs two thirds of a full one or more, and no launch less than one; partial products are written and read at 2.8 TB/s.
 // The constants are a fit to 4100 timed prefills (TinyLlama, 1B and 8B shapes, 300 to 2036 ids, both modes, each tile and cut
-// for each of the four products in turn): a prefill is within 1 % of what that product's fastest launch makes it, and faster
-// than by rules that cut K only while all ranges fit the device at once: exact mode, 8B shape 370 ids 11.9 -> 10.7 ms,
+// for each of the four products in turn; a column of 256 x 128, and that tile's last round in the fast mode, adjusted since to
+// its trips of 64 columns).  By the fit a prefill was within 1 % of what that product's fastest launch makes it, and it is
+// faster than by rules that cut K only while all ranges fit the device at once: exact mode, 8B shape 370 ids 11.9 -> 10.7 ms,
 // 600 18.6 -> 17.1, 750 20.4 -> 19.6; 1B 1140 5.21 -> 4.91; TinyLlama 1530 7.53 -> 7.17.
 // W1+W3, tiles against blocks: 1B shape 1024 ids 127 / 81 and 118 / 67 us, 1280 ids (a quarter of a second round) 163 / 108
 // and 187 / 113, 2048 ids 236 / 156 and 217 / 127; 8B 512 ids 224 / 152 and 196 / 122, 1024 ids 426 / 280 and 369 / 224.
 //
 // Up to 256 tokens the choice is made by what a launch of each would take.  A workgroup is paced by its bytes from L2 into
-// LDS, one of k_gemm_pipe, in the exact mode up to 128 tokens, by its MFMA clocks where they take longer; a
-// last round of workgroups that does not fill the device counts almost whole; k_gemm_few's sums meet in LDS, a tile of 32 x 32
-// at a time; every partial product of a cut K is written, in many short runs, and read once more.  No launch is faster than
+// LDS, one of k_gemm_pipe, in the exact mode up to 128 tokens, by its MFMA clocks where they take longer; a last round of
+// workgroups that does not fill the device counts almost whole; k_gemm_few's sums meet in LDS, a tile of 32 x 32 at a time;
+// every partial product of a cut K is written, in many short runs, and read once more.  No launch is faster than
 // its weights, and of two that are bound by them the one with less to do is taken.  The constants are a fit to 10000 timed
 // prefills (TinyLlama, 1B and 8B shapes, 10 to 256 ids, both modes, every tile of the list for each of the four products in
 // turn): up to 128 tokens a prefill is 0.3 % slower on average than with that product's fastest launch.  In the exact mode
