@@ -351,8 +351,9 @@ __global__ __launch_bounds__(256) void k_gemm(const half_t* __restrict__ w, cons
 // v_mfma_f32_16x16x32_f16, remainder right behind head in the same accumulator: 32 x 32 x 16 needs a lower clock for the same
 // work (the exact mode's W1+W3, 512 ids: 1B shape 69 -> 63 us, 8B 252 -> 224; of 2048 ids of the 1B shape 260 -> 236, W2 127 ->
 // 112; the fast mode, half of it data, 2 to 5 %).  A trip covers 64 columns, a whole cache line of every row: L2 gives a compute
-// unit 100 bytes a nanosecond in requests of whole lines and 70 in halves of lines.  The rows of the three operand
-// tiles lie one after the other in a stage of LDS, and a requesting wavefront fills 1 KiB of it
+// unit 100 bytes a nanosecond in requests of whole lines and 70 in halves of lines (256 workgroups of eight wavefronts that do
+// nothing but request rows 4 KiB apart from 256 KiB to 2 MiB; contiguous, 105 to 111).  The rows of the three operand tiles lie
+// one after the other in a stage of LDS, and a requesting wavefront fills 1 KiB of it
 // with one global_load_lds_dwordx4 (lane i -> 16 bytes at M0 + 16 i): no registers are staged
 // and nothing waits for the data but the s_waitcnt ahead of the trip that multiplies it.  As
 // many stages as 160 KiB hold, five at most.  Of 256 x 128 tiles in the exact mode a stage would be 64 KiB, two of them too few:
